@@ -188,6 +188,31 @@ hipError_t launch_gather_columns(const T *dense, T *out, const LevelPlan &plan, 
 template <typename T>
 hipError_t launch_scatter_columns(const T *grad, T *dense, const LevelPlan &plan, int64_t d, const int64_t *codes,
                                   int64_t rows, hipStream_t stream);
+// Long chains of chunk signatures (chain_kernels.hip).  `src`: [rows, n] dense-layout rows `src_stride` elements
+// apart.  left: products of the elements up to and including c (inclusive), or, at c >= 1, of those before c;
+// right (may be null): of those after c; both [rows, n, levels below depth].  total (may be null): product of all,
+// below the top level, into rows `total_stride` apart.  temp: one array like `left` (two with `right`, the second
+// temp_elems further on).
+template <typename T>
+hipError_t launch_chain(const T *src, int64_t src_stride, int64_t rows, int n, int64_t d, int depth, T *left,
+                        bool left_inclusive, T *right, T *total, int64_t total_stride, T *temp, int64_t temp_elems,
+                        hipStream_t stream);
+// Where the product of everything left of element c lies: row c * step + shift of the per_row rows of its path.
+// total: the last of these rows is the product of all, and launch_chain_top copies it below the top level too.
+template <typename T>
+struct ChainLeft {
+    const T *first;
+    int64_t per_row, step, shift;
+    bool total;
+};
+// top level of the product of all, from the elements and the left products
+template <typename T>
+hipError_t launch_chain_top(const T *elements, int64_t stride, const ChainLeft<T> &left, T *out, int64_t out_stride, int64_t rows,
+                            int n, int64_t d, int depth, hipStream_t stream);
+// whether these launches exist for a chain of n elements, and what they take (estimates, us)
+bool chain_possible(int64_t rows, int n, int64_t d, int depth);
+double chain_us(size_t elem, int64_t rows, int n, int64_t d, int depth, int directions);
+double chain_top_us(size_t elem, int64_t rows, int n, int64_t d, int depth);
 template <typename TI, typename T>
 hipError_t launch_increments_to_path(const TI *grad_inc, T *grad_path, int64_t B, int64_t L, int64_t d,
                                      hipStream_t stream);

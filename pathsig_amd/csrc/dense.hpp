@@ -13,6 +13,7 @@ struct DenseChoice {
                                 // signature, which the forward keeps or the backward computes again
     int variant;                // index into the table of compiled shapes
     int fwd_chunks;             // time chunks per (path, window) in the forward
+    bool chains;                // the products of the chunks may use the launches for long chains of them
     int bwd_chunks;             // ... and in the backward (at least 2 when embedding: no dense signature is saved)
     size_t dense_bytes;         // embed: bytes of one dense [rows, S] buffer
     size_t forward_workspace;   // bytes of scratch the forward needs (including the dense buffer)

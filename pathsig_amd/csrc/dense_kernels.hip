@@ -2207,10 +2207,10 @@ __global__ void __launch_bounds__((Geometry<D, N, P, sizeof(T), MAXW>::kBlock))
 // rows to fill the GPU with it; otherwise the longer prefix (more lanes per row, a few more chain FMAs per
 // lane) is taken.
 #define PSIG_VARIANTS(X) \
-    X(0, 4, 6, 3, 5, 4) X(1, 8, 4, 2, 3, 2) X(2, 6, 5, 3, 3, 3) X(3, 4, 4, 2, 3, 2) X(4, 3, 5, 3, 4, 3) \
+    X(0, 4, 6, 3, 5, 4) X(1, 8, 4, 2, 3, 2) X(2, 6, 5, 3, 4, 3) X(3, 4, 4, 2, 3, 2) X(4, 3, 5, 3, 4, 3) \
     X(5, 2, 8, 5, 7, 6) X(6, 8, 5, 3, 4, 3) X(7, 8, 4, 3, 3, 2) X(8, 3, 6, 3, 5, 4) X(9, 4, 5, 3, 4, 3) \
-    X(10, 5, 4, 2, 3, 2) X(11, 5, 5, 3, 4, 3) X(12, 5, 6, 4, 4, 4) X(13, 6, 4, 2, 3, 2) X(14, 7, 4, 2, 3, 2) \
-    X(15, 7, 5, 3, 3, 3) X(16, 2, 2, 1, 1, 1) X(17, 3, 2, 1, 1, 1) X(18, 4, 2, 1, 1, 1) X(19, 5, 2, 1, 1, 1) \
+    X(10, 5, 4, 2, 3, 2) X(11, 5, 5, 3, 4, 3) X(12, 5, 6, 4, 5, 4) X(13, 6, 4, 2, 3, 2) X(14, 7, 4, 2, 3, 2) \
+    X(15, 7, 5, 3, 4, 3) X(16, 2, 2, 1, 1, 1) X(17, 3, 2, 1, 1, 1) X(18, 4, 2, 1, 1, 1) X(19, 5, 2, 1, 1, 1) \
     X(20, 6, 2, 1, 1, 1) X(21, 7, 2, 1, 1, 1) X(22, 8, 2, 1, 1, 1) X(23, 2, 3, 2, 2, 1) X(24, 3, 3, 2, 2, 1) \
     X(25, 4, 3, 2, 2, 1) X(26, 5, 3, 2, 2, 1) X(27, 6, 3, 2, 2, 1) X(28, 7, 3, 2, 2, 1) X(29, 8, 3, 2, 2, 1) \
     X(30, 2, 4, 3, 3, 2) X(31, 3, 4, 3, 3, 2) X(32, 2, 5, 4, 4, 3) X(33, 2, 6, 4, 5, 4) X(34, 6, 6, 4, 4, 3) \
@@ -2222,7 +2222,7 @@ __global__ void __launch_bounds__((Geometry<D, N, P, sizeof(T), MAXW>::kBlock))
     X(55, 11, 4, 2, 3, 2) X(56, 12, 4, 2, 3, 2) X(57, 13, 4, 2, 3, 2) X(58, 14, 4, 2, 3, 2) \
     X(59, 15, 4, 2, 3, 2) X(60, 16, 4, 2, 3, 2) X(61, 9, 5, 3, 3, 3) X(62, 10, 5, 3, 3, 3) \
     X(63, 11, 5, 3, 3, 3) X(64, 12, 5, 3, 3, 3) X(65, 2, 7, 5, 6, 5) X(66, 3, 7, 4, 5, 4) \
-    X(67, 4, 7, 4, 5, 4) X(68, 3, 8, 5, 6, 5) X(69, 2, 9, 6, 8, 7) X(70, 2, 10, 6, 8, 7) \
+    X(67, 4, 7, 4, 6, 4) X(68, 3, 8, 5, 6, 5) X(69, 2, 9, 6, 8, 7) X(70, 2, 10, 6, 8, 7) \
     X(71, 17, 2, 1, 1, 1) X(72, 18, 2, 1, 1, 1) X(73, 19, 2, 1, 1, 1) X(74, 20, 2, 1, 1, 1) \
     X(75, 21, 2, 1, 1, 1) X(76, 22, 2, 1, 1, 1) X(77, 23, 2, 1, 1, 1) X(78, 24, 2, 1, 1, 1) \
     X(79, 25, 2, 1, 1, 1) X(80, 26, 2, 1, 1, 1) X(81, 27, 2, 1, 1, 1) X(82, 28, 2, 1, 1, 1) \
@@ -2291,6 +2291,7 @@ struct VariantInfo {
     int d, depth, block;  // block: threads of one unit
     int unit_blocks;      // blocks a unit is spread over (more than one: swept in one piece, dense only)
     int64_t sig_size, low_size;
+    int sub_size;         // values below the prefix of a lane
     bool bounds_ok;       // the sweeps can leave out top-level words by letter bounds
     bool chunks_ok[2];    // fp32, fp64: rows can be cut into time chunks
     bool fp64_fits;       // a lane's state fits the register file in fp64 too (else a later entry of the shape serves fp64)
@@ -2319,7 +2320,7 @@ template <int D, int N, int P, int PC, int PS>
 constexpr VariantInfo variant_info() {
     using G = Geometry<D, N, P>;
     using G64 = Geometry<D, N, P, 8>;
-    return VariantInfo{D, N, G::kUnitWaves * kWave, G::kUnitBlocks, G::kSigSize, G::kLowSize,
+    return VariantInfo{D, N, G::kUnitWaves * kWave, G::kUnitBlocks, G::kSigSize, G::kLowSize, G::kFwdSub,
                        LetterBounds<D, P>::kUsable && !G::kOnePiece && D <= 16,
                        {!G::kOnePiece && scan_fits<float, D, N, PS>(),
                         !G64::kOnePiece && scan_fits<double, D, N, PS>()},
@@ -2361,7 +2362,7 @@ constexpr bool shape_enabled(int, int) { return true; }
 template <int D, int N, int P, int PC, int PS>
 constexpr VariantInfo variant_info_if_enabled() {
     if constexpr (shape_enabled(D, N)) return variant_info<D, N, P, PC, PS>();
-    else return VariantInfo{-1, -1, 0, 0, 0, 0, false, {false, false}, false, false};
+    else return VariantInfo{-1, -1, 0, 0, 0, 0, 0, false, {false, false}, false, false};
 }
 
 #define PSIG_INFO(I, D, N, P, PC, PS) variant_info_if_enabled<D, N, P, PC, PS>(),
@@ -2387,30 +2388,57 @@ void profile_mark(bool begin, hipStream_t stream) {
 }
 
 // number of time chunks per row: enough waves to give every SIMD of the GPU about two (want_waves = 2048), but
-// chunks of at least 16 increments
-int pick_chunks(int64_t rows, int block, int64_t L, int64_t want_waves) {
+// chunks of at least 16 increments, and of at least 32 where there are more than 64 of them (`many`: their products
+// then take some five launches, chain_kernels.hip)
+constexpr int64_t kMostChunks = 1024;
+int pick_chunks(int64_t rows, int block, int64_t L, int64_t want_waves, bool many) {
     const int64_t waves_per_row = block / kWave;
     int64_t c = (want_waves + rows * waves_per_row - 1) / (rows * waves_per_row);
     const int64_t max_c = (L - 1) / 16;
     if (c > max_c) c = max_c;
-    if (c > 64) c = 64;
+    const int64_t most = many ? std::max<int64_t>(64, std::min<int64_t>(kMostChunks, (L - 1) / 32)) : 64;
+    if (c > most) c = most;
     if (c >= 4) c = (c + 3) / 4 * 4 <= max_c ? (c + 3) / 4 * 4 : c / 4 * 4;  // whole blocks of four chunks
     if (c < 1) c = 1;
     return (int)c;
 }
 
+// A path gradient is the difference of neighbouring increment sums, sqrt(L) times smaller than they are for a
+// Brownian path, so in fp32 whatever moves the boundaries of the chunks or the order of their products moves the
+// gradient by 1e-7 sqrt(L) of its norm: 1e-5 from some 10 000 increments on.  fp32 calls keep to 64 chunks and to
+// one product after the other beyond this length.
+constexpr int64_t kChainsUpToSteps = 4096;
+
 #endif
+
+// Estimates of the launches that multiply one chunk after the other.  A product of a scan over 64 chunks took 0.14 us
+// at depth 2, 0.35 at depth 3 and 4, 0.3 (rows of 100 bytes) to 0.85 (19 kB) at depth 5, 0.7 at depth 6; of a combine about as much when it stages
+// its rows in LDS, else what it takes to load a row at addresses of the lane's own ((6, 5) 2.1, (4, 6) in fp64 1.7,
+// (7, 5) in fp64 3.7 us).
+inline double scan_us(int n, int depth, double row_bytes) {
+    return 2.0 + (0.02 + 0.11 * depth + 1.5e-5 * row_bytes) * (n - 1);
+}
+template <typename T>
+double combine_us(int n, int depth, int64_t sig_size, bool staged) {
+    return staged ? scan_us(n, depth, 0) : 2.0 + (n - 1) * (0.8 + 0.02e-3 * (double)sig_size * sizeof(T));
+}
 
 template <typename T, int D, int N, int P, int GW>
 constexpr bool group_fits() {
     return Geometry<D, N, P, sizeof(T)>::kBlock * GW <= 1024 && forward_lds_bytes<D, N, P, GW, T>() <= 64 * 1024;
 }
 
-// Prefix products edgeA and suffix products edgeZ of the chunk signatures below the top level (dense_scan_kernel).
-template <typename T, int D, int N, int PS>
-hipError_t launch_scan(const T *chunk_low, T *edgeA, T *edgeZ, int64_t rows, int chunks, hipStream_t stream) {
-    using GC = Geometry<D, N, PS>;
 
+// Prefix products edgeA and (unless null) suffix products edgeZ of the chunk signatures below the top level (dense_scan_kernel).
+// chains: long chains of chunks may take the launches of chain_kernels.hip, with `temp` for their scratch.
+template <typename T, int D, int N, int PS>
+hipError_t launch_scan(const T *chunk_low, T *edgeA, T *edgeZ, int64_t rows, int chunks, T *temp, bool chains,
+                       hipStream_t stream) {
+    using GC = Geometry<D, N, PS>;
+    // (whether or not the second direction is asked for: a forward returns the same bits with and without it)
+    if (chains && chain_us(sizeof(T), rows, chunks, D, N, 2) < scan_us(chunks, N, GC::kLowSize * sizeof(T)))
+        return launch_chain<T>(chunk_low, GC::kLowSize, rows, chunks, D, N, edgeA, true, edgeZ, (T *)nullptr, 0, temp,
+                               rows * chunks * GC::kLowSize, stream);
     // all chunk rows of a row go to LDS at once when they fit (a little under the 160 KB of a CU)
     const size_t resident_bytes = (size_t)chunks * GC::kLowSize * sizeof(T);
     const size_t fixed_bytes = 2 * GC::kLowSize * sizeof(T) + 1024;
@@ -2420,10 +2448,10 @@ hipError_t launch_scan(const T *chunk_low, T *edgeA, T *edgeZ, int64_t rows, int
             hipError_t e = allow_dynamic_lds<dense_scan_kernel<T, D, N, PS, true>>(resident_bytes);
             if (e != hipSuccess) return e;
         }
-        hipLaunchKernelGGL(kernel, dim3((unsigned)rows, 2), dim3(GC::kBlock + kCopyThreads), resident_bytes, stream,
+        hipLaunchKernelGGL(kernel, dim3((unsigned)rows, edgeZ ? 2 : 1), dim3(GC::kBlock + kCopyThreads), resident_bytes, stream,
                            chunk_low, edgeA, edgeZ, chunks, (T *)nullptr, (int64_t)0);
     } else {
-        hipLaunchKernelGGL((dense_scan_kernel<T, D, N, PS, false>), dim3((unsigned)rows, 2),
+        hipLaunchKernelGGL((dense_scan_kernel<T, D, N, PS, false>), dim3((unsigned)rows, edgeZ ? 2 : 1),
                            dim3(GC::kBlock + kCopyThreads), 0, stream, chunk_low, edgeA, edgeZ, chunks, (T *)nullptr,
                            (int64_t)0);
     }
@@ -2435,7 +2463,7 @@ hipError_t launch_scan(const T *chunk_low, T *edgeA, T *edgeZ, int64_t rows, int
 // pad256 bytes after the start of the first.
 template <typename T, int D, int N, int P, int PC, int PS>
 hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks, const int *bounds, T *keep,
-                       void *workspace, hipStream_t stream, bool grouped) {
+                       void *workspace, hipStream_t stream, bool grouped, bool chains) {
     using G = Geometry<D, N, P, sizeof(T)>;
     using GC = Geometry<D, N, PC>;
     constexpr bool kStaged = 2 * GC::kSigSize * sizeof(T) <= 48 * 1024;
@@ -2461,25 +2489,51 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
     // a row that fits one block goes straight to the output, without the combine launch
     T *chunk_sig = (T *)workspace;
     // the chunks' own signatures below the top level, from which the products for the backward are made
-    T *chunk_low = keep ? (T *)((unsigned char *)workspace + pad256((size_t)rows * chunks * G::kSigSize * sizeof(T)))
-                        : (T *)nullptr;
+    T *const low_space = (T *)((unsigned char *)workspace + pad256((size_t)rows * chunks * G::kSigSize * sizeof(T)));
+    T *chunk_low = keep ? low_space : (T *)nullptr;
+    // scratch of a long chain of products (present when chain_possible says so for the chunks)
+    const int64_t low_elems = rows * chunks * G::kLowSize;
+    T *const chain_temp = (T *)((unsigned char *)low_space + pad256((size_t)low_elems * sizeof(T)));
+    const int gw = bounds ? 1
+                   : (group_fits<T, D, N, P, 4>() && chunks % 4 == 0) ? 4
+                   : (group_fits<T, D, N, P, 2>() && chunks % 2 == 0) ? 2 : 1;
+    bool top_sums = false;  // see below
+    if constexpr (scan_fits<T, D, N, PS>()) {
+        const double left_us =
+            std::min(scan_us(chunks, N, G::kLowSize * sizeof(T)), chain_us(sizeof(T), rows, chunks, D, N, 2));
+        top_sums = chains && chunks > gw && chain_top_us(sizeof(T), rows, chunks / gw, D, N) + 0.25 * left_us <
+                                                combine_us<T>(chunks / gw, N, G::kSigSize, kStaged);
+    }
     if constexpr (sizeof(T) == 4 && grouped_handover_ok<D, N, P, PC, PS>()) {
-        if (keep && grouped && !bounds && chunks % 4 == 0 && chunks >= 8) {
+        const int groups4 = chunks / 4;
+        const bool in_groups = grouped && !bounds && chunks % 4 == 0 && chunks >= 8;
+        const bool in_chain = in_groups && chains &&
+                              chain_us(sizeof(T), rows, groups4, D, N, 2) + chain_top_us(sizeof(T), rows, groups4, D, N) <
+                                  scan_us(groups4, N, 0);
+        if (in_groups) top_sums = false;
+        if (in_groups && (keep || in_chain)) {
             // grouped hand-over: keep = [in-group prefix products][in-group suffix products], both
             // [rows, chunks, low], then [products of the groups to the left][.. to the right], both
             // [rows, chunks / 4, low]
             using ES = EdgesShape<T, D, N, PS, PC>;
-            const int groups4 = chunks / 4;
             const size_t unit_bytes = pad256((size_t)rows * chunks * G::kLowSize * sizeof(T));
             const size_t group_bytes = pad256((size_t)rows * groups4 * G::kLowSize * sizeof(T));
-            T *in_suffix = (T *)((unsigned char *)keep + unit_bytes);
-            T *edgeL = (T *)((unsigned char *)keep + 2 * unit_bytes);
-            T *edgeR = (T *)((unsigned char *)keep + 2 * unit_bytes + group_bytes);
+            // (a forward that keeps nothing makes the products of the groups to the left alone)
+            T *in_suffix = keep ? (T *)((unsigned char *)keep + unit_bytes) : (T *)nullptr;
+            T *edgeL = keep ? (T *)((unsigned char *)keep + 2 * unit_bytes) : chain_temp;
+            T *edgeR = keep ? (T *)((unsigned char *)keep + 2 * unit_bytes + group_bytes) : (T *)nullptr;
             hipLaunchKernelGGL((dense_forward_kernel<T, D, N, P, 4>), dim3((unsigned)(rows * groups4)),
                                dim3(G::kBlock * 4), 0, stream, path, chunk_sig, shape, chunks, (T *)nullptr,
                                (const int *)nullptr, keep, in_suffix);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
+            if (in_chain) {
+                e = launch_chain<T>((const T *)chunk_sig, G::kSigSize, rows, groups4, D, N, edgeL, false, edgeR, sig,
+                                    G::kSigSize, low_space, rows * groups4 * G::kLowSize, stream);
+                if (e != hipSuccess) return e;
+                return launch_chain_top<T>((const T *)chunk_sig, G::kSigSize, ChainLeft<T>{edgeL, groups4, 1, 0, false}, sig,
+                                           G::kSigSize, rows, groups4, D, N, stream);
+            }
             auto kernel = dense_group_edges_kernel<T, D, N, PS, PC>;
             if (ES::kCombineBytes > 48 * 1024) {
                 e = allow_dynamic_lds<dense_group_edges_kernel<T, D, N, PS, PC>>(ES::kCombineBytes);
@@ -2490,6 +2544,7 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
             return hipGetLastError();
         }
     }
+    if (top_sums) chunk_low = low_space;
     int groups = chunks;
     if constexpr (kBoundsOk) {
         if (bounds) {
@@ -2530,6 +2585,19 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (groups < 0) groups = chunks;
+    if (top_sums) {
+        // The products left of every chunk give the top level as a sum over the partial signatures; they are made for a
+        // backward anyway.
+        if constexpr (scan_fits<T, D, N, PS>()) {
+            T *edgeA = keep ? keep : chain_temp + low_elems;
+            T *edgeZ = keep ? (T *)((unsigned char *)keep + pad256((size_t)low_elems * sizeof(T))) : (T *)nullptr;
+            e = launch_scan<T, D, N, PS>((const T *)chunk_low, edgeA, edgeZ, rows, chunks, chain_temp, true, stream);
+            if (e != hipSuccess) return e;
+            return launch_chain_top<T>((const T *)chunk_sig, G::kSigSize,
+                                       ChainLeft<T>{edgeA, chunks, chunks / groups, -1, true}, sig, G::kSigSize, rows,
+                                       groups, D, N, stream);
+        }
+    }
     if (keep) {
         if constexpr (scan_fits<T, D, N, PS>()) {
             T *edgeZ = (T *)((unsigned char *)keep + pad256((size_t)rows * chunks * G::kLowSize * sizeof(T)));
@@ -2553,7 +2621,8 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
                     return hipGetLastError();
                 }
             }
-            e = launch_scan<T, D, N, PS>((const T *)chunk_low, keep, edgeZ, rows, chunks, stream);
+            e = launch_scan<T, D, N, PS>((const T *)chunk_low, keep, edgeZ, rows, chunks, chain_temp, chains,
+                                         stream);
             if (e != hipSuccess) return e;
         } else {
             return hipErrorNotSupported;  // such shapes are never cut into time chunks (dense_choice)
@@ -2573,7 +2642,7 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
 template <typename T, int D, int N, int P, int PC, int PS>
 hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_inc, T *grad_path, bool *wrote_path,
                         const SigShape &shape, int chunks, const int *bounds, const T *kept, void *workspace,
-                        hipStream_t stream, bool grouped, bool inc_cleared) {
+                        hipStream_t stream, bool grouped, bool chains, bool inc_cleared) {
     using G = Geometry<D, N, P, sizeof(T)>;
     using GC = Geometry<D, N, PS>;
     constexpr bool kBoundsOk = LetterBounds<D, P>::kUsable && !G::kOnePiece;
@@ -2643,7 +2712,8 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
             }
             e = hipGetLastError();
             if (e != hipSuccess) return e;
-            e = launch_scan<T, D, N, PS>((const T *)chunk_low, edgeA, edgeZ, rows, chunks, stream);
+            e = launch_scan<T, D, N, PS>((const T *)chunk_low, edgeA, edgeZ, rows, chunks, (T *)(ws + 3 * edge_bytes),
+                                         chains, stream);
             if (e != hipSuccess) return e;
             dumpA = edgeA;
             dumpH = edgeZ;
@@ -2762,8 +2832,22 @@ DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, cons
             dc.bounded = chunks_ok && v.bounds_ok && level_sizes[depth] > 0 && level_sizes[depth] < top_dense &&
                          options().letter_bounds != 0;
         }
+        // an increment takes some 0.2 us of both sweeps and 0.013 us for every value below a lane's prefix, twice that
+        // in fp64
+        const double step_us = (0.2 + 0.013 * v.sub_size) * (elem == 8 ? 2.0 : 1.0);
+        const double low_bytes = (double)v.low_size * elem;
+        const bool may_chain = elem == 8 || L - 1 <= kChainsUpToSteps;
+        bool many = false;  // more than 64 chunks
+        if (chunks_ok && L - 1 > 2048) {
+            // what the shorter sweeps save against what the longer chains of products cost
+            const int most = pick_chunks(rows, v.block, L, 2048, true);
+            many = most > 64 && (double)(L - 1) * (1.0 / 64 - 1.0 / most) * step_us >
+                                    5.0 + chain_us(elem, rows, most, d, depth, 2) -
+                                        std::min(scan_us(64, depth, low_bytes), chain_us(elem, rows, 64, d, depth, 2));
+        }
         // (letter blocks: twice the waves that fit the GPU at once, so that the short ones fill in behind the long)
-        int chunks = pick_chunks(rows, v.block, L, dc.bounded && elem == 4 ? 4096 : 2048);
+        const int64_t want_waves = dc.bounded && elem == 4 ? 4096 : 2048;
+        int chunks = pick_chunks(rows, v.block, L, want_waves, many && may_chain);
         // deep fp32 shapes: the reverse sweep rebuilds A_t = A_{t+1} (x) exp(-dx_t) step by step, and over a span of
         // large increments that roll-back loses digits at depth 9 and more (d = 2, depth 12, five increments of
         // size 0.8: gradient off by 1.5e-5 in one piece, 1e-6 in two or more); four chunks at least
@@ -2772,6 +2856,10 @@ DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, cons
         // not chunked: units of several blocks (a row is dozens of waves already), rows too long for the scan
         // kernel's LDS
         if (!chunks_ok) chunks = 1;
+        // A step of training whose launches take less than the 60 us that autograd takes to get through its own
+        // forward and backward gains nothing from shorter ones, and the chains are three to five launches more.
+        // (The values a call returns do not depend on whether it keeps anything for a backward, so neither may this.)
+        dc.chains = may_chain && (double)(L - 1) / chunks * step_us + 8.0 + 1.3 * scan_us(chunks, depth, low_bytes) > 55.0;
         if (rows * (chunks + 1) >= (int64_t(1) << 31)) return dc;
         dc.usable = true;
         dc.variant = i;
@@ -2781,10 +2869,14 @@ DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, cons
         dc.backward_workspace = (dc.resweep ? 2 : 1) * dc.dense_bytes + (dc.bounded ? kBoundsBytes : 0);
         // forward: the chunk signatures, and those below the top level from which a keeping forward makes the
         // products its backward starts from; backward: the latter and the two arrays of products
+        // (long chains of products take two more such arrays)
         if (dc.fwd_chunks > 1)
             dc.forward_workspace += pad256((size_t)rows * dc.fwd_chunks * v.sig_size * elem) +
-                                    pad256((size_t)rows * dc.fwd_chunks * v.low_size * elem);
-        if (dc.bwd_chunks > 1) dc.backward_workspace += 3 * pad256((size_t)rows * dc.bwd_chunks * v.low_size * elem);
+                                    (chain_possible(rows, dc.fwd_chunks, d, depth) ? 3 : 1) *
+                                        pad256((size_t)rows * dc.fwd_chunks * v.low_size * elem);
+        if (dc.bwd_chunks > 1)
+            dc.backward_workspace += (chain_possible(rows, dc.bwd_chunks, d, depth) ? 5 : 3) *
+                                     pad256((size_t)rows * dc.bwd_chunks * v.low_size * elem);
         // the forward can hand those products to the backward when both cut the rows the same way
         if (dc.bwd_chunks > 1 && dc.fwd_chunks == dc.bwd_chunks) {
             dc.keep_bytes = 2 * pad256((size_t)rows * dc.bwd_chunks * v.low_size * elem);
@@ -2880,15 +2972,16 @@ static_assert(PSIG_GROUP < kDenseGroups, "group index out of range");
 #define PSIG_CASE_FWD(I, D, N, P, PC, PS)                                                                         \
     case I:                                                                                                       \
         if constexpr (I % kDenseGroups == PSIG_GROUP && shape_enabled(D, N))                                      \
-            return run_forward<T, D, N, P, PC, PS>(path, sig, shape, dc.fwd_chunks, bounds, keep, workspace,    \
-                                                   stream, dc.grouped);                                           \
+            return run_forward<T, D, N, P, PC, PS>(path, sig, shape, dc.fwd_chunks,                               \
+                                                   bounds, keep, workspace, stream, dc.grouped,                   \
+                                                   dc.chains);                                                    \
         break;
 #define PSIG_CASE_BWD(I, D, N, P, PC, PS)                                                                          \
     case I:                                                                                                        \
         if constexpr (I % kDenseGroups == PSIG_GROUP && shape_enabled(D, N))                                       \
             return run_backward<T, D, N, P, PC, PS>(path, sig, grad_sig, grad_inc, grad_path, wrote_path, shape,   \
                                                     dc.bwd_chunks, bounds, kept, workspace, stream, dc.grouped,    \
-                                                    inc_cleared);                                                  \
+                                                    dc.chains, inc_cleared);                                                  \
         break;
 
 template <int GROUP, typename T>
