@@ -165,6 +165,33 @@ int pathsig_logsig_backward_kept(const void *logsig, const void *cache, const vo
                                  const int64_t *top_words, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
+ * The log-signature in one call (no counterpart in the reference, whose module calls the two operators and selects
+ * columns): path -> the wanted columns of the log-signature, and their gradients -> path gradient.  The signature
+ * stays in dense rows in between; nothing of the hybrid layout is written.  level_sizes, W, windows: as for the
+ * signature (levels below depth dense, NULL: all); top_words: codes of the top level where it is listed; picked
+ * [n_out]: hybrid column of every output, NULL with a dense layout (then n_out = all columns).
+ *   pathsig_logsignature_sizes   bytes of `saved` and of the two workspaces; PATHSIG_ERR_UNSUPPORTED for calls that
+ *                                are not available in this form (compiled shapes of depth 2 to 8 are).  A forward
+ *                                with saved == NULL takes forward_workspace + saved bytes of workspace.
+ *   pathsig_logsignature_lists   what a caller keeps with a list of wanted columns (device memory, a few ints per
+ *                                column): made once for (top_words, picked), read by every call with them
+ */
+int pathsig_logsignature_sizes(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
+                               int64_t W, size_t *saved, size_t *forward_workspace, size_t *backward_workspace);
+size_t pathsig_logsignature_lists_bytes(int64_t d, int depth, int64_t n_out);
+int pathsig_logsignature_lists(const int64_t *top_words, int64_t top_size, const int64_t *picked, int64_t n_out,
+                               int64_t d, int depth, void *lists, void *stream);
+int pathsig_logsignature_forward(const void *path, void *out, int dtype, int64_t B, int64_t L, int64_t d, int depth,
+                                 const int64_t *level_sizes, const int64_t *top_words, const int64_t *picked,
+                                 int64_t n_out, const void *lists, const int32_t *windows, int64_t W, void *saved,
+                                 void *workspace, size_t workspace_bytes, void *stream);
+int pathsig_logsignature_backward(const void *path, const void *saved, size_t saved_bytes, const void *grad_out,
+                                  void *grad_path, int dtype, int64_t B, int64_t L, int64_t d, int depth,
+                                  const int64_t *level_sizes, const int64_t *top_words, const int64_t *picked,
+                                  int64_t n_out, const void *lists, const int32_t *windows, int64_t W, void *workspace,
+                                  size_t workspace_bytes, void *stream);
+
+/*
  * Tuning switches (no counterpart in the reference, whose two heuristics are hard-coded:
  * src/pathsig/forward/sig_launch.cu:23-27, src/pathsig/backward/sig_backward_launch.cu:171).  They are process
  * wide and meant for tests and measurements; the defaults need no call.  Initial values come from the environment

@@ -8,6 +8,7 @@ There is no fallback: if the library is missing, importing the package fails.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import pathlib
 import threading
 
@@ -107,6 +108,7 @@ def lib() -> ctypes.CDLL:
 
 _TORCH_LIB_NAME = "libpathsig_torch.so"
 _torch_ops_loaded = False
+direct = None  # the extension module of that library: calls without the boxing of an operator (csrc/torch_ops.cpp)
 
 
 def load_torch_ops() -> None:
@@ -122,9 +124,13 @@ def load_torch_ops() -> None:
         raise RuntimeError(
             f"Could not find the operator library {path}. Build it with `python pathsig_amd/build_ext.py` "
             "(needs g++ and the torch headers).")
+    global direct
     try:
         torch.ops.load_library(str(path))
-    except OSError as exc:  # built against another torch or an older libpathsig_hip.so
+        spec = importlib.util.spec_from_file_location("libpathsig_torch", path)
+        direct = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(direct)
+    except (OSError, ImportError) as exc:  # built against another torch or an older libpathsig_hip.so
         raise RuntimeError(f"{path} could not be loaded ({exc}); rebuild it with "
                            "`python pathsig_amd/build_ext.py`.") from exc
     _torch_ops_loaded = True

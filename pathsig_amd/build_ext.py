@@ -11,6 +11,7 @@ import concurrent.futures
 import pathlib
 import subprocess
 import sys
+import sysconfig
 
 PKG = pathlib.Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
@@ -83,14 +84,15 @@ def build_torch_ops(verbose: bool = False, out_dir: pathlib.Path | None = None) 
 
     if torch.version.hip is None:
         raise RuntimeError("the operator library needs a ROCm build of PyTorch")
-    includes = [f"-I{p}" for p in cpp_extension.include_paths()] + ["-I/opt/rocm/include", f"-I{INCLUDE}"]
+    includes = ([f"-I{p}" for p in cpp_extension.include_paths()]
+                + [f"-I{sysconfig.get_paths()['include']}", "-I/opt/rocm/include", f"-I{INCLUDE}"])
     lib_dirs = cpp_extension.library_paths()
     pkg = PKG if out_dir is None else pathlib.Path(out_dir)
     torch_lib = pkg / TORCH_LIB.name
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes,
            str(CSRC / "torch_ops.cpp"), "-o", str(torch_lib),
-           *[f"-L{d}" for d in lib_dirs], "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch",
+           *[f"-L{d}" for d in lib_dirs], "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python",
            f"-L{pkg}", "-lpathsig_hip", "-Wl,-rpath,$ORIGIN", *[f"-Wl,-rpath,{d}" for d in lib_dirs]]
     if verbose:
         print(" ".join(cmd), flush=True)

@@ -48,11 +48,14 @@ struct OptionCells {
           deep_fp64(getenv("PATHSIG_NO_DEEP_FP64") ? 0 : 1),
           grouped(getenv("PATHSIG_NO_GROUPED") ? 0 : 1) {}
 };
+std::atomic<int64_t> g_options_epoch{0};
 OptionCells &option_cells() {
     static OptionCells cells;  // the environment is read here, once
     return cells;
 }
 }  // namespace
+
+int64_t options_epoch() { return g_options_epoch.load(std::memory_order_relaxed); }
 
 const Options &options() {
     thread_local Options snapshot;
@@ -533,6 +536,116 @@ int check_logsig(int dtype, int64_t rows, int64_t d, int depth, int64_t top_size
     return PATHSIG_OK;
 }
 
+// Signature and log-signature in one call: the signature is swept into dense rows, the logarithm reads them there and
+// computes the wanted columns; the backward expands the gradients of these columns into dense rows, on which the
+// adjoint of the logarithm and that of the signature work in place.  Nothing is gathered, scattered or cleared in
+// between, and no row of the hybrid layout is ever written.
+struct LogPlan {
+    bool usable;
+    DenseChoice dc;      // with the number of backward chunks of this call
+    int64_t rows, columns, lower, top;
+    bool keep_products;  // the forward hands the products of its chunks to the backward ..
+    bool keep_rows;      // .. or the dense signature rows (swept in one piece)
+    // byte offsets into `saved`: [products of the chunks, or the dense rows][log-signature][its cache]
+    size_t lg_at, cache_at, saved_bytes;
+    size_t rows_bytes;   // of one dense buffer
+    size_t forward_bytes;          // scratch of a forward that saves (one that does not adds saved_bytes)
+    size_t inc_bytes, adjoint_bytes, backward_bytes;
+};
+
+LogPlan log_plan(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes, int64_t W) {
+    LogPlan lp{};
+    if (check_common(dtype, B, L, d, depth) != PATHSIG_OK || d < 2 || d > 64) return lp;
+    const size_t elem = elem_size(dtype);
+    LevelPlan plan;
+    bool all_dense;
+    if (build_plan(d, depth, level_sizes, INT64_MAX, true, &plan, &all_dense) != PATHSIG_OK) return lp;
+    const int64_t windows = W > 0 ? W : 1;
+    lp.rows = B * windows;
+    if (lp.rows <= 0 || !picked_logsig_possible(elem, lp.rows, d, depth) || check_grid(plan, lp.rows) != PATHSIG_OK)
+        return lp;
+    // (levels below the top are dense in the hybrid layout)
+    for (int k = 1; k < depth; ++k)
+        if (plan.code_off[k] >= 0) return lp;
+    lp.dc = dense_choice(elem, d, depth, all_dense, level_sizes, B, L, windows, W > 0);
+    if (!lp.dc.usable) return lp;
+    lp.lower = plan.out_off[depth];
+    lp.top = checked_pow(d, depth);
+    lp.columns = lp.lower + lp.top;
+    lp.rows_bytes = align_up((size_t)lp.rows * lp.columns * elem);
+    // rows enough to fill the device are swept in one piece, from the dense rows that the logarithm reads too
+    if (lp.dc.fwd_chunks == 1 && !lp.dc.bounded) lp.dc.bwd_chunks = 1;
+    lp.keep_rows = lp.dc.bwd_chunks == 1;
+    lp.keep_products = !lp.keep_rows && lp.dc.keep_bytes > 0;
+    const size_t kept = align_up(lp.keep_rows ? lp.rows_bytes : lp.keep_products ? lp.dc.keep_bytes : 0);
+    const size_t lg = align_up((size_t)lp.rows * lp.lower * elem);
+    lp.lg_at = kept;
+    lp.cache_at = kept + lg;
+    lp.saved_bytes = lp.cache_at + align_up((size_t)lp.rows * lp.lower * depth * elem);
+    // (the dense rows of the forward are saved or scratch; what dense_choice asks for a dense buffer is not needed)
+    lp.forward_bytes = (lp.keep_rows ? 0 : lp.rows_bytes) + align_up(lp.dc.forward_workspace - lp.dc.dense_bytes);
+    lp.inc_bytes = inc_buffer_bytes(elem, B, L, d, false);
+    const LogsigBackwardPlan ap = logsig_backward_plan(elem, lp.rows, d, depth, lp.top);
+    lp.adjoint_bytes = align_up((size_t)(ap.a_elems + ap.q_elems) * elem);
+    lp.backward_bytes = lp.inc_bytes + lp.rows_bytes + lp.adjoint_bytes +
+                        align_up(lp.dc.backward_workspace - (lp.dc.resweep ? 2 : 1) * lp.dc.dense_bytes);
+    lp.usable = true;
+    return lp;
+}
+
+// what a module keeps: the letter bounds of the word list (16 ints) and the lists of outputs per dense column
+const int *bounds_of(const void *lists) { return (const int *)lists; }
+const int *heads_of(const void *lists) { return (const int *)lists + 16; }
+
+template <typename T>
+int log_forward_t(const LogPlan &lp, const void *path, void *out, int64_t n_out, int64_t B, int64_t L, int64_t d, int depth,
+                  const int64_t *top_words, int64_t top_size, const int64_t *picked, const void *lists,
+                  const int32_t *windows, int64_t W, void *saved, void *workspace, hipStream_t stream) {
+    const SigShape shape{B, L, d, windows ? W : 1, windows};
+    unsigned char *ws = (unsigned char *)workspace;
+    const bool save = saved != nullptr;
+    unsigned char *keep = save ? (unsigned char *)saved : ws + lp.forward_bytes;
+    T *rows = (T *)(lp.keep_rows ? keep : ws);
+    void *rest = ws + (lp.keep_rows ? 0 : lp.rows_bytes);
+    DenseChoice dc = lp.dc;
+    hipError_t e = launch_dense_forward<T>((const T *)path, rows, shape, dc, top_words, top_size,
+                                           save && lp.keep_products ? (T *)keep : (T *)nullptr, rest, stream,
+                                           lists ? bounds_of(lists) : nullptr);
+    if (e != hipSuccess) return launch_failed(e, "dense forward launch");
+    e = launch_picked_logsig<T>(rows, lp.columns, (T *)(keep + lp.lg_at), (T *)(keep + lp.cache_at), (T *)out, n_out,
+                                lp.rows, d, depth, top_size, top_words, picked, stream);
+    if (e != hipSuccess) return launch_failed(e, "logsig forward launch");
+    return PATHSIG_OK;
+}
+
+template <typename T>
+int log_backward_t(const LogPlan &lp, const void *path, const void *saved, const void *grad_out, int64_t n_out,
+                   void *grad_path, int64_t B, int64_t L, int64_t d, int depth, const int64_t *top_words, int64_t top_size,
+                   const void *lists, const int32_t *windows, int64_t W, void *workspace, hipStream_t stream) {
+    const SigShape shape{B, L, d, windows ? W : 1, windows};
+    unsigned char *ws = (unsigned char *)workspace;
+    const unsigned char *keep = (const unsigned char *)saved;
+    T *ginc = (T *)ws;
+    T *dense = (T *)(ws + lp.inc_bytes);
+    T *adjoint_ws = (T *)(ws + lp.inc_bytes + lp.rows_bytes);
+    void *rest = ws + lp.inc_bytes + lp.rows_bytes + lp.adjoint_bytes;
+    const int *head = lists ? heads_of(lists) : nullptr;
+    hipError_t e = launch_picked_adjoint<T>((const T *)(keep + lp.lg_at), (const T *)(keep + lp.cache_at),
+                                            (const T *)grad_out, n_out, dense, adjoint_ws, lp.rows, d, depth, head,
+                                            head ? head + lp.columns : nullptr, stream);
+    if (e != hipSuccess) return launch_failed(e, "logsig backward launch");
+    bool wrote_path = false;
+    e = launch_dense_backward<T>((const T *)path, lp.keep_rows ? (const T *)keep : (const T *)nullptr, dense, ginc,
+                                 (T *)grad_path, &wrote_path, shape, lp.dc, top_words, top_size,
+                                 lp.keep_products ? (const T *)keep : (const T *)nullptr, rest, false, stream,
+                                 lists ? bounds_of(lists) : nullptr);
+    if (e != hipSuccess) return launch_failed(e, "dense backward launch");
+    if (wrote_path) return PATHSIG_OK;
+    e = launch_increments_to_path<T, T>(ginc, (T *)grad_path, B, L, d, stream);
+    if (e != hipSuccess) return launch_failed(e, "path-gradient launch");
+    return PATHSIG_OK;
+}
+
 size_t logsig_backward_bytes(int dtype, int64_t rows, int64_t d, int depth, int64_t top_size) {
     const LogsigBackwardPlan lp = logsig_backward_plan(elem_size(dtype), rows, d, depth, top_size);
     return (size_t)(lp.a_elems + lp.q_elems + lp.top_elems) * elem_size(dtype);
@@ -581,6 +694,7 @@ int pathsig_set_option(const char *name, int64_t value) {
         set_error("unknown option or value out of range: %s = %lld", name, (long long)value);
         return PATHSIG_ERR_ARGUMENT;
     }
+    g_options_epoch.fetch_add(1, std::memory_order_relaxed);
     return PATHSIG_OK;
 }
 
@@ -906,6 +1020,115 @@ int pathsig_logsig_forward_keep(const void *sig, void *logsig, void *cache, int 
     }
     return logsig_forward_any(sig, logsig, cache, nullptr, dtype, rows, d, depth, top_size, top_words,
                               (hipStream_t)stream);
+}
+
+int pathsig_logsignature_sizes(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes, int64_t W,
+                               size_t *saved, size_t *forward_workspace, size_t *backward_workspace) {
+    const LogPlan lp = log_plan(dtype, B, L, d, depth, level_sizes, W);
+    if (saved) *saved = lp.usable ? lp.saved_bytes : 0;
+    if (forward_workspace) *forward_workspace = lp.usable ? lp.forward_bytes : 0;
+    if (backward_workspace) *backward_workspace = lp.usable ? lp.backward_bytes : 0;
+    if (!lp.usable) set_error("log-signature in one call: not available for this shape");
+    return lp.usable ? PATHSIG_OK : PATHSIG_ERR_UNSUPPORTED;
+}
+
+size_t pathsig_logsignature_lists_bytes(int64_t d, int depth, int64_t n_out) {
+    if (d < 2 || depth < 1 || depth > kMaxDepth || n_out < 0) return 0;
+    const int64_t top = checked_pow(d, depth);
+    if (top < 0 || top > (int64_t(1) << 31)) return 0;
+    return (size_t)(16 + hybrid_size(d, depth, top) + n_out) * sizeof(int);
+}
+
+int pathsig_logsignature_lists(const int64_t *top_words, int64_t top_size, const int64_t *picked, int64_t n_out, int64_t d,
+                               int depth, void *lists, void *stream) {
+    if (pathsig_logsignature_lists_bytes(d, depth, n_out) == 0 || top_size < 0) {
+        set_error("lists of wanted columns: bad sizes");
+        return PATHSIG_ERR_ARGUMENT;
+    }
+    const int64_t top = checked_pow(d, depth), columns = hybrid_size(d, depth, top);
+    const bool listed = top_size != top;
+    if (!lists || (n_out > 0 && !picked) || (listed && top_size > 0 && !top_words)) {
+        set_error("lists of wanted columns: NULL pointer");
+        return PATHSIG_ERR_ARGUMENT;
+    }
+    if (!listed) top_words = nullptr;
+    int *at = (int *)lists;
+    hipStream_t st = (hipStream_t)stream;
+    if (d <= 16 && listed) {
+        const hipError_t e = launch_letter_bounds(top_words, top_size, (int)d, depth, at, st);
+        if (e != hipSuccess) return launch_failed(e, "letter bounds launch");
+    }
+    const hipError_t e =
+        launch_pick_lists(top_words, picked, n_out, columns - top, columns, at + 16, at + 16 + columns, st);
+    if (e != hipSuccess) return launch_failed(e, "pick list launch");
+    return PATHSIG_OK;
+}
+
+namespace {
+int check_logsignature(const LogPlan &lp, const int64_t *top_words, int64_t top_size, const int64_t *picked,
+                       const void *lists, const void *workspace, size_t workspace_bytes, size_t need) {
+    if (!lp.usable) {
+        set_error("log-signature in one call: not available for this shape");
+        return PATHSIG_ERR_UNSUPPORTED;
+    }
+    const bool listed = top_size != lp.top;
+    if ((listed && !picked) || ((picked != nullptr) != (lists != nullptr)) || (listed && top_size > 0 && !top_words)) {
+        set_error("log-signature in one call: word list, wanted columns and their lists go together");
+        return PATHSIG_ERR_ARGUMENT;
+    }
+    if (need > 0 && (!workspace || workspace_bytes < need)) {
+        set_error("workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
+        return PATHSIG_ERR_WORKSPACE;
+    }
+    return PATHSIG_OK;
+}
+}  // namespace
+
+int pathsig_logsignature_forward(const void *path, void *out, int dtype, int64_t B, int64_t L, int64_t d, int depth,
+                                 const int64_t *level_sizes, const int64_t *top_words, const int64_t *picked, int64_t n_out,
+                                 const void *lists, const int32_t *windows, int64_t W, void *saved, void *workspace,
+                                 size_t workspace_bytes, void *stream) {
+    const LogPlan lp = log_plan(dtype, B, L, d, depth, level_sizes, windows ? W : 0);
+    const int64_t top_size = level_sizes ? level_sizes[depth] : lp.top;
+    const int rc = check_logsignature(lp, top_words, top_size, picked, lists, workspace, workspace_bytes,
+                                      lp.forward_bytes + (saved ? 0 : lp.saved_bytes));
+    if (rc != PATHSIG_OK) return rc;
+    if (!path || !out) {
+        set_error("path and out must not be NULL");
+        return PATHSIG_ERR_ARGUMENT;
+    }
+    if (dtype == PATHSIG_F32)
+        return log_forward_t<float>(lp, path, out, n_out, B, L, d, depth, top_words, top_size, picked, lists, windows, W,
+                                    saved, workspace, (hipStream_t)stream);
+    return log_forward_t<double>(lp, path, out, n_out, B, L, d, depth, top_words, top_size, picked, lists, windows, W, saved,
+                                 workspace, (hipStream_t)stream);
+}
+
+int pathsig_logsignature_backward(const void *path, const void *saved, size_t saved_bytes, const void *grad_out,
+                                  void *grad_path, int dtype, int64_t B, int64_t L, int64_t d, int depth,
+                                  const int64_t *level_sizes,
+                                  const int64_t *top_words, const int64_t *picked, int64_t n_out, const void *lists,
+                                  const int32_t *windows, int64_t W, void *workspace, size_t workspace_bytes,
+                                  void *stream) {
+    const LogPlan lp = log_plan(dtype, B, L, d, depth, level_sizes, windows ? W : 0);
+    const int64_t top_size = level_sizes ? level_sizes[depth] : lp.top;
+    const int rc =
+        check_logsignature(lp, top_words, top_size, picked, lists, workspace, workspace_bytes, lp.backward_bytes);
+    if (rc != PATHSIG_OK) return rc;
+    if (!path || !saved || !grad_out || !grad_path) {
+        set_error("path, saved, grad_out and grad_path must not be NULL");
+        return PATHSIG_ERR_ARGUMENT;
+    }
+    if (saved_bytes != lp.saved_bytes) {
+        set_error("saved buffer: the forward of this call saves %zu bytes, got %zu (made under other options?)",
+                  lp.saved_bytes, saved_bytes);
+        return PATHSIG_ERR_ARGUMENT;
+    }
+    if (dtype == PATHSIG_F32)
+        return log_backward_t<float>(lp, path, saved, grad_out, n_out, grad_path, B, L, d, depth, top_words, top_size, lists,
+                                     windows, W, workspace, (hipStream_t)stream);
+    return log_backward_t<double>(lp, path, saved, grad_out, n_out, grad_path, B, L, d, depth, top_words, top_size, lists,
+                                  windows, W, workspace, (hipStream_t)stream);
 }
 
 size_t pathsig_logsig_backward_kept_workspace(int dtype, int64_t rows, int64_t d, int depth, int64_t top_size) {

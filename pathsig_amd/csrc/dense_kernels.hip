@@ -26,6 +26,7 @@
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <type_traits>
 
 #include "dense.hpp"
@@ -400,6 +401,13 @@ __global__ void __launch_bounds__(1024)
     letter_bounds_kernel(const int64_t *__restrict__ codes, int64_t count, int d, int depth, bool narrow,
                          int *__restrict__ bounds) {
     letter_bounds_block(codes, count, d, depth, narrow, bounds);
+}
+
+// The letter bounds of a word list, for callers that keep them (16 ints).
+hipError_t launch_letter_bounds_impl(const int64_t *codes, int64_t count, int d, int depth, int *bounds, hipStream_t stream) {
+    const bool narrow = (double)depth * std::log2((double)d) < 32.0;
+    hipLaunchKernelGGL(letter_bounds_kernel, dim3(1), dim3(1024), 0, stream, codes, count, d, depth, narrow, bounds);
+    return hipGetLastError();
 }
 
 // The last block computes the letter bounds (when asked for: bounds != nullptr), the others clear ptr[0..n).
@@ -1711,7 +1719,7 @@ __device__ __forceinline__ void dense_backward_body(
     constexpr int KS = N - P;
     constexpr int kParts = BS::kParts;
     constexpr int kBwdTile = BS::kBwdTile;
-    constexpr bool kToPath = CHUNKED && !ACCUMULATE;  // writes the path gradient itself (see the tile flush)
+    constexpr bool kToPath = !ACCUMULATE;  // writes the path gradient itself (see the tile flush)
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;  // within the block
     // first level split between lanes: pu_unit counts (part of the children, prefix); pu is the prefix
@@ -2106,7 +2114,7 @@ __device__ __forceinline__ void dense_backward_body(
         // cell of (increment, letter) number idx in a row of `sg`
         auto cell = [](int idx) { return BS::kLetters == D ? idx : (idx / D) * BS::kLetters + idx % D; };
         if constexpr (kToPath) {
-            // Time-chunked, no windows: the path gradient dL/dx[t] = g[t-1] - g[t] leaves the kernel directly.
+            // No windows, one block to a unit: the path gradient dL/dx[t] = g[t-1] - g[t] leaves the kernel directly.
             // Tiles are flushed from the right end of the chunk to its left end; `carry` holds g of the first
             // increment of the tile flushed before (the one to the right), whose point is written now.
             for (int idx = tid; idx < nt * D; idx += G::kBlock) {
@@ -2338,9 +2346,7 @@ const int *stage_letter_bounds(const DenseChoice &dc, const int64_t *top_codes, 
     if (!dc.bounded) return nullptr;
     int *bounds = (int *)*workspace;
     *workspace = (unsigned char *)*workspace + kBoundsBytes;
-    const bool narrow = (double)depth * std::log2((double)d) < 32.0;
-    hipLaunchKernelGGL(letter_bounds_kernel, dim3(1), dim3(1024), 0, stream, top_codes, top_count, d, depth, narrow,
-                       bounds);
+    (void)launch_letter_bounds_impl(top_codes, top_count, d, depth, bounds, stream);
     return bounds;
 }
 
@@ -2670,7 +2676,8 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
             if constexpr (G::kUnitBlocks == 1)
                 hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, false, false>), dim3((unsigned)rows),
                                    dim3(G::kBlock), 0, stream, path, sig, grad_sig, (const T *)nullptr,
-                                   (const T *)nullptr, grad_inc, shape, 1);
+                                   (const T *)nullptr, grad_inc, shape, 1, grad_path);
+            *wrote_path = true;
         }
         profile_bracket(false, stream);
         return hipGetLastError();
@@ -2759,6 +2766,10 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
 }  // namespace
 
 #if PSIG_GROUP < 0
+hipError_t launch_letter_bounds(const int64_t *codes, int64_t count, int d, int depth, int *bounds, hipStream_t stream) {
+    return launch_letter_bounds_impl(codes, count, d, depth, bounds, stream);
+}
+
 void profile_bracket(bool begin, hipStream_t stream) { profile_mark(begin, stream); }
 
 void profile_enable(bool on) {
@@ -2774,8 +2785,8 @@ float profile_sweep_ms() {
     return ms;
 }
 
-DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes, int64_t B,
-                         int64_t L, int64_t W, bool) {
+static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes,
+                                     int64_t B, int64_t L, int64_t W) {
     DenseChoice dc{};
     dc.variant = -1;
     dc.fwd_chunks = dc.bwd_chunks = 1;
@@ -2891,6 +2902,38 @@ DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, cons
     return dc;
 }
 
+// A step of training asks for the same choice seven times (sizes of buffers, then the launches), and a small call is
+// bound by its host time: the last few choices of a thread are remembered.
+DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes, int64_t B,
+                         int64_t L, int64_t W, bool) {
+    struct Key {
+        int64_t elem, d, depth, all_dense, B, L, W, options, sizes[kMaxDepth];
+    };
+    constexpr int kRemembered = 8;
+    thread_local Key keys[kRemembered];
+    thread_local DenseChoice choices[kRemembered];
+    thread_local unsigned used = 0, next = 0;
+    Key key;
+    std::memset(&key, 0, sizeof key);
+    key.elem = (int64_t)elem;
+    key.d = d;
+    key.depth = depth;
+    key.all_dense = all_dense ? 1 : 0;
+    key.B = B;
+    key.L = L;
+    key.W = W;
+    key.options = options_epoch();
+    if (!all_dense && level_sizes) std::memcpy(key.sizes, level_sizes + 1, (size_t)depth * sizeof(int64_t));
+    for (unsigned i = 0; i < used; ++i)
+        if (!std::memcmp(&keys[i], &key, sizeof key)) return choices[i];
+    const DenseChoice dc = make_dense_choice(elem, d, depth, all_dense, level_sizes, B, L, W);
+    keys[next] = key;
+    choices[next] = dc;
+    next = (next + 1) % kRemembered;
+    if (used < kRemembered) ++used;
+    return dc;
+}
+
 // f(std::integral_constant<int, g>) for the group g of a shape
 template <int GI = 0, typename F>
 void dispatch_group(int group, F &&f) {
@@ -2905,11 +2948,13 @@ void dispatch_group(int group, F &&f) {
 template <typename T>
 hipError_t launch_dense_forward(const T *path, T *sig, const SigShape &shape, const DenseChoice &dc,
                                 const int64_t *top_codes, int64_t top_count, T *keep, void *workspace,
-                                hipStream_t stream) {
+                                hipStream_t stream, const int *ready_bounds) {
     if (dc.variant < 0 || dc.variant >= kNumVariants) return hipErrorNotSupported;
     if (keep && dc.keep_bytes == 0) return hipErrorInvalidValue;
-    const int *bounds = stage_letter_bounds(dc, top_codes, top_count, kVariants[dc.variant].d,
-                                            kVariants[dc.variant].depth, &workspace, stream);
+    const int *bounds = dc.bounded && ready_bounds
+                            ? ready_bounds
+                            : stage_letter_bounds(dc, top_codes, top_count, kVariants[dc.variant].d,
+                                                  kVariants[dc.variant].depth, &workspace, stream);
     hipError_t e = hipErrorNotSupported;
     dispatch_group(dc.variant % kDenseGroups, [&](auto g) {
         e = launch_dense_forward_group<decltype(g)::value, T>(path, sig, shape, dc, bounds, keep, workspace, stream);
@@ -2921,11 +2966,13 @@ template <typename T>
 hipError_t launch_dense_backward(const T *path, const T *sig, const T *grad_sig, T *grad_inc, T *grad_path,
                                  bool *wrote_path, const SigShape &shape, const DenseChoice &dc,
                                  const int64_t *top_codes, int64_t top_count, const T *kept, void *workspace,
-                                 bool prepared, hipStream_t stream) {
+                                 bool prepared, hipStream_t stream, const int *ready_bounds) {
     if (dc.variant < 0 || dc.variant >= kNumVariants) return hipErrorNotSupported;
     if (kept && dc.keep_bytes == 0) return hipErrorInvalidValue;
     const int *bounds = nullptr;
-    if (prepared && dc.bounded) {
+    if (dc.bounded && ready_bounds) {
+        bounds = ready_bounds;
+    } else if (prepared && dc.bounded) {
         bounds = (const int *)workspace;
         workspace = (unsigned char *)workspace + kBoundsBytes;
     } else {
@@ -2955,10 +3002,10 @@ hipError_t prepare_dense_backward(const DenseChoice &dc, T *zero, int64_t count,
 
 #define PSIG_INSTANTIATE(T)                                                                                      \
     template hipError_t launch_dense_forward<T>(const T *, T *, const SigShape &, const DenseChoice &,            \
-                                                const int64_t *, int64_t, T *, void *, hipStream_t);             \
+                                                const int64_t *, int64_t, T *, void *, hipStream_t, const int *); \
     template hipError_t launch_dense_backward<T>(const T *, const T *, const T *, T *, T *, bool *, const SigShape &, \
                                                  const DenseChoice &, const int64_t *, int64_t, const T *, void *,  \
-                                                 bool, hipStream_t);                                                \
+                                                 bool, hipStream_t, const int *);                                   \
     template hipError_t prepare_dense_backward<T>(const DenseChoice &, T *, int64_t, const int64_t *, int64_t,      \
                                                   void *, hipStream_t);
 PSIG_INSTANTIATE(float)

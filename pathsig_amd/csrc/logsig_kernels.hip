@@ -27,6 +27,7 @@
 //   * scatter form (any size): every word pushes its terms to its prefixes and suffixes with atomics.
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -52,6 +53,8 @@ struct HybridPlan {
     int64_t total;     // S of the hybrid layout
     int64_t lower;     // columns of the levels below `depth`
     int top_is_list;   // top level takes its codes from top_words
+    int64_t lg_stride, cache_stride;  // elements from row to row of the log-signature and of its cache
+    bool summed;       // adjoint: the gradient row already holds the upstream gradient, and sums are added to it
 };
 
 // 1/k! for the exponential series
@@ -83,6 +86,32 @@ __device__ __forceinline__ void word_splits(IDX code, IDX d, IDX (&pidx)[DEG + 1
     }
 }
 
+// acc = value of one word of DEG letters in the Q form (STABLE) from its signature value sw; put(m, Q_m) for m = 2 .. DEG;
+// qc = -sum_{m=2}^{DEG} Q_m / (m + 1)!.  `right`, C: as in logsig_forward_level.
+template <typename T, int DEG, bool STABLE, typename IDX, typename Put>
+__device__ __forceinline__ T word_value(IDX code, T sw, const T *right, const T *C, int depth, IDX d, T &qc, Put &&put) {
+    // dense column of every proper prefix, right factor of every proper suffix
+    IDX pidx[DEG + 1], sidx[DEG + 1];
+    T sufv[DEG + 1];
+    word_splits<IDX, DEG>(code, d, pidx, sidx);
+#pragma unroll
+    for (int k = 1; k < DEG; ++k) sufv[k] = right[sidx[k]];
+    T acc = sw;
+    qc = T(0);
+#pragma unroll
+    for (int m = 2; m <= DEG; ++m) {
+        T pv = T(0);
+#pragma unroll
+        for (int k = m - 1; k < DEG; ++k) pv += C[pidx[k] * (IDX)depth + (IDX)(m - 2)] * sufv[DEG - k];
+        if constexpr (STABLE) {
+            acc -= inv_factorial<T>(m) * pv;
+            qc -= inv_factorial<T>(m + 1) * pv;
+        }
+        put(m, pv);
+    }
+    return acc;
+}
+
 // One level of one row.  STABLE: C is the cache of the Q form (entry k - 1 of a row holds Q_k; entry 0 the
 // log-signature itself), the right factors are log-signature values of the levels below, read from lg, and
 // lg receives the level.  Otherwise C is the power cache P of the reference, the right factors are signature
@@ -97,31 +126,16 @@ __device__ void logsig_forward_level(const T *__restrict__ s, T *C, T *lg, const
     // the blocks of one row (gridDim.y of them) share the words of the level
     for (int64_t i = (int64_t)blockIdx.y * (int)blockDim.x + threadIdx.x; i < hp.size[DEG]; i += (int64_t)gridDim.y * (int)blockDim.x) {
         const IDX code = listed ? (IDX)top_words[i] : (IDX)i;
-        // dense column of every proper prefix, right factor of every proper suffix
-        IDX pidx[DEG + 1], sidx[DEG + 1];
-        T sufv[DEG + 1];
-        word_splits<IDX, DEG>(code, d, pidx, sidx);
-#pragma unroll
-        for (int k = 1; k < DEG; ++k) sufv[k] = right[sidx[k]];
         const IDX own = (IDX)(hp.off[DEG] + i);
         const T sw = s[own];
         T *Cw = C + own * (IDX)depth;
         // the Q form never reads the cache rows of the top level (nothing is longer than a top-level word), so
         // they are not written: for many rows the cache is most of what this kernel moves
         const bool keep_row = !STABLE || DEG < depth;
-        T acc = sw;
-        T qc = T(0);  // -sum_{m=2}^{DEG} Q_m(w) / (m + 1)!
-#pragma unroll
-        for (int m = 2; m <= DEG; ++m) {
-            T pv = T(0);
-#pragma unroll
-            for (int k = m - 1; k < DEG; ++k) pv += C[pidx[k] * (IDX)depth + (IDX)(m - 2)] * sufv[DEG - k];
-            if constexpr (STABLE) {
-                acc -= inv_factorial<T>(m) * pv;
-                qc -= inv_factorial<T>(m + 1) * pv;
-            }
+        T qc;  // -sum_{m=2}^{DEG} Q_m(w) / (m + 1)!
+        const T acc = word_value<T, DEG, STABLE, IDX>(code, sw, right, C, depth, d, qc, [&](int m, T pv) {
             if (keep_row) Cw[m - 1] = pv;
-        }
+        });
         if constexpr (STABLE) {
             if (keep_row) {
                 // entry |w| of the row, which no product reads: Qc(w) = -sum_{m=1}^{|w|} Q_m(w) / (m + 1)!, the
@@ -148,8 +162,8 @@ __global__ void __launch_bounds__(kLogBlock) logsig_forward_kernel(const T *__re
                                                                    int last) {
     const int64_t row = blockIdx.x;
     const T *s = sig + row * hp.total;
-    T *lg = logsig + row * hp.total;
-    T *Cr = C + row * hp.total * hp.depth;
+    T *lg = logsig + row * hp.lg_stride;
+    T *Cr = C + row * hp.cache_stride;
     for (int deg = first; deg <= last; ++deg) {
         switch (deg) {
 #define PSIG_CASE(N) \
@@ -161,6 +175,89 @@ __global__ void __launch_bounds__(kLogBlock) logsig_forward_kernel(const T *__re
         }
         __threadfence_block();
         __syncthreads();
+    }
+}
+
+// The log-signature of a call whose signature rows are dense (stride sig_stride), and of which n_out columns are wanted:
+// column picked[j] of the hybrid layout for output j (all columns of the dense layout when picked is null).  The
+// levels below the top are computed whole, into lg and the cache C (rows of hp.lower and hp.lower * depth elements);
+// of the top level only the words that are wanted, straight from the dense signature into the output.
+// Levels first .. last (below the top) of one row per blockIdx.x, then, with_out, the outputs, which gridDim.y blocks
+// of a row share.
+template <typename T, typename IDX>
+__global__ void __launch_bounds__(kLogBlock)
+    logsig_picked_kernel(const T *__restrict__ sig, int64_t sig_stride, T *lg_all, T *C_all, T *__restrict__ out,
+                         int64_t n_out, HybridPlan hp, const int64_t *__restrict__ top_words,
+                         const int64_t *__restrict__ picked, int first, int last, bool with_out) {
+    const int64_t row = blockIdx.x;
+    const T *s = sig + row * sig_stride;
+    T *lg = lg_all + row * hp.lg_stride;
+    T *C = C_all + row * hp.cache_stride;
+    for (int deg = first; deg <= last; ++deg) {
+        switch (deg) {
+#define PSIG_CASE(N) \
+    case N: logsig_forward_level<T, N, true, IDX>(s, C, lg, hp, top_words); break;
+            PSIG_CASE(1) PSIG_CASE(2) PSIG_CASE(3) PSIG_CASE(4) PSIG_CASE(5) PSIG_CASE(6) PSIG_CASE(7)
+#undef PSIG_CASE
+            default: break;
+        }
+        __threadfence_block();
+        __syncthreads();
+    }
+    if (!with_out) return;
+    T *o = out + row * n_out;
+    const T *s_top = s + hp.off[hp.depth];
+    auto outputs = [&](auto degc) {
+        constexpr int DEG = decltype(degc)::value;
+        for (int64_t j = (int64_t)blockIdx.y * (int)blockDim.x + threadIdx.x; j < n_out; j += (int64_t)gridDim.y * (int)blockDim.x) {
+            const IDX col = picked ? (IDX)picked[j] : (IDX)j;
+            if (col < (IDX)hp.lower) {
+                o[j] = lg[col];
+            } else {
+                const IDX i = col - (IDX)hp.lower;
+                const IDX code = hp.top_is_list ? (IDX)top_words[i] : i;
+                T qc;
+                o[j] = word_value<T, DEG, true, IDX>(code, s_top[code], lg, C, DEG, (IDX)hp.d, qc, [](int, T) {});
+            }
+        }
+    };
+    switch (hp.depth) {
+#define PSIG_CASE(N) \
+    case N: outputs(std::integral_constant<int, N>{}); break;
+        PSIG_CASE(2) PSIG_CASE(3) PSIG_CASE(4) PSIG_CASE(5) PSIG_CASE(6) PSIG_CASE(7) PSIG_CASE(8)
+#undef PSIG_CASE
+        default: break;
+    }
+}
+
+// Which outputs feed a dense column: head[column] is one of them (-1: none) and next[output] the following one, so
+// that an output asked for twice counts twice.  top_words is null where the top level is dense too.  One block.
+__global__ void __launch_bounds__(1024)
+    pick_lists_kernel(const int64_t *__restrict__ top_words, const int64_t *__restrict__ picked, int64_t n_out,
+                      int64_t lower, int64_t columns, int *__restrict__ head, int *__restrict__ next) {
+    for (int64_t i = threadIdx.x; i < columns; i += 1024) head[i] = -1;
+    __threadfence_block();
+    __syncthreads();
+    for (int64_t j = threadIdx.x; j < n_out; j += 1024) {
+        const int64_t col = picked[j];
+        const int64_t at = col < lower || !top_words ? col : lower + top_words[col - lower];
+        next[j] = atomicExch(&head[at], (int)j);
+    }
+}
+
+// dense gradient rows from the gradients of the outputs: every column is written, in one pass
+template <typename T>
+__global__ void __launch_bounds__(256)
+    expand_picked_kernel(const T *__restrict__ grad, T *__restrict__ dense, const int *__restrict__ head,
+                         const int *__restrict__ next, int64_t rows, int64_t columns, int64_t n_out) {
+    for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < columns; c += (int64_t)gridDim.x * 256) {
+        const int first = head[c];
+        const int second = first >= 0 ? next[first] : -1;
+        for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) {
+            T v = first >= 0 ? grad[row * n_out + first] : T(0);
+            for (int j = second; j >= 0; j = next[j]) v += grad[row * n_out + j];
+            dense[row * columns + c] = v;
+        }
     }
 }
 
@@ -236,8 +333,8 @@ __global__ void __launch_bounds__(kLogBlock) logsig_backward_kernel(const T *__r
                                                                     int64_t lds_cols) {
     extern __shared__ __align__(16) unsigned char logsig_smem[];
     const int64_t row = blockIdx.x;
-    const T *s = logsig + row * hp.total;
-    const T *Pr = cache + row * hp.total * hp.depth;
+    const T *s = logsig + row * hp.lg_stride;
+    const T *Pr = cache + row * hp.cache_stride;
     const T *gl = grad_logsig + row * hp.total;
     AdjointSink<T> sink;
     sink.gs = grad_sig + row * hp.total;
@@ -442,7 +539,7 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_top_kernel(const T *_
     const int64_t row = blockIdx.x;
     const int j = (int)blockIdx.y + 1, i = N - j;
     const bool suffix_side = blockIdx.z == 1;
-    {
+    if (!hp.summed) {
         // the gradient of a top-level word is its upstream gradient: every block of the row copies a slice
         const int64_t slices = 2 * (int64_t)gridDim.y, slice = 2 * (int64_t)blockIdx.y + blockIdx.z;
         const int64_t per = (hp.size[N] + slices - 1) / slices;
@@ -452,7 +549,7 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_top_kernel(const T *_
         if (from < to)
             batched_rounds<4>(to - from, [&](int64_t e) { return gl[from + e]; }, [&](int64_t e, T v) { gs[from + e] = v; });
     }
-    const T *lgs = logsig + row * hp.total;
+    const T *lgs = logsig + row * hp.lg_stride;
     const T *gtop = gtop_all + row * top_dense;
     int64_t wi = 1, wj = 1;
     for (int k = 0; k < i; ++k) wi *= hp.d;
@@ -463,8 +560,8 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_top_kernel(const T *_
                         [&](int64_t, int64_t o, T r) { R[o] = r; });
     } else {
         T *gsi = grad_sig + row * hp.total + hp.off[i];
-        block_matvec<T>(gtop, cache + (row * hp.total + hp.off[j]) * N + j, MatvecShape{1, wi, wj, 1, 0, 1, wi, 0, 0, N, 0}, red,
-                        [&](int64_t, int64_t o, T r) { gsi[o] = r; });
+        block_matvec<T>(gtop, cache + row * hp.cache_stride + hp.off[j] * N + j, MatvecShape{1, wi, wj, 1, 0, 1, wi, 0, 0, N, 0},
+                        red, [&](int64_t, int64_t o, T r) { gsi[o] = hp.summed ? gsi[o] + r : r; });
     }
 }
 
@@ -481,7 +578,7 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_top_rows_kernel(
     T *gtop = reinterpret_cast<T *>(top_smem);
     const int N = hp.depth;
     const int64_t row = blockIdx.x;
-    const T *lgs = logsig + row * hp.total;
+    const T *lgs = logsig + row * hp.lg_stride;
     const T *gl = grad_logsig + row * hp.total + hp.off[N];
     if (hp.size[N] != top_dense) {  // a listed top level (possibly empty)
         for (int64_t i = threadIdx.x; i < top_dense; i += (int)blockDim.x) gtop[i] = T(0);
@@ -500,8 +597,8 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_top_rows_kernel(
         block_matvec<T>(gtop, lgs + hp.off[i], MatvecShape{1, wj, wi, 1, 0, wi, 1, 0, 0, 1, 0}, red,
                         [&](int64_t, int64_t o, T r) { R[o] = r; });
         T *gsi = grad_sig + row * hp.total + hp.off[i];
-        block_matvec<T>(gtop, cache + (row * hp.total + hp.off[j]) * N + j, MatvecShape{1, wi, wj, 1, 0, 1, wi, 0, 0, N, 0}, red,
-                        [&](int64_t, int64_t o, T r) { gsi[o] = r; });
+        block_matvec<T>(gtop, cache + row * hp.cache_stride + hp.off[j] * N + j, MatvecShape{1, wi, wj, 1, 0, 1, wi, 0, 0, N, 0},
+                        red, [&](int64_t, int64_t o, T r) { gsi[o] = hp.summed ? gsi[o] + r : r; });
     }
 }
 
@@ -523,10 +620,11 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_kernel(const T *__res
     __shared__ T red[kLogBlock];
     const int N = hp.depth;
     const int64_t row = blockIdx.x;
-    const T *lgs = logsig + row * hp.total;
-    const T *Cr = cache + row * hp.total * N;
+    const T *lgs = logsig + row * hp.lg_stride;
+    const T *Cr = cache + row * hp.cache_stride;
     const T *gl = grad_logsig + row * hp.total;
     T *gs = grad_sig + row * hp.total;
+    const bool summed = hp.summed;  // gs holds the upstream gradient already
     // the address space of `a` is fixed at compile time, so that its loads are LDS loads and not generic ones
     static_assert(A_IN_LDS || !STAGED, "the staged form keeps `a` in LDS too");
     T *a;
@@ -540,7 +638,7 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_kernel(const T *__res
         T *gs_l = a + hp.lower * N, *lgs_l = gs_l + hp.lower, *C_l = lgs_l + few;
         batched_rounds<4>(few, [&](int64_t i) { return lgs[i]; }, [&](int64_t i, T v) { lgs_l[i] = v; });
         batched_rounds<8>(few * N, [&](int64_t i) { return Cr[i]; }, [&](int64_t i, T v) { C_l[i] = v; });
-        batched_rounds<8>(hp.lower, [&](int64_t i) { return gs[i] + gl[i]; }, [&](int64_t i, T v) { gs_l[i] = v; });
+        batched_rounds<8>(hp.lower, [&](int64_t i) { return summed ? gs[i] : gs[i] + gl[i]; }, [&](int64_t i, T v) { gs_l[i] = v; });
         lgsp = lgs_l;
         Crp = C_l;
         gsp = gs_l;
@@ -662,7 +760,7 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_kernel(const T *__res
         }
         // lam(w) = g(w) + a_1(w) + the sums above is the gradient of the word; a_k(w) -= lam(w) / k! for k >= 2
         for (int i = tid; i < wn; i += BLK) {
-            const T lam = (STAGED ? T(0) : gl[hp.off[n] + i]) + an[i * N] + gsn[i];
+            const T lam = (STAGED || summed ? T(0) : gl[hp.off[n] + i]) + an[i * N] + gsn[i];
             gsn[i] = lam;
             for (int k = 2; k <= n; ++k) an[i * N + k - 1] -= invf[k] * lam;
         }
@@ -713,6 +811,9 @@ HybridPlan make_hybrid(int64_t d, int depth, int64_t top_size, const int64_t *to
         off += hp.size[k];
     }
     hp.total = off;
+    hp.lg_stride = off;
+    hp.cache_stride = off * depth;
+    hp.summed = false;
     return hp;
 }
 
@@ -794,6 +895,13 @@ LogsigBackwardPlan logsig_backward_plan(size_t elem, int64_t rows, int64_t d, in
     return lp;
 }
 
+namespace {
+template <typename T>
+hipError_t launch_adjoint(const T *logsig, const T *cache, const T *grad_logsig, T *grad_sig, T *workspace, int64_t rows,
+                          const HybridPlan &hp, const LogsigBackwardPlan &lp, const int64_t *top_words,
+                          hipStream_t stream);
+}
+
 // logsig and cache are the outputs of launch_logsig_forward for the same signature
 template <typename T>
 hipError_t launch_logsig_backward(const T *logsig, const T *cache, const T *grad_logsig, T *grad_sig, T *workspace,
@@ -802,6 +910,16 @@ hipError_t launch_logsig_backward(const T *logsig, const T *cache, const T *grad
     if (rows <= 0) return hipSuccess;
     const HybridPlan hp = make_hybrid(d, depth, top_size, top_words);
     const LogsigBackwardPlan lp = logsig_backward_plan(sizeof(T), rows, d, depth, top_size);
+    return launch_adjoint<T>(logsig, cache, grad_logsig, grad_sig, workspace, rows, hp, lp, top_words, stream);
+}
+
+namespace {
+template <typename T>
+hipError_t launch_adjoint(const T *logsig, const T *cache, const T *grad_logsig, T *grad_sig, T *workspace, int64_t rows,
+                          const HybridPlan &hp, const LogsigBackwardPlan &lp, const int64_t *top_words,
+                          hipStream_t stream) {
+    const int64_t d = hp.d, top_size = hp.size[hp.depth];
+    const int depth = hp.depth;
     const int blk = logsig_block(hp.total, rows);
     T *gradP = workspace;
     if (lp.gather) {
@@ -810,7 +928,7 @@ hipError_t launch_logsig_backward(const T *logsig, const T *cache, const T *grad
         // top-level products: with many rows of a small layout one block per row with the row's dense top-level
         // gradient in LDS; else one block per (row, split, side) over a dense copy of that gradient in memory
         const size_t top_bytes = (size_t)lp.top_dense * sizeof(T);
-        bool copy_top = true;  // the lower-level kernel copies the top-level part of the gradient
+        bool copy_top = !hp.summed;  // the lower-level kernel copies the top-level part of the gradient
         if (rows >= 256 && top_bytes <= 64 * 1024) {
             if (top_bytes > 32 * 1024) {
                 e = allow_dynamic_lds<logsig_gather_top_rows_kernel<T>>(top_bytes);
@@ -873,12 +991,80 @@ hipError_t launch_logsig_backward(const T *logsig, const T *cache, const T *grad
                        grad_logsig, grad_sig, gradP, hp, top_words, lds_cols);
     return hipGetLastError();
 }
+}  // namespace
+
+// ---------------------------------------------------------------------------------------------
+// the log-signature of dense signature rows, wanted columns only
+// ---------------------------------------------------------------------------------------------
+namespace {
+HybridPlan picked_plan(int64_t d, int depth, int64_t top_size, const int64_t *top_words) {
+    HybridPlan hp = make_hybrid(d, depth, top_size, top_words);
+    hp.lg_stride = hp.lower;
+    hp.cache_stride = hp.lower * depth;
+    return hp;
+}
+}  // namespace
+
+bool picked_logsig_possible(size_t elem, int64_t rows, int64_t d, int depth) {
+    if (depth < 2 || depth > 8 || options().logsig_scatter != 0) return false;
+    // 32-bit columns everywhere, and the gather form of the adjoint
+    const double top = std::pow((double)d, (double)depth);
+    return top * depth < 2e9 && rows < (int64_t(1) << 31) && logsig_backward_plan(elem, rows, d, depth, (int64_t)top).gather;
+}
+
+hipError_t launch_pick_lists(const int64_t *top_words, const int64_t *picked, int64_t n_out, int64_t lower,
+                             int64_t columns, int *head, int *next, hipStream_t stream) {
+    hipLaunchKernelGGL(pick_lists_kernel, dim3(1), dim3(1024), 0, stream, top_words, picked, n_out, lower, columns, head,
+                       next);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_picked_logsig(const T *sig, int64_t sig_stride, T *lg, T *cache, T *out, int64_t n_out, int64_t rows,
+                                int64_t d, int depth, int64_t top_size, const int64_t *top_words, const int64_t *picked,
+                                hipStream_t stream) {
+    const HybridPlan hp = picked_plan(d, depth, top_size, top_words);
+    const int blk = logsig_block(hp.total, rows);
+    int64_t slices = (n_out + 4 * blk - 1) / (4 * blk);
+    if (slices > 16) slices = 16;
+    const bool together = slices < 2;
+    hipLaunchKernelGGL((logsig_picked_kernel<T, uint32_t>), dim3((unsigned)rows), dim3(blk), 0, stream, sig, sig_stride, lg,
+                       cache, out, n_out, hp, top_words, picked, 1, depth - 1, together);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || together) return e;
+    hipLaunchKernelGGL((logsig_picked_kernel<T, uint32_t>), dim3((unsigned)rows, (unsigned)slices), dim3(blk), 0, stream,
+                       sig, sig_stride, lg, cache, out, n_out, hp, top_words, picked, 1, 0, true);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_picked_adjoint(const T *lg, const T *cache, const T *grad_out, int64_t n_out, T *dense, T *workspace,
+                                 int64_t rows, int64_t d, int depth, const int *head, const int *next,
+                                 hipStream_t stream) {
+    int64_t top = 1;
+    for (int k = 0; k < depth; ++k) top *= d;
+    HybridPlan hp = picked_plan(d, depth, top, nullptr);
+    const LogsigBackwardPlan lp = logsig_backward_plan(sizeof(T), rows, d, depth, top);
+    if (head) {
+        hipLaunchKernelGGL(expand_picked_kernel<T>, columns_by_rows_grid(hp.total, rows), dim3(256), 0, stream, grad_out,
+                           dense, head, next, rows, hp.total, n_out);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        hp.summed = true;
+        grad_out = dense;
+    }
+    return launch_adjoint<T>(lg, cache, grad_out, dense, workspace, rows, hp, lp, nullptr, stream);
+}
 
 #define PSIG_INSTANTIATE(T)                                                                                       \
     template hipError_t launch_logsig_forward<T>(const T *, T *, T *, T *, int64_t, int64_t, int, int64_t,        \
                                                  const int64_t *, hipStream_t);                                   \
     template hipError_t launch_logsig_backward<T>(const T *, const T *, const T *, T *, T *, int64_t, int64_t, int, \
-                                                  int64_t, const int64_t *, hipStream_t);
+                                                  int64_t, const int64_t *, hipStream_t);                             \
+    template hipError_t launch_picked_logsig<T>(const T *, int64_t, T *, T *, T *, int64_t, int64_t, int64_t, int,    \
+                                                int64_t, const int64_t *, const int64_t *, hipStream_t);             \
+    template hipError_t launch_picked_adjoint<T>(const T *, const T *, const T *, int64_t, T *, T *, int64_t, int64_t, \
+                                                 int, const int *, const int *, hipStream_t);
 PSIG_INSTANTIATE(float)
 PSIG_INSTANTIATE(double)
 #undef PSIG_INSTANTIATE

@@ -11,8 +11,12 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/autograd.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/python_arg_parser.h>
 #include <torch/library.h>
 
+#include <cstdlib>
 #include <limits>
 #include <tuple>
 #include <vector>
@@ -476,6 +480,286 @@ std::tuple<Tensor, Tensor> sig_to_logsig_keep_autograd(const Tensor &signature, 
     return {out[0], out[1]};
 }
 
+
+// ---- calls from the modules --------------------------------------------------------------------------------
+// A small call is bound by its host time, and a good part of that is the boxed call of an operator from Python (the
+// schema, a stack of values, two rounds of dispatch).  The modules therefore call the functions of this extension
+// (PyInit_libpathsig_torch below), which hand plain CUDA tensors straight to the device implementations and their
+// autograd nodes.  Everything that is not a plain CUDA tensor in plain eager mode (subclasses, fake tensors, function
+// transforms, tracing, dispatch or torch-function modes) is left to the registered operators: the functions return
+// None and the module takes that way.
+bool plain_call(const Tensor &path) {
+    using c10::DispatchKey;
+    if (!path.defined() || path.scalar_type() == at::kHalf) return false;
+    if (at::impl::torch_function_mode_enabled()) return false;
+    const auto tls = c10::impl::tls_local_dispatch_key_set();
+    const c10::DispatchKeySet ordinary({DispatchKey::CUDA, DispatchKey::ADInplaceOrView, DispatchKey::AutogradCUDA,
+                                        DispatchKey::AutogradOther, DispatchKey::BackendSelect, DispatchKey::AutocastCUDA,
+                                        DispatchKey::AutocastCPU});
+    const c10::DispatchKeySet rest = ((path.key_set() | tls.included_) - tls.excluded_) - ordinary;
+    return path.is_cuda() && (rest.raw_repr() & ~c10::full_backend_mask) == 0;
+}
+
+// the signature with its hand-over, as SignatureKeepFunction, without a second dispatch
+struct SignatureKeepDirectFunction : public torch::autograd::Function<SignatureKeepDirectFunction> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &path, int64_t depth, bool alt, const Tensor &words,
+                          std::vector<int64_t> level_sizes, bool use_windows, const Tensor &windows) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        auto [out, chunks] = sig_forward(path, depth, alt, words, level_sizes, use_windows, windows, true);
+        ctx->save_for_backward({path, out, chunks, windows, words});
+        level_sizes.push_back(depth);
+        level_sizes.push_back(alt ? 1 : 0);
+        level_sizes.push_back(use_windows ? 1 : 0);
+        ctx->saved_data["call"] = std::move(level_sizes);
+        ctx->set_materialize_grads(false);
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        Tensor grad_path;
+        if (ctx->needs_input_grad(0) && grads[0].defined()) {
+            const auto saved = ctx->get_saved_variables();
+            const auto call = ctx->saved_data["call"].toIntVector();
+            const size_t n = call.size() - 3;
+            const at::IntArrayRef level_sizes(call.data(), n);
+            if (at::GradMode::is_enabled()) {
+                // a graph of the gradient is asked for: the operator says what it makes of that
+                static auto op = typed_op<SigBackwardKept>("pathsig::signature_backward_kept");
+                grad_path = op.call(saved[0], saved[1], grads[0], saved[2], call[n], call[n + 1] != 0, saved[4], level_sizes,
+                                    call[n + 2] != 0, saved[3]);
+            } else {
+                grad_path = sig_backward(saved[0], saved[1], grads[0], saved[2], call[n], call[n + 1] != 0, saved[4],
+                                         level_sizes, call[n + 2] != 0, saved[3]);
+            }
+        }
+        return {grad_path, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// ---- the log-signature in one call (pathsig_logsignature_*) -------------------------------------------------------
+struct LogOne {
+    SigCall c;
+    Tensor picked, lists;
+    int64_t n_out;
+    const int64_t *sizes;  // host, or nullptr for the dense layout
+    int64_t top;
+    size_t saved, forward_ws, backward_ws;
+};
+
+// false: not available in this form
+bool log_one(LogOne &o, const Tensor &path, int64_t depth, bool alt, const Tensor &top_words, at::IntArrayRef level_sizes,
+             const Tensor &picked, const Tensor &lists, bool use_windows, const Tensor &windows) {
+    if (depth < 2 || path.dim() != 3 || path.size(1) < 2 ||
+        (path.scalar_type() != at::kFloat && path.scalar_type() != at::kDouble))
+        return false;
+    o.c = sig_call(path, depth, alt, top_words, level_sizes, use_windows, windows);
+    if (use_windows && o.c.W == 0) return false;
+    o.sizes = alt ? level_sizes.data() : nullptr;
+    o.top = alt ? level_sizes[depth] : 0;
+    if (alt) {
+        o.picked = picked;
+        o.lists = lists;
+        o.n_out = picked.numel();
+        if (!picked.is_cuda() || picked.scalar_type() != at::kLong || !picked.is_contiguous() || o.n_out == 0 ||
+            picked.device() != path.device() || top_words.device() != path.device() || lists.device() != path.device() ||
+            level_sizes[1] != o.c.d || (o.top != dense_size(o.c.d, depth, depth) && o.c.n_words < o.top) ||
+            !lists.defined() ||
+            (size_t)lists.numel() * sizeof(int32_t) < pathsig_logsignature_lists_bytes(o.c.d, (int)depth, o.n_out))
+            return false;
+    } else {
+        o.n_out = o.c.sig_size;
+    }
+    return pathsig_logsignature_sizes(o.c.dt, o.c.B, o.c.L, o.c.d, (int)depth, o.sizes, o.c.W, &o.saved, &o.forward_ws,
+                                      &o.backward_ws) == PATHSIG_OK;
+}
+
+std::tuple<Tensor, Tensor> log_one_forward(const LogOne &o, bool save) {
+    const SigCall &c = o.c;
+    c10::DeviceGuard guard(c.path.device());
+    Tensor out = c.W > 0 ? at::empty({c.B, c.W, o.n_out}, c.path.options()) : at::empty({c.B, o.n_out}, c.path.options());
+    Tensor saved = save ? scratch(o.saved, c.path) : Tensor();
+    const size_t ws_bytes = o.forward_ws + (save ? 0 : o.saved);
+    Tensor ws = scratch(ws_bytes, c.path);
+    check_rc(pathsig_logsignature_forward(ptr(c.path), ptr(out), c.dt, c.B, c.L, c.d, (int)c.depth, o.sizes,
+                                          (const int64_t *)ptr(c.words), (const int64_t *)ptr(o.picked), o.n_out,
+                                          ptr(o.lists), c.W > 0 ? (const int32_t *)ptr(c.win) : nullptr, c.W, ptr(saved),
+                                          ptr(ws), ws_bytes, stream_of(c.path)));
+    return {out, saved};
+}
+
+// the same gradient through the operators, for a backward that meets other tuning switches than its forward did or is
+// asked for a graph of the gradient
+Tensor log_backward_composed(const SigCall &c, const Tensor &grad, bool alt, const Tensor &top_words,
+                             at::IntArrayRef level_sizes, const Tensor &picked, bool use_windows, const Tensor &windows) {
+    static auto sig_op = typed_op<SigForwardKeep>("pathsig::compute_signature_keep");
+    static auto log_op = typed_op<LogForward>("pathsig::sig_to_logsig_keep");
+    static auto log_back = typed_op<LogBackward>("pathsig::logsig_backward_kept");
+    static auto sig_back = typed_op<SigBackwardKept>("pathsig::signature_backward_kept");
+    std::vector<int64_t> sizes(level_sizes.begin(), level_sizes.end());
+    if (!alt) {
+        sizes.assign(1, 0);
+        for (int64_t k = 1; k <= c.depth; ++k) sizes.push_back(dense_size(c.d, k, k));
+    }
+    auto [sig, chunks] = sig_op.call(c.path, c.depth, alt, top_words, sizes, use_windows, windows);
+    auto [logsig, cache] = log_op.call(sig, c.depth, c.d, alt, top_words, sizes);
+    Tensor grad_logsig = alt ? at::zeros_like(logsig).index_add(-1, picked, grad) : grad;
+    Tensor grad_sig = log_back.call(logsig, cache, grad_logsig, c.depth, alt, top_words, sizes);
+    return sig_back.call(c.path, sig, grad_sig, chunks, c.depth, alt, top_words, sizes, use_windows, windows);
+}
+
+struct LogSignatureKeepDirectFunction : public torch::autograd::Function<LogSignatureKeepDirectFunction> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &path, const LogOne *one, bool alt, const Tensor &words,
+                          std::vector<int64_t> level_sizes, const Tensor &windows) {
+        at::AutoDispatchBelowADInplaceOrView below;
+        auto [out, saved] = log_one_forward(*one, true);
+        ctx->save_for_backward({path, saved, windows, words, one->picked, one->lists});
+        level_sizes.push_back(one->c.depth);
+        level_sizes.push_back(alt ? 1 : 0);
+        level_sizes.push_back(one->c.W > 0 ? 1 : 0);
+        ctx->saved_data["call"] = std::move(level_sizes);
+        ctx->set_materialize_grads(false);
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        Tensor grad_path;
+        if (ctx->needs_input_grad(0) && grads[0].defined()) {
+            const auto saved = ctx->get_saved_variables();
+            const auto call = ctx->saved_data["call"].toIntVector();
+            const size_t n = call.size() - 3;
+            const at::IntArrayRef level_sizes(call.data(), n);
+            const bool alt = call[n + 1] != 0, use_windows = call[n + 2] != 0;
+            Tensor grad = grads[0].contiguous();
+            LogOne o;
+            const bool one = log_one(o, saved[0], call[n], alt, saved[3], level_sizes, saved[4], saved[5], use_windows, saved[2]);
+            c10::DeviceGuard guard(saved[0].device());
+            if (one && (size_t)saved[1].numel() == o.saved && !at::GradMode::is_enabled()) {
+                const SigCall &c = o.c;
+                grad_path = at::empty_like(c.path);
+                Tensor ws = scratch(o.backward_ws, c.path);
+                check_rc(pathsig_logsignature_backward(
+                    ptr(c.path), ptr(saved[1]), o.saved, ptr(grad), ptr(grad_path), c.dt, c.B, c.L, c.d, (int)c.depth,
+                    o.sizes, (const int64_t *)ptr(c.words), (const int64_t *)ptr(o.picked), o.n_out, ptr(o.lists),
+                    c.W > 0 ? (const int32_t *)ptr(c.win) : nullptr, c.W, ptr(ws), o.backward_ws, stream_of(c.path)));
+            } else {
+                const SigCall c = sig_call(saved[0], call[n], alt, saved[3], level_sizes, use_windows, saved[2]);
+                grad_path = log_backward_composed(c, grad, alt, saved[3], level_sizes, saved[4], use_windows, saved[2]);
+            }
+        }
+        return {grad_path, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+bool wants_keep(const Tensor &path) { return at::GradMode::is_enabled() && path.requires_grad(); }
+
+// PATHSIG_NO_KEEP switches the hand-over off: the module then calls the operator without it
+bool no_keep() {
+    const char *v = std::getenv("PATHSIG_NO_KEEP");
+    return v && *v;
+}
+
+// The functions of the extension.  All arguments positional; None when the call is not one for this way.
+bool tensor_arg(PyObject *obj, Tensor &out) {
+    if (!THPVariable_CheckExact(obj)) return false;
+    out = THPVariable_Unpack(obj);
+    return true;
+}
+
+bool ints_arg(PyObject *obj, std::vector<int64_t> &out) {
+    if (!PyList_Check(obj)) return false;
+    const Py_ssize_t n = PyList_GET_SIZE(obj);
+    out.reserve((size_t)n + 3);
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        const long long v = PyLong_AsLongLong(PyList_GET_ITEM(obj, i));
+        if (v == -1 && PyErr_Occurred()) {
+            PyErr_Clear();
+            return false;
+        }
+        out.push_back(v);
+    }
+    return true;
+}
+
+// (path, depth, alt, words, level_sizes, use_windows, windows)
+PyObject *py_signature(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    Tensor path, words, windows, out;
+    std::vector<int64_t> sizes;
+    if (nargs != 7 || !tensor_arg(args[0], path) || !tensor_arg(args[3], words) || !tensor_arg(args[6], windows) ||
+        !PyLong_Check(args[1]) || !ints_arg(args[4], sizes) || !plain_call(path) ||
+        (wants_keep(path) && no_keep()))
+        Py_RETURN_NONE;
+    const int64_t depth = PyLong_AsLongLong(args[1]);
+    const bool alt = args[2] == Py_True, use_windows = args[5] == Py_True;
+    {
+        pybind11::gil_scoped_release no_gil;
+        if (wants_keep(path)) {
+            out = SignatureKeepDirectFunction::apply(path, depth, alt, words, std::move(sizes), use_windows, windows);
+        } else {
+            at::AutoDispatchBelowADInplaceOrView below;
+            out = std::get<0>(sig_forward(path, depth, alt, words, sizes, use_windows, windows, false));
+        }
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// (path, depth, alt, top_words, level_sizes, picked, lists, use_windows, windows)
+PyObject *py_logsignature(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    Tensor path, words, picked, lists, windows, out;
+    std::vector<int64_t> sizes;
+    if (nargs != 9 || !tensor_arg(args[0], path) || !tensor_arg(args[3], words) || !tensor_arg(args[5], picked) ||
+        !tensor_arg(args[6], lists) || !tensor_arg(args[8], windows) || !PyLong_Check(args[1]) ||
+        !ints_arg(args[4], sizes) || !plain_call(path) ||
+        (wants_keep(path) && no_keep()))
+        Py_RETURN_NONE;
+    const int64_t depth = PyLong_AsLongLong(args[1]);
+    const bool alt = args[2] == Py_True, use_windows = args[7] == Py_True;
+    bool done = false;
+    {
+        pybind11::gil_scoped_release no_gil;
+        LogOne o;
+        if (log_one(o, path, depth, alt, words, sizes, picked, lists, use_windows, windows)) {
+            done = true;
+            if (wants_keep(path)) {
+                out = LogSignatureKeepDirectFunction::apply(path, &o, alt, words, std::move(sizes), windows);
+            } else {
+                at::AutoDispatchBelowADInplaceOrView below;
+                out = std::get<0>(log_one_forward(o, false));
+            }
+        }
+    }
+    if (!done) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// (top_words, top_size, picked, d, depth): the lists of pathsig_logsignature_lists, or None where there are none
+PyObject *py_lists(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    Tensor words, picked;
+    if (nargs != 5 || !tensor_arg(args[0], words) || !tensor_arg(args[2], picked) || !words.is_cuda() ||
+        !picked.is_cuda() || words.scalar_type() != at::kLong || picked.scalar_type() != at::kLong)
+        Py_RETURN_NONE;
+    const int64_t top = PyLong_AsLongLong(args[1]), d = PyLong_AsLongLong(args[3]), depth = PyLong_AsLongLong(args[4]);
+    const size_t bytes = pathsig_logsignature_lists_bytes(d, (int)depth, picked.numel());
+    if (bytes == 0 || picked.numel() == 0 || d > 64 || depth < 2 || depth > 8) Py_RETURN_NONE;
+    c10::DeviceGuard guard(picked.device());
+    Tensor w = words.contiguous(), p = picked.contiguous();
+    Tensor lists = at::empty({(int64_t)(bytes / sizeof(int32_t))}, p.options().dtype(at::kInt));
+    if (top != dense_size(d, depth, depth) && w.numel() < top) Py_RETURN_NONE;
+    check_rc(pathsig_logsignature_lists((const int64_t *)ptr(w), top, (const int64_t *)ptr(p), p.numel(),
+                                        d, (int)depth, ptr(lists), stream_of(p)));
+    return THPVariable_Wrap(std::move(lists));
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef kMethods[] = {
+    {"signature", (PyCFunction)(void (*)(void))py_signature, METH_FASTCALL, nullptr},
+    {"logsignature", (PyCFunction)(void (*)(void))py_logsignature, METH_FASTCALL, nullptr},
+    {"logsignature_lists", (PyCFunction)(void (*)(void))py_lists, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "libpathsig_torch", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
 }  // namespace
 
 TORCH_LIBRARY(pathsig, m) {
@@ -521,3 +805,5 @@ TORCH_LIBRARY_IMPL(pathsig, Autograd, m) {
     m.impl("compute_signature_keep", &compute_signature_keep_autograd);
     m.impl("sig_to_logsig_keep", &sig_to_logsig_keep_autograd);
 }
+
+extern "C" __attribute__((visibility("default"))) PyObject *PyInit_libpathsig_torch(void) { return PyModule_Create(&kModule); }

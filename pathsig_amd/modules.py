@@ -5,6 +5,7 @@ from __future__ import annotations
 import torch
 from torch import nn
 
+from . import _load
 from .ops import _logsig_of, compute_signature
 
 _DEVICE = "cuda"
@@ -42,6 +43,13 @@ def _projection_words(projection):
     return True, words.contiguous()
 
 
+_direct = _load.direct
+
+
+def _version(t: torch.Tensor) -> int:
+    return -1 if t.is_inference() else t._version
+
+
 class Signature(nn.Module):
     """Truncated signature of a batch of paths (B, L, d) -> (B, S) or, with windows, (B, W, S)."""
 
@@ -57,8 +65,15 @@ class Signature(nn.Module):
         self._level_sizes = projection.level_sizes if self.alternative_projection else []
 
     def forward(self, path: torch.Tensor) -> torch.Tensor:
-        return compute_signature(path, self.depth, self.alternative_projection, self._encoded_words,
-                                 self._level_sizes, self.use_windows, self._windows)
+        held = self._buffers
+        if not torch.compiler.is_compiling():
+            # plain tensors in plain eager mode skip the boxed operator call (None: not such a call)
+            out = _direct.signature(path, self.depth, self.alternative_projection, held["_encoded_words"],
+                                    self._level_sizes, self.use_windows, held["_windows"])
+            if out is not None:
+                return out
+        return compute_signature(path, self.depth, self.alternative_projection, held["_encoded_words"],
+                                 self._level_sizes, self.use_windows, held["_windows"])
 
 
 class LogSignature(nn.Module):
@@ -79,6 +94,7 @@ class LogSignature(nn.Module):
                 self.register_buffer(name, _no_tensor(torch.int64), persistent=False)
             self._level_sizes: list[int] = []
             self._ext_level_sizes: list[int] = []
+            self._lists = None
             return
 
         self.register_buffer("_encoded_words", words, persistent=True)
@@ -91,8 +107,37 @@ class LogSignature(nn.Module):
         picked = projection.logsig_indices()
         self.register_buffer("_indices_from_sig", picked.to(device=_DEVICE, dtype=torch.int64).contiguous(),
                              persistent=True)
+        self._make_lists()
+
+    def _make_lists(self):
+        """What the one-call form reads beside the words and the wanted columns: made from both, again when either
+        is replaced or written to."""
+        words, picked = self._buffers["_top_words"], self._buffers["_indices_from_sig"]
+        lists = _direct.logsignature_lists(words, self._ext_level_sizes[self.depth], picked, self._path_dim, self.depth)
+        self._lists = (words, _version(words), picked, _version(picked), lists)
+        return lists
+
+    def _one_call(self, path: torch.Tensor):
+        """Signature, logarithm and selection in one call; None where that form does not apply."""
+        held = self._buffers
+        words, picked = held["_top_words"], held["_indices_from_sig"]
+        if self.alternative_projection:
+            made = self._lists
+            lists = made[4]
+            if made[0] is not words or made[2] is not picked or made[1] != _version(words) or made[3] != _version(picked):
+                lists = self._make_lists()
+            if lists is None:
+                return None
+        else:
+            lists = picked
+        return _direct.logsignature(path, self.depth, self.alternative_projection, words, self._ext_level_sizes, picked,
+                                    lists, self.use_windows, held["_windows"])
 
     def forward(self, path: torch.Tensor) -> torch.Tensor:
+        if not torch.compiler.is_compiling():
+            out = self._one_call(path)
+            if out is not None:
+                return out
         if self.alternative_projection:
             d = self._path_dim
             sizes = self._ext_level_sizes
