@@ -546,6 +546,7 @@ struct LogPlan {
     int64_t rows, columns, lower, top;
     bool keep_products;  // the forward hands the products of its chunks to the backward ..
     bool keep_rows;      // .. or the dense signature rows (swept in one piece)
+    bool small;          // one block per row, everything in LDS (logsig_rows.hip)
     // byte offsets into `saved`: [products of the chunks, or the dense rows][log-signature][its cache]
     size_t lg_at, cache_at, saved_bytes;
     size_t rows_bytes;   // of one dense buffer
@@ -581,12 +582,13 @@ LogPlan log_plan(int dtype, int64_t B, int64_t L, int64_t d, int depth, const in
     const size_t lg = align_up((size_t)lp.rows * lp.lower * elem);
     lp.lg_at = kept;
     lp.cache_at = kept + lg;
-    lp.saved_bytes = lp.cache_at + align_up((size_t)lp.rows * lp.lower * depth * elem);
+    lp.small = elem == 8 ? log_rows_possible<double>(d, depth) : log_rows_possible<float>(d, depth);
+    lp.saved_bytes = lp.cache_at + (lp.small ? 0 : align_up((size_t)lp.rows * lp.lower * depth * elem));
     // (the dense rows of the forward are saved or scratch; what dense_choice asks for a dense buffer is not needed)
     lp.forward_bytes = (lp.keep_rows ? 0 : lp.rows_bytes) + align_up(lp.dc.forward_workspace - lp.dc.dense_bytes);
     lp.inc_bytes = inc_buffer_bytes(elem, B, L, d, false);
     const LogsigBackwardPlan ap = logsig_backward_plan(elem, lp.rows, d, depth, lp.top);
-    lp.adjoint_bytes = align_up((size_t)(ap.a_elems + ap.q_elems) * elem);
+    lp.adjoint_bytes = lp.small ? 0 : align_up((size_t)(ap.a_elems + ap.q_elems) * elem);
     lp.backward_bytes = lp.inc_bytes + lp.rows_bytes + lp.adjoint_bytes +
                         align_up(lp.dc.backward_workspace - (lp.dc.resweep ? 2 : 1) * lp.dc.dense_bytes);
     lp.usable = true;
@@ -612,7 +614,11 @@ int log_forward_t(const LogPlan &lp, const void *path, void *out, int64_t n_out,
                                            save && lp.keep_products ? (T *)keep : (T *)nullptr, rest, stream,
                                            lists ? bounds_of(lists) : nullptr);
     if (e != hipSuccess) return launch_failed(e, "dense forward launch");
-    e = launch_picked_logsig<T>(rows, lp.columns, (T *)(keep + lp.lg_at), (T *)(keep + lp.cache_at), (T *)out, n_out,
+    if (lp.small)
+        e = launch_log_rows_forward<T>(rows, save ? (T *)(keep + lp.lg_at) : (T *)nullptr, (T *)out, n_out, lp.rows, d, depth,
+                                       top_size != lp.top ? top_words : nullptr, picked, stream);
+    else
+        e = launch_picked_logsig<T>(rows, lp.columns, (T *)(keep + lp.lg_at), (T *)(keep + lp.cache_at), (T *)out, n_out,
                                 lp.rows, d, depth, top_size, top_words, picked, stream);
     if (e != hipSuccess) return launch_failed(e, "logsig forward launch");
     return PATHSIG_OK;
@@ -621,7 +627,7 @@ int log_forward_t(const LogPlan &lp, const void *path, void *out, int64_t n_out,
 template <typename T>
 int log_backward_t(const LogPlan &lp, const void *path, const void *saved, const void *grad_out, int64_t n_out,
                    void *grad_path, int64_t B, int64_t L, int64_t d, int depth, const int64_t *top_words, int64_t top_size,
-                   const void *lists, const int32_t *windows, int64_t W, void *workspace, hipStream_t stream) {
+                   const int64_t *picked, const void *lists, const int32_t *windows, int64_t W, void *workspace, hipStream_t stream) {
     const SigShape shape{B, L, d, windows ? W : 1, windows};
     unsigned char *ws = (unsigned char *)workspace;
     const unsigned char *keep = (const unsigned char *)saved;
@@ -630,9 +636,14 @@ int log_backward_t(const LogPlan &lp, const void *path, const void *saved, const
     T *adjoint_ws = (T *)(ws + lp.inc_bytes + lp.rows_bytes);
     void *rest = ws + lp.inc_bytes + lp.rows_bytes + lp.adjoint_bytes;
     const int *head = lists ? heads_of(lists) : nullptr;
-    hipError_t e = launch_picked_adjoint<T>((const T *)(keep + lp.lg_at), (const T *)(keep + lp.cache_at),
-                                            (const T *)grad_out, n_out, dense, adjoint_ws, lp.rows, d, depth, head,
-                                            head ? head + lp.columns : nullptr, stream);
+    hipError_t e;
+    if (lp.small)
+        e = launch_log_rows_adjoint<T>((const T *)(keep + lp.lg_at), (const T *)grad_out, dense, n_out, lp.rows, d, depth,
+                                       top_size != lp.top ? top_words : nullptr, picked, stream);
+    else
+        e = launch_picked_adjoint<T>((const T *)(keep + lp.lg_at), (const T *)(keep + lp.cache_at), (const T *)grad_out,
+                                     n_out, dense, adjoint_ws, lp.rows, d, depth, head,
+                                     head ? head + lp.columns : nullptr, stream);
     if (e != hipSuccess) return launch_failed(e, "logsig backward launch");
     bool wrote_path = false;
     e = launch_dense_backward<T>((const T *)path, lp.keep_rows ? (const T *)keep : (const T *)nullptr, dense, ginc,
@@ -1125,10 +1136,10 @@ int pathsig_logsignature_backward(const void *path, const void *saved, size_t sa
         return PATHSIG_ERR_ARGUMENT;
     }
     if (dtype == PATHSIG_F32)
-        return log_backward_t<float>(lp, path, saved, grad_out, n_out, grad_path, B, L, d, depth, top_words, top_size, lists,
-                                     windows, W, workspace, (hipStream_t)stream);
-    return log_backward_t<double>(lp, path, saved, grad_out, n_out, grad_path, B, L, d, depth, top_words, top_size, lists,
-                                  windows, W, workspace, (hipStream_t)stream);
+        return log_backward_t<float>(lp, path, saved, grad_out, n_out, grad_path, B, L, d, depth, top_words, top_size, picked,
+                                     lists, windows, W, workspace, (hipStream_t)stream);
+    return log_backward_t<double>(lp, path, saved, grad_out, n_out, grad_path, B, L, d, depth, top_words, top_size, picked,
+                                  lists, windows, W, workspace, (hipStream_t)stream);
 }
 
 size_t pathsig_logsig_backward_kept_workspace(int dtype, int64_t rows, int64_t d, int depth, int64_t top_size) {

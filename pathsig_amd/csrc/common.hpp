@@ -249,5 +249,31 @@ template <typename T>
 hipError_t launch_picked_adjoint(const T *lg, const T *cache, const T *grad_out, int64_t n_out, T *dense, T *workspace,
                                  int64_t rows, int64_t d, int depth, const int *head, const int *next,
                                  hipStream_t stream);
+// The same for small layouts (logsig_rows.hip; specialised for float and double): one block per row, no cache and no
+// lists.  top_words: null where the top level is dense.
+template <typename T>
+bool log_rows_possible(int64_t d, int depth);
+template <typename T>
+hipError_t launch_log_rows_forward(const T *sig, T *lg, T *out, int64_t n_out, int64_t rows, int64_t d, int depth,
+                                   const int64_t *top_words, const int64_t *picked, hipStream_t stream);
+template <typename T>
+hipError_t launch_log_rows_adjoint(const T *lg, const T *grad, T *dense, int64_t n_out, int64_t rows, int64_t d, int depth,
+                                   const int64_t *top_words, const int64_t *picked, hipStream_t stream);
+template <>
+bool log_rows_possible<float>(int64_t d, int depth);
+template <>
+bool log_rows_possible<double>(int64_t d, int depth);
+template <>
+hipError_t launch_log_rows_forward<float>(const float *, float *, float *, int64_t, int64_t, int64_t, int,
+                                          const int64_t *, const int64_t *, hipStream_t);
+template <>
+hipError_t launch_log_rows_forward<double>(const double *, double *, double *, int64_t, int64_t, int64_t, int,
+                                           const int64_t *, const int64_t *, hipStream_t);
+template <>
+hipError_t launch_log_rows_adjoint<float>(const float *, const float *, float *, int64_t, int64_t, int64_t, int,
+                                          const int64_t *, const int64_t *, hipStream_t);
+template <>
+hipError_t launch_log_rows_adjoint<double>(const double *, const double *, double *, int64_t, int64_t, int64_t, int,
+                                           const int64_t *, const int64_t *, hipStream_t);
 
 }  // namespace psig

@@ -39,7 +39,7 @@ def _projection(ps, kind, d, depth):
     return None
 
 
-# (8, 5): letter bounds; (8, 4): few rows and many (more than one block of a row shares the top level, a block per
+# (8, 5): letter bounds; (8, 4): few rows (several blocks of a row share its outputs); (3, 3): many (a block per
 # row); (13, 4): swept in one piece; (2, 2): the smallest layout
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("kind", ["dense", "lyndon", "twice", "full_top"])
@@ -85,3 +85,23 @@ def test_lists_follow_the_buffers_and_switches(ps, set_option):
         (grad,) = torch.autograd.grad(out, x, G.cuda())
         assert rel_err(grad, want_grad) < 2e-12
         set_option("tiled", 1)
+
+
+# a block per row compiled for the layout: the longest and the shortest of every depth, those that fit in fp32 only
+# ((3, 7), (4, 6)), tiny ones whose rows are less than a wave, more rows than share the device by slices
+@pytest.mark.parametrize("kind", ["dense", "lyndon"])
+@pytest.mark.parametrize("d,depth", [(2, 2), (16, 2), (2, 3), (16, 3), (7, 4), (2, 5), (5, 5), (3, 6), (4, 6), (2, 7), (3, 7),
+                                     (2, 8)])
+def test_small_layouts(ps, kind, d, depth):
+    proj = _projection(ps, kind, d, depth)
+    module = ps.LogSignature(depth=depth, projection=proj)
+    for B in (1, 530 if d ** depth < 300 else 5):
+        path = brownian_path(B, 7, d, seed=840 + d)
+        xr, want = _want(path, depth, None, proj)
+        G = randn(tuple(want.shape), seed=83)
+        (want_grad,) = torch.autograd.grad(want, xr, G)
+        for dtype in (torch.float64, torch.float32):
+            x = path.to(dtype).cuda().requires_grad_(True)
+            out = module(x)
+            (grad,) = torch.autograd.grad(out, x, G.to(dtype).cuda())
+            assert rel_err(out, want) < TOL[dtype] and rel_err(grad, want_grad) < 2 * TOL[dtype]
