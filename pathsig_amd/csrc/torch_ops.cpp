@@ -487,10 +487,10 @@ std::tuple<Tensor, Tensor> sig_to_logsig_keep_autograd(const Tensor &signature, 
 // (PyInit_libpathsig_torch below), which hand plain CUDA tensors straight to the device implementations and their
 // autograd nodes.  Everything that is not a plain CUDA tensor in plain eager mode (subclasses, fake tensors, function
 // transforms, tracing, dispatch or torch-function modes) is left to the registered operators: the functions return
-// None and the module takes that way.
+// None and the module takes that way.  So are tensors with a forward-mode tangent, which the operators refuse.
 bool plain_call(const Tensor &path) {
     using c10::DispatchKey;
-    if (!path.defined() || path.scalar_type() == at::kHalf) return false;
+    if (!path.defined() || path.scalar_type() == at::kHalf || path._fw_grad(/*level=*/0).defined()) return false;
     if (at::impl::torch_function_mode_enabled()) return false;
     const auto tls = c10::impl::tls_local_dispatch_key_set();
     const c10::DispatchKeySet ordinary({DispatchKey::CUDA, DispatchKey::ADInplaceOrView, DispatchKey::AutogradCUDA,

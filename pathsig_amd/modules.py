@@ -46,8 +46,8 @@ def _projection_words(projection):
 _direct = _load.direct
 
 
-def _version(t: torch.Tensor) -> int:
-    return -1 if t.is_inference() else t._version
+def _version(t: torch.Tensor):
+    return None if t.is_inference() else t._version  # (a write to an inference tensor leaves no trace)
 
 
 class Signature(nn.Module):
@@ -122,10 +122,14 @@ class LogSignature(nn.Module):
         held = self._buffers
         words, picked = held["_top_words"], held["_indices_from_sig"]
         if self.alternative_projection:
-            made = self._lists
-            lists = made[4]
-            if made[0] is not words or made[2] is not picked or made[1] != _version(words) or made[3] != _version(picked):
+            made = self.__dict__.get("_lists")  # (a module unpickled from an older file has none)
+            at = (_version(words), _version(picked))
+            if None in at:
+                return None
+            if made is None or made[0] is not words or made[2] is not picked or (made[1], made[3]) != at:
                 lists = self._make_lists()
+            else:
+                lists = made[4]
             if lists is None:
                 return None
         else:

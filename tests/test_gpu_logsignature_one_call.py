@@ -105,3 +105,24 @@ def test_small_layouts(ps, kind, d, depth):
             out = module(x)
             (grad,) = torch.autograd.grad(out, x, G.to(dtype).cuda())
             assert rel_err(out, want) < TOL[dtype] and rel_err(grad, want_grad) < 2 * TOL[dtype]
+
+
+def test_modules_and_tensors_the_direct_call_leaves_to_the_operators(ps):
+    """A module from a file without the derived lists, buffers whose writes leave no trace, and tangents."""
+    d, depth = 3, 3
+    first = ps.projections.words([(0, 1, 2), (2, 2, 0)], depth=depth, path_dim=d)
+    other = ps.projections.words([(1, 1, 2), (2, 0, 1)], depth=depth, path_dim=d)
+    path = brownian_path(2, 9, d, seed=830)
+    older = ps.LogSignature(depth=depth, projection=first)
+    del older.__dict__["_lists"]
+    assert rel_err(older(path.cuda()), _want(path, depth, None, first)[1]) < 1e-12
+    with torch.inference_mode():
+        written = ps.LogSignature(depth=depth, projection=first)
+        written(path.cuda())
+        written._top_words.copy_(ps.LogSignature(depth=depth, projection=other)._top_words)
+        assert rel_err(written(path.cuda()), _want(path, depth, None, other)[1]) < 1e-12
+    for module in (ps.Signature(depth=depth), ps.LogSignature(depth=depth)):
+        with torch.autograd.forward_ad.dual_level():
+            x = torch.autograd.forward_ad.make_dual(path.cuda(), path.cuda())
+            with pytest.raises(RuntimeError):
+                module(x)
