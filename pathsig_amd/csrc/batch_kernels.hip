@@ -1,4 +1,5 @@
-// Signature backward for word projections with lanes on paths.
+// Signature backward for word projections with lanes on paths, over more than sixteen letters (batch_lists.hip: up to
+// sixteen; the figures below are of sixteen letters, before that one was there).
 //
 // The kernels in words_kernels.hip put one lane on each requested word, so every increment ends in a
 // sum over lanes per letter.  With a batch of paths there is a cheaper arrangement: a group of G lanes
@@ -294,6 +295,8 @@ bool batch_backward_usable(size_t elem, int64_t B, int64_t d, int64_t W) {
 template <typename T, typename ACC>
 hipError_t launch_batch_backward(const T *path, const T *sig, const T *grad_sig, ACC *grad_inc, const SigShape &shape,
                                  const LevelPlan &plan_in, const int64_t *codes, hipStream_t stream) {
+    // (over sixteen letters and fewer the entries are sorted by letter once and added up in rows: 757 against 959 us)
+    if (shape.d <= 16) return launch_batch_lists<T, ACC>(path, sig, grad_sig, grad_inc, shape, plan_in, codes, stream);
     const int G = batch_group<T>(shape.B);
     LevelPlan plan = plan_in;
     int64_t blocks = 0;

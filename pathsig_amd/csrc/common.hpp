@@ -49,7 +49,8 @@ struct Options {
     int64_t chunks;          // forced number of time chunks of the register-tiled kernels (0: chosen per call)
     int64_t letter_bounds;   // embedded projections leave out top-level words by letter bounds (default 1)
     int64_t logsig_scatter;  // log-signature adjoint in its scatter form even where the gather form fits (default 0)
-    int64_t batch_tile;      // cap on the increments per tile of the lanes-on-paths backward (0: no cap)
+    int64_t batch_tile;      // cap on the increments per tile of the lanes-on-paths backward over more than sixteen
+                             // letters (0: no cap)
     int64_t embed_share;     // a projection runs on the register-tiled kernels when its top level keeps at least
                              // 1/embed_share of the dense one (0: never; -1: the library's own rule)
     int64_t tiled;           // 0: every call takes the per-word kernels, whatever its shape (default 1)
@@ -151,6 +152,10 @@ bool batch_wide_sums(size_t elem, const LevelPlan &plan);
 template <typename T, typename ACC>
 hipError_t launch_batch_backward(const T *path, const T *sig, const T *grad_sig, ACC *grad_inc, const SigShape &shape,
                                  const LevelPlan &plan, const int64_t *codes, hipStream_t stream);
+// the same over at most sixteen letters (batch_lists.hip)
+template <typename T, typename ACC>
+hipError_t launch_batch_lists(const T *path, const T *sig, const T *grad_sig, ACC *grad_inc, const SigShape &shape,
+                               const LevelPlan &plan, const int64_t *codes, hipStream_t stream);
 template <typename T>
 hipError_t launch_fill_zero(T *ptr, int64_t n, hipStream_t stream);
 // Grid of the kernels that run x over the columns of a row (256 threads to a block, a thread per column while
