@@ -35,12 +35,12 @@ import torch
 PEAK_TFLOPS = {"f32": 157.3, "f64": 78.6}
 # HBM bytes per launch of the dominant kernel, keyed by workload: rocprofv3 FETCH_SIZE + WRITE_SIZE counters scaled
 # on a copy of known size (FETCH_SIZE x 2.00, WRITE_SIZE x 1.00).  These are figures from the committed counter
-# summaries, not measured in this run; `source` names the summary.  c4 counts the float atomics of the slab flush as
-# written bytes (268 MB of the 377), c5 those of the letter blocks' per-increment sums (33.5 MB of the 152.6).
+# summaries, not measured in this run; `source` names the summary.  c4 counts the float atomics of the letter sums as
+# written bytes (477 MB of the 497), c5 those of the letter blocks' per-increment sums (33.5 MB of the 152.6).
 TRAFFIC = {
     ("c2", "f32"): {"bytes": 33.9e6, "source": "profiles/dense_backward_kernel_c2.md"},
     ("c3", "f32"): {"bytes": 189.7e6, "source": "profiles/dense_kernels_c3_c5.md"},
-    ("c4", "f32"): {"bytes": 377.4e6, "source": "profiles/batch_backward_kernel_c4.md"},
+    ("c4", "f32"): {"bytes": 496.8e6, "source": "profiles/list_backward_kernel_words.md"},
     ("c5", "f32"): {"bytes": 152.6e6, "source": "profiles/dense_kernels_c3_c5.md"},
 }
 
@@ -329,7 +329,7 @@ def run_config(name, dtype_name, args, with_graph, with_cpu, settle_ms):
             sweep_ms = sum(sweep) / len(sweep)
             ach_k = 3.0 * wl["fwd_flops"] / (sweep_ms * 1e-3) / 1e12
             kernel = ("dense_backward_kernel (reverse sweep)" if cfg.get("words") is None
-                      else "batch_backward_kernel (reverse sweep, lanes on paths)")
+                      else "list_backward_kernel (reverse sweep, lanes on paths)")
             traffic = TRAFFIC.get((name, dtype_name))
             result["roofline"] = {"bound": "valu", "achieved": ach_k, "peak": peak, "unit": "TFLOP/s",
                                   "frac": ach_k / peak, "traffic": None if traffic is None else traffic["bytes"],

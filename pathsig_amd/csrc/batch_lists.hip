@@ -9,13 +9,13 @@
 // up the rows: a lane takes four paths of a row, sixteen bytes of an entry at a time.  A letter that most words share
 // takes more rows, so the time does not depend on the words.  The sums of the rows are stored in LDS, added up per
 // letter and sent to memory by atomics in the order of the output, whole cache lines at a time (atomics from the lanes
-// that add the rows, four paths and a few letters to an instruction, took 380 us of 1137).
+// that add the rows, four paths and a few letters to an instruction, took a third of the kernel's time).
 //
-// 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32: 757 us against 959 us with the cells
-// (351 M vector instructions against 464 M, four waves to a SIMD against two).  The chains alone take 540 us: bound by
-// vector issue and by blocks of unequal length, not by memory.  The same sums on the matrix cores (16x16x4 fp32, the
-// entries times a matrix of zeros and ones) were built and are slower: fp32 matrix instructions take as long as the
-// vector ALU would for sixteen letters and do not run beside it.
+// 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32: 643 us against 959 us with the cells; fp64 step
+// 1749 against 2368 us.  The chains alone take 70 % of that: bound by vector issue and by blocks of unequal length, not
+// by memory.  The same sums on the matrix cores (16x16x4 fp32, the entries times a matrix of zeros and ones) were built
+// and are slower: fp32 matrix instructions take as long as the vector
+// ALU would for sixteen letters and do not run beside it.
 #include <type_traits>
 
 #include "common.hpp"
@@ -38,7 +38,7 @@ static_assert(kTile == 2 && kStage % kTile == 0, "the increments of a tile are r
 static_assert(kTile * kRows * 4 == kThreads, "a thread per increment of the tile, row and four paths");
 
 // Entries of a lane: with twelve, four blocks share a CU's LDS and the registers of four waves to a SIMD suffice
-// (eighteen, three blocks: 791 against 757 us in the example above).
+// (eighteen, three blocks: 4 % slower in the example above).
 constexpr int kEntries = 12;
 constexpr int kBlockEntries = kWaves * kSlots * kEntries;
 // The rows suffice however the entries fall to the letters: a letter with n entries leaves at most kRowLen - 1 places
