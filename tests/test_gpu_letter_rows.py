@@ -1,5 +1,5 @@
 """Backward of word projections with lanes on paths over at most sixteen letters (batch_lists.hip): the entries of an
-increment sorted by letter into rows, against the CPU checker."""
+increment sorted by letter into rows, against the oracle."""
 import random
 
 import pytest
