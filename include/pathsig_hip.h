@@ -173,8 +173,9 @@ int pathsig_logsig_backward_kept(const void *logsig, const void *cache, const vo
  *   pathsig_logsignature_sizes   bytes of `saved` and of the two workspaces; PATHSIG_ERR_UNSUPPORTED for calls that
  *                                are not available in this form (compiled shapes of depth 2 to 8 are).  A forward
  *                                with saved == NULL takes forward_workspace + saved bytes of workspace.
- *   pathsig_logsignature_lists   what a caller keeps with a list of wanted columns (device memory, a few ints per
- *                                column): made once for (top_words, picked), read by every call with them
+ * top_words and picked are read by the launches of each call; nothing derived from them outlives it.  `lists` is
+ * therefore left unread and may be NULL, and pathsig_logsignature_lists only checks its arguments; both are there
+ * for callers of the version that read tables made once per list.
  */
 int pathsig_logsignature_sizes(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
                                int64_t W, size_t *saved, size_t *forward_workspace, size_t *backward_workspace);

@@ -537,9 +537,11 @@ int check_logsig(int dtype, int64_t rows, int64_t d, int depth, int64_t top_size
 }
 
 // Signature and log-signature in one call: the signature is swept into dense rows, the logarithm reads them there and
-// computes the wanted columns; the backward expands the gradients of these columns into dense rows, on which the
-// adjoint of the logarithm and that of the signature work in place.  Nothing is gathered, scattered or cleared in
-// between, and no row of the hybrid layout is ever written.
+// computes the wanted columns; the backward adds the gradients of these columns into dense rows, on which the adjoint
+// of the logarithm and that of the signature work in place.  No row of the hybrid layout is ever written.  Everything
+// that follows from the lists of words and columns (letter bounds, places in the dense rows) is worked out by the
+// launches of each call: the lists are device memory that may be rewritten between two calls, or between two replays
+// of a captured graph.
 struct LogPlan {
     bool usable;
     DenseChoice dc;      // with the number of backward chunks of this call
@@ -595,14 +597,10 @@ LogPlan log_plan(int dtype, int64_t B, int64_t L, int64_t d, int depth, const in
     return lp;
 }
 
-// what a module keeps: the letter bounds of the word list (16 ints) and the lists of outputs per dense column
-const int *bounds_of(const void *lists) { return (const int *)lists; }
-const int *heads_of(const void *lists) { return (const int *)lists + 16; }
-
 template <typename T>
 int log_forward_t(const LogPlan &lp, const void *path, void *out, int64_t n_out, int64_t B, int64_t L, int64_t d, int depth,
-                  const int64_t *top_words, int64_t top_size, const int64_t *picked, const void *lists,
-                  const int32_t *windows, int64_t W, void *saved, void *workspace, hipStream_t stream) {
+                  const int64_t *top_words, int64_t top_size, const int64_t *picked, const int32_t *windows, int64_t W,
+                  void *saved, void *workspace, hipStream_t stream) {
     const SigShape shape{B, L, d, windows ? W : 1, windows};
     unsigned char *ws = (unsigned char *)workspace;
     const bool save = saved != nullptr;
@@ -611,8 +609,7 @@ int log_forward_t(const LogPlan &lp, const void *path, void *out, int64_t n_out,
     void *rest = ws + (lp.keep_rows ? 0 : lp.rows_bytes);
     DenseChoice dc = lp.dc;
     hipError_t e = launch_dense_forward<T>((const T *)path, rows, shape, dc, top_words, top_size,
-                                           save && lp.keep_products ? (T *)keep : (T *)nullptr, rest, stream,
-                                           lists ? bounds_of(lists) : nullptr);
+                                           save && lp.keep_products ? (T *)keep : (T *)nullptr, rest, stream);
     if (e != hipSuccess) return launch_failed(e, "dense forward launch");
     if (lp.small)
         e = launch_log_rows_forward<T>(rows, save ? (T *)(keep + lp.lg_at) : (T *)nullptr, (T *)out, n_out, lp.rows, d, depth,
@@ -627,7 +624,7 @@ int log_forward_t(const LogPlan &lp, const void *path, void *out, int64_t n_out,
 template <typename T>
 int log_backward_t(const LogPlan &lp, const void *path, const void *saved, const void *grad_out, int64_t n_out,
                    void *grad_path, int64_t B, int64_t L, int64_t d, int depth, const int64_t *top_words, int64_t top_size,
-                   const int64_t *picked, const void *lists, const int32_t *windows, int64_t W, void *workspace, hipStream_t stream) {
+                   const int64_t *picked, const int32_t *windows, int64_t W, void *workspace, hipStream_t stream) {
     const SigShape shape{B, L, d, windows ? W : 1, windows};
     unsigned char *ws = (unsigned char *)workspace;
     const unsigned char *keep = (const unsigned char *)saved;
@@ -635,21 +632,28 @@ int log_backward_t(const LogPlan &lp, const void *path, const void *saved, const
     T *dense = (T *)(ws + lp.inc_bytes);
     T *adjoint_ws = (T *)(ws + lp.inc_bytes + lp.rows_bytes);
     void *rest = ws + lp.inc_bytes + lp.rows_bytes + lp.adjoint_bytes;
-    const int *head = lists ? heads_of(lists) : nullptr;
+    // the adjoint adds to cleared rows, or (small layouts, all columns) writes every element itself
+    const bool clear_rows = picked && !lp.small;
+    // one launch clears the increment sums and the dense rows behind them and computes the letter bounds
+    const bool prepared = clear_rows || lp.dc.bounded;
     hipError_t e;
+    if (prepared) {
+        e = prepare_dense_backward<T>(lp.dc, ginc, (int64_t)((lp.inc_bytes + (clear_rows ? lp.rows_bytes : 0)) / sizeof(T)),
+                                      top_words, top_size, rest, stream);
+        if (e != hipSuccess) return launch_failed(e, "fill launch");
+    }
     if (lp.small)
         e = launch_log_rows_adjoint<T>((const T *)(keep + lp.lg_at), (const T *)grad_out, dense, n_out, lp.rows, d, depth,
                                        top_size != lp.top ? top_words : nullptr, picked, stream);
     else
         e = launch_picked_adjoint<T>((const T *)(keep + lp.lg_at), (const T *)(keep + lp.cache_at), (const T *)grad_out,
-                                     n_out, dense, adjoint_ws, lp.rows, d, depth, head,
-                                     head ? head + lp.columns : nullptr, stream);
+                                     n_out, dense, adjoint_ws, lp.rows, d, depth, top_size != lp.top ? top_words : nullptr,
+                                     picked, stream);
     if (e != hipSuccess) return launch_failed(e, "logsig backward launch");
     bool wrote_path = false;
     e = launch_dense_backward<T>((const T *)path, lp.keep_rows ? (const T *)keep : (const T *)nullptr, dense, ginc,
                                  (T *)grad_path, &wrote_path, shape, lp.dc, top_words, top_size,
-                                 lp.keep_products ? (const T *)keep : (const T *)nullptr, rest, false, stream,
-                                 lists ? bounds_of(lists) : nullptr);
+                                 lp.keep_products ? (const T *)keep : (const T *)nullptr, rest, prepared, stream);
     if (e != hipSuccess) return launch_failed(e, "dense backward launch");
     if (wrote_path) return PATHSIG_OK;
     e = launch_increments_to_path<T, T>(ginc, (T *)grad_path, B, L, d, stream);
@@ -1056,35 +1060,25 @@ int pathsig_logsignature_lists(const int64_t *top_words, int64_t top_size, const
         set_error("lists of wanted columns: bad sizes");
         return PATHSIG_ERR_ARGUMENT;
     }
-    const int64_t top = checked_pow(d, depth), columns = hybrid_size(d, depth, top);
-    const bool listed = top_size != top;
+    const bool listed = top_size != checked_pow(d, depth);
     if (!lists || (n_out > 0 && !picked) || (listed && top_size > 0 && !top_words)) {
         set_error("lists of wanted columns: NULL pointer");
         return PATHSIG_ERR_ARGUMENT;
     }
-    if (!listed) top_words = nullptr;
-    int *at = (int *)lists;
-    hipStream_t st = (hipStream_t)stream;
-    if (d <= 16 && listed) {
-        const hipError_t e = launch_letter_bounds(top_words, top_size, (int)d, depth, at, st);
-        if (e != hipSuccess) return launch_failed(e, "letter bounds launch");
-    }
-    const hipError_t e =
-        launch_pick_lists(top_words, picked, n_out, columns - top, columns, at + 16, at + 16 + columns, st);
-    if (e != hipSuccess) return launch_failed(e, "pick list launch");
+    (void)stream;  // nothing to make: see pathsig_logsignature_forward
     return PATHSIG_OK;
 }
 
 namespace {
 int check_logsignature(const LogPlan &lp, const int64_t *top_words, int64_t top_size, const int64_t *picked,
-                       const void *lists, const void *workspace, size_t workspace_bytes, size_t need) {
+                       const void *workspace, size_t workspace_bytes, size_t need) {
     if (!lp.usable) {
         set_error("log-signature in one call: not available for this shape");
         return PATHSIG_ERR_UNSUPPORTED;
     }
     const bool listed = top_size != lp.top;
-    if ((listed && !picked) || ((picked != nullptr) != (lists != nullptr)) || (listed && top_size > 0 && !top_words)) {
-        set_error("log-signature in one call: word list, wanted columns and their lists go together");
+    if ((listed && !picked) || (listed && top_size > 0 && !top_words)) {
+        set_error("log-signature in one call: a listed top level needs its words and the wanted columns");
         return PATHSIG_ERR_ARGUMENT;
     }
     if (need > 0 && (!workspace || workspace_bytes < need)) {
@@ -1097,11 +1091,11 @@ int check_logsignature(const LogPlan &lp, const int64_t *top_words, int64_t top_
 
 int pathsig_logsignature_forward(const void *path, void *out, int dtype, int64_t B, int64_t L, int64_t d, int depth,
                                  const int64_t *level_sizes, const int64_t *top_words, const int64_t *picked, int64_t n_out,
-                                 const void *lists, const int32_t *windows, int64_t W, void *saved, void *workspace,
+                                 const void *, const int32_t *windows, int64_t W, void *saved, void *workspace,
                                  size_t workspace_bytes, void *stream) {
     const LogPlan lp = log_plan(dtype, B, L, d, depth, level_sizes, windows ? W : 0);
     const int64_t top_size = level_sizes ? level_sizes[depth] : lp.top;
-    const int rc = check_logsignature(lp, top_words, top_size, picked, lists, workspace, workspace_bytes,
+    const int rc = check_logsignature(lp, top_words, top_size, picked, workspace, workspace_bytes,
                                       lp.forward_bytes + (saved ? 0 : lp.saved_bytes));
     if (rc != PATHSIG_OK) return rc;
     if (!path || !out) {
@@ -1109,22 +1103,22 @@ int pathsig_logsignature_forward(const void *path, void *out, int dtype, int64_t
         return PATHSIG_ERR_ARGUMENT;
     }
     if (dtype == PATHSIG_F32)
-        return log_forward_t<float>(lp, path, out, n_out, B, L, d, depth, top_words, top_size, picked, lists, windows, W,
-                                    saved, workspace, (hipStream_t)stream);
-    return log_forward_t<double>(lp, path, out, n_out, B, L, d, depth, top_words, top_size, picked, lists, windows, W, saved,
+        return log_forward_t<float>(lp, path, out, n_out, B, L, d, depth, top_words, top_size, picked, windows, W, saved,
+                                    workspace, (hipStream_t)stream);
+    return log_forward_t<double>(lp, path, out, n_out, B, L, d, depth, top_words, top_size, picked, windows, W, saved,
                                  workspace, (hipStream_t)stream);
 }
 
 int pathsig_logsignature_backward(const void *path, const void *saved, size_t saved_bytes, const void *grad_out,
                                   void *grad_path, int dtype, int64_t B, int64_t L, int64_t d, int depth,
                                   const int64_t *level_sizes,
-                                  const int64_t *top_words, const int64_t *picked, int64_t n_out, const void *lists,
+                                  const int64_t *top_words, const int64_t *picked, int64_t n_out, const void *,
                                   const int32_t *windows, int64_t W, void *workspace, size_t workspace_bytes,
                                   void *stream) {
     const LogPlan lp = log_plan(dtype, B, L, d, depth, level_sizes, windows ? W : 0);
     const int64_t top_size = level_sizes ? level_sizes[depth] : lp.top;
     const int rc =
-        check_logsignature(lp, top_words, top_size, picked, lists, workspace, workspace_bytes, lp.backward_bytes);
+        check_logsignature(lp, top_words, top_size, picked, workspace, workspace_bytes, lp.backward_bytes);
     if (rc != PATHSIG_OK) return rc;
     if (!path || !saved || !grad_out || !grad_path) {
         set_error("path, saved, grad_out and grad_path must not be NULL");
@@ -1137,9 +1131,9 @@ int pathsig_logsignature_backward(const void *path, const void *saved, size_t sa
     }
     if (dtype == PATHSIG_F32)
         return log_backward_t<float>(lp, path, saved, grad_out, n_out, grad_path, B, L, d, depth, top_words, top_size, picked,
-                                     lists, windows, W, workspace, (hipStream_t)stream);
+                                     windows, W, workspace, (hipStream_t)stream);
     return log_backward_t<double>(lp, path, saved, grad_out, n_out, grad_path, B, L, d, depth, top_words, top_size, picked,
-                                  lists, windows, W, workspace, (hipStream_t)stream);
+                                  windows, W, workspace, (hipStream_t)stream);
 }
 
 size_t pathsig_logsig_backward_kept_workspace(int dtype, int64_t rows, int64_t d, int depth, int64_t top_size) {

@@ -241,21 +241,19 @@ hipError_t launch_logsig_backward(const T *logsig, const T *cache, const T *grad
 // The log-signature in one go with its signature: from dense signature rows to the wanted columns of the hybrid layout,
 // and from the gradients of those columns to dense gradient rows.  lg, cache: [rows, columns below the top level] and
 // [rows, the same, depth], written by the first and read by the second.  picked (null: the whole dense layout): hybrid
-// column of every output.  head, next: the lists of launch_pick_lists over the dense columns (null with picked).
-// workspace: a_elems + q_elems of logsig_backward_plan for the dense top level.
+// column of every output; dense is cleared before where picked is given.  top_words (adjoint): null where the top level
+// is dense.  workspace: a_elems + q_elems of logsig_backward_plan for the dense top level.
 bool picked_logsig_possible(size_t elem, int64_t rows, int64_t d, int depth);
-hipError_t launch_pick_lists(const int64_t *top_words, const int64_t *picked, int64_t n_out, int64_t lower,
-                             int64_t columns, int *head, int *next, hipStream_t stream);
 template <typename T>
 hipError_t launch_picked_logsig(const T *sig, int64_t sig_stride, T *lg, T *cache, T *out, int64_t n_out, int64_t rows,
                                 int64_t d, int depth, int64_t top_size, const int64_t *top_words, const int64_t *picked,
                                 hipStream_t stream);
 template <typename T>
 hipError_t launch_picked_adjoint(const T *lg, const T *cache, const T *grad_out, int64_t n_out, T *dense, T *workspace,
-                                 int64_t rows, int64_t d, int depth, const int *head, const int *next,
+                                 int64_t rows, int64_t d, int depth, const int64_t *top_words, const int64_t *picked,
                                  hipStream_t stream);
-// The same for small layouts (logsig_rows.hip; specialised for float and double): one block per row, no cache and no
-// lists.  top_words: null where the top level is dense.
+// The same for small layouts (logsig_rows.hip; specialised for float and double): one block per row, no cache, every
+// element of the dense rows written.  top_words: null where the top level is dense.
 template <typename T>
 bool log_rows_possible(int64_t d, int depth);
 template <typename T>

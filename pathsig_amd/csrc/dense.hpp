@@ -29,14 +29,13 @@ DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, cons
 
 // `sig` / `grad_sig` are dense-layout rows; `workspace` is the part of the scratch after any dense buffer.
 // top_codes / top_count: the word list of the top level (device memory), read only when dc.bounded.
-// ready_bounds (optional, device memory): the letter bounds of a bounded call where the caller has them already.
 // keep (optional, dc.keep_bytes bytes): receives, per time chunk, the signature of the row up to the chunk's right
 // edge and that of the rest of the row, below the top level; passing the same buffer as `kept` to the backward of
 // the same call saves it the launches that recompute them.
 template <typename T>
 hipError_t launch_dense_forward(const T *path, T *sig, const SigShape &shape, const DenseChoice &dc,
                                 const int64_t *top_codes, int64_t top_count, T *keep, void *workspace,
-                                hipStream_t stream, const int *ready_bounds = nullptr);
+                                hipStream_t stream);
 // The backward fills grad_inc ([B, L-1, d] increment gradients), or, for calls without windows whose units are one
 // block, writes grad_path ([B, L, d]) itself and reports that in *wrote_path.
 // prepared: prepare_dense_backward has run for this call (grad_inc is zero, the letter bounds of a bounded call
@@ -45,9 +44,7 @@ template <typename T>
 hipError_t launch_dense_backward(const T *path, const T *sig, const T *grad_sig, T *grad_inc, T *grad_path,
                                  bool *wrote_path, const SigShape &shape, const DenseChoice &dc,
                                  const int64_t *top_codes, int64_t top_count, const T *kept, void *workspace,
-                                 bool prepared, hipStream_t stream, const int *ready_bounds = nullptr);
-// letter bounds of a word list over at most sixteen letters (16 ints)
-hipError_t launch_letter_bounds(const int64_t *codes, int64_t count, int d, int depth, int *bounds, hipStream_t stream);
+                                 bool prepared, hipStream_t stream);
 // One launch in front of the backward of an embedded projection, in place of three: clears zero[0..count) (the
 // per-increment sums and the dense gradient buffer behind them) and, for a bounded call, computes the letter
 // bounds into bounds_at (the head of the workspace that launch_dense_backward will be given).

@@ -403,13 +403,6 @@ __global__ void __launch_bounds__(1024)
     letter_bounds_block(codes, count, d, depth, narrow, bounds);
 }
 
-// The letter bounds of a word list, for callers that keep them (16 ints).
-hipError_t launch_letter_bounds_impl(const int64_t *codes, int64_t count, int d, int depth, int *bounds, hipStream_t stream) {
-    const bool narrow = (double)depth * std::log2((double)d) < 32.0;
-    hipLaunchKernelGGL(letter_bounds_kernel, dim3(1), dim3(1024), 0, stream, codes, count, d, depth, narrow, bounds);
-    return hipGetLastError();
-}
-
 // The last block computes the letter bounds (when asked for: bounds != nullptr), the others clear ptr[0..n).
 template <typename T>
 __global__ void __launch_bounds__(1024)
@@ -2346,7 +2339,9 @@ const int *stage_letter_bounds(const DenseChoice &dc, const int64_t *top_codes, 
     if (!dc.bounded) return nullptr;
     int *bounds = (int *)*workspace;
     *workspace = (unsigned char *)*workspace + kBoundsBytes;
-    (void)launch_letter_bounds_impl(top_codes, top_count, d, depth, bounds, stream);
+    const bool narrow = (double)depth * std::log2((double)d) < 32.0;
+    hipLaunchKernelGGL(letter_bounds_kernel, dim3(1), dim3(1024), 0, stream, top_codes, top_count, d, depth, narrow,
+                       bounds);
     return bounds;
 }
 
@@ -2766,10 +2761,6 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
 }  // namespace
 
 #if PSIG_GROUP < 0
-hipError_t launch_letter_bounds(const int64_t *codes, int64_t count, int d, int depth, int *bounds, hipStream_t stream) {
-    return launch_letter_bounds_impl(codes, count, d, depth, bounds, stream);
-}
-
 void profile_bracket(bool begin, hipStream_t stream) { profile_mark(begin, stream); }
 
 void profile_enable(bool on) {
@@ -2948,13 +2939,11 @@ void dispatch_group(int group, F &&f) {
 template <typename T>
 hipError_t launch_dense_forward(const T *path, T *sig, const SigShape &shape, const DenseChoice &dc,
                                 const int64_t *top_codes, int64_t top_count, T *keep, void *workspace,
-                                hipStream_t stream, const int *ready_bounds) {
+                                hipStream_t stream) {
     if (dc.variant < 0 || dc.variant >= kNumVariants) return hipErrorNotSupported;
     if (keep && dc.keep_bytes == 0) return hipErrorInvalidValue;
-    const int *bounds = dc.bounded && ready_bounds
-                            ? ready_bounds
-                            : stage_letter_bounds(dc, top_codes, top_count, kVariants[dc.variant].d,
-                                                  kVariants[dc.variant].depth, &workspace, stream);
+    const int *bounds = stage_letter_bounds(dc, top_codes, top_count, kVariants[dc.variant].d,
+                                            kVariants[dc.variant].depth, &workspace, stream);
     hipError_t e = hipErrorNotSupported;
     dispatch_group(dc.variant % kDenseGroups, [&](auto g) {
         e = launch_dense_forward_group<decltype(g)::value, T>(path, sig, shape, dc, bounds, keep, workspace, stream);
@@ -2966,13 +2955,11 @@ template <typename T>
 hipError_t launch_dense_backward(const T *path, const T *sig, const T *grad_sig, T *grad_inc, T *grad_path,
                                  bool *wrote_path, const SigShape &shape, const DenseChoice &dc,
                                  const int64_t *top_codes, int64_t top_count, const T *kept, void *workspace,
-                                 bool prepared, hipStream_t stream, const int *ready_bounds) {
+                                 bool prepared, hipStream_t stream) {
     if (dc.variant < 0 || dc.variant >= kNumVariants) return hipErrorNotSupported;
     if (kept && dc.keep_bytes == 0) return hipErrorInvalidValue;
     const int *bounds = nullptr;
-    if (dc.bounded && ready_bounds) {
-        bounds = ready_bounds;
-    } else if (prepared && dc.bounded) {
+    if (prepared && dc.bounded) {
         bounds = (const int *)workspace;
         workspace = (unsigned char *)workspace + kBoundsBytes;
     } else {
@@ -3002,10 +2989,10 @@ hipError_t prepare_dense_backward(const DenseChoice &dc, T *zero, int64_t count,
 
 #define PSIG_INSTANTIATE(T)                                                                                      \
     template hipError_t launch_dense_forward<T>(const T *, T *, const SigShape &, const DenseChoice &,            \
-                                                const int64_t *, int64_t, T *, void *, hipStream_t, const int *); \
+                                                const int64_t *, int64_t, T *, void *, hipStream_t);             \
     template hipError_t launch_dense_backward<T>(const T *, const T *, const T *, T *, T *, bool *, const SigShape &, \
                                                  const DenseChoice &, const int64_t *, int64_t, const T *, void *,  \
-                                                 bool, hipStream_t, const int *);                                   \
+                                                 bool, hipStream_t);                                                \
     template hipError_t prepare_dense_backward<T>(const DenseChoice &, T *, int64_t, const int64_t *, int64_t,      \
                                                   void *, hipStream_t);
 PSIG_INSTANTIATE(float)

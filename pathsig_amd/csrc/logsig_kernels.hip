@@ -230,34 +230,16 @@ __global__ void __launch_bounds__(kLogBlock)
     }
 }
 
-// Which outputs feed a dense column: head[column] is one of them (-1: none) and next[output] the following one, so
-// that an output asked for twice counts twice.  top_words is null where the top level is dense too.  One block.
-__global__ void __launch_bounds__(1024)
-    pick_lists_kernel(const int64_t *__restrict__ top_words, const int64_t *__restrict__ picked, int64_t n_out,
-                      int64_t lower, int64_t columns, int *__restrict__ head, int *__restrict__ next) {
-    for (int64_t i = threadIdx.x; i < columns; i += 1024) head[i] = -1;
-    __threadfence_block();
-    __syncthreads();
-    for (int64_t j = threadIdx.x; j < n_out; j += 1024) {
-        const int64_t col = picked[j];
-        const int64_t at = col < lower || !top_words ? col : lower + top_words[col - lower];
-        next[j] = atomicExch(&head[at], (int)j);
-    }
-}
-
-// dense gradient rows from the gradients of the outputs: every column is written, in one pass
+// Adds the gradients of the outputs to cleared dense gradient rows (an output may be asked for twice).  The place of
+// an output is worked out once for all rows of its block.  top_words is null where the top level is dense too.
 template <typename T>
 __global__ void __launch_bounds__(256)
-    expand_picked_kernel(const T *__restrict__ grad, T *__restrict__ dense, const int *__restrict__ head,
-                         const int *__restrict__ next, int64_t rows, int64_t columns, int64_t n_out) {
-    for (int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x; c < columns; c += (int64_t)gridDim.x * 256) {
-        const int first = head[c];
-        const int second = first >= 0 ? next[first] : -1;
-        for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) {
-            T v = first >= 0 ? grad[row * n_out + first] : T(0);
-            for (int j = second; j >= 0; j = next[j]) v += grad[row * n_out + j];
-            dense[row * columns + c] = v;
-        }
+    scatter_picked_kernel(const T *__restrict__ grad, T *__restrict__ dense, const int64_t *__restrict__ top_words,
+                          const int64_t *__restrict__ picked, int64_t rows, int64_t lower, int64_t columns, int64_t n_out) {
+    for (int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x; j < n_out; j += (int64_t)gridDim.x * 256) {
+        const int64_t col = picked[j];
+        const int64_t at = col < lower || !top_words ? col : lower + top_words[col - lower];
+        for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) atomicAdd(&dense[row * columns + at], grad[row * n_out + j]);
     }
 }
 
@@ -1012,13 +994,6 @@ bool picked_logsig_possible(size_t elem, int64_t rows, int64_t d, int depth) {
     return top * depth < 2e9 && rows < (int64_t(1) << 31) && logsig_backward_plan(elem, rows, d, depth, (int64_t)top).gather;
 }
 
-hipError_t launch_pick_lists(const int64_t *top_words, const int64_t *picked, int64_t n_out, int64_t lower,
-                             int64_t columns, int *head, int *next, hipStream_t stream) {
-    hipLaunchKernelGGL(pick_lists_kernel, dim3(1), dim3(1024), 0, stream, top_words, picked, n_out, lower, columns, head,
-                       next);
-    return hipGetLastError();
-}
-
 template <typename T>
 hipError_t launch_picked_logsig(const T *sig, int64_t sig_stride, T *lg, T *cache, T *out, int64_t n_out, int64_t rows,
                                 int64_t d, int depth, int64_t top_size, const int64_t *top_words, const int64_t *picked,
@@ -1039,15 +1014,15 @@ hipError_t launch_picked_logsig(const T *sig, int64_t sig_stride, T *lg, T *cach
 
 template <typename T>
 hipError_t launch_picked_adjoint(const T *lg, const T *cache, const T *grad_out, int64_t n_out, T *dense, T *workspace,
-                                 int64_t rows, int64_t d, int depth, const int *head, const int *next,
+                                 int64_t rows, int64_t d, int depth, const int64_t *top_words, const int64_t *picked,
                                  hipStream_t stream) {
     int64_t top = 1;
     for (int k = 0; k < depth; ++k) top *= d;
     HybridPlan hp = picked_plan(d, depth, top, nullptr);
     const LogsigBackwardPlan lp = logsig_backward_plan(sizeof(T), rows, d, depth, top);
-    if (head) {
-        hipLaunchKernelGGL(expand_picked_kernel<T>, columns_by_rows_grid(hp.total, rows), dim3(256), 0, stream, grad_out,
-                           dense, head, next, rows, hp.total, n_out);
+    if (picked) {
+        hipLaunchKernelGGL(scatter_picked_kernel<T>, columns_by_rows_grid(n_out, rows), dim3(256), 0, stream, grad_out,
+                           dense, top_words, picked, rows, hp.lower, hp.total, n_out);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         hp.summed = true;
@@ -1064,7 +1039,7 @@ hipError_t launch_picked_adjoint(const T *lg, const T *cache, const T *grad_out,
     template hipError_t launch_picked_logsig<T>(const T *, int64_t, T *, T *, T *, int64_t, int64_t, int64_t, int,    \
                                                 int64_t, const int64_t *, const int64_t *, hipStream_t);             \
     template hipError_t launch_picked_adjoint<T>(const T *, const T *, const T *, int64_t, T *, T *, int64_t, int64_t, \
-                                                 int, const int *, const int *, hipStream_t);
+                                                 int, const int64_t *, const int64_t *, hipStream_t);
 PSIG_INSTANTIATE(float)
 PSIG_INSTANTIATE(double)
 #undef PSIG_INSTANTIATE

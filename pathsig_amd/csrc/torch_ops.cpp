@@ -538,7 +538,7 @@ struct SignatureKeepDirectFunction : public torch::autograd::Function<SignatureK
 // ---- the log-signature in one call (pathsig_logsignature_*) -------------------------------------------------------
 struct LogOne {
     SigCall c;
-    Tensor picked, lists;
+    Tensor picked;
     int64_t n_out;
     const int64_t *sizes;  // host, or nullptr for the dense layout
     int64_t top;
@@ -547,7 +547,7 @@ struct LogOne {
 
 // false: not available in this form
 bool log_one(LogOne &o, const Tensor &path, int64_t depth, bool alt, const Tensor &top_words, at::IntArrayRef level_sizes,
-             const Tensor &picked, const Tensor &lists, bool use_windows, const Tensor &windows) {
+             const Tensor &picked, bool use_windows, const Tensor &windows) {
     if (depth < 2 || path.dim() != 3 || path.size(1) < 2 ||
         (path.scalar_type() != at::kFloat && path.scalar_type() != at::kDouble))
         return false;
@@ -557,13 +557,10 @@ bool log_one(LogOne &o, const Tensor &path, int64_t depth, bool alt, const Tenso
     o.top = alt ? level_sizes[depth] : 0;
     if (alt) {
         o.picked = picked;
-        o.lists = lists;
         o.n_out = picked.numel();
         if (!picked.is_cuda() || picked.scalar_type() != at::kLong || !picked.is_contiguous() || o.n_out == 0 ||
-            picked.device() != path.device() || top_words.device() != path.device() || lists.device() != path.device() ||
-            level_sizes[1] != o.c.d || (o.top != dense_size(o.c.d, depth, depth) && o.c.n_words < o.top) ||
-            !lists.defined() ||
-            (size_t)lists.numel() * sizeof(int32_t) < pathsig_logsignature_lists_bytes(o.c.d, (int)depth, o.n_out))
+            picked.device() != path.device() || top_words.device() != path.device() || level_sizes[1] != o.c.d ||
+            (o.top != dense_size(o.c.d, depth, depth) && o.c.n_words < o.top))
             return false;
     } else {
         o.n_out = o.c.sig_size;
@@ -581,7 +578,7 @@ std::tuple<Tensor, Tensor> log_one_forward(const LogOne &o, bool save) {
     Tensor ws = scratch(ws_bytes, c.path);
     check_rc(pathsig_logsignature_forward(ptr(c.path), ptr(out), c.dt, c.B, c.L, c.d, (int)c.depth, o.sizes,
                                           (const int64_t *)ptr(c.words), (const int64_t *)ptr(o.picked), o.n_out,
-                                          ptr(o.lists), c.W > 0 ? (const int32_t *)ptr(c.win) : nullptr, c.W, ptr(saved),
+                                          nullptr, c.W > 0 ? (const int32_t *)ptr(c.win) : nullptr, c.W, ptr(saved),
                                           ptr(ws), ws_bytes, stream_of(c.path)));
     return {out, saved};
 }
@@ -611,7 +608,7 @@ struct LogSignatureKeepDirectFunction : public torch::autograd::Function<LogSign
                           std::vector<int64_t> level_sizes, const Tensor &windows) {
         at::AutoDispatchBelowADInplaceOrView below;
         auto [out, saved] = log_one_forward(*one, true);
-        ctx->save_for_backward({path, saved, windows, words, one->picked, one->lists});
+        ctx->save_for_backward({path, saved, windows, words, one->picked});
         level_sizes.push_back(one->c.depth);
         level_sizes.push_back(alt ? 1 : 0);
         level_sizes.push_back(one->c.W > 0 ? 1 : 0);
@@ -629,7 +626,7 @@ struct LogSignatureKeepDirectFunction : public torch::autograd::Function<LogSign
             const bool alt = call[n + 1] != 0, use_windows = call[n + 2] != 0;
             Tensor grad = grads[0].contiguous();
             LogOne o;
-            const bool one = log_one(o, saved[0], call[n], alt, saved[3], level_sizes, saved[4], saved[5], use_windows, saved[2]);
+            const bool one = log_one(o, saved[0], call[n], alt, saved[3], level_sizes, saved[4], use_windows, saved[2]);
             c10::DeviceGuard guard(saved[0].device());
             if (one && (size_t)saved[1].numel() == o.saved && !at::GradMode::is_enabled()) {
                 const SigCall &c = o.c;
@@ -637,7 +634,7 @@ struct LogSignatureKeepDirectFunction : public torch::autograd::Function<LogSign
                 Tensor ws = scratch(o.backward_ws, c.path);
                 check_rc(pathsig_logsignature_backward(
                     ptr(c.path), ptr(saved[1]), o.saved, ptr(grad), ptr(grad_path), c.dt, c.B, c.L, c.d, (int)c.depth,
-                    o.sizes, (const int64_t *)ptr(c.words), (const int64_t *)ptr(o.picked), o.n_out, ptr(o.lists),
+                    o.sizes, (const int64_t *)ptr(c.words), (const int64_t *)ptr(o.picked), o.n_out, nullptr,
                     c.W > 0 ? (const int32_t *)ptr(c.win) : nullptr, c.W, ptr(ws), o.backward_ws, stream_of(c.path)));
             } else {
                 const SigCall c = sig_call(saved[0], call[n], alt, saved[3], level_sizes, use_windows, saved[2]);
@@ -702,23 +699,22 @@ PyObject *py_signature(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// (path, depth, alt, top_words, level_sizes, picked, lists, use_windows, windows)
+// (path, depth, alt, top_words, level_sizes, picked, use_windows, windows)
 PyObject *py_logsignature(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
-    Tensor path, words, picked, lists, windows, out;
+    Tensor path, words, picked, windows, out;
     std::vector<int64_t> sizes;
-    if (nargs != 9 || !tensor_arg(args[0], path) || !tensor_arg(args[3], words) || !tensor_arg(args[5], picked) ||
-        !tensor_arg(args[6], lists) || !tensor_arg(args[8], windows) || !PyLong_Check(args[1]) ||
-        !ints_arg(args[4], sizes) || !plain_call(path) ||
+    if (nargs != 8 || !tensor_arg(args[0], path) || !tensor_arg(args[3], words) || !tensor_arg(args[5], picked) ||
+        !tensor_arg(args[7], windows) || !PyLong_Check(args[1]) || !ints_arg(args[4], sizes) || !plain_call(path) ||
         (wants_keep(path) && no_keep()))
         Py_RETURN_NONE;
     const int64_t depth = PyLong_AsLongLong(args[1]);
-    const bool alt = args[2] == Py_True, use_windows = args[7] == Py_True;
+    const bool alt = args[2] == Py_True, use_windows = args[6] == Py_True;
     bool done = false;
     {
         pybind11::gil_scoped_release no_gil;
         LogOne o;
-        if (log_one(o, path, depth, alt, words, sizes, picked, lists, use_windows, windows)) {
+        if (log_one(o, path, depth, alt, words, sizes, picked, use_windows, windows)) {
             done = true;
             if (wants_keep(path)) {
                 out = LogSignatureKeepDirectFunction::apply(path, &o, alt, words, std::move(sizes), windows);
@@ -733,30 +729,9 @@ PyObject *py_logsignature(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// (top_words, top_size, picked, d, depth): the lists of pathsig_logsignature_lists, or None where there are none
-PyObject *py_lists(PyObject *, PyObject *const *args, Py_ssize_t nargs) {
-    HANDLE_TH_ERRORS
-    Tensor words, picked;
-    if (nargs != 5 || !tensor_arg(args[0], words) || !tensor_arg(args[2], picked) || !words.is_cuda() ||
-        !picked.is_cuda() || words.scalar_type() != at::kLong || picked.scalar_type() != at::kLong)
-        Py_RETURN_NONE;
-    const int64_t top = PyLong_AsLongLong(args[1]), d = PyLong_AsLongLong(args[3]), depth = PyLong_AsLongLong(args[4]);
-    const size_t bytes = pathsig_logsignature_lists_bytes(d, (int)depth, picked.numel());
-    if (bytes == 0 || picked.numel() == 0 || d > 64 || depth < 2 || depth > 8) Py_RETURN_NONE;
-    c10::DeviceGuard guard(picked.device());
-    Tensor w = words.contiguous(), p = picked.contiguous();
-    Tensor lists = at::empty({(int64_t)(bytes / sizeof(int32_t))}, p.options().dtype(at::kInt));
-    if (top != dense_size(d, depth, depth) && w.numel() < top) Py_RETURN_NONE;
-    check_rc(pathsig_logsignature_lists((const int64_t *)ptr(w), top, (const int64_t *)ptr(p), p.numel(),
-                                        d, (int)depth, ptr(lists), stream_of(p)));
-    return THPVariable_Wrap(std::move(lists));
-    END_HANDLE_TH_ERRORS
-}
-
 PyMethodDef kMethods[] = {
     {"signature", (PyCFunction)(void (*)(void))py_signature, METH_FASTCALL, nullptr},
     {"logsignature", (PyCFunction)(void (*)(void))py_logsignature, METH_FASTCALL, nullptr},
-    {"logsignature_lists", (PyCFunction)(void (*)(void))py_lists, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "libpathsig_torch", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 

@@ -46,10 +46,6 @@ def _projection_words(projection):
 _direct = _load.direct
 
 
-def _version(t: torch.Tensor):
-    return None if t.is_inference() else t._version  # (a write to an inference tensor leaves no trace)
-
-
 class Signature(nn.Module):
     """Truncated signature of a batch of paths (B, L, d) -> (B, S) or, with windows, (B, W, S)."""
 
@@ -94,7 +90,6 @@ class LogSignature(nn.Module):
                 self.register_buffer(name, _no_tensor(torch.int64), persistent=False)
             self._level_sizes: list[int] = []
             self._ext_level_sizes: list[int] = []
-            self._lists = None
             return
 
         self.register_buffer("_encoded_words", words, persistent=True)
@@ -107,39 +102,17 @@ class LogSignature(nn.Module):
         picked = projection.logsig_indices()
         self.register_buffer("_indices_from_sig", picked.to(device=_DEVICE, dtype=torch.int64).contiguous(),
                              persistent=True)
-        self._make_lists()
-
-    def _make_lists(self):
-        """What the one-call form reads beside the words and the wanted columns: made from both, again when either
-        is replaced or written to."""
-        words, picked = self._buffers["_top_words"], self._buffers["_indices_from_sig"]
-        lists = _direct.logsignature_lists(words, self._ext_level_sizes[self.depth], picked, self._path_dim, self.depth)
-        self._lists = (words, _version(words), picked, _version(picked), lists)
-        return lists
-
-    def _one_call(self, path: torch.Tensor):
-        """Signature, logarithm and selection in one call; None where that form does not apply."""
-        held = self._buffers
-        words, picked = held["_top_words"], held["_indices_from_sig"]
-        if self.alternative_projection:
-            made = self.__dict__.get("_lists")  # (a module unpickled from an older file has none)
-            at = (_version(words), _version(picked))
-            if None in at:
-                return None
-            if made is None or made[0] is not words or made[2] is not picked or (made[1], made[3]) != at:
-                lists = self._make_lists()
-            else:
-                lists = made[4]
-            if lists is None:
-                return None
-        else:
-            lists = picked
-        return _direct.logsignature(path, self.depth, self.alternative_projection, words, self._ext_level_sizes, picked,
-                                    lists, self.use_windows, held["_windows"])
+        # What follows from the buffers is worked out on the device in every call, never kept here: they may be
+        # rewritten in any way.  (Modules pickled by earlier versions carry tables under this name.)
+        self._lists = None
 
     def forward(self, path: torch.Tensor) -> torch.Tensor:
         if not torch.compiler.is_compiling():
-            out = self._one_call(path)
+            # signature, logarithm and selection in one call (None: that form does not apply)
+            held = self._buffers
+            out = _direct.logsignature(path, self.depth, self.alternative_projection, held["_top_words"],
+                                       self._ext_level_sizes, held["_indices_from_sig"], self.use_windows,
+                                       held["_windows"])
             if out is not None:
                 return out
         if self.alternative_projection:
