@@ -613,7 +613,7 @@ int log_forward_t(const LogPlan &lp, const void *path, void *out, int64_t n_out,
     if (e != hipSuccess) return launch_failed(e, "dense forward launch");
     if (lp.small)
         e = launch_log_rows_forward<T>(rows, save ? (T *)(keep + lp.lg_at) : (T *)nullptr, (T *)out, n_out, lp.rows, d, depth,
-                                       top_size != lp.top ? top_words : nullptr, picked, stream);
+                                       top_size, top_size != lp.top ? top_words : nullptr, picked, stream);
     else
         e = launch_picked_logsig<T>(rows, lp.columns, (T *)(keep + lp.lg_at), (T *)(keep + lp.cache_at), (T *)out, n_out,
                                 lp.rows, d, depth, top_size, top_words, picked, stream);
@@ -644,11 +644,11 @@ int log_backward_t(const LogPlan &lp, const void *path, const void *saved, const
     }
     if (lp.small)
         e = launch_log_rows_adjoint<T>((const T *)(keep + lp.lg_at), (const T *)grad_out, dense, n_out, lp.rows, d, depth,
-                                       top_size != lp.top ? top_words : nullptr, picked, stream);
+                                       top_size, top_size != lp.top ? top_words : nullptr, picked, stream);
     else
         e = launch_picked_adjoint<T>((const T *)(keep + lp.lg_at), (const T *)(keep + lp.cache_at), (const T *)grad_out,
-                                     n_out, dense, adjoint_ws, lp.rows, d, depth, top_size != lp.top ? top_words : nullptr,
-                                     picked, stream);
+                                     n_out, dense, adjoint_ws, lp.rows, d, depth, top_size,
+                                     top_size != lp.top ? top_words : nullptr, picked, stream);
     if (e != hipSuccess) return launch_failed(e, "logsig backward launch");
     bool wrote_path = false;
     e = launch_dense_backward<T>((const T *)path, lp.keep_rows ? (const T *)keep : (const T *)nullptr, dense, ginc,

@@ -63,6 +63,17 @@ const Options &options();
 int64_t options_epoch();  // changes with every pathsig_set_option
 
 #if defined(__HIPCC__)
+// Column of the dense layout that an output asked for as column `col` of the hybrid layout stands for (`lower` columns
+// below the top level, `columns` in all, `top` words of the top level; top_words null: dense), or -1: the lists are
+// buffers that a caller may load from a file, and nothing on the way here has looked at them.
+__device__ __forceinline__ int64_t picked_column(int64_t col, const int64_t *__restrict__ top_words, int64_t lower,
+                                                 int64_t columns, int64_t top) {
+    if ((uint64_t)col >= (uint64_t)columns) return -1;
+    if (col < lower) return col;
+    const int64_t code = top_words ? top_words[col - lower] : col - lower;
+    return (uint64_t)code < (uint64_t)top ? lower + code : -1;
+}
+
 // Wave-wide sum of one value per lane; the total is valid in lane 63 only.
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ float dpp_add_c(float v) {
@@ -241,8 +252,8 @@ hipError_t launch_logsig_backward(const T *logsig, const T *cache, const T *grad
 // The log-signature in one go with its signature: from dense signature rows to the wanted columns of the hybrid layout,
 // and from the gradients of those columns to dense gradient rows.  lg, cache: [rows, columns below the top level] and
 // [rows, the same, depth], written by the first and read by the second.  picked (null: the whole dense layout): hybrid
-// column of every output; dense is cleared before where picked is given.  top_words (adjoint): null where the top level
-// is dense.  workspace: a_elems + q_elems of logsig_backward_plan for the dense top level.
+// column of every output (one that is no column, or a word that is none: NaN, and no gradient); dense is cleared before
+// where picked is given.  top_words: top_size codes, null (adjoint) where the top level is dense.  workspace: a_elems + q_elems of logsig_backward_plan for the dense top level.
 bool picked_logsig_possible(size_t elem, int64_t rows, int64_t d, int depth);
 template <typename T>
 hipError_t launch_picked_logsig(const T *sig, int64_t sig_stride, T *lg, T *cache, T *out, int64_t n_out, int64_t rows,
@@ -250,33 +261,35 @@ hipError_t launch_picked_logsig(const T *sig, int64_t sig_stride, T *lg, T *cach
                                 hipStream_t stream);
 template <typename T>
 hipError_t launch_picked_adjoint(const T *lg, const T *cache, const T *grad_out, int64_t n_out, T *dense, T *workspace,
-                                 int64_t rows, int64_t d, int depth, const int64_t *top_words, const int64_t *picked,
-                                 hipStream_t stream);
+                                 int64_t rows, int64_t d, int depth, int64_t top_size, const int64_t *top_words,
+                                 const int64_t *picked, hipStream_t stream);
 // The same for small layouts (logsig_rows.hip; specialised for float and double): one block per row, no cache, every
 // element of the dense rows written.  top_words: null where the top level is dense.
 template <typename T>
 bool log_rows_possible(int64_t d, int depth);
 template <typename T>
 hipError_t launch_log_rows_forward(const T *sig, T *lg, T *out, int64_t n_out, int64_t rows, int64_t d, int depth,
-                                   const int64_t *top_words, const int64_t *picked, hipStream_t stream);
+                                   int64_t top_size, const int64_t *top_words, const int64_t *picked,
+                                   hipStream_t stream);
 template <typename T>
 hipError_t launch_log_rows_adjoint(const T *lg, const T *grad, T *dense, int64_t n_out, int64_t rows, int64_t d, int depth,
-                                   const int64_t *top_words, const int64_t *picked, hipStream_t stream);
+                                   int64_t top_size, const int64_t *top_words, const int64_t *picked,
+                                   hipStream_t stream);
 template <>
 bool log_rows_possible<float>(int64_t d, int depth);
 template <>
 bool log_rows_possible<double>(int64_t d, int depth);
 template <>
 hipError_t launch_log_rows_forward<float>(const float *, float *, float *, int64_t, int64_t, int64_t, int,
-                                          const int64_t *, const int64_t *, hipStream_t);
+                                          int64_t, const int64_t *, const int64_t *, hipStream_t);
 template <>
 hipError_t launch_log_rows_forward<double>(const double *, double *, double *, int64_t, int64_t, int64_t, int,
-                                           const int64_t *, const int64_t *, hipStream_t);
+                                           int64_t, const int64_t *, const int64_t *, hipStream_t);
 template <>
 hipError_t launch_log_rows_adjoint<float>(const float *, const float *, float *, int64_t, int64_t, int64_t, int,
-                                          const int64_t *, const int64_t *, hipStream_t);
+                                          int64_t, const int64_t *, const int64_t *, hipStream_t);
 template <>
 hipError_t launch_log_rows_adjoint<double>(const double *, const double *, double *, int64_t, int64_t, int64_t, int,
-                                           const int64_t *, const int64_t *, hipStream_t);
+                                           int64_t, const int64_t *, const int64_t *, hipStream_t);
 
 }  // namespace psig

@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(kLogBlock) logsig_forward_kernel(const T *__re
 template <typename T, typename IDX>
 __global__ void __launch_bounds__(kLogBlock)
     logsig_picked_kernel(const T *__restrict__ sig, int64_t sig_stride, T *lg_all, T *C_all, T *__restrict__ out,
-                         int64_t n_out, HybridPlan hp, const int64_t *__restrict__ top_words,
+                         int64_t n_out, HybridPlan hp, int64_t top, const int64_t *__restrict__ top_words,
                          const int64_t *__restrict__ picked, int first, int last, bool with_out) {
     const int64_t row = blockIdx.x;
     const T *s = sig + row * sig_stride;
@@ -210,12 +210,13 @@ __global__ void __launch_bounds__(kLogBlock)
     auto outputs = [&](auto degc) {
         constexpr int DEG = decltype(degc)::value;
         for (int64_t j = (int64_t)blockIdx.y * (int)blockDim.x + threadIdx.x; j < n_out; j += (int64_t)gridDim.y * (int)blockDim.x) {
-            const IDX col = picked ? (IDX)picked[j] : (IDX)j;
-            if (col < (IDX)hp.lower) {
-                o[j] = lg[col];
+            const int64_t at = picked ? picked_column(picked[j], hp.top_is_list ? top_words : nullptr, hp.lower, hp.total, top) : j;
+            if (at < 0) {
+                o[j] = (T)NAN;
+            } else if (at < hp.lower) {
+                o[j] = lg[at];
             } else {
-                const IDX i = col - (IDX)hp.lower;
-                const IDX code = hp.top_is_list ? (IDX)top_words[i] : i;
+                const IDX code = (IDX)(at - hp.lower);
                 T qc;
                 o[j] = word_value<T, DEG, true, IDX>(code, s_top[code], lg, C, DEG, (IDX)hp.d, qc, [](int, T) {});
             }
@@ -235,10 +236,11 @@ __global__ void __launch_bounds__(kLogBlock)
 template <typename T>
 __global__ void __launch_bounds__(256)
     scatter_picked_kernel(const T *__restrict__ grad, T *__restrict__ dense, const int64_t *__restrict__ top_words,
-                          const int64_t *__restrict__ picked, int64_t rows, int64_t lower, int64_t columns, int64_t n_out) {
+                          const int64_t *__restrict__ picked, int64_t rows, int64_t lower, int64_t columns,
+                          int64_t top_size, int64_t n_out) {
     for (int64_t j = (int64_t)blockIdx.x * 256 + threadIdx.x; j < n_out; j += (int64_t)gridDim.x * 256) {
-        const int64_t col = picked[j];
-        const int64_t at = col < lower || !top_words ? col : lower + top_words[col - lower];
+        const int64_t at = picked_column(picked[j], top_words, lower, lower + top_size, columns - lower);
+        if (at < 0) continue;
         for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) atomicAdd(&dense[row * columns + at], grad[row * n_out + j]);
     }
 }
@@ -999,30 +1001,31 @@ hipError_t launch_picked_logsig(const T *sig, int64_t sig_stride, T *lg, T *cach
                                 int64_t d, int depth, int64_t top_size, const int64_t *top_words, const int64_t *picked,
                                 hipStream_t stream) {
     const HybridPlan hp = picked_plan(d, depth, top_size, top_words);
+    const int64_t top = sig_stride - hp.lower;  // words of the dense top level
     const int blk = logsig_block(hp.total, rows);
     int64_t slices = (n_out + 4 * blk - 1) / (4 * blk);
     if (slices > 16) slices = 16;
     const bool together = slices < 2;
     hipLaunchKernelGGL((logsig_picked_kernel<T, uint32_t>), dim3((unsigned)rows), dim3(blk), 0, stream, sig, sig_stride, lg,
-                       cache, out, n_out, hp, top_words, picked, 1, depth - 1, together);
+                       cache, out, n_out, hp, top, top_words, picked, 1, depth - 1, together);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || together) return e;
     hipLaunchKernelGGL((logsig_picked_kernel<T, uint32_t>), dim3((unsigned)rows, (unsigned)slices), dim3(blk), 0, stream,
-                       sig, sig_stride, lg, cache, out, n_out, hp, top_words, picked, 1, 0, true);
+                       sig, sig_stride, lg, cache, out, n_out, hp, top, top_words, picked, 1, 0, true);
     return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_picked_adjoint(const T *lg, const T *cache, const T *grad_out, int64_t n_out, T *dense, T *workspace,
-                                 int64_t rows, int64_t d, int depth, const int64_t *top_words, const int64_t *picked,
-                                 hipStream_t stream) {
+                                 int64_t rows, int64_t d, int depth, int64_t top_size, const int64_t *top_words,
+                                 const int64_t *picked, hipStream_t stream) {
     int64_t top = 1;
     for (int k = 0; k < depth; ++k) top *= d;
     HybridPlan hp = picked_plan(d, depth, top, nullptr);
     const LogsigBackwardPlan lp = logsig_backward_plan(sizeof(T), rows, d, depth, top);
     if (picked) {
         hipLaunchKernelGGL(scatter_picked_kernel<T>, columns_by_rows_grid(n_out, rows), dim3(256), 0, stream, grad_out,
-                           dense, top_words, picked, rows, hp.lower, hp.total, n_out);
+                           dense, top_words, picked, rows, hp.lower, hp.total, top_size, n_out);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         hp.summed = true;
@@ -1039,7 +1042,7 @@ hipError_t launch_picked_adjoint(const T *lg, const T *cache, const T *grad_out,
     template hipError_t launch_picked_logsig<T>(const T *, int64_t, T *, T *, T *, int64_t, int64_t, int64_t, int,    \
                                                 int64_t, const int64_t *, const int64_t *, hipStream_t);             \
     template hipError_t launch_picked_adjoint<T>(const T *, const T *, const T *, int64_t, T *, T *, int64_t, int64_t, \
-                                                 int, const int64_t *, const int64_t *, hipStream_t);
+                                                 int, int64_t, const int64_t *, const int64_t *, hipStream_t);
 PSIG_INSTANTIATE(float)
 PSIG_INSTANTIATE(double)
 #undef PSIG_INSTANTIATE

@@ -85,11 +85,11 @@ __device__ __forceinline__ T weight_of_word(const T *L, const T *Q, int col) {
 }
 
 // sig: dense rows; lg (may be null): [rows, kLow] log-signature below the top level; out: [rows, n_out].
-// picked: hybrid column of every output (null: all columns, dense); top_words: codes of a listed top level.
+// picked: hybrid column of every output (null: all columns, dense); top_words: top_size codes of a listed top level.
 // The gridDim.y blocks of a row share its outputs (each computes the levels below the top for itself).
 template <typename T, int D, int N>
 __global__ void __launch_bounds__((Rows<T, D, N>::kThreads))
-    log_rows_forward_kernel(const T *__restrict__ sig, T *__restrict__ lg, T *__restrict__ out, int n_out,
+    log_rows_forward_kernel(const T *__restrict__ sig, T *__restrict__ lg, T *__restrict__ out, int n_out, int64_t top_size,
                             const int64_t *__restrict__ top_words, const int64_t *__restrict__ picked) {
     using R = Rows<T, D, N>;
     __shared__ T mem[R::kForward];
@@ -136,11 +136,13 @@ __global__ void __launch_bounds__((Rows<T, D, N>::kThreads))
         return;
     }
     for (int j = first; j < n_out; j += stride) {
-        const int col = (int)picked[j];
-        if (col < R::kLow) {
-            o[j] = L[col];
+        const int at = (int)picked_column(picked[j], top_words, R::kLow, R::kLow + top_size, R::kTop);
+        if (at < 0) {
+            o[j] = (T)NAN;
+        } else if (at < R::kLow) {
+            o[j] = L[at];
         } else {
-            const int w = top_words ? (int)top_words[col - R::kLow] : col - R::kLow;
+            const int w = at - R::kLow;
             T acc = s[R::kLow + w];
             static_for<1, N>([&](auto jc) {
                 constexpr int p = decltype(jc)::value;
@@ -169,7 +171,7 @@ __device__ __forceinline__ T sum_of_lanes(T v) {
 // grad: [rows, n_out]; dense: [rows, kLow + kTop], the gradient of the dense signature rows (every column written)
 template <typename T, int D, int N>
 __global__ void __launch_bounds__((Rows<T, D, N>::kThreads))
-    log_rows_adjoint_kernel(const T *__restrict__ lg, const T *__restrict__ grad, T *__restrict__ dense, int n_out,
+    log_rows_adjoint_kernel(const T *__restrict__ lg, const T *__restrict__ grad, T *__restrict__ dense, int n_out, int64_t top_size,
                             const int64_t *__restrict__ top_words, const int64_t *__restrict__ picked) {
     using R = Rows<T, D, N>;
     extern __shared__ __align__(16) unsigned char rows_smem[];
@@ -191,10 +193,10 @@ __global__ void __launch_bounds__((Rows<T, D, N>::kThreads))
     __syncthreads();
     if (picked) {
         for (int j = tid; j < n_out; j += R::kThreads) {
-            const int col = (int)picked[j];
+            const int at = (int)picked_column(picked[j], top_words, R::kLow, R::kLow + top_size, R::kTop);
             // (an output may be asked for twice)
-            if (col < R::kLow) atomicAdd(&lam[col], gin[j]);
-            else atomicAdd(&g[top_words ? (int)top_words[col - R::kLow] : col - R::kLow], gin[j]);
+            if (at >= R::kLow) atomicAdd(&g[at - R::kLow], gin[j]);
+            else if (at >= 0) atomicAdd(&lam[at], gin[j]);
         }
     }
     static_for<2, N>([&](auto kc) {
@@ -329,7 +331,7 @@ bool log_rows_possible<PSIG_ROWS_TYPE>(int64_t d, int depth) {
 
 template <>
 hipError_t launch_log_rows_forward<PSIG_ROWS_TYPE>(const PSIG_ROWS_TYPE *sig, PSIG_ROWS_TYPE *lg, PSIG_ROWS_TYPE *out,
-                                                   int64_t n_out, int64_t rows, int64_t d, int depth,
+                                                   int64_t n_out, int64_t rows, int64_t d, int depth, int64_t top_size,
                                                    const int64_t *top_words, const int64_t *picked, hipStream_t stream) {
     return with_layout<PSIG_ROWS_TYPE, 2, 2>(
         d, depth,
@@ -340,7 +342,7 @@ hipError_t launch_log_rows_forward<PSIG_ROWS_TYPE>(const PSIG_ROWS_TYPE *sig, PS
             const int64_t slices = rows >= 512 ? 1 : std::max<int64_t>(1, std::min<int64_t>(rounds, 512 / rows));
             hipLaunchKernelGGL((log_rows_forward_kernel<PSIG_ROWS_TYPE, decltype(dc)::value, decltype(nc)::value>),
                                dim3((unsigned)rows, (unsigned)slices), dim3(R::kThreads), 0, stream, sig, lg, out,
-                               (int)n_out, top_words, picked);
+                               (int)n_out, top_size, top_words, picked);
             return hipGetLastError();
         },
         hipErrorNotSupported);
@@ -349,7 +351,7 @@ hipError_t launch_log_rows_forward<PSIG_ROWS_TYPE>(const PSIG_ROWS_TYPE *sig, PS
 template <>
 hipError_t launch_log_rows_adjoint<PSIG_ROWS_TYPE>(const PSIG_ROWS_TYPE *lg, const PSIG_ROWS_TYPE *grad,
                                                    PSIG_ROWS_TYPE *dense, int64_t n_out, int64_t rows, int64_t d, int depth,
-                                                   const int64_t *top_words, const int64_t *picked, hipStream_t stream) {
+                                                   int64_t top_size, const int64_t *top_words, const int64_t *picked, hipStream_t stream) {
     return with_layout<PSIG_ROWS_TYPE, 2, 2>(
         d, depth,
         [&](auto dc, auto nc) {
@@ -361,7 +363,7 @@ hipError_t launch_log_rows_adjoint<PSIG_ROWS_TYPE>(const PSIG_ROWS_TYPE *lg, con
                 if (e != hipSuccess) return e;
             }
             hipLaunchKernelGGL((log_rows_adjoint_kernel<PSIG_ROWS_TYPE, D, N>), dim3((unsigned)rows), dim3(R::kThreads),
-                               bytes, stream, lg, grad, dense, (int)n_out, top_words, picked);
+                               bytes, stream, lg, grad, dense, (int)n_out, top_size, top_words, picked);
             return hipGetLastError();
         },
         hipErrorNotSupported);

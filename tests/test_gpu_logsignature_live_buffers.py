@@ -140,3 +140,35 @@ def test_calls_on_several_streams_after_a_rewrite(ps, pair):
     torch.cuda.synchronize()
     for out, grad in results:
         assert rel_err(out, want) < 1e-12 and rel_err(grad, want_grad) < 2e-12
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("pair", SHAPES, indirect=True)
+def test_columns_and_words_that_are_none(ps, pair, dtype):
+    """Wanted columns and words out of range (a damaged state_dict) are NaN and have no gradient; the others are as
+    they were."""
+    depth, first, _, path, G = pair
+    module = ps.LogSignature(depth=depth, projection=first())
+    d, columns = path.shape[2], sum(module._ext_level_sizes)
+    x, g = path.to(dtype).cuda().requires_grad_(True), G.to(dtype).cuda()
+    good = module(x)
+    assert "LogSignatureKeepDirect" in good.grad_fn.name()  # (the launches that check)
+    picked, words = module._indices_from_sig, module._top_words
+    n = picked.numel()
+    bad_columns = {0: -1, 2: columns, 3: 2 ** 40}
+    bad_words = {4: -1, 6: d ** depth, 8: 2 ** 40}  # of the outputs 5, 7 and 9
+    lost = torch.zeros(n, dtype=torch.bool, device="cuda")
+    lost[[*bad_columns, *(at + 1 for at in bad_words)]] = True
+    (want_grad,) = torch.autograd.grad(good, x, g.masked_fill(lost, 0))
+    for at, column in bad_columns.items():
+        picked[at] = column
+    for at, code in bad_words.items():
+        words[at] = code
+    with torch.no_grad():
+        plain = module(x)
+    out = module(x)
+    (grad,) = torch.autograd.grad(out, x, g)
+    assert torch.equal(out.isnan(), lost.expand_as(out)) and torch.equal(plain.isnan(), out.isnan())
+    tol = 1e-12 if dtype == torch.float64 else 1e-5
+    assert rel_err(out[:, ~lost], good[:, ~lost].detach().cpu().double()) < tol
+    assert rel_err(grad, want_grad.cpu().double()) < 2 * tol
