@@ -488,17 +488,22 @@ std::tuple<Tensor, Tensor> sig_to_logsig_keep_autograd(const Tensor &signature, 
 // autograd nodes.  Everything that is not a plain CUDA tensor in plain eager mode (subclasses, fake tensors, function
 // transforms, tracing, dispatch or torch-function modes) is left to the registered operators: the functions return
 // None and the module takes that way.  So are tensors with a forward-mode tangent, which the operators refuse.
-bool plain_call(const Tensor &path) {
+// The backward of these nodes looks at its tensors in the same way: an upstream gradient can be a batched tensor
+// (is_grads_batched), a view whose sign bit is still to be applied, or one that a mode is watching, and saved-tensor
+// hooks can hand back anything.
+bool plain(const Tensor &t) {
     using c10::DispatchKey;
-    if (!path.defined() || path.scalar_type() == at::kHalf || path._fw_grad(/*level=*/0).defined()) return false;
+    if (!t.defined() || !t.is_cuda() || t._fw_grad(/*level=*/0).defined()) return false;
     if (at::impl::torch_function_mode_enabled()) return false;
     const auto tls = c10::impl::tls_local_dispatch_key_set();
     const c10::DispatchKeySet ordinary({DispatchKey::CUDA, DispatchKey::ADInplaceOrView, DispatchKey::AutogradCUDA,
                                         DispatchKey::AutogradOther, DispatchKey::BackendSelect, DispatchKey::AutocastCUDA,
                                         DispatchKey::AutocastCPU});
-    const c10::DispatchKeySet rest = ((path.key_set() | tls.included_) - tls.excluded_) - ordinary;
-    return path.is_cuda() && (rest.raw_repr() & ~c10::full_backend_mask) == 0;
+    const c10::DispatchKeySet rest = ((t.key_set() | tls.included_) - tls.excluded_) - ordinary;
+    return (rest.raw_repr() & ~c10::full_backend_mask) == 0;
 }
+
+bool plain_call(const Tensor &path) { return plain(path) && path.scalar_type() != at::kHalf; }
 
 // the signature with its hand-over, as SignatureKeepFunction, without a second dispatch
 struct SignatureKeepDirectFunction : public torch::autograd::Function<SignatureKeepDirectFunction> {
@@ -521,8 +526,10 @@ struct SignatureKeepDirectFunction : public torch::autograd::Function<SignatureK
             const auto call = ctx->saved_data["call"].toIntVector();
             const size_t n = call.size() - 3;
             const at::IntArrayRef level_sizes(call.data(), n);
-            if (at::GradMode::is_enabled()) {
-                // a graph of the gradient is asked for: the operator says what it makes of that
+            if (at::GradMode::is_enabled() || !plain(grads[0]) || !plain(saved[0]) || !plain(saved[1]) ||
+                !plain(saved[2])) {
+                // a graph of the gradient is asked for, or the tensors are not plain: the operator says what it makes
+                // of that
                 static auto op = typed_op<SigBackwardKept>("pathsig::signature_backward_kept");
                 grad_path = op.call(saved[0], saved[1], grads[0], saved[2], call[n], call[n + 1] != 0, saved[4], level_sizes,
                                     call[n + 2] != 0, saved[3]);
@@ -583,8 +590,8 @@ std::tuple<Tensor, Tensor> log_one_forward(const LogOne &o, bool save) {
     return {out, saved};
 }
 
-// the same gradient through the operators, for a backward that meets other tuning switches than its forward did or is
-// asked for a graph of the gradient
+// the same gradient through the operators, for a backward that meets other tuning switches than its forward did, is
+// asked for a graph of the gradient or gets tensors that are not plain
 Tensor log_backward_composed(const SigCall &c, const Tensor &grad, bool alt, const Tensor &top_words,
                              at::IntArrayRef level_sizes, const Tensor &picked, bool use_windows, const Tensor &windows) {
     static auto sig_op = typed_op<SigForwardKeep>("pathsig::compute_signature_keep");
@@ -624,12 +631,13 @@ struct LogSignatureKeepDirectFunction : public torch::autograd::Function<LogSign
             const size_t n = call.size() - 3;
             const at::IntArrayRef level_sizes(call.data(), n);
             const bool alt = call[n + 1] != 0, use_windows = call[n + 2] != 0;
-            Tensor grad = grads[0].contiguous();
             LogOne o;
-            const bool one = log_one(o, saved[0], call[n], alt, saved[3], level_sizes, saved[4], use_windows, saved[2]);
+            const bool one = !at::GradMode::is_enabled() && plain(grads[0]) && plain(saved[0]) && plain(saved[1]) &&
+                             log_one(o, saved[0], call[n], alt, saved[3], level_sizes, saved[4], use_windows, saved[2]);
             c10::DeviceGuard guard(saved[0].device());
-            if (one && (size_t)saved[1].numel() == o.saved && !at::GradMode::is_enabled()) {
+            if (one && (size_t)saved[1].numel() == o.saved) {
                 const SigCall &c = o.c;
+                Tensor grad = grads[0].contiguous();
                 grad_path = at::empty_like(c.path);
                 Tensor ws = scratch(o.backward_ws, c.path);
                 check_rc(pathsig_logsignature_backward(
@@ -638,7 +646,7 @@ struct LogSignatureKeepDirectFunction : public torch::autograd::Function<LogSign
                     c.W > 0 ? (const int32_t *)ptr(c.win) : nullptr, c.W, ptr(ws), o.backward_ws, stream_of(c.path)));
             } else {
                 const SigCall c = sig_call(saved[0], call[n], alt, saved[3], level_sizes, use_windows, saved[2]);
-                grad_path = log_backward_composed(c, grad, alt, saved[3], level_sizes, saved[4], use_windows, saved[2]);
+                grad_path = log_backward_composed(c, grads[0], alt, saved[3], level_sizes, saved[4], use_windows, saved[2]);
             }
         }
         return {grad_path, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
