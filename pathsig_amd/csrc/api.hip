@@ -185,6 +185,11 @@ int launch_failed(hipError_t e, const char *what) {
     return PATHSIG_ERR_LAUNCH;
 }
 
+// bytes that the per-word forward keeps (prefix values)
+size_t words_keep_bytes(const LevelPlan &plan, int64_t rows, size_t elem) {
+    return plan.keep_size == 0 ? 0 : kept_bytes((size_t)(rows * plan.keep_size) * elem, elem, 0, Kept::values);
+}
+
 template <typename T>
 int sig_forward_t(const void *path, void *sig, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
                   const int64_t *codes, int64_t n_encoded, const int32_t *windows, int64_t W, void *keep,
@@ -198,7 +203,7 @@ int sig_forward_t(const void *path, void *sig, int64_t B, int64_t L, int64_t d, 
     rc = check_grid(plan, B * shape.W);
     if (rc != PATHSIG_OK) return rc;
     const DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
-    const size_t keep_need = dc.usable ? dc.keep_bytes : (size_t)(B * shape.W * plan.keep_size) * sizeof(T);
+    const size_t keep_need = dc.usable ? dc.keep_bytes : words_keep_bytes(plan, B * shape.W, sizeof(T));
     if (keep && (keep_need == 0 || keep_bytes < keep_need)) {
         set_error("chunk buffer: this call keeps %zu bytes, got %zu", keep_need, keep_bytes);
         return PATHSIG_ERR_ARGUMENT;
@@ -248,11 +253,10 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
     rc = check_grid(plan, B * shape.W);
     if (rc != PATHSIG_OK) return rc;
     const DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
-    const size_t keep_need = dc.usable ? dc.keep_bytes : (size_t)(B * shape.W * plan.keep_size) * sizeof(T);
+    const size_t keep_need = dc.usable ? dc.keep_bytes : words_keep_bytes(plan, B * shape.W, sizeof(T));
     // The layout of what a forward keeps follows from the choice of kernels, which the tuning switches can change
     // between the two calls.  A buffer of another size than this call would have kept comes from a forward that
-    // chose differently and is refused (every such choice keeps a different number of bytes: prefix values per
-    // word, two rows of products per chunk, or the dense signature).
+    // chose differently and is refused (kept_bytes: no two choices keep the same number of bytes).
     if (kept && (keep_need == 0 || kept_bytes != keep_need)) {
         set_error("chunk buffer: the forward of this call keeps %zu bytes, got %zu (made under other options?)", keep_need,
                   kept_bytes);
@@ -585,7 +589,12 @@ LogPlan log_plan(int dtype, int64_t B, int64_t L, int64_t d, int depth, const in
     lp.lg_at = kept;
     lp.cache_at = kept + lg;
     lp.small = elem == 8 ? log_rows_possible<double>(d, depth) : log_rows_possible<float>(d, depth);
-    lp.saved_bytes = lp.cache_at + (lp.small ? 0 : align_up((size_t)lp.rows * lp.lower * depth * elem));
+    lp.saved_bytes = kept_bytes(lp.cache_at + (lp.small ? 0 : align_up((size_t)lp.rows * lp.lower * depth * elem)), elem,
+                                lp.dc.bwd_chunks,
+                                lp.keep_rows        ? Kept::rows
+                                : !lp.keep_products ? Kept::values
+                                : lp.dc.grouped     ? Kept::groups
+                                                    : Kept::products);
     // (the dense rows of the forward are saved or scratch; what dense_choice asks for a dense buffer is not needed)
     lp.forward_bytes = (lp.keep_rows ? 0 : lp.rows_bytes) + align_up(lp.dc.forward_workspace - lp.dc.dense_bytes);
     lp.inc_bytes = inc_buffer_bytes(elem, B, L, d, false);
@@ -737,7 +746,7 @@ size_t pathsig_sig_chunks_bytes(int dtype, int64_t B, int64_t L, int64_t d, int 
     const DenseChoice dc =
         dense_choice(elem_size(dtype), d, depth, all_dense, level_sizes, B, L, W > 0 ? W : 1, W > 0);
     if (dc.usable) return dc.keep_bytes;
-    return (size_t)(B * (W > 0 ? W : 1) * plan.keep_size) * elem_size(dtype);
+    return words_keep_bytes(plan, B * (W > 0 ? W : 1), elem_size(dtype));
 }
 
 int pathsig_sig_forward(const void *path, void *sig, int dtype, int64_t B, int64_t L, int64_t d, int depth,

@@ -24,6 +24,15 @@ struct DenseChoice {
                                 // (four arrays: [rows, chunks, low] twice, then [rows, chunks / 4, low] twice)
 };
 
+// What a forward hands to its backward has a layout that the tuning switches decide (time chunks and their hand-over),
+// and they may change in between, so the size of the buffer says which it is: rounded up to 4096 elements, and an
+// element more for every (chunk count, kind).  Chunk counts go up to 1024, so no two layouts of a call share a size.
+enum class Kept { values = 0, products = 1, groups = 2, rows = 3 };  // values: of words, or none
+inline size_t kept_bytes(size_t raw, size_t elem, int chunks, Kept kind) {
+    const size_t unit = 4096 * elem;
+    return (raw + unit - 1) / unit * unit + (size_t)(chunks % 1024 * 4 + (int)kind) * elem;
+}
+
 DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes, int64_t B,
                          int64_t L, int64_t W, bool windowed);
 

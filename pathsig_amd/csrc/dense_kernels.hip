@@ -2886,8 +2886,9 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
             dc.grouped = elem == 4 && v.grouped_ok && !dc.embed && chunks % 4 == 0 && chunks >= 8 &&
                          options().grouped != 0;
             if (dc.grouped) dc.keep_bytes += 2 * pad256((size_t)rows * (chunks / 4) * v.low_size * elem);
+            dc.keep_bytes = kept_bytes(dc.keep_bytes, elem, chunks, dc.grouped ? Kept::groups : Kept::products);
         }
-        if (dc.resweep) dc.keep_bytes = (size_t)rows * v.sig_size * elem;
+        if (dc.resweep) dc.keep_bytes = kept_bytes((size_t)rows * v.sig_size * elem, elem, 1, Kept::rows);
         return dc;
     }
     return dc;
