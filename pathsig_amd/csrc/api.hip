@@ -185,9 +185,13 @@ int launch_failed(hipError_t e, const char *what) {
     return PATHSIG_ERR_LAUNCH;
 }
 
-// bytes that the per-word forward keeps (prefix values)
-size_t words_keep_bytes(const LevelPlan &plan, int64_t rows, size_t elem) {
-    return plan.keep_size == 0 ? 0 : kept_bytes((size_t)(rows * plan.keep_size) * elem, elem, 0, Kept::values);
+// bytes that the per-word forward keeps (prefix values): not as many as the dense rows that the same call may keep
+size_t words_keep_bytes(const LevelPlan &plan, int64_t rows, int64_t d, size_t elem) {
+    if (plan.keep_size == 0) return 0;
+    const size_t bytes = kept_bytes((size_t)(rows * plan.keep_size) * elem, elem, 0, Kept::values);
+    double dense = 0;
+    for (int k = plan.depth; k >= 1; --k) dense = (dense + 1.0) * (double)d;
+    return (double)bytes == dense * (double)rows * (double)elem ? bytes + 4096 * elem : bytes;
 }
 
 template <typename T>
@@ -203,7 +207,7 @@ int sig_forward_t(const void *path, void *sig, int64_t B, int64_t L, int64_t d, 
     rc = check_grid(plan, B * shape.W);
     if (rc != PATHSIG_OK) return rc;
     const DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
-    const size_t keep_need = dc.usable ? dc.keep_bytes : words_keep_bytes(plan, B * shape.W, sizeof(T));
+    const size_t keep_need = dc.usable ? dc.keep_bytes : words_keep_bytes(plan, B * shape.W, d, sizeof(T));
     if (keep && (keep_need == 0 || keep_bytes < keep_need)) {
         set_error("chunk buffer: this call keeps %zu bytes, got %zu", keep_need, keep_bytes);
         return PATHSIG_ERR_ARGUMENT;
@@ -253,7 +257,7 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
     rc = check_grid(plan, B * shape.W);
     if (rc != PATHSIG_OK) return rc;
     const DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
-    const size_t keep_need = dc.usable ? dc.keep_bytes : words_keep_bytes(plan, B * shape.W, sizeof(T));
+    const size_t keep_need = dc.usable ? dc.keep_bytes : words_keep_bytes(plan, B * shape.W, d, sizeof(T));
     // The layout of what a forward keeps follows from the choice of kernels, which the tuning switches can change
     // between the two calls.  A buffer of another size than this call would have kept comes from a forward that
     // chose differently and is refused (kept_bytes: no two choices keep the same number of bytes).
@@ -746,7 +750,7 @@ size_t pathsig_sig_chunks_bytes(int dtype, int64_t B, int64_t L, int64_t d, int 
     const DenseChoice dc =
         dense_choice(elem_size(dtype), d, depth, all_dense, level_sizes, B, L, W > 0 ? W : 1, W > 0);
     if (dc.usable) return dc.keep_bytes;
-    return words_keep_bytes(plan, B * (W > 0 ? W : 1), elem_size(dtype));
+    return words_keep_bytes(plan, B * (W > 0 ? W : 1), d, elem_size(dtype));
 }
 
 int pathsig_sig_forward(const void *path, void *sig, int dtype, int64_t B, int64_t L, int64_t d, int depth,

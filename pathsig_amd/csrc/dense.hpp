@@ -27,6 +27,7 @@ struct DenseChoice {
 // What a forward hands to its backward has a layout that the tuning switches decide (time chunks and their hand-over),
 // and they may change in between, so the size of the buffer says which it is: rounded up to 4096 elements, and an
 // element more for every (chunk count, kind).  Chunk counts go up to 1024, so no two layouts of a call share a size.
+// (rows: of the log-signature in one call; the dense rows of a projection are a buffer of exactly their size.)
 enum class Kept { values = 0, products = 1, groups = 2, rows = 3 };  // values: of words, or none
 inline size_t kept_bytes(size_t raw, size_t elem, int chunks, Kept kind) {
     const size_t unit = 4096 * elem;

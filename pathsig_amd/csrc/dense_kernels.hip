@@ -2888,7 +2888,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
             if (dc.grouped) dc.keep_bytes += 2 * pad256((size_t)rows * (chunks / 4) * v.low_size * elem);
             dc.keep_bytes = kept_bytes(dc.keep_bytes, elem, chunks, dc.grouped ? Kept::groups : Kept::products);
         }
-        if (dc.resweep) dc.keep_bytes = kept_bytes((size_t)rows * v.sig_size * elem, elem, 1, Kept::rows);
+        if (dc.resweep) dc.keep_bytes = (size_t)rows * v.sig_size * elem;  // (such a shape has no time chunks to tell apart)
         return dc;
     }
     return dc;
