@@ -859,7 +859,10 @@ int pathsig_sig_backward_noalloc(const void *path, const void *sig, const void *
                                  void *stream) {
     int rc = check_common(dtype, B, L, d, depth);
     if (rc != PATHSIG_OK) return rc;
-    const size_t need = pathsig_sig_backward_workspace(dtype, B, L, d, depth, level_sizes, windows ? W : 0);
+    size_t need = pathsig_sig_backward_workspace(dtype, B, L, d, depth, level_sizes, windows ? W : 0);
+    // (the launches for long chains of chunks take scratch for speed: a call that fits without them goes without)
+    const PlainChunks plain(need > (size_t)PATHSIG_STATIC_SCRATCH_BYTES);
+    if (plain.active()) need = pathsig_sig_backward_workspace(dtype, B, L, d, depth, level_sizes, windows ? W : 0);
     if (need > (size_t)PATHSIG_STATIC_SCRATCH_BYTES) {
         set_error("this call needs %zu bytes of scratch; the static buffer of pathsig_sig_backward_noalloc holds %zu "
                   "(use pathsig_sig_backward with a workspace of your own)", need, (size_t)PATHSIG_STATIC_SCRATCH_BYTES);

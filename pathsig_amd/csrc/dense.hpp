@@ -13,7 +13,6 @@ struct DenseChoice {
                                 // signature, which the forward keeps or the backward computes again
     int variant;                // index into the table of compiled shapes
     int fwd_chunks;             // time chunks per (path, window) in the forward
-    bool chains;                // the products of the chunks may use the launches for long chains of them
     int bwd_chunks;             // ... and in the backward (at least 2 when embedding: no dense signature is saved)
     size_t dense_bytes;         // embed: bytes of one dense [rows, S] buffer
     size_t forward_workspace;   // bytes of scratch the forward needs (including the dense buffer)
@@ -22,6 +21,22 @@ struct DenseChoice {
                                 // chunk signatures below the top level, or (resweep) the dense signature (0: none)
     bool grouped;               // the kept products are those within groups of four chunks plus those of whole groups
                                 // (four arrays: [rows, chunks, low] twice, then [rows, chunks / 4, low] twice)
+    // the launches for long chains of chunks (chain_kernels.hip), whose scratch the workspaces hold where they are taken
+    bool chain_scan;            // products of the chunks to the left and to the right of every chunk
+    bool chain_groups;          // grouped: those of the groups, and the top level of the row as a sum over the groups
+    bool chain_top;             // not grouped: the top level of the row as a sum over the partial signatures
+    bool forward_chains;        // any of them in the forward
+};
+
+// While one that is on lives, the choices made on its thread take at most 64 chunks to a row and no launches for long
+// chains of them, and need none of their scratch.
+class PlainChunks {
+public:
+    explicit PlainChunks(bool on);
+    ~PlainChunks();
+    PlainChunks(const PlainChunks &) = delete;
+    PlainChunks &operator=(const PlainChunks &) = delete;
+    static bool active();
 };
 
 // What a forward hands to its backward has a layout that the tuning switches decide (time chunks and their hand-over),

@@ -2297,6 +2297,7 @@ struct VariantInfo {
     bool chunks_ok[2];    // fp32, fp64: rows can be cut into time chunks
     bool fp64_fits;       // a lane's state fits the register file in fp64 too (else a later entry of the shape serves fp64)
     bool grouped_ok;      // fp32: the hand-over of chunk products by groups of four chunks is compiled
+    int group_sizes[2];   // fp32, fp64: see group_sizes()
 };
 
 // Grouped hand-over (fp32): the forward sweep, four chunks to a block, leaves the products of every chunk with its
@@ -2317,6 +2318,18 @@ constexpr bool grouped_handover_ok() {
     }
 }
 
+template <typename T, int D, int N, int P, int GW>
+constexpr bool group_fits() {
+    return Geometry<D, N, P, sizeof(T)>::kBlock * GW <= 1024 && forward_lds_bytes<D, N, P, GW, T>() <= 64 * 1024;
+}
+
+// numbers of chunks (2 and 4 as bits) that the forward sweep can put into one block
+template <typename T, int D, int N, int P>
+constexpr int group_sizes() {
+    if constexpr (Geometry<D, N, P, sizeof(T)>::kOnePiece) return 0;
+    else return (group_fits<T, D, N, P, 4>() ? 4 : 0) | (group_fits<T, D, N, P, 2>() ? 2 : 0);
+}
+
 template <int D, int N, int P, int PC, int PS>
 constexpr VariantInfo variant_info() {
     using G = Geometry<D, N, P>;
@@ -2326,7 +2339,8 @@ constexpr VariantInfo variant_info() {
                        {!G::kOnePiece && scan_fits<float, D, N, PS>(),
                         !G64::kOnePiece && scan_fits<double, D, N, PS>()},
                        G::kSplit || trie_size(D, N - P) <= 132,
-                       grouped_handover_ok<D, N, P, PC, PS>()};
+                       grouped_handover_ok<D, N, P, PC, PS>(),
+                       {group_sizes<float, D, N, P>(), group_sizes<double, D, N, P>()}};
 }
 
 constexpr size_t kBoundsBytes = 256;  // scratch for the letter bounds (16 ints, padded)
@@ -2363,7 +2377,7 @@ constexpr bool shape_enabled(int, int) { return true; }
 template <int D, int N, int P, int PC, int PS>
 constexpr VariantInfo variant_info_if_enabled() {
     if constexpr (shape_enabled(D, N)) return variant_info<D, N, P, PC, PS>();
-    else return VariantInfo{-1, -1, 0, 0, 0, 0, 0, false, {false, false}, false, false};
+    else return VariantInfo{-1, -1, 0, 0, 0, 0, 0, false, {false, false}, false, false, {0, 0}};
 }
 
 #define PSIG_INFO(I, D, N, P, PC, PS) variant_info_if_enabled<D, N, P, PC, PS>(),
@@ -2410,34 +2424,26 @@ int pick_chunks(int64_t rows, int block, int64_t L, int64_t want_waves, bool man
 // one product after the other beyond this length.
 constexpr int64_t kChainsUpToSteps = 4096;
 
-#endif
-
 // Estimates of the launches that multiply one chunk after the other.  A product of a scan over 64 chunks took 0.14 us
 // at depth 2, 0.35 at depth 3 and 4, 0.3 (rows of 100 bytes) to 0.85 (19 kB) at depth 5, 0.7 at depth 6; of a combine about as much when it stages
 // its rows in LDS, else what it takes to load a row at addresses of the lane's own ((6, 5) 2.1, (4, 6) in fp64 1.7,
 // (7, 5) in fp64 3.7 us).
-inline double scan_us(int n, int depth, double row_bytes) {
+double scan_us(int n, int depth, double row_bytes) {
     return 2.0 + (0.02 + 0.11 * depth + 1.5e-5 * row_bytes) * (n - 1);
 }
-template <typename T>
-double combine_us(int n, int depth, int64_t sig_size, bool staged) {
-    return staged ? scan_us(n, depth, 0) : 2.0 + (n - 1) * (0.8 + 0.02e-3 * (double)sig_size * sizeof(T));
+double combine_us(size_t elem, int n, int depth, int64_t sig_size, bool staged) {
+    return staged ? scan_us(n, depth, 0) : 2.0 + (n - 1) * (0.8 + 0.02e-3 * (double)(sig_size * elem));
 }
 
-template <typename T, int D, int N, int P, int GW>
-constexpr bool group_fits() {
-    return Geometry<D, N, P, sizeof(T)>::kBlock * GW <= 1024 && forward_lds_bytes<D, N, P, GW, T>() <= 64 * 1024;
-}
-
+#endif
 
 // Prefix products edgeA and (unless null) suffix products edgeZ of the chunk signatures below the top level (dense_scan_kernel).
-// chains: long chains of chunks may take the launches of chain_kernels.hip, with `temp` for their scratch.
+// chain: by the launches of chain_kernels.hip, with `temp` for their scratch.
 template <typename T, int D, int N, int PS>
-hipError_t launch_scan(const T *chunk_low, T *edgeA, T *edgeZ, int64_t rows, int chunks, T *temp, bool chains,
+hipError_t launch_scan(const T *chunk_low, T *edgeA, T *edgeZ, int64_t rows, int chunks, T *temp, bool chain,
                        hipStream_t stream) {
     using GC = Geometry<D, N, PS>;
-    // (whether or not the second direction is asked for: a forward returns the same bits with and without it)
-    if (chains && chain_us(sizeof(T), rows, chunks, D, N, 2) < scan_us(chunks, N, GC::kLowSize * sizeof(T)))
+    if (chain)
         return launch_chain<T>(chunk_low, GC::kLowSize, rows, chunks, D, N, edgeA, true, edgeZ, (T *)nullptr, 0, temp,
                                rows * chunks * GC::kLowSize, stream);
     // all chunk rows of a row go to LDS at once when they fit (a little under the 160 KB of a CU)
@@ -2463,13 +2469,14 @@ hipError_t launch_scan(const T *chunk_low, T *edgeA, T *edgeZ, int64_t rows, int
 // time-chunked backward of the same call starts its chunks from: [rows, chunks, low] twice, the second array
 // pad256 bytes after the start of the first.
 template <typename T, int D, int N, int P, int PC, int PS>
-hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks, const int *bounds, T *keep,
-                       void *workspace, hipStream_t stream, bool grouped, bool chains) {
+hipError_t run_forward(const T *path, T *sig, const SigShape &shape, const DenseChoice &dc, const int *bounds, T *keep,
+                       void *workspace, hipStream_t stream) {
     using G = Geometry<D, N, P, sizeof(T)>;
     using GC = Geometry<D, N, PC>;
     constexpr bool kStaged = 2 * GC::kSigSize * sizeof(T) <= 48 * 1024;
     constexpr bool kBoundsOk = LetterBounds<D, P>::kUsable && !G::kOnePiece;
     const int64_t rows = shape.B * shape.W;
+    const int chunks = dc.fwd_chunks;
     if (bounds && !kBoundsOk) return hipErrorInvalidValue;
     if (chunks <= 1) {
         if constexpr (kBoundsOk) {
@@ -2491,28 +2498,13 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
     T *chunk_sig = (T *)workspace;
     // the chunks' own signatures below the top level, from which the products for the backward are made
     T *const low_space = (T *)((unsigned char *)workspace + pad256((size_t)rows * chunks * G::kSigSize * sizeof(T)));
-    T *chunk_low = keep ? low_space : (T *)nullptr;
-    // scratch of a long chain of products (present when chain_possible says so for the chunks)
+    T *chunk_low = keep || dc.chain_top ? low_space : (T *)nullptr;
+    // scratch of a long chain of products (two arrays of low_elems, there where dc.forward_chains)
     const int64_t low_elems = rows * chunks * G::kLowSize;
     T *const chain_temp = (T *)((unsigned char *)low_space + pad256((size_t)low_elems * sizeof(T)));
-    const int gw = bounds ? 1
-                   : (group_fits<T, D, N, P, 4>() && chunks % 4 == 0) ? 4
-                   : (group_fits<T, D, N, P, 2>() && chunks % 2 == 0) ? 2 : 1;
-    bool top_sums = false;  // see below
-    if constexpr (scan_fits<T, D, N, PS>()) {
-        const double left_us =
-            std::min(scan_us(chunks, N, G::kLowSize * sizeof(T)), chain_us(sizeof(T), rows, chunks, D, N, 2));
-        top_sums = chains && chunks > gw && chain_top_us(sizeof(T), rows, chunks / gw, D, N) + 0.25 * left_us <
-                                                combine_us<T>(chunks / gw, N, G::kSigSize, kStaged);
-    }
     if constexpr (sizeof(T) == 4 && grouped_handover_ok<D, N, P, PC, PS>()) {
         const int groups4 = chunks / 4;
-        const bool in_groups = grouped && !bounds && chunks % 4 == 0 && chunks >= 8;
-        const bool in_chain = in_groups && chains &&
-                              chain_us(sizeof(T), rows, groups4, D, N, 2) + chain_top_us(sizeof(T), rows, groups4, D, N) <
-                                  scan_us(groups4, N, 0);
-        if (in_groups) top_sums = false;
-        if (in_groups && (keep || in_chain)) {
+        if (dc.grouped && (keep || dc.chain_groups)) {
             // grouped hand-over: keep = [in-group prefix products][in-group suffix products], both
             // [rows, chunks, low], then [products of the groups to the left][.. to the right], both
             // [rows, chunks / 4, low]
@@ -2528,7 +2520,7 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
                                (const int *)nullptr, keep, in_suffix);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
-            if (in_chain) {
+            if (dc.chain_groups) {
                 e = launch_chain<T>((const T *)chunk_sig, G::kSigSize, rows, groups4, D, N, edgeL, false, edgeR, sig,
                                     G::kSigSize, low_space, rows * groups4 * G::kLowSize, stream);
                 if (e != hipSuccess) return e;
@@ -2545,7 +2537,6 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
             return hipGetLastError();
         }
     }
-    if (top_sums) chunk_low = low_space;
     int groups = chunks;
     if constexpr (kBoundsOk) {
         if (bounds) {
@@ -2586,13 +2577,14 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (groups < 0) groups = chunks;
-    if (top_sums) {
+    if (dc.chain_top) {
         // The products left of every chunk give the top level as a sum over the partial signatures; they are made for a
         // backward anyway.
         if constexpr (scan_fits<T, D, N, PS>()) {
             T *edgeA = keep ? keep : chain_temp + low_elems;
             T *edgeZ = keep ? (T *)((unsigned char *)keep + pad256((size_t)low_elems * sizeof(T))) : (T *)nullptr;
-            e = launch_scan<T, D, N, PS>((const T *)chunk_low, edgeA, edgeZ, rows, chunks, chain_temp, true, stream);
+            e = launch_scan<T, D, N, PS>((const T *)chunk_low, edgeA, edgeZ, rows, chunks, chain_temp, dc.chain_scan,
+                                        stream);
             if (e != hipSuccess) return e;
             return launch_chain_top<T>((const T *)chunk_sig, G::kSigSize,
                                        ChainLeft<T>{edgeA, chunks, chunks / groups, -1, true}, sig, G::kSigSize, rows,
@@ -2622,7 +2614,7 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
                     return hipGetLastError();
                 }
             }
-            e = launch_scan<T, D, N, PS>((const T *)chunk_low, keep, edgeZ, rows, chunks, chain_temp, chains,
+            e = launch_scan<T, D, N, PS>((const T *)chunk_low, keep, edgeZ, rows, chunks, chain_temp, dc.chain_scan,
                                          stream);
             if (e != hipSuccess) return e;
         } else {
@@ -2642,12 +2634,13 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, int chunks,
 
 template <typename T, int D, int N, int P, int PC, int PS>
 hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_inc, T *grad_path, bool *wrote_path,
-                        const SigShape &shape, int chunks, const int *bounds, const T *kept, void *workspace,
-                        hipStream_t stream, bool grouped, bool chains, bool inc_cleared) {
+                        const SigShape &shape, const DenseChoice &dc, const int *bounds, const T *kept, void *workspace,
+                        hipStream_t stream, bool inc_cleared) {
     using G = Geometry<D, N, P, sizeof(T)>;
     using GC = Geometry<D, N, PS>;
     constexpr bool kBoundsOk = LetterBounds<D, P>::kUsable && !G::kOnePiece;
     const int64_t rows = shape.B * shape.W;
+    const int chunks = dc.bwd_chunks;
     // per-increment sums are added in memory for overlapping windows and for units spread over several blocks
     // (among them the letter blocks of a sweep with letter bounds)
     const bool accumulate =
@@ -2691,7 +2684,7 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
             dumpA = kept;
             dumpH = (const T *)((const unsigned char *)kept + edge_bytes);
             if constexpr (sizeof(T) == 4 && grouped_handover_ok<D, N, P, PC, PS>()) {
-                if (grouped && !bounds && chunks % 4 == 0 && chunks >= 8) {
+                if (dc.grouped) {
                     const size_t group_bytes = pad256((size_t)rows * (chunks / 4) * G::kLowSize * sizeof(T));
                     edgeL = (const T *)((const unsigned char *)kept + 2 * edge_bytes);
                     edgeR = (const T *)((const unsigned char *)kept + 2 * edge_bytes + group_bytes);
@@ -2715,7 +2708,7 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
             e = hipGetLastError();
             if (e != hipSuccess) return e;
             e = launch_scan<T, D, N, PS>((const T *)chunk_low, edgeA, edgeZ, rows, chunks, (T *)(ws + 3 * edge_bytes),
-                                         chains, stream);
+                                         dc.chain_scan, stream);
             if (e != hipSuccess) return e;
             dumpA = edgeA;
             dumpH = edgeZ;
@@ -2777,7 +2770,7 @@ float profile_sweep_ms() {
 }
 
 static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes,
-                                     int64_t B, int64_t L, int64_t W) {
+                                     int64_t B, int64_t L, int64_t W, bool plain) {
     DenseChoice dc{};
     dc.variant = -1;
     dc.fwd_chunks = dc.bwd_chunks = 1;
@@ -2838,7 +2831,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         // in fp64
         const double step_us = (0.2 + 0.013 * v.sub_size) * (elem == 8 ? 2.0 : 1.0);
         const double low_bytes = (double)v.low_size * elem;
-        const bool may_chain = elem == 8 || L - 1 <= kChainsUpToSteps;
+        const bool may_chain = !plain && (elem == 8 || L - 1 <= kChainsUpToSteps);
         bool many = false;  // more than 64 chunks
         if (chunks_ok && L - 1 > 2048) {
             // what the shorter sweeps save against what the longer chains of products cost
@@ -2861,7 +2854,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         // A step of training whose launches take less than the 60 us that autograd takes to get through its own
         // forward and backward gains nothing from shorter ones, and the chains are three to five launches more.
         // (The values a call returns do not depend on whether it keeps anything for a backward, so neither may this.)
-        dc.chains = may_chain && (double)(L - 1) / chunks * step_us + 8.0 + 1.3 * scan_us(chunks, depth, low_bytes) > 55.0;
+        const bool chains = may_chain && chunks > 1 && (double)(L - 1) / chunks * step_us + 8.0 + 1.3 * scan_us(chunks, depth, low_bytes) > 55.0;
         if (rows * (chunks + 1) >= (int64_t(1) << 31)) return dc;
         dc.usable = true;
         dc.variant = i;
@@ -2869,16 +2862,6 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         dc.bwd_chunks = (dc.embed && !dc.resweep && chunks < 2) ? 2 : chunks;
         dc.forward_workspace = dc.dense_bytes + (dc.bounded ? kBoundsBytes : 0);
         dc.backward_workspace = (dc.resweep ? 2 : 1) * dc.dense_bytes + (dc.bounded ? kBoundsBytes : 0);
-        // forward: the chunk signatures, and those below the top level from which a keeping forward makes the
-        // products its backward starts from; backward: the latter and the two arrays of products
-        // (long chains of products take two more such arrays)
-        if (dc.fwd_chunks > 1)
-            dc.forward_workspace += pad256((size_t)rows * dc.fwd_chunks * v.sig_size * elem) +
-                                    (chain_possible(rows, dc.fwd_chunks, d, depth) ? 3 : 1) *
-                                        pad256((size_t)rows * dc.fwd_chunks * v.low_size * elem);
-        if (dc.bwd_chunks > 1)
-            dc.backward_workspace += (chain_possible(rows, dc.bwd_chunks, d, depth) ? 5 : 3) *
-                                     pad256((size_t)rows * dc.bwd_chunks * v.low_size * elem);
         // the forward can hand those products to the backward when both cut the rows the same way
         if (dc.bwd_chunks > 1 && dc.fwd_chunks == dc.bwd_chunks) {
             dc.keep_bytes = 2 * pad256((size_t)rows * dc.bwd_chunks * v.low_size * elem);
@@ -2888,18 +2871,53 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
             if (dc.grouped) dc.keep_bytes += 2 * pad256((size_t)rows * (chunks / 4) * v.low_size * elem);
             dc.keep_bytes = kept_bytes(dc.keep_bytes, elem, chunks, dc.grouped ? Kept::groups : Kept::products);
         }
+        if (chains) {
+            // (whether or not the backward asks for the second direction: a forward returns the same bits with and
+            // without a hand-over)
+            const double chain = chain_us(elem, rows, chunks, d, depth, 2), scan = scan_us(chunks, depth, low_bytes);
+            dc.chain_scan = chain < scan;
+            if (dc.grouped) {
+                const int groups = chunks / 4;
+                dc.chain_groups = chain_us(elem, rows, groups, d, depth, 2) + chain_top_us(elem, rows, groups, d, depth) <
+                                  scan_us(groups, depth, 0);
+            } else {
+                const int most = dc.bounded ? 0 : v.group_sizes[elem == 8 ? 1 : 0];
+                const int in_block = (most & 4) && chunks % 4 == 0 ? 4 : (most & 2) && chunks % 2 == 0 ? 2 : 1;
+                const bool staged = 2 * (size_t)v.sig_size * elem <= 48 * 1024;  // (run_forward: kStaged)
+                dc.chain_top = chunks > in_block &&
+                               chain_top_us(elem, rows, chunks / in_block, d, depth) + 0.25 * std::min(scan, chain) <
+                                   combine_us(elem, chunks / in_block, depth, v.sig_size, staged);
+            }
+        }
+        dc.forward_chains = dc.grouped ? dc.chain_groups : dc.chain_scan || dc.chain_top;
+        // forward: the chunk signatures, and those below the top level from which a keeping forward makes the
+        // products its backward starts from; backward: the latter and the two arrays of products.  Where the launches
+        // of long chains are taken they need two more such arrays.
+        if (dc.fwd_chunks > 1)
+            dc.forward_workspace += pad256((size_t)rows * dc.fwd_chunks * v.sig_size * elem) +
+                                    (dc.forward_chains ? 3 : 1) * pad256((size_t)rows * dc.fwd_chunks * v.low_size * elem);
+        if (dc.bwd_chunks > 1)
+            dc.backward_workspace += (dc.chain_scan ? 5 : 3) * pad256((size_t)rows * dc.bwd_chunks * v.low_size * elem);
         if (dc.resweep) dc.keep_bytes = (size_t)rows * v.sig_size * elem;  // (such a shape has no time chunks to tell apart)
         return dc;
     }
     return dc;
 }
 
+static bool &plain_chunks() {
+    thread_local bool on = false;
+    return on;
+}
+PlainChunks::PlainChunks(bool on) { plain_chunks() = on; }
+PlainChunks::~PlainChunks() { plain_chunks() = false; }
+bool PlainChunks::active() { return plain_chunks(); }
+
 // A step of training asks for the same choice seven times (sizes of buffers, then the launches), and a small call is
 // bound by its host time: the last few choices of a thread are remembered.
 DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes, int64_t B,
                          int64_t L, int64_t W, bool) {
     struct Key {
-        int64_t elem, d, depth, all_dense, B, L, W, options, sizes[kMaxDepth];
+        int64_t elem, d, depth, all_dense, B, L, W, plain, options, sizes[kMaxDepth];
     };
     constexpr int kRemembered = 8;
     thread_local Key keys[kRemembered];
@@ -2914,11 +2932,12 @@ DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, cons
     key.B = B;
     key.L = L;
     key.W = W;
+    key.plain = PlainChunks::active();
     key.options = options_epoch();
     if (!all_dense && level_sizes) std::memcpy(key.sizes, level_sizes + 1, (size_t)depth * sizeof(int64_t));
     for (unsigned i = 0; i < used; ++i)
         if (!std::memcmp(&keys[i], &key, sizeof key)) return choices[i];
-    const DenseChoice dc = make_dense_choice(elem, d, depth, all_dense, level_sizes, B, L, W);
+    const DenseChoice dc = make_dense_choice(elem, d, depth, all_dense, level_sizes, B, L, W, key.plain != 0);
     keys[next] = key;
     choices[next] = dc;
     next = (next + 1) % kRemembered;
@@ -3007,16 +3026,13 @@ static_assert(PSIG_GROUP < kDenseGroups, "group index out of range");
 #define PSIG_CASE_FWD(I, D, N, P, PC, PS)                                                                         \
     case I:                                                                                                       \
         if constexpr (I % kDenseGroups == PSIG_GROUP && shape_enabled(D, N))                                      \
-            return run_forward<T, D, N, P, PC, PS>(path, sig, shape, dc.fwd_chunks,                               \
-                                                   bounds, keep, workspace, stream, dc.grouped,                   \
-                                                   dc.chains);                                                    \
+            return run_forward<T, D, N, P, PC, PS>(path, sig, shape, dc, bounds, keep, workspace, stream);        \
         break;
 #define PSIG_CASE_BWD(I, D, N, P, PC, PS)                                                                          \
     case I:                                                                                                        \
         if constexpr (I % kDenseGroups == PSIG_GROUP && shape_enabled(D, N))                                       \
             return run_backward<T, D, N, P, PC, PS>(path, sig, grad_sig, grad_inc, grad_path, wrote_path, shape,   \
-                                                    dc.bwd_chunks, bounds, kept, workspace, stream, dc.grouped,    \
-                                                    dc.chains, inc_cleared);                                                  \
+                                                    dc, bounds, kept, workspace, stream, inc_cleared);             \
         break;
 
 template <int GROUP, typename T>

@@ -1,0 +1,36 @@
+"""Scratch of the launches for long chains of time chunks: asked for where they are taken, and never at the price of a call
+that the allocation-free backward can serve without them."""
+import pytest
+import torch
+
+from .helpers import rel_err
+from .test_zz_no_alloc import STATIC_BYTES, TOL, _both
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from pathsig_amd import _load
+    return _load.lib()
+
+
+# Sixteen chunks, whose products take one launch: the increment sums and three arrays of [rows, chunks, 1364] values.
+@pytest.mark.parametrize("B", [128, 160])
+def test_no_scratch_for_launches_that_are_not_made(lib, B):
+    L, d, depth, low = 1024, 4, 6, 1364
+    chunks = lib.pathsig_sig_forward_workspace(0, B, L, d, depth, None, 0) // (B * 4 * (low + 4 ** 6 + low))
+    assert chunks == 16
+    need = lib.pathsig_sig_backward_workspace(0, B, L, d, depth, None, 0)
+    assert need <= B * (L - 1) * d * 4 + 3 * B * chunks * low * 4 + 4 * 256
+    assert need < STATIC_BYTES
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,B,L,beyond", [(torch.float32, 160, 1024, False), (torch.float64, 8, 6000, True),
+                                              (torch.float64, 4, 12001, True)])
+def test_allocation_free_backward_goes_without_the_chains(lib, dtype, B, L, beyond):
+    rc, need, got, want = _both(lib, dtype, B, L, 4, 6)
+    assert (need > STATIC_BYTES) == beyond  # what the call takes with a workspace of its own
+    assert rc == 0, lib.pathsig_last_error()
+    assert rel_err(got, want) < TOL[dtype]
+    # (the choice ends with the call)
+    assert lib.pathsig_sig_backward_workspace(0 if dtype == torch.float32 else 1, B, L, 4, 6, None, 0) == need
