@@ -185,13 +185,20 @@ int launch_failed(hipError_t e, const char *what) {
     return PATHSIG_ERR_LAUNCH;
 }
 
-// bytes that the per-word forward keeps (prefix values): not as many as the dense rows that the same call may keep
+// Bytes that the per-word forward keeps (prefix values).  Under other tuning switches the same call keeps whole arrays
+// [rows, levels below the top] or dense rows (DenseChoice::keep_bytes): one or two elements more where the size would be
+// one of those.
 size_t words_keep_bytes(const LevelPlan &plan, int64_t rows, int64_t d, size_t elem) {
-    if (plan.keep_size == 0) return 0;
-    const size_t bytes = kept_bytes((size_t)(rows * plan.keep_size) * elem, elem, 0, Kept::values);
-    double dense = 0;
-    for (int k = plan.depth; k >= 1; --k) dense = (dense + 1.0) * (double)d;
-    return (double)bytes == dense * (double)rows * (double)elem ? bytes + 4096 * elem : bytes;
+    if (plan.keep_size == 0 || rows == 0) return 0;
+    uint64_t low = 0, top = 1;  // (modulo 2^64 where no shape is compiled)
+    for (int k = 1; k <= plan.depth; ++k) {
+        if (k > 1) low += top;
+        top *= (uint64_t)d;
+    }
+    const uint64_t unit = (uint64_t)rows * low, dense = unit + (uint64_t)rows * top;
+    uint64_t count = (uint64_t)(rows * plan.keep_size);
+    while (unit > 1 && (count % unit == 0 || count == dense)) ++count;
+    return (size_t)count * elem;
 }
 
 template <typename T>
@@ -260,7 +267,7 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
     const size_t keep_need = dc.usable ? dc.keep_bytes : words_keep_bytes(plan, B * shape.W, d, sizeof(T));
     // The layout of what a forward keeps follows from the choice of kernels, which the tuning switches can change
     // between the two calls.  A buffer of another size than this call would have kept comes from a forward that
-    // chose differently and is refused (kept_bytes: no two choices keep the same number of bytes).
+    // chose differently and is refused (no two choices keep the same number of bytes).
     if (kept && (keep_need == 0 || kept_bytes != keep_need)) {
         set_error("chunk buffer: the forward of this call keeps %zu bytes, got %zu (made under other options?)", keep_need,
                   kept_bytes);
@@ -550,6 +557,14 @@ int check_logsig(int dtype, int64_t rows, int64_t d, int depth, int64_t top_size
 // that follows from the lists of words and columns (letter bounds, places in the dense rows) is worked out by the
 // launches of each call: the lists are device memory that may be rewritten between two calls, or between two replays
 // of a captured graph.
+// What the forward saves has a layout that the tuning switches decide (time chunks and their hand-over), and they may
+// change before the backward, so the size of the buffer says which it is: rounded up to 4096 elements, and an element
+// more for every (chunk count, kind).  Chunk counts go up to 1024, so no two layouts of a call share a size.
+enum class Saved { values = 0, products = 1, groups = 2, rows = 3 };  // beside the log-signature; values: nothing
+size_t tagged_bytes(size_t raw, size_t elem, int chunks, Saved kind) {
+    return align_up(raw, 4096 * elem) + (size_t)(chunks % 1024 * 4 + (int)kind) * elem;
+}
+
 struct LogPlan {
     bool usable;
     DenseChoice dc;      // with the number of backward chunks of this call
@@ -593,12 +608,12 @@ LogPlan log_plan(int dtype, int64_t B, int64_t L, int64_t d, int depth, const in
     lp.lg_at = kept;
     lp.cache_at = kept + lg;
     lp.small = elem == 8 ? log_rows_possible<double>(d, depth) : log_rows_possible<float>(d, depth);
-    lp.saved_bytes = kept_bytes(lp.cache_at + (lp.small ? 0 : align_up((size_t)lp.rows * lp.lower * depth * elem)), elem,
-                                lp.dc.bwd_chunks,
-                                lp.keep_rows        ? Kept::rows
-                                : !lp.keep_products ? Kept::values
-                                : lp.dc.grouped     ? Kept::groups
-                                                    : Kept::products);
+    lp.saved_bytes = tagged_bytes(lp.cache_at + (lp.small ? 0 : align_up((size_t)lp.rows * lp.lower * depth * elem)), elem,
+                                  lp.dc.bwd_chunks,
+                                  lp.keep_rows        ? Saved::rows
+                                  : !lp.keep_products ? Saved::values
+                                  : lp.dc.grouped     ? Saved::groups
+                                                      : Saved::products);
     // (the dense rows of the forward are saved or scratch; what dense_choice asks for a dense buffer is not needed)
     lp.forward_bytes = (lp.keep_rows ? 0 : lp.rows_bytes) + align_up(lp.dc.forward_workspace - lp.dc.dense_bytes);
     lp.inc_bytes = inc_buffer_bytes(elem, B, L, d, false);

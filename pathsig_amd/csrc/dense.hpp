@@ -18,7 +18,9 @@ struct DenseChoice {
     size_t forward_workspace;   // bytes of scratch the forward needs (including the dense buffer)
     size_t backward_workspace;  // bytes of scratch the backward needs beyond the increment accumulator
     size_t keep_bytes;          // bytes the forward can keep for the backward: the prefix and suffix products of the
-                                // chunk signatures below the top level, or (resweep) the dense signature (0: none)
+                                // chunk signatures below the top level, or (resweep) the dense signature (0: none).
+                                // The layout follows from the tuning switches, which may change before the backward,
+                                // so no two layouts of a call take the same number of bytes
     bool grouped;               // the kept products are those within groups of four chunks plus those of whole groups
                                 // (four arrays: [rows, chunks, low] twice, then [rows, chunks / 4, low] twice)
     // the launches for long chains of chunks (chain_kernels.hip), whose scratch the workspaces hold where they are taken
@@ -38,16 +40,6 @@ public:
     PlainChunks &operator=(const PlainChunks &) = delete;
     static bool active();
 };
-
-// What a forward hands to its backward has a layout that the tuning switches decide (time chunks and their hand-over),
-// and they may change in between, so the size of the buffer says which it is: rounded up to 4096 elements, and an
-// element more for every (chunk count, kind).  Chunk counts go up to 1024, so no two layouts of a call share a size.
-// (rows: of the log-signature in one call; the dense rows of a projection are a buffer of exactly their size.)
-enum class Kept { values = 0, products = 1, groups = 2, rows = 3 };  // values: of words, or none
-inline size_t kept_bytes(size_t raw, size_t elem, int chunks, Kept kind) {
-    const size_t unit = 4096 * elem;
-    return (raw + unit - 1) / unit * unit + (size_t)(chunks % 1024 * 4 + (int)kind) * elem;
-}
 
 DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes, int64_t B,
                          int64_t L, int64_t W, bool windowed);

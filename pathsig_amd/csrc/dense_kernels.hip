@@ -2864,12 +2864,16 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         dc.backward_workspace = (dc.resweep ? 2 : 1) * dc.dense_bytes + (dc.bounded ? kBoundsBytes : 0);
         // the forward can hand those products to the backward when both cut the rows the same way
         if (dc.bwd_chunks > 1 && dc.fwd_chunks == dc.bwd_chunks) {
-            dc.keep_bytes = 2 * pad256((size_t)rows * dc.bwd_chunks * v.low_size * elem);
             // grouped hand-over (see grouped_handover_ok): whole groups of four chunks, two groups at least
             dc.grouped = elem == 4 && v.grouped_ok && !dc.embed && chunks % 4 == 0 && chunks >= 8 &&
                          options().grouped != 0;
-            if (dc.grouped) dc.keep_bytes += 2 * pad256((size_t)rows * (chunks / 4) * v.low_size * elem);
-            dc.keep_bytes = kept_bytes(dc.keep_bytes, elem, chunks, dc.grouped ? Kept::groups : Kept::products);
+            // In units of one array [rows, low]: an even number for two arrays to a chunk, an odd one for groups, and
+            // in either case the same few more for the padding of the arrays to 256 bytes, so that the size tells the
+            // layout.  (Padded sizes alone coincide: rows of 24 bytes in two to ten chunks, or eight chunks in groups
+            // and ten without.)
+            const size_t unit = (size_t)rows * v.low_size * elem;
+            const size_t spare = unit % 256 == 0 ? 0 : 2 * ((512 + unit - 1) / unit);
+            dc.keep_bytes = unit * (spare + (dc.grouped ? (size_t)(chunks / 4 * 10 + 1) : (size_t)chunks * 2));
         }
         if (chains) {
             // (whether or not the backward asks for the second direction: a forward returns the same bits with and
@@ -2898,7 +2902,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
                                     (dc.forward_chains ? 3 : 1) * pad256((size_t)rows * dc.fwd_chunks * v.low_size * elem);
         if (dc.bwd_chunks > 1)
             dc.backward_workspace += (dc.chain_scan ? 5 : 3) * pad256((size_t)rows * dc.bwd_chunks * v.low_size * elem);
-        if (dc.resweep) dc.keep_bytes = (size_t)rows * v.sig_size * elem;  // (such a shape has no time chunks to tell apart)
+        if (dc.resweep) dc.keep_bytes = (size_t)rows * v.sig_size * elem;
         return dc;
     }
     return dc;
