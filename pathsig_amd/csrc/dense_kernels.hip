@@ -2918,8 +2918,10 @@ bool PlainChunks::active() { return plain_chunks(); }
 
 // A step of training asks for the same choice seven times (sizes of buffers, then the launches), and a small call is
 // bound by its host time: the last few choices of a thread are remembered.
+// Windows lie in device memory: what follows from the length of a row (more than 64 chunks, chains of them) cannot be
+// judged by that of the path, so windowed calls make the plain choice.
 DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes, int64_t B,
-                         int64_t L, int64_t W, bool) {
+                         int64_t L, int64_t W, bool windowed) {
     struct Key {
         int64_t elem, d, depth, all_dense, B, L, W, plain, options, sizes[kMaxDepth];
     };
@@ -2936,7 +2938,7 @@ DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, cons
     key.B = B;
     key.L = L;
     key.W = W;
-    key.plain = PlainChunks::active();
+    key.plain = windowed || PlainChunks::active() ? 1 : 0;
     key.options = options_epoch();
     if (!all_dense && level_sizes) std::memcpy(key.sizes, level_sizes + 1, (size_t)depth * sizeof(int64_t));
     for (unsigned i = 0; i < used; ++i)
