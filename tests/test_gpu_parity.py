@@ -164,9 +164,11 @@ def test_projection_with_windows(ps, set_option, route):
     assert rel_err(grad, TO.signature_vjp(path, G, depth, sizes, codes, wins)) < 1e-12
 
 
-# Batches of a dozen paths or more take the backward kernels that put lanes on paths (groups of 16 or 32
-# paths per word); the cases cover both group sizes, ragged last groups, dense and listed levels, prefixes
-# read from the saved signature and prefixes rebuilt by a forward sweep, long words and wide alphabets.
+# Batches of a dozen paths or more take the backward kernels that put lanes on paths: up to sixteen letters
+# groups of sixteen paths (batch_lists.hip), above that, here only dense levels over 66 and 70 letters, groups of
+# 16 or 32 (batch_kernels.hip; its listed and long words are in test_gpu_wide_words.py).  The cases cover ragged
+# last groups, dense and listed levels, prefixes read from the saved signature and prefixes rebuilt by a forward
+# sweep, long words and wide alphabets.
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("case", [
     dict(d=3, depth=4, L=15, B=13, kind="words"),
