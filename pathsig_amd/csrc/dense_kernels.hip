@@ -2770,7 +2770,7 @@ float profile_sweep_ms() {
 }
 
 static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes,
-                                     int64_t B, int64_t L, int64_t W, bool plain) {
+                                     int64_t B, int64_t L, int64_t W, bool windowed, bool plain) {
     DenseChoice dc{};
     dc.variant = -1;
     dc.fwd_chunks = dc.bwd_chunks = 1;
@@ -2833,7 +2833,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         const double low_bytes = (double)v.low_size * elem;
         const bool may_chain = !plain && (elem == 8 || L - 1 <= kChainsUpToSteps);
         bool many = false;  // more than 64 chunks
-        if (chunks_ok && L - 1 > 2048) {
+        if (chunks_ok && !windowed && L - 1 > 2048) {
             // what the shorter sweeps save against what the longer chains of products cost
             const int most = pick_chunks(rows, v.block, L, 2048, true);
             many = most > 64 && (double)(L - 1) * (1.0 / 64 - 1.0 / most) * step_us >
@@ -2851,10 +2851,6 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         // not chunked: units of several blocks (a row is dozens of waves already), rows too long for the scan
         // kernel's LDS
         if (!chunks_ok) chunks = 1;
-        // A step of training whose launches take less than the 60 us that autograd takes to get through its own
-        // forward and backward gains nothing from shorter ones, and the chains are three to five launches more.
-        // (The values a call returns do not depend on whether it keeps anything for a backward, so neither may this.)
-        const bool chains = may_chain && chunks > 1 && (double)(L - 1) / chunks * step_us + 8.0 + 1.3 * scan_us(chunks, depth, low_bytes) > 55.0;
         if (rows * (chunks + 1) >= (int64_t(1) << 31)) return dc;
         dc.usable = true;
         dc.variant = i;
@@ -2875,22 +2871,31 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
             const size_t spare = unit % 256 == 0 ? 0 : 2 * ((512 + unit - 1) / unit);
             dc.keep_bytes = unit * (spare + (dc.grouped ? (size_t)(chunks / 4 * 10 + 1) : (size_t)chunks * 2));
         }
-        if (chains) {
+        const int most_in_block = dc.bounded ? 0 : v.group_sizes[elem == 8 ? 1 : 0];
+        const int in_block = (most_in_block & 4) && chunks % 4 == 0 ? 4 : (most_in_block & 2) && chunks % 2 == 0 ? 2 : 1;
+        const bool staged = 2 * (size_t)v.sig_size * elem <= 48 * 1024;  // (run_forward: kStaged)
+        const double scan = scan_us(chunks, depth, low_bytes);
+        const double combine = combine_us(elem, chunks / in_block, depth, v.sig_size, staged);
+        // A step of training whose launches take less than the 60 us that autograd takes to get through its own
+        // forward and backward gains nothing from shorter ones, and the chains are three to five launches more.
+        // (The values a call returns do not depend on whether it keeps anything for a backward, so neither may this.)
+        // Windows lie in device memory: a row may be of any length up to the path's and counts as a short one, so the
+        // products alone decide.  (One window of 64 of 20001 points, (4, 4) in fp64, without gradient: 12 us, 35 when the
+        // path was taken for the row; ten of (6, 5) on two paths of 4001 points, a step: 123 us without chains, 90 with.)
+        const double launches_us = windowed ? scan + (dc.grouped ? 0.3 * scan : combine)
+                                            : (double)(L - 1) / chunks * step_us + 1.3 * scan;
+        if (may_chain && chunks > 1 && launches_us + 8.0 > 55.0) {
             // (whether or not the backward asks for the second direction: a forward returns the same bits with and
             // without a hand-over)
-            const double chain = chain_us(elem, rows, chunks, d, depth, 2), scan = scan_us(chunks, depth, low_bytes);
+            const double chain = chain_us(elem, rows, chunks, d, depth, 2);
             dc.chain_scan = chain < scan;
             if (dc.grouped) {
                 const int groups = chunks / 4;
                 dc.chain_groups = chain_us(elem, rows, groups, d, depth, 2) + chain_top_us(elem, rows, groups, d, depth) <
                                   scan_us(groups, depth, 0);
             } else {
-                const int most = dc.bounded ? 0 : v.group_sizes[elem == 8 ? 1 : 0];
-                const int in_block = (most & 4) && chunks % 4 == 0 ? 4 : (most & 2) && chunks % 2 == 0 ? 2 : 1;
-                const bool staged = 2 * (size_t)v.sig_size * elem <= 48 * 1024;  // (run_forward: kStaged)
                 dc.chain_top = chunks > in_block &&
-                               chain_top_us(elem, rows, chunks / in_block, d, depth) + 0.25 * std::min(scan, chain) <
-                                   combine_us(elem, chunks / in_block, depth, v.sig_size, staged);
+                               chain_top_us(elem, rows, chunks / in_block, d, depth) + 0.25 * std::min(scan, chain) < combine;
             }
         }
         dc.forward_chains = dc.grouped ? dc.chain_groups : dc.chain_scan || dc.chain_top;
@@ -2918,12 +2923,10 @@ bool PlainChunks::active() { return plain_chunks(); }
 
 // A step of training asks for the same choice seven times (sizes of buffers, then the launches), and a small call is
 // bound by its host time: the last few choices of a thread are remembered.
-// Windows lie in device memory: what follows from the length of a row (more than 64 chunks, chains of them) cannot be
-// judged by that of the path, so windowed calls make the plain choice.
 DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes, int64_t B,
                          int64_t L, int64_t W, bool windowed) {
     struct Key {
-        int64_t elem, d, depth, all_dense, B, L, W, plain, options, sizes[kMaxDepth];
+        int64_t elem, d, depth, all_dense, B, L, W, windowed, plain, options, sizes[kMaxDepth];
     };
     constexpr int kRemembered = 8;
     thread_local Key keys[kRemembered];
@@ -2938,12 +2941,13 @@ DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, cons
     key.B = B;
     key.L = L;
     key.W = W;
-    key.plain = windowed || PlainChunks::active() ? 1 : 0;
+    key.windowed = windowed ? 1 : 0;
+    key.plain = PlainChunks::active() ? 1 : 0;
     key.options = options_epoch();
     if (!all_dense && level_sizes) std::memcpy(key.sizes, level_sizes + 1, (size_t)depth * sizeof(int64_t));
     for (unsigned i = 0; i < used; ++i)
         if (!std::memcmp(&keys[i], &key, sizeof key)) return choices[i];
-    const DenseChoice dc = make_dense_choice(elem, d, depth, all_dense, level_sizes, B, L, W, key.plain != 0);
+    const DenseChoice dc = make_dense_choice(elem, d, depth, all_dense, level_sizes, B, L, W, windowed, key.plain != 0);
     keys[next] = key;
     choices[next] = dc;
     next = (next + 1) % kRemembered;

@@ -37,15 +37,18 @@ def test_allocation_free_backward_goes_without_the_chains(lib, dtype, B, L, beyo
 
 
 # Windows lie in device memory, so their lengths are not known where the chunks are chosen: a few short windows of a long
-# path must not be cut into the hundreds of chunks that the whole path would be worth.
+# path must not be cut into the hundreds of chunks that the whole path would be worth, nor take the launches for long
+# chains where only the length of the path would pay for them.
 @pytest.mark.parametrize("dtype,elem", [(0, 4), (1, 8)])
-@pytest.mark.parametrize("B,W,L,d,depth", [(1, 10, 20001, 4, 4), (1, 1, 20001, 4, 4), (2, 3, 4000, 6, 5), (1, 5, 3500, 3, 6)])
-def test_windows_keep_to_64_chunks_and_take_no_chains(lib, dtype, elem, B, W, L, d, depth):
+@pytest.mark.parametrize("B,W,L,d,depth,chains", [(1, 10, 20001, 4, 4, False), (1, 1, 20001, 4, 4, False), (1, 3, 4000, 6, 5, True),
+                                                  (1, 5, 3500, 3, 6, True)])
+def test_windows_are_not_taken_for_rows_as_long_as_the_path(lib, dtype, elem, B, W, L, d, depth, chains):
     whole = lib.pathsig_sig_forward_workspace(dtype, B * W, L, d, depth, None, 0)
     low, rows = sum(d ** k for k in range(1, depth)), B * W
-    bound = rows * 64 * (low + d ** depth + low) * elem + 2 * 256
+    arrays = 3 if chains else 1  # of the levels below the top, beside the chunk signatures
+    bound = rows * 64 * (low + d ** depth + arrays * low) * elem + (1 + arrays) * 256
     assert whole > bound or (elem == 4 and L - 1 > 4096)  # (paths of that length are cut further)
     assert 0 < lib.pathsig_sig_forward_workspace(dtype, B, L, d, depth, None, W) <= bound
-    products = 3 * (rows * 64 * low * elem + 256)
+    products = (2 + arrays) * (rows * 64 * low * elem + 256)
     assert lib.pathsig_sig_backward_workspace(dtype, B, L, d, depth, None, W) <= B * (L - 1) * d * elem + 256 + products
     assert lib.pathsig_sig_forward_workspace(dtype, B * W, L, d, depth, None, 0) == whole
