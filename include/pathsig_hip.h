@@ -201,7 +201,8 @@ int pathsig_logsignature_backward(const void *path, const void *saved, size_t sa
  *                     (PATHSIG_CHUNKS)
  *   "letter_bounds"   1 = embedded projections leave out unwanted top-level words (PATHSIG_NO_LETTER_BOUNDS sets 0)
  *   "logsig_scatter"  1 = the log-signature adjoint always takes its scatter form (PATHSIG_LOGSIG_SCATTER=1)
- *   "batch_tile"      cap on the increments per tile of the lanes-on-paths backward, 0 = none (PATHSIG_BATCH_TILE)
+ *   "batch_tile"      cap on the increments per tile of the lanes-on-paths backward over more than sixteen letters,
+ *                     0 = none (PATHSIG_BATCH_TILE)
  *   "embed_share"     which word projections run on the register-tiled kernels (dense sweep + gather of the
  *                     wanted columns) instead of the per-word kernels: -1 = the library's rule (top level keeps
  *                     1/8 of the dense one, or the dense sweep is estimated cheaper), 0 = none, n > 0 = those whose
