@@ -1,5 +1,7 @@
 // Signature backward for word projections with lanes on paths, over more than sixteen letters (batch_lists.hip: up to
-// sixteen; the figures below are of sixteen letters, before that one was there).
+// sixteen; the figures below, those behind the words per lane included, are of sixteen letters, before that one was
+// there).  256 paths of 512 points, fp32: 1064 us for 2468 words up to length 6 over 20 letters, 1818 us for 2664 up to
+// length 5 over 40, where the slabs leave room for one increment to a tile.
 //
 // The kernels in words_kernels.hip put one lane on each requested word, so every increment ends in a
 // sum over lanes per letter.  With a batch of paths there is a cheaper arrangement: a group of G lanes

@@ -12,8 +12,11 @@
 // that add the rows, four paths and a few letters to an instruction, took a third of the kernel's time).
 //
 // 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32: 643 us against 959 us with the cells; fp64 step
-// 1749 against 2368 us.  The chains alone take 70 % of that: bound by vector issue and by blocks of unequal length, not
-// by memory.  The same sums on the matrix cores (16x16x4 fp32, the entries times a matrix of zeros and ones) were built
+// 1749 against 2368 us.  The chains alone take 70 % of that.  Not bound by memory, nor by the vector ALU's own rate: a
+// SIMD issues a vector instruction every 1.7 ns, where four resident waves can issue one in 0.9.  The LDS works for
+// 0.35 of the 0.64 ms, 36 % of that in bank conflicts (a staged letter is 34 words after the one before, so the parity
+// of a letter decides which half of the banks its 32 words take, and the four words of a wave have letters of their
+// own), and two barriers per two increments and blocks of unequal length (912 on 1024 places) add to it.  The same sums on the matrix cores (16x16x4 fp32, the entries times a matrix of zeros and ones) were built
 // and are slower: fp32 matrix instructions take as long as the vector
 // ALU would for sixteen letters and do not run beside it.
 #include <type_traits>

@@ -253,7 +253,8 @@ hipError_t launch_logsig_backward(const T *logsig, const T *cache, const T *grad
 // and from the gradients of those columns to dense gradient rows.  lg, cache: [rows, columns below the top level] and
 // [rows, the same, depth], written by the first and read by the second.  picked (null: the whole dense layout): hybrid
 // column of every output (one that is no column, or a word that is none: NaN, and no gradient); dense is cleared before
-// where picked is given.  top_words: top_size codes, null (adjoint) where the top level is dense.  workspace: a_elems + q_elems of logsig_backward_plan for the dense top level.
+// where picked is given.  top_words: top_size codes, null (adjoint) where the top level is dense.  workspace: a_elems +
+// q_elems of logsig_backward_plan for the dense top level.
 bool picked_logsig_possible(size_t elem, int64_t rows, int64_t d, int depth);
 template <typename T>
 hipError_t launch_picked_logsig(const T *sig, int64_t sig_stride, T *lg, T *cache, T *out, int64_t n_out, int64_t rows,
