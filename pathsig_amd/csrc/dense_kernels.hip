@@ -2418,10 +2418,14 @@ int pick_chunks(int64_t rows, int block, int64_t L, int64_t want_waves, bool man
     return (int)c;
 }
 
-// A path gradient is the difference of neighbouring increment sums, sqrt(L) times smaller than they are for a
-// Brownian path, so in fp32 whatever moves the boundaries of the chunks or the order of their products moves the
-// gradient by 1e-7 sqrt(L) of its norm: 1e-5 from some 10 000 increments on.  fp32 calls keep to 64 chunks and to
-// one product after the other beyond this length.
+// fp32 calls keep to 64 chunks and to one product after the other beyond this length: a cautious limit, not one that
+// precision asks for.  A path gradient is the difference of neighbouring increment sums, sqrt(L) times smaller than
+// they are for a Brownian path, so fp32 gradients are off by about 1e-7 sqrt(L) of their norm, and two ways of cutting a
+// path differ by as much from each other.  Against 64 bits neither is the better one: (3, 6), 4 paths of 20001 points,
+// largest error of three draws 1.10e-5 with 64 chunks (values 3.6e-7) and 1.10e-5 with 512 in chains (1.0e-7); (2, 8)
+// 1.25e-5 both, (4, 4) 1.08e-5 both, (5, 5), 2 of 10001, 9.3e-6 and 9.4e-6.  What the limit costs, us a step: 302
+// against 135, 288 against 139, 135 against 85, 162 against 83; (3, 6) 120 against 73 at 4098 points, so there is a step
+// in time at 4097 increments.  The other way round (8, 3), 8 of 12001: 100 us here, 107 without the limit.
 constexpr int64_t kChainsUpToSteps = 4096;
 
 // Estimates of the launches that multiply one chunk after the other.  A product of a scan over 64 chunks took 0.14 us
