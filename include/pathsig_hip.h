@@ -169,7 +169,7 @@ int pathsig_logsig_backward_kept(const void *logsig, const void *cache, const vo
  * columns): path -> the wanted columns of the log-signature, and their gradients -> path gradient.  The signature
  * stays in dense rows in between; nothing of the hybrid layout is written.  level_sizes, W, windows: as for the
  * signature (levels below depth dense, NULL: all); top_words: codes of the top level where it is listed; picked
- * [n_out]: hybrid column of every output, NULL with a dense layout (then n_out = all columns).
+ * [n_out]: hybrid column of every output, NULL with a dense layout (then n_out must be the number of all columns).
  *   pathsig_logsignature_sizes   bytes of `saved` and of the two workspaces; PATHSIG_ERR_UNSUPPORTED for calls that
  *                                are not available in this form (compiled shapes of depth 2 to 8 are).  A forward
  *                                with saved == NULL takes forward_workspace + saved bytes of workspace.

@@ -1101,8 +1101,8 @@ int pathsig_logsignature_lists(const int64_t *top_words, int64_t top_size, const
 }
 
 namespace {
-int check_logsignature(const LogPlan &lp, const int64_t *top_words, int64_t top_size, const int64_t *picked,
-                       const void *workspace, size_t workspace_bytes, size_t need) {
+int check_logsignature(const LogPlan &lp, const int64_t *top_words, int64_t top_size, const int64_t *picked, int64_t n_out,
+                       const int32_t *windows, int64_t W, const void *workspace, size_t workspace_bytes, size_t need) {
     if (!lp.usable) {
         set_error("log-signature in one call: not available for this shape");
         return PATHSIG_ERR_UNSUPPORTED;
@@ -1110,6 +1110,14 @@ int check_logsignature(const LogPlan &lp, const int64_t *top_words, int64_t top_
     const bool listed = top_size != lp.top;
     if ((listed && !picked) || (listed && top_size > 0 && !top_words)) {
         set_error("log-signature in one call: a listed top level needs its words and the wanted columns");
+        return PATHSIG_ERR_ARGUMENT;
+    }
+    if (n_out < 0 || (!picked && n_out != lp.columns)) {
+        set_error("log-signature in one call: %lld outputs of %lld columns", (long long)n_out, (long long)lp.columns);
+        return PATHSIG_ERR_ARGUMENT;
+    }
+    if (windows && W <= 0) {
+        set_error("log-signature in one call: %lld windows", (long long)W);
         return PATHSIG_ERR_ARGUMENT;
     }
     if (need > 0 && (!workspace || workspace_bytes < need)) {
@@ -1126,7 +1134,7 @@ int pathsig_logsignature_forward(const void *path, void *out, int dtype, int64_t
                                  size_t workspace_bytes, void *stream) {
     const LogPlan lp = log_plan(dtype, B, L, d, depth, level_sizes, windows ? W : 0);
     const int64_t top_size = level_sizes ? level_sizes[depth] : lp.top;
-    const int rc = check_logsignature(lp, top_words, top_size, picked, workspace, workspace_bytes,
+    const int rc = check_logsignature(lp, top_words, top_size, picked, n_out, windows, W, workspace, workspace_bytes,
                                       lp.forward_bytes + (saved ? 0 : lp.saved_bytes));
     if (rc != PATHSIG_OK) return rc;
     if (!path || !out) {
@@ -1149,7 +1157,7 @@ int pathsig_logsignature_backward(const void *path, const void *saved, size_t sa
     const LogPlan lp = log_plan(dtype, B, L, d, depth, level_sizes, windows ? W : 0);
     const int64_t top_size = level_sizes ? level_sizes[depth] : lp.top;
     const int rc =
-        check_logsignature(lp, top_words, top_size, picked, workspace, workspace_bytes, lp.backward_bytes);
+        check_logsignature(lp, top_words, top_size, picked, n_out, windows, W, workspace, workspace_bytes, lp.backward_bytes);
     if (rc != PATHSIG_OK) return rc;
     if (!path || !saved || !grad_out || !grad_path) {
         set_error("path, saved, grad_out and grad_path must not be NULL");

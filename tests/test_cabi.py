@@ -124,3 +124,21 @@ def test_sparse_projections_take_the_dense_kernels_when_that_is_cheaper(lib):
     finally:
         assert lib.pathsig_set_option(b"embed_share", -1) == 0
         assert lib.pathsig_set_option(b"tiled", 1) == 0
+
+
+@pytest.mark.parametrize("n_out,picked,windows,W", [
+    (38, 0, 0, 0), (40, 0, 0, 0), (0, 0, 0, 0),  # all columns: 39 of them
+    (-1, 1, 0, 0),
+    (39, 0, 1, 0), (39, 0, 1, -1),  # windows, but none
+])
+def test_logsignature_in_one_call_checks_its_sizes(lib, n_out, picked, windows, W):
+    B, L, d, depth, ptr, size = 2, 12, 3, 3, ctypes.c_void_p, ctypes.c_size_t
+    i64 = ctypes.c_int64
+    saved, forward, backward = size(), size(), size()
+    assert lib.pathsig_logsignature_sizes(0, i64(B), i64(L), i64(d), depth, None, i64(0), ctypes.byref(saved),
+                                          ctypes.byref(forward), ctypes.byref(backward)) == 0
+    shape = (0, i64(B), i64(L), i64(d), depth, None, None, ptr(picked), i64(n_out), None, ptr(windows), i64(W))
+    assert lib.pathsig_logsignature_forward(ptr(1), ptr(1), *shape, ptr(1), ptr(1), forward, None) == -1
+    assert b"log-signature in one call" in lib.pathsig_last_error()
+    assert lib.pathsig_logsignature_backward(ptr(1), ptr(1), saved, ptr(1), ptr(1), *shape, ptr(1), backward, None) == -1
+    assert b"log-signature in one call" in lib.pathsig_last_error()
