@@ -1651,28 +1651,41 @@ __global__ void __launch_bounds__(kWave) chunk_level1_kernel(const T *__restrict
 // vector instruction for a long run of multiply-adds, 1.7 to 1.8 ns as soon as one instruction in sixty-four
 // is a DPP move, which is what one wave alone gets; LDS reads, writes and swizzles cost about three instruction
 // slots each and leave the overlap alone.  The loop of the depth-6 sweep over four letters: 1.39 ns per vector
-// instruction as compiled, 1.11 ns with its twelve DPP instructions replaced by plain ones.  So fp32 units of up
-// to four waves over at most fifteen letters take another way: every lane stores its D terms of an increment,
+// instruction as compiled, 1.11 ns with its twelve DPP instructions replaced by plain ones.  So units of up to four
+// waves over at most fifteen letters take another way: every lane stores its D terms of an increment,
 // padded to kDP, into a slab of its wave (one or more 16-byte LDS stores), and once kSubTile increments have
 // gathered there the lanes read the slab back across the lanes, eight 16-byte reads each, and leave eight
 // partial sums per increment and letter in `sg`.
+// Units of five to eight waves do so too where a lane's state leaves no more than two waves to a SIMD: one such block
+// then fills a CU whatever LDS it takes.  (8, 5), fp32, 256 paths of 2048 points: reverse sweep 1734 -> 1588 us (307
+// -> 293 vector instructions per increment and wave); letters 16 bytes apart instead of 32, which halves the bank
+// conflicts, 1631.
+// fp64: the exchanges move two registers to a value, the slab 16 bytes to two letters, and the chain's terms are added
+// to the lane's row there.  It pays from seven letters on, with eight values to exchange, and over two: a step of 512
+// paths of 2000 points, us, DPP / slab: (7, 2) 489 / 372, (8, 3) 543 / 480, (10, 2) 726 / 570, (9, 3) 1640 / 1268,
+// (2, 4) 267 / 249; (8, 5) with letter bounds, 128 of 1024, 951 / 905.  Not over three to six letters ((4, 3) 244 /
+// 332, (6, 3) 315 / 375) nor, with sixteen padded letters, for thirteen letters and more at depth 3 ((15, 3) 1388 /
+// 1483) and nine and more at depth 4 and 5 ((9, 4) 526 / 570).
 template <typename T, int D, int N, int P, int MAXW = 0>
 struct BackwardShape {
     using G = Geometry<D, N, P, sizeof(T), MAXW>;
     static constexpr int KS = N - P;
-    static constexpr int kDP = D <= 4 ? 4 : D <= 8 ? 8 : 16;  // letters padded to whole 16-byte pieces
-    // (blocks of eight waves, their 64 KB of slabs in dynamic LDS and sums tiled by sixteen increments, measured
-    // slower than the DPP form: the depth-5 sweep over eight letters 359 us against 336 us)
-    static constexpr bool kSlab = sizeof(T) == 4 && D <= 15 && !G::kSplit && G::kWaves <= 4;
-    static constexpr int kGroups = kDP / 4;        // 16-byte pieces per lane and increment
-    static constexpr int kSubTile = 32 / kDP;      // increments that wait in the slab: 8, 4 or 2 (8 KB per wave)
+    static constexpr int kVW = 16 / (int)sizeof(T);  // letters of a 16-byte piece
+    // letters padded to a power of two of whole 16-byte pieces
+    static constexpr int kDP = D <= kVW ? kVW : D <= 4 ? 4 : D <= 8 ? 8 : 16;
+    static constexpr bool kSlabLetters =
+        sizeof(T) == 4 || D == 2 || D == 7 || D == 8 || (D >= 9 && (N == 2 || (N == 3 && D <= 12)));
+    static constexpr bool kSlab = kSlabLetters && D <= 15 && !G::kSplit &&
+                                  (G::kWaves <= 4 || (G::kWaves <= 8 && G::kSubTrie > 40));
+    static constexpr int kGroups = kDP / kVW;      // 16-byte pieces per lane and increment
+    static constexpr int kSubTile = 8 / kGroups;   // increments that wait in the slab: 8, 4, 2 or 1 (8 KB per wave)
     static constexpr int kSlabElems = kSlab ? G::kWaves * kSubTile * kWave * kDP : 4;
     static constexpr int kParts = kSlab ? 8 : 4;
     static constexpr int kLetters = kSlab ? kDP : D;  // cells of one increment in a row of `sg`
     // LDS bytes of the parts of one increment
     static constexpr int kRowBytes = G::kWaves * kParts * kLetters * (int)sizeof(T);
     // (letter blocks: eight one-wave blocks and their 8 KB slabs share a CU, so the sums of a tile take 4 KB)
-    static constexpr int kTileBytes = G::kLetterBlocks ? 4096 : 8192;
+    static constexpr int kTileBytes = G::kLetterBlocks ? 4096 : G::kWaves > 4 ? 8192 * (int)sizeof(T) : 8192;
     static constexpr int kBwdTile =
         kSlab ? (kRowBytes * 32 <= kTileBytes ? 32 : kRowBytes * 16 <= kTileBytes ? 16 : 8)
               : (kRowBytes * 64 <= 49152 ? 64 : kRowBytes * 32 <= 49152 ? 32
@@ -1686,12 +1699,12 @@ struct BackwardShape {
     static constexpr int kStage = kStageTiles * kTileStage + (kStageTiles > 1 ? KS * D : 0);
     static constexpr int kSums = G::kWaves * kParts;
     static constexpr int kSumRow = kBwdTile * kLetters;
-    // fp64: the chain's P terms reach their letters through LDS (a row of D cells per lane, letter-major so that
-    // a wave's accesses never share a bank).  A lane's prefix never changes, so it only ever touches the same
-    // P cells and the others stay zero: P LDS adds, D loads and P clearing stores replace 3 * P * D selects and
-    // adds of a kernel that is bound by vector instruction issue.  fp32 multiplies by one-hot constants instead
-    // where those fit the register file.
-    static constexpr bool kChainCells = sizeof(T) == 8 && D <= 8 && D * G::kBlock * (int)sizeof(T) <= 32 * 1024;
+    // fp64: the chain's P terms reach their letters through LDS (the lane's row of the slab where there is one, else a row
+    // of D cells per lane, letter-major so that a wave's accesses never share a bank).  A lane's prefix never changes, so
+    // it only ever touches the same P cells and the others stay zero: P LDS adds, D loads and P clearing stores replace
+    // 3 * P * D selects and adds of a kernel that is bound by vector instruction issue.  fp32 multiplies by one-hot
+    // constants instead where those fit the register file.
+    static constexpr bool kChainCells = sizeof(T) == 8 && !kSlab && D <= 8 && D * G::kBlock * (int)sizeof(T) <= 32 * 1024;
     static constexpr int kCells = kChainCells ? D * G::kBlock : 1;
 };
 
@@ -1726,6 +1739,8 @@ __device__ __forceinline__ void dense_backward_body(
     prefix_letters<D, P>(active ? pu : 0, u);
     // chain terms through LDS (see BackwardShape): the lane's cells start at zero
     constexpr bool kCellChain = BS::kChainCells && !(sizeof(T) == 4 && P * D <= 24);
+    // (the rows of the slab are written anew for every increment)
+    constexpr bool kSlabChain = BS::kSlab && sizeof(T) == 8;
     T *my_cells = cells + (BS::kChainCells ? tid : 0);  // cell of letter k: my_cells[k * G::kBlock]
     if constexpr (kCellChain) {
 #pragma unroll
@@ -1900,6 +1915,12 @@ __device__ __forceinline__ void dense_backward_body(
             with_first[j] = u[j] == uf[j];
         }
     }
+    // element of the lane's slab row where the term of prefix letter j belongs (fp64 layout)
+    int chain_at[kSlabChain ? P : 1];
+    if constexpr (kSlabChain) {
+#pragma unroll
+        for (int j = 0; j < P; ++j) chain_at[j] = (u[j] / BS::kVW) * (kWave * BS::kVW) + u[j] % BS::kVW;
+    }
     if constexpr (kOneHot) {
 #pragma unroll
         for (int j = 0; j < P; ++j)
@@ -1952,7 +1973,7 @@ __device__ __forceinline__ void dense_backward_body(
 #pragma unroll
                 for (int j = 0; j < (kLastDirect ? 0 : P); ++j) {
                     if constexpr (kOneHot) v = fmad<T>(onehot[j][k], gpre[j], v);
-                    else if constexpr (!BS::kChainCells) v += (u[j] == k) ? gpre[j] : T(0);
+                    else if constexpr (!BS::kChainCells && !kSlabChain) v += (u[j] == k) ? gpre[j] : T(0);
                 }
                 tot[k] = v;
             }
@@ -1969,16 +1990,26 @@ __device__ __forceinline__ void dense_backward_body(
             if constexpr (BS::kSlab) {
                 // the lane's terms of this increment go to its row of the wave's slab; the increment that completes
                 // a group of kSubTile sums the group over the lanes
-                using V4 = typename VecOf<T, 4>::type;
-                constexpr int kSub = BS::kSubTile, kGroups = BS::kGroups;
-                V4 *mine = reinterpret_cast<V4 *>(slab) +
-                           (size_t)(((wave * kSub + (tt & (kSub - 1))) * kWave + lane) * kGroups);
+                using V = typename VecOf<T, BS::kVW>::type;
+                constexpr int kSub = BS::kSubTile, kGroups = BS::kGroups, kVW = BS::kVW;
+                // fp32: a lane's pieces lie side by side.  fp64: [piece][lane], because lanes 64 bytes apart would meet in
+                // a quarter of the banks (fp32 measured the same with its 32 bytes either way).
+                constexpr int kLaneStep = sizeof(T) == 8 ? 1 : kGroups, kPieceStep = sizeof(T) == 8 ? kWave : 1;
+                V *mine = reinterpret_cast<V *>(slab) +
+                          (size_t)((wave * kSub + (tt & (kSub - 1))) * kWave * kGroups + lane * kLaneStep);
 #pragma unroll
                 for (int g = 0; g < kGroups; ++g) {
-                    V4 v;
+                    V v;
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = 4 * g + e < D ? tot[4 * g + e < D ? 4 * g + e : 0] : T(0);
-                    mine[g] = v;
+                    for (int e = 0; e < kVW; ++e) v[e] = kVW * g + e < D ? tot[kVW * g + e < D ? kVW * g + e : 0] : T(0);
+                    mine[g * kPieceStep] = v;
+                }
+                if constexpr (kSlabChain) {
+                    // the chain's terms are added to the letters of the lane's prefix where they lie (LDS adds, because
+                    // two positions may carry the same letter; no other lane touches this row)
+                    T *row = reinterpret_cast<T *>(mine);
+#pragma unroll
+                    for (int j = 0; j < P; ++j) atomicAdd(row + chain_at[j], gpre[j]);
                 }
                 if ((tt & (kSub - 1)) == 0) {
                     // (the LDS operations of a wave complete in order; the fence keeps the compiler from moving
@@ -1988,15 +2019,19 @@ __device__ __forceinline__ void dense_backward_body(
                     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                     // lane -> (increment of the group, one eighth of the lanes, 16-byte piece of the letters)
                     constexpr int kPer = kWave / kSub;  // lanes that share an increment: 8 * kGroups
-                    const int ttl = lane / kPer, part = (lane % kPer) / kGroups, piece = lane % kGroups;
-                    const V4 *rows = reinterpret_cast<const V4 *>(slab) +
-                                     (size_t)((wave * kSub + ttl) * kWave) * kGroups + piece;
+                    const int ttl = lane / kPer;
+                    const int part = sizeof(T) == 8 ? lane & 7 : (lane % kPer) / kGroups;
+                    const int piece = sizeof(T) == 8 ? (lane % kPer) / 8 : lane % kGroups;
+                    const V *rows = reinterpret_cast<const V *>(slab) +
+                                    (size_t)((wave * kSub + ttl) * kWave) * kGroups + piece * kPieceStep;
                     // source lanes 8 s + (part + s) % 8: the eight lanes that read together hit different banks
-                    V4 acc = rows[(size_t)(part & 7) * kGroups];
+                    // (fp64: 8 s + part, 128 bytes in one piece)
+                    auto source = [&](int s8) { return (sizeof(T) == 8 ? 8 * s8 + part : 8 * s8 + ((part + s8) & 7)) * kLaneStep; };
+                    V acc = rows[(size_t)source(0)];
 #pragma unroll
-                    for (int s8 = 1; s8 < 8; ++s8) acc += rows[(size_t)(8 * s8 + ((part + s8) & 7)) * kGroups];
+                    for (int s8 = 1; s8 < 8; ++s8) acc += rows[(size_t)source(s8)];
                     if (tt + ttl < nt)  // (rows beyond the last increment of the tile hold nothing of this tile)
-                        reinterpret_cast<V4 *>(&sg[wave * 8 + part][0])[(tt + ttl) * kGroups + piece] = acc;
+                        reinterpret_cast<V *>(&sg[wave * 8 + part][0])[(tt + ttl) * kGroups + piece] = acc;
                 }
             } else if constexpr (kParts == 4) {
                 // up to sixteen letters in one pass of exchanges (padded to a power of two with zeros), wider

@@ -1,0 +1,50 @@
+"""Per-increment sums over the letters in the reverse sweep, against the CPU checker: the lanes leave their terms in a slab
+in LDS (fp32 up to fifteen letters, fp64 over the alphabets where that is the faster way) or exchange them."""
+import pytest
+import torch
+
+from oracle import tensor_oracle as TO
+
+from .helpers import brownian_path, randn, rel_err
+
+pytestmark = pytest.mark.gpu
+TOL = {torch.float32: 1e-5, torch.float64: 1e-12}
+
+
+# Alphabets on both sides of every padding of the slab (2, 4, 8, 16 letters), blocks of one to eight waves; lengths around
+# the increments that wait in the slab (1 to 8) and the tiles of 8, 16 and 32 increments; time chunks with a ghost step.
+@pytest.mark.parametrize("d,depth,dtype", [(8, 5, torch.float32), (7, 5, torch.float32), (2, 4, torch.float64),
+                                           (3, 3, torch.float64), (7, 4, torch.float64), (8, 3, torch.float64),
+                                           (8, 5, torch.float64), (10, 3, torch.float64), (12, 2, torch.float64),
+                                           (15, 3, torch.float64)])
+@pytest.mark.parametrize("L,chunks", [(2, 1), (8, 1), (10, 1), (34, 1), (35, 3), (65, 2)])
+def test_lengths_around_the_tiles(set_option, d, depth, dtype, L, chunks):
+    import pathsig_amd as ps
+    set_option("chunks", chunks)
+    B = 2
+    path = brownian_path(B, L, d, seed=40 + d + L)
+    want = TO.signature(path, depth)
+    G = randn(tuple(want.shape), seed=41)
+    x = path.to(dtype).cuda().requires_grad_(True)
+    out = ps.Signature(depth=depth)(x)
+    (grad,) = torch.autograd.grad(out, x, G.to(dtype).cuda())
+    assert rel_err(out, want) < TOL[dtype]
+    assert rel_err(grad, TO.signature_vjp(path, G, depth)) < TOL[dtype]
+
+
+@pytest.mark.parametrize("d,depth,dtype", [(8, 5, torch.float32), (8, 4, torch.float64), (2, 5, torch.float64),
+                                           (11, 3, torch.float64)])
+def test_overlapping_windows(d, depth, dtype):
+    import pathsig_amd as ps
+    B, L = 2, 40
+    path = brownian_path(B, L, d, seed=60 + d)
+    spans = [(0, 40), (3, 20), (5, 5), (7, 8), (11, 29)]
+    x = path.to(dtype).cuda().requires_grad_(True)
+    out = ps.Signature(depth=depth, windows=torch.tensor(spans, device="cuda"))(x)
+    G = randn(tuple(out.shape), seed=61)
+    (grad,) = torch.autograd.grad(out, x, G.to(dtype).cuda())
+    want = torch.zeros_like(path)
+    for w, (start, end) in enumerate(spans):
+        if end - start > 1:
+            want[:, start:end] += TO.signature_vjp(path[:, start:end], G[:, w], depth)
+    assert rel_err(grad, want) < TOL[dtype]
