@@ -165,14 +165,15 @@ struct StepTargets {
 // ---------------------------------------------------------------------------------------------
 // adjoint of one Chen step
 // ---------------------------------------------------------------------------------------------
-template <typename T, int D, int P, int M, int J, int LO = 0, int K = D>
+// BACK: the leaves of the target (level M of A) are taken back by the step on the way.
+template <typename T, int D, int P, int M, int J, int LO = 0, int K = D, bool BACK = false>
 struct AdjDescend {
     // pt = Horner value of the parent; returns its adjoint.  gdxk[q][a] collects the gradient with respect
     // to dxs[q][a]; the caller folds the 1/(q+1) back in.
     template <int ASUB, int HSUB, int KS>
     // (with the first level split between lanes: dxf / gdxf are the increments of the lane's own K letters and
     // their gradients; otherwise they are dxs / gdxk themselves)
-    static __device__ __forceinline__ T run(T pt, int idx0, const T (&asub)[ASUB], T (&hsub)[HSUB],
+    static __device__ __forceinline__ T run(T pt, int idx0, T (&asub)[ASUB], T (&hsub)[HSUB],
                                             const T (&dxs)[KS][D], const T (&dxf)[KS][K], T (&gdxk)[KS][D],
                                             T (&gdxf)[KS][K]) {
         constexpr int off = sub_size(D, K, J - P - 1);
@@ -186,10 +187,11 @@ struct AdjDescend {
             T g;
             if constexpr (J == M) {
                 g = hsub[off + idx0 + a];
+                if constexpr (BACK) asub[off + idx0 + a] = fmad<T>(-pt, inc, asub[off + idx0 + a]);
             } else {
                 const T tmp = fmad<T>(pt, inc, asub[off + idx0 + a]);
-                g = AdjDescend<T, D, P, M, J + 1, LO, K>::template run<ASUB, HSUB, KS>(tmp, (idx0 + a) * D, asub, hsub,
-                                                                                       dxs, dxf, gdxk, gdxf);
+                g = AdjDescend<T, D, P, M, J + 1, LO, K, BACK>::template run<ASUB, HSUB, KS>(tmp, (idx0 + a) * D, asub,
+                                                                                            hsub, dxs, dxf, gdxk, gdxf);
                 hsub[off + idx0 + a] += g;
             }
             if constexpr (kFirst) gdxf[M - J][a] = fmad<T>(g, pt, gdxf[M - J][a]);
@@ -200,12 +202,14 @@ struct AdjDescend {
     }
 };
 
-template <typename T, int D, int N, int P, int M, int LO = 0, int K = D>
+// BACK: A is still the signature after the step; each target below the top takes its level back once the levels it
+// reads have been: A_M <- A_M - tmp_{M-1} dx, with the Horner values tmp that the adjoint needs anyway.
+template <typename T, int D, int N, int P, int M, int LO = 0, int K = D, bool BACK = false>
 struct AdjTargets {
     // targets ascending: the seed of target M (adjoint of level M) is only changed by targets above M;
     // LO applies to the top target (M = N), whose left-out words have a zero upstream gradient
     template <int ASUB, int HSUB, int KS>
-    static __device__ __forceinline__ void run(const T (&a)[P + 1], const T (&asub)[ASUB], T (&hc)[P + 1],
+    static __device__ __forceinline__ void run(T (&a)[P + 1], T (&asub)[ASUB], T (&hc)[P + 1],
                                                T (&hsub)[HSUB], const T (&dxs)[KS][D], const T (&dxf)[KS][K],
                                                const T (&dxp)[P], T (&gdxk)[KS][D], T (&gdxf)[KS][K],
                                                T (&gpre)[P]) {
@@ -222,8 +226,9 @@ struct AdjTargets {
         constexpr int JS = (M <= P) ? M : P;  // chain level where the walk back starts
         if constexpr (M <= P) {
             g = hc[M];
+            if constexpr (BACK && M < N) a[M] = fmad<T>(-ps[M], dxp[M - 1], a[M]);
         } else {
-            g = AdjDescend<T, D, P, M, P + 1, (M == N ? LO : 0), K>::template run<ASUB, HSUB, KS>(
+            g = AdjDescend<T, D, P, M, P + 1, (M == N ? LO : 0), K, BACK && M < N>::template run<ASUB, HSUB, KS>(
                 tmp, 0, asub, hsub, dxs, dxf, gdxk, gdxf);
             hc[P] += g;
         }
@@ -236,7 +241,7 @@ struct AdjTargets {
             }
         }
         if constexpr (M < N)
-            AdjTargets<T, D, N, P, M + 1, LO, K>::template run<ASUB, HSUB, KS>(a, asub, hc, hsub, dxs, dxf, dxp, gdxk,
+            AdjTargets<T, D, N, P, M + 1, LO, K, BACK>::template run<ASUB, HSUB, KS>(a, asub, hc, hsub, dxs, dxf, dxp, gdxk,
                                                                                  gdxf, gpre);
     }
 };
@@ -1710,7 +1715,13 @@ struct BackwardShape {
 
 // BOUND: the upstream gradient is zero on every top-level word that has a letter below BOUND after the
 // prefix's first letter, and the sweep leaves those words out; the LDS arrays belong to the calling kernel.
-template <typename T, int D, int N, int P, bool ACCUMULATE, bool CHUNKED, int BOUND, int MAXW = 0>
+// SHARED: A_t = A_{t+1} (x) exp(-dx_t) is taken back target by target inside the adjoint of the step, on the Horner values
+// that the adjoint computes anyway (AdjTargets: BACK), in place of a pass with exp(-dx) that computes such values of its
+// own: 12 of 293 vector instructions less per increment for (8, 5), 22 of some 260 for (4, 6).  Reverse sweeps, us, a pass of
+// its own / shared: fp32 (8, 5), 256 paths of 2048 points, 1728 / 1691; (4, 6), 128 of 1024, 88.8 / 85.2; (3, 6), 4 of
+// 20001, 177 / 167; (6, 5), 64 of 2048 in windows of 64, 340 / 335; (8, 5) with letter bounds 337 / 327; fp64 (6, 5) 95.3 /
+// 90.9, (3, 6) 54.5 / 50.8, (8, 4) 123.5 / 120.6.  Not shared: see run_backward.
+template <typename T, int D, int N, int P, bool ACCUMULATE, bool CHUNKED, int BOUND, int MAXW = 0, bool SHARED = true>
 __device__ __forceinline__ void dense_backward_body(
     const T *__restrict__ path, const T *__restrict__ sig, const T *__restrict__ grad_sig, const T *__restrict__ edgeA,
     const T *__restrict__ edgeZ, T *__restrict__ grad_inc, const SigShape &shape, int chunks, T *__restrict__ grad_path,
@@ -1937,8 +1948,8 @@ __device__ __forceinline__ void dense_backward_body(
         const T *sdx = sdx_all + (t0 - staged_from) * (KS * D);
         lds_barrier();
         auto step = [&](int tt, const T (&dxs)[KS][D], const T (&dxp)[P], const T (&dxf)[FQ][FK]) {
-            // A_t = A_{t+1} (x) exp(-dx_t), levels < N
-            if constexpr (N > 1) {
+            if constexpr (!SHARED) {
+                // A_t = A_{t+1} (x) exp(-dx_t), levels < N
                 if constexpr (G::kSplit)
                     StepTargets<T, D, P, N - 1, true, 0, KF>::template run<kAS, KS>(a, asub, dxs, dxf, dxp);
                 else
@@ -1957,10 +1968,10 @@ __device__ __forceinline__ void dense_backward_body(
 #pragma unroll
             for (int j = 0; j < P; ++j) gpre[j] = T(0);
             if constexpr (G::kSplit)
-                AdjTargets<T, D, N, P, 1, BOUND, KF>::template run<kAS, G::kFwdSub, KS>(a, asub, hc, hsub, dxs, dxf, dxp,
+                AdjTargets<T, D, N, P, 1, BOUND, KF, SHARED>::template run<kAS, G::kFwdSub, KS>(a, asub, hc, hsub, dxs, dxf, dxp,
                                                                                         gdxk, gdxf, gpre);
             else
-                AdjTargets<T, D, N, P, 1, BOUND>::template run<kAS, G::kFwdSub, KS>(a, asub, hc, hsub, dxs, dxs, dxp,
+                AdjTargets<T, D, N, P, 1, BOUND, D, SHARED>::template run<kAS, G::kFwdSub, KS>(a, asub, hc, hsub, dxs, dxs, dxp,
                                                                                     gdxk, gdxk, gpre);
             // letter k collects the sub-trie sums (with the 1/(q+1) of their increments) and the chain
             // positions whose letter is k
@@ -2196,7 +2207,8 @@ __device__ __forceinline__ void dense_backward_body(
 // BOUNDED: the upstream gradient is zero on every top-level word outside the letter bounds in `bounds` (see
 // LetterBounds).  Every wave runs the copy of the sweep compiled for its bound; all copies meet at the same
 // barriers.
-template <typename T, int D, int N, int P, bool ACCUMULATE, bool CHUNKED, bool BOUNDED = false, int MAXW = 0>
+template <typename T, int D, int N, int P, bool ACCUMULATE, bool CHUNKED, bool BOUNDED = false, int MAXW = 0,
+          bool SHARED = true>
 __global__ void __launch_bounds__((Geometry<D, N, P, sizeof(T), MAXW>::kBlock))
     dense_backward_kernel(const T *__restrict__ path, const T *__restrict__ sig, const T *__restrict__ grad_sig,
                           const T *__restrict__ edgeA, const T *__restrict__ edgeZ, T *__restrict__ grad_inc,
@@ -2220,15 +2232,15 @@ __global__ void __launch_bounds__((Geometry<D, N, P, sizeof(T), MAXW>::kBlock))
         const int pu = G::kLetterBlocks ? tid + part_of_block<G>() * G::kBlock : LetterBounds<D, P>::prefix_of_thread(tid);
         const int lo = LetterBounds<D, P>::of_wave(bounds, pu);
         dispatch_value<0, D>(lo, [&](auto loc) {
-            dense_backward_body<T, D, N, P, ACCUMULATE, CHUNKED, decltype(loc)::value, MAXW>(
+            dense_backward_body<T, D, N, P, ACCUMULATE, CHUNKED, decltype(loc)::value, MAXW, SHARED>(
                 path, sig, grad_sig, edgeA, edgeZ, grad_inc, shape, chunks, grad_path, pu, tid, sdx, sg, cells, slab, carry,
                 edgeL, edgeR);
         });
     } else {
         const int pu = G::kUnitBlocks > 1 ? tid + part_of_block<G>() * G::kBlock : tid;
-        dense_backward_body<T, D, N, P, ACCUMULATE, CHUNKED, 0, MAXW>(path, sig, grad_sig, edgeA, edgeZ, grad_inc,
-                                                                      shape, chunks, grad_path, pu, tid, sdx, sg, cells,
-                                                                      slab, carry, edgeL, edgeR);
+        dense_backward_body<T, D, N, P, ACCUMULATE, CHUNKED, 0, MAXW, SHARED>(
+            path, sig, grad_sig, edgeA, edgeZ, grad_inc, shape, chunks, grad_path, pu, tid, sdx, sg, cells, slab, carry, edgeL,
+            edgeR);
     }
 }
 
@@ -2422,6 +2434,17 @@ constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
 size_t pad256(size_t n) { return (n + 255) / 256 * 256; }
 
+// fp32 calls keep to 64 chunks, to one product after the other and to a roll-back of its own beyond this length: a
+// cautious limit, not one that precision asks for.  A path gradient is the difference of neighbouring increment sums,
+// sqrt(L) times smaller than they are for a Brownian path, so fp32 gradients are off by about 1e-7 sqrt(L) of their
+// norm, and two ways of cutting a path differ by as much from each other.  Against 64 bits neither is the better one:
+// (3, 6), 4 paths of 20001 points, largest error of three draws 1.10e-5 with 64 chunks (values 3.6e-7) and 1.10e-5 with
+// 512 in chains (1.0e-7); (2, 8) 1.25e-5 both, (4, 4) 1.08e-5 both, (5, 5), 2 of 10001, 9.3e-6 and 9.4e-6.  What the
+// limit costs, us a step: 302 against 135, 288 against 139, 135 against 85, 162 against 83; (3, 6) 120 against 73 at
+// 4098 points, so there is a step in time at 4097 increments.  The other way round (8, 3), 8 of 12001: 100 us here, 107
+// without the limit. The shared roll-back alone would take 10 of the 177 us of the reverse sweep at (3, 6).
+constexpr int64_t kSameBitsFromSteps = 4096;
+
 #if PSIG_GROUP < 0
 struct SweepProfile {
     bool enabled = false, valid = false;
@@ -2452,16 +2475,6 @@ int pick_chunks(int64_t rows, int block, int64_t L, int64_t want_waves, bool man
     if (c < 1) c = 1;
     return (int)c;
 }
-
-// fp32 calls keep to 64 chunks and to one product after the other beyond this length: a cautious limit, not one that
-// precision asks for.  A path gradient is the difference of neighbouring increment sums, sqrt(L) times smaller than
-// they are for a Brownian path, so fp32 gradients are off by about 1e-7 sqrt(L) of their norm, and two ways of cutting a
-// path differ by as much from each other.  Against 64 bits neither is the better one: (3, 6), 4 paths of 20001 points,
-// largest error of three draws 1.10e-5 with 64 chunks (values 3.6e-7) and 1.10e-5 with 512 in chains (1.0e-7); (2, 8)
-// 1.25e-5 both, (4, 4) 1.08e-5 both, (5, 5), 2 of 10001, 9.3e-6 and 9.4e-6.  What the limit costs, us a step: 302
-// against 135, 288 against 139, 135 against 85, 162 against 83; (3, 6) 120 against 73 at 4098 points, so there is a step
-// in time at 4097 increments.  The other way round (8, 3), 8 of 12001: 100 us here, 107 without the limit.
-constexpr int64_t kChainsUpToSteps = 4096;
 
 // Estimates of the launches that multiply one chunk after the other.  A product of a scan over 64 chunks took 0.14 us
 // at depth 2, 0.35 at depth 3 and 4, 0.3 (rows of 100 bytes) to 0.85 (19 kB) at depth 5, 0.7 at depth 6; of a combine about as much when it stages
@@ -2763,11 +2776,14 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
                                        dim3((unsigned)(units * GL::kUnitBlocks)), dim3(GL::kBlock), 0, stream, path, sig,
                                        grad_sig, dumpA, dumpH, grad_inc, shape, chunks, (T *)nullptr, bounds);
                 } else if (accumulate) {
-                    hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, true, true>), dim3((unsigned)units),
+                    // (fp64: the levels of A held until their target comes leave the copies of the body for the
+                    // smaller bounds more than the register file; all words of weight 6.25 and below over eight letters, 72
+                    // paths of 500 points: 403 us, shared 428)
+                    hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, true, true, 0, false>), dim3((unsigned)units),
                                        dim3(G::kBlock), 0, stream, path, sig, grad_sig, dumpA,
                                        dumpH, grad_inc, shape, chunks, (T *)nullptr, bounds);
                 } else {
-                    hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, false, true, true>), dim3((unsigned)units),
+                    hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, false, true, true, 0, false>), dim3((unsigned)units),
                                        dim3(G::kBlock), 0, stream, path, sig, grad_sig, dumpA,
                                        dumpH, grad_inc, shape, chunks, grad_path, bounds);
                 }
@@ -2779,10 +2795,20 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
                 hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, true>), dim3((unsigned)units),
                                    dim3(G::kBlock), 0, stream, path, sig, grad_sig, dumpA, dumpH,
                                    grad_inc, shape, chunks, (T *)nullptr, (const int *)nullptr, edgeL, edgeR);
-            else
-                hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, false, true>), dim3((unsigned)units),
-                                   dim3(G::kBlock), 0, stream, path, sig, grad_sig, dumpA, dumpH,
-                                   grad_inc, shape, chunks, grad_path, (const int *)nullptr, edgeL, edgeR);
+            else {
+                auto launch = [&](auto shared) {
+                    hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, false, true, false, 0, decltype(shared)::value>),
+                                       dim3((unsigned)units), dim3(G::kBlock), 0, stream, path, sig, grad_sig, dumpA, dumpH,
+                                       grad_inc, shape, chunks, grad_path, (const int *)nullptr, edgeL, edgeR);
+                };
+                if constexpr (sizeof(T) == 4) {
+                    // Rows beyond kSameBitsFromSteps keep the order of operations that they had: see there.
+                    if (shape.L - 1 > kSameBitsFromSteps) launch(std::false_type{});
+                    else launch(std::true_type{});
+                } else {
+                    launch(std::true_type{});
+                }
+            }
         }
         if (!accumulate) *wrote_path = true;
         profile_bracket(false, stream);
@@ -2870,7 +2896,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         // in fp64
         const double step_us = (0.2 + 0.013 * v.sub_size) * (elem == 8 ? 2.0 : 1.0);
         const double low_bytes = (double)v.low_size * elem;
-        const bool may_chain = !plain && (elem == 8 || L - 1 <= kChainsUpToSteps);
+        const bool may_chain = !plain && (elem == 8 || L - 1 <= kSameBitsFromSteps);
         bool many = false;  // more than 64 chunks
         if (chunks_ok && !windowed && L - 1 > 2048) {
             // what the shorter sweeps save against what the longer chains of products cost

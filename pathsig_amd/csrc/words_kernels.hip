@@ -58,7 +58,7 @@ __device__ void forward_body(const T *__restrict__ path, T *__restrict__ sig, co
                 for (int k = 0; k < DEG; ++k) dl[k] = dxr[l[k]];
                 T dq[DEG][DEG];
                 scale_letters<T, DEG>(dl, dq);
-                chain_step<T, DEG, DEG, true>(p, dq);
+                chain_step<T, DEG, DEG>(p, dq);
             }
         }
     }
@@ -200,7 +200,7 @@ __device__ void backward_body(const T *__restrict__ path, const T *__restrict__ 
                 for (int k = 0; k < DEG; ++k) dl[k] = dxr[l[k]];
                 T dq[DEG][DEG];
                 scale_letters<T, DEG>(dl, dq);
-                chain_step<T, DEG, DEG - 1, true>(p, dq);
+                chain_step<T, DEG, DEG - 1>(p, dq);
             }
         }
     }
@@ -228,10 +228,9 @@ __device__ void backward_body(const T *__restrict__ path, const T *__restrict__ 
             T dl[DEG];
 #pragma unroll
             for (int k = 0; k < DEG; ++k) dl[k] = dxr[l[k]];
-            // S_t = S_{t+1} (x) exp(-dx_t) on the chain (levels < DEG are all the adjoint needs)
+            // S_t = S_{t+1} (x) exp(-dx_t) on the chain (levels < DEG are all the adjoint needs), and the adjoint
             T dq[DEG][DEG];
             scale_letters<T, DEG>(dl, dq);
-            chain_step<T, DEG, DEG - 1, false>(p, dq);
             T gl[DEG];
             chain_step_adjoint<T, DEG>(p, h, dl, dq, gl);
             if (sorted) {
