@@ -1683,6 +1683,7 @@ struct BackwardShape {
     static constexpr bool kSlab = kSlabLetters && D <= 15 && !G::kSplit &&
                                   (G::kWaves <= 4 || (G::kWaves <= 8 && G::kSubTrie > 40));
     static constexpr int kGroups = kDP / kVW;      // 16-byte pieces per lane and increment
+    static constexpr bool kByPiece = sizeof(T) == 8 || kGroups >= 4;  // layout of the slab: [piece][lane]
     static constexpr int kSubTile = 8 / kGroups;   // increments that wait in the slab: 8, 4, 2 or 1 (8 KB per wave)
     static constexpr int kSlabElems = kSlab ? G::kWaves * kSubTile * kWave * kDP : 4;
     static constexpr int kParts = kSlab ? 8 : 4;
@@ -1703,7 +1704,9 @@ struct BackwardShape {
     static constexpr int kStageTiles = !kSlab || kStageRoom < 1 ? 1 : kStageRoom > 8 ? 8 : kStageRoom;
     static constexpr int kStage = kStageTiles * kTileStage + (kStageTiles > 1 ? KS * D : 0);
     static constexpr int kSums = G::kWaves * kParts;
-    static constexpr int kSumRow = kBwdTile * kLetters;
+    // (by piece, the eight lanes that store together hold eight parts of a sum: a piece of padding puts them into
+    // different banks)
+    static constexpr int kSumRow = kBwdTile * kLetters + (kSlab && kByPiece ? kVW : 0);
     // fp64: the chain's P terms reach their letters through LDS (the lane's row of the slab where there is one, else a row
     // of D cells per lane, letter-major so that a wave's accesses never share a bank).  A lane's prefix never changes, so
     // it only ever touches the same P cells and the others stay zero: P LDS adds, D loads and P clearing stores replace
@@ -1749,7 +1752,7 @@ __device__ __forceinline__ void dense_backward_body(
     int u[P];
     prefix_letters<D, P>(active ? pu : 0, u);
     // chain terms through LDS (see BackwardShape): the lane's cells start at zero
-    constexpr bool kCellChain = BS::kChainCells && !(sizeof(T) == 4 && P * D <= 24);
+    constexpr bool kCellChain = BS::kChainCells;
     // (the rows of the slab are written anew for every increment)
     constexpr bool kSlabChain = BS::kSlab && sizeof(T) == 8;
     T *my_cells = cells + (BS::kChainCells ? tid : 0);  // cell of letter k: my_cells[k * G::kBlock]
@@ -1898,8 +1901,9 @@ __device__ __forceinline__ void dense_backward_body(
     }
     a[0] = T(1);
     // onehot[j][k] = 1 when the j-th letter of the lane's prefix is k (kept in registers only where
-    // registers are plentiful; otherwise the letters are compared every time)
-    constexpr bool kOneHot = sizeof(T) == 4 && P * D <= 24;
+    // registers are plentiful: few of them, or few values below the prefix; otherwise the letters are compared every time,
+    // a select and an add in place of a multiply-add: 30 of 140 vector instructions of an increment at (15, 3))
+    constexpr bool kOneHot = sizeof(T) == 4 && (P * D <= 24 || (P * D <= 30 && G::kSubTrie <= 16));
     T onehot[kOneHot ? P : 1][kOneHot ? D : 1];
     // Wide alphabets compare every letter with the prefix letters to route the chain's terms (P * D selects and
     // adds per increment).  The last prefix letter is different in every lane of a row of sixteen, so its term
@@ -2003,9 +2007,13 @@ __device__ __forceinline__ void dense_backward_body(
                 // a group of kSubTile sums the group over the lanes
                 using V = typename VecOf<T, BS::kVW>::type;
                 constexpr int kSub = BS::kSubTile, kGroups = BS::kGroups, kVW = BS::kVW;
-                // fp32: a lane's pieces lie side by side.  fp64: [piece][lane], because lanes 64 bytes apart would meet in
-                // a quarter of the banks (fp32 measured the same with its 32 bytes either way).
-                constexpr int kLaneStep = sizeof(T) == 8 ? 1 : kGroups, kPieceStep = sizeof(T) == 8 ? kWave : 1;
+                // A lane's pieces lie side by side up to 32 bytes of fp32 (which measured the same either way), else
+                // [piece][lane]: lanes 64 bytes apart meet in a quarter of the banks, and so do the eight parts of a sum in
+                // `sg` without its padding.  us a step, side by side / by piece, fp32: (15, 3), 3105 windows of 54 points,
+                // 273 / 191 for the sweep (with the letters of the prefix in registers, see kOneHot); (15, 2), 512 paths of 1000
+                // points, 207 / 150; (10, 2), 256 of 1000, 94 / 68; (12, 3), 128 of 300, 48 / 35; (9, 4) 57 / 51.
+                constexpr bool kByPiece = BS::kByPiece;
+                constexpr int kLaneStep = kByPiece ? 1 : kGroups, kPieceStep = kByPiece ? kWave : 1;
                 V *mine = reinterpret_cast<V *>(slab) +
                           (size_t)((wave * kSub + (tt & (kSub - 1))) * kWave * kGroups + lane * kLaneStep);
 #pragma unroll
@@ -2031,8 +2039,8 @@ __device__ __forceinline__ void dense_backward_body(
                     // lane -> (increment of the group, one eighth of the lanes, 16-byte piece of the letters)
                     constexpr int kPer = kWave / kSub;  // lanes that share an increment: 8 * kGroups
                     const int ttl = lane / kPer;
-                    const int part = sizeof(T) == 8 ? lane & 7 : (lane % kPer) / kGroups;
-                    const int piece = sizeof(T) == 8 ? (lane % kPer) / 8 : lane % kGroups;
+                    const int part = kByPiece ? lane & 7 : (lane % kPer) / kGroups;
+                    const int piece = kByPiece ? (lane % kPer) / 8 : lane % kGroups;
                     const V *rows = reinterpret_cast<const V *>(slab) +
                                     (size_t)((wave * kSub + ttl) * kWave) * kGroups + piece * kPieceStep;
                     // source lanes 8 s + (part + s) % 8: the eight lanes that read together hit different banks
@@ -2152,16 +2160,33 @@ __device__ __forceinline__ void dense_backward_body(
         lds_barrier();
         // cell of (increment, letter) number idx in a row of `sg`
         auto cell = [](int idx) { return BS::kLetters == D ? idx : (idx / D) * BS::kLetters + idx % D; };
+        // Sum of the parts of all waves.  More than 32 of them meet per wave first: one after the other, 64 terms left the
+        // gradient of (8, 5), 64 paths of 500 points, off by 2.5e-6 of its norm instead of 1.8e-6 (with sums by DPP 2.0e-6).
+        auto sum_of_parts = [&](int at) {
+            if constexpr (BS::kSums > 32) {
+                T v = T(0);
+#pragma unroll
+                for (int wv = 0; wv < G::kWaves; ++wv) {
+                    T of_wave = sg[wv * kParts][at];
+#pragma unroll
+                    for (int q = 1; q < kParts; ++q) of_wave += sg[wv * kParts + q][at];
+                    v = wv == 0 ? of_wave : v + of_wave;
+                }
+                return v;
+            } else {
+                T v = sg[0][at];
+#pragma unroll
+                for (int q = 1; q < BS::kSums; ++q) v += sg[q][at];
+                return v;
+            }
+        };
         if constexpr (kToPath) {
             // No windows, one block to a unit: the path gradient dL/dx[t] = g[t-1] - g[t] leaves the kernel directly.
             // Tiles are flushed from the right end of the chunk to its left end; `carry` holds g of the first
             // increment of the tile flushed before (the one to the right), whose point is written now.
             for (int idx = tid; idx < nt * D; idx += G::kBlock) {
                 const int at = cell(idx);
-                T v = sg[0][at];
-#pragma unroll
-                for (int q = 1; q < G::kWaves * kParts; ++q) v += sg[q][at];
-                sg[0][at] = v;
+                sg[0][at] = sum_of_parts(at);
             }
             lds_barrier();
             T *gp = grad_path + (b * shape.L + span.start + t0) * D;
@@ -2190,10 +2215,7 @@ __device__ __forceinline__ void dense_backward_body(
             }
         } else {
             for (int idx = tid; idx < nt * D; idx += G::kBlock) {
-                const int at = cell(idx);
-                T v = sg[0][at];
-#pragma unroll
-                for (int q = 1; q < G::kWaves * kParts; ++q) v += sg[q][at];
+                const T v = sum_of_parts(cell(idx));
                 if constexpr (ACCUMULATE) {
                     atomicAdd(&ginc[t0 * D + idx], v);
                 } else {

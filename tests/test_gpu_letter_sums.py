@@ -16,7 +16,8 @@ TOL = {torch.float32: 1e-5, torch.float64: 1e-12}
 @pytest.mark.parametrize("d,depth,dtype", [(8, 5, torch.float32), (7, 5, torch.float32), (2, 4, torch.float64),
                                            (3, 3, torch.float64), (7, 4, torch.float64), (8, 3, torch.float64),
                                            (8, 5, torch.float64), (10, 3, torch.float64), (12, 2, torch.float64),
-                                           (15, 3, torch.float64)])
+                                           (15, 3, torch.float64), (9, 3, torch.float32), (10, 4, torch.float32),
+                                           (15, 3, torch.float32), (15, 2, torch.float32)])
 @pytest.mark.parametrize("L,chunks", [(2, 1), (8, 1), (10, 1), (34, 1), (35, 3), (65, 2)])
 def test_lengths_around_the_tiles(set_option, d, depth, dtype, L, chunks):
     import pathsig_amd as ps
