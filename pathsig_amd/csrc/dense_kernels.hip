@@ -1901,9 +1901,9 @@ __device__ __forceinline__ void dense_backward_body(
     }
     a[0] = T(1);
     // onehot[j][k] = 1 when the j-th letter of the lane's prefix is k (kept in registers only where
-    // registers are plentiful: few of them, or few values below the prefix; otherwise the letters are compared every time,
-    // a select and an add in place of a multiply-add: 30 of 140 vector instructions of an increment at (15, 3))
-    constexpr bool kOneHot = sizeof(T) == 4 && (P * D <= 24 || (P * D <= 30 && G::kSubTrie <= 16));
+    // registers are plentiful; otherwise the letters are compared every time, which also keeps an infinite term of one
+    // letter out of the sums of the others)
+    constexpr bool kOneHot = sizeof(T) == 4 && P * D <= 24;
     T onehot[kOneHot ? P : 1][kOneHot ? D : 1];
     // Wide alphabets compare every letter with the prefix letters to route the chain's terms (P * D selects and
     // adds per increment).  The last prefix letter is different in every lane of a row of sixteen, so its term
@@ -2009,9 +2009,9 @@ __device__ __forceinline__ void dense_backward_body(
                 constexpr int kSub = BS::kSubTile, kGroups = BS::kGroups, kVW = BS::kVW;
                 // A lane's pieces lie side by side up to 32 bytes of fp32 (which measured the same either way), else
                 // [piece][lane]: lanes 64 bytes apart meet in a quarter of the banks, and so do the eight parts of a sum in
-                // `sg` without its padding.  us a step, side by side / by piece, fp32: (15, 3), 3105 windows of 54 points,
-                // 273 / 191 for the sweep (with the letters of the prefix in registers, see kOneHot); (15, 2), 512 paths of 1000
-                // points, 207 / 150; (10, 2), 256 of 1000, 94 / 68; (12, 3), 128 of 300, 48 / 35; (9, 4) 57 / 51.
+                // `sg` without its padding.  us a step of forward and reverse sweep, side by side / by piece, fp32: (15, 3),
+                // 3105 windows of 54 points, 318 / 246; (14, 3), 256 paths of 1000, 495 / 378; (15, 2), 512 of 1000, 243 / 184.
+                // The reverse sweep alone: (10, 2), 256 of 1000, 94 / 68; (12, 3), 128 of 300, 48 / 35; (9, 4) 57 / 51.
                 constexpr bool kByPiece = BS::kByPiece;
                 constexpr int kLaneStep = kByPiece ? 1 : kGroups, kPieceStep = kByPiece ? kWave : 1;
                 V *mine = reinterpret_cast<V *>(slab) +

@@ -49,3 +49,21 @@ def test_overlapping_windows(d, depth, dtype):
         if end - start > 1:
             want[:, start:end] += TO.signature_vjp(path[:, start:end], G[:, w], depth)
     assert rel_err(grad, want) < TOL[dtype]
+
+
+@pytest.mark.parametrize("d,depth,dtype", [(14, 3, torch.float32), (15, 3, torch.float32), (12, 4, torch.float32),
+                                           (8, 4, torch.float64)])
+def test_an_infinite_gradient_stays_with_its_letters(d, depth, dtype):
+    import pathsig_amd as ps
+    L, word = 12, [0, 2, 1, 0][:depth]
+    x = brownian_path(1, L, d, seed=80 + d).to(dtype).cuda().requires_grad_(True)
+    out = ps.Signature(depth=depth)(x)
+    G = randn(tuple(out.shape), seed=81).to(dtype).cuda()
+    column = sum(d ** k for k in range(1, depth))
+    for k, letter in enumerate(word):
+        column += letter * d ** (depth - 1 - k)
+    G[0, column] = float("inf")
+    (grad,) = torch.autograd.grad(out, x, G)
+    # the words of the other letters do not meet this gradient; its own letters do
+    assert torch.isfinite(grad[..., 3:]).all()
+    assert not torch.isfinite(grad[..., :3]).any(dim=1).all()
