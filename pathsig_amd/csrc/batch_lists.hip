@@ -208,9 +208,7 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
                     T dl[DEG];
 #pragma unroll
                     for (int k = 0; k < DEG; ++k) dl[k] = steps[aoff[i][k] + (tt / 2) * kPair + tt % 2];
-                    T dq[DEG][DEG];
-                    scale_letters<T, DEG>(dl, dq);
-                    chain_step<T, DEG, DEG - 1>(p[i], dq);
+                    chain_step<T, DEG, DEG - 1>(p[i], dl);
                 }
             }
             lds_barrier();
@@ -272,9 +270,7 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
 #pragma unroll
                 for (int k = 0; k < DEG; ++k) dl[k] = both[i][k][tt];
                 // S_t = S_{t+1} (x) exp(-dx_t) on the chain (levels < DEG are all the adjoint needs), and the adjoint
-                T dq[DEG][DEG];
-                scale_letters<T, DEG>(dl, dq);
-                chain_step_adjoint<T, DEG>(p[i], h[i], dl, dq, gl);
+                chain_step_adjoint<T, DEG>(p[i], h[i], dl, gl);
 #pragma unroll
                 for (int k = 0; k < DEG; ++k) to[(i * DEG + k) * kWave] = gl[k];
             }

@@ -56,9 +56,7 @@ __device__ void forward_body(const T *__restrict__ path, T *__restrict__ sig, co
                 T dl[DEG];
 #pragma unroll
                 for (int k = 0; k < DEG; ++k) dl[k] = dxr[l[k]];
-                T dq[DEG][DEG];
-                scale_letters<T, DEG>(dl, dq);
-                chain_step<T, DEG, DEG>(p, dq);
+                chain_step<T, DEG, DEG>(p, dl);
             }
         }
     }
@@ -198,9 +196,7 @@ __device__ void backward_body(const T *__restrict__ path, const T *__restrict__ 
                 T dl[DEG];
 #pragma unroll
                 for (int k = 0; k < DEG; ++k) dl[k] = dxr[l[k]];
-                T dq[DEG][DEG];
-                scale_letters<T, DEG>(dl, dq);
-                chain_step<T, DEG, DEG - 1>(p, dq);
+                chain_step<T, DEG, DEG - 1>(p, dl);
             }
         }
     }
@@ -229,10 +225,8 @@ __device__ void backward_body(const T *__restrict__ path, const T *__restrict__ 
 #pragma unroll
             for (int k = 0; k < DEG; ++k) dl[k] = dxr[l[k]];
             // S_t = S_{t+1} (x) exp(-dx_t) on the chain (levels < DEG are all the adjoint needs), and the adjoint
-            T dq[DEG][DEG];
-            scale_letters<T, DEG>(dl, dq);
             T gl[DEG];
-            chain_step_adjoint<T, DEG>(p, h, dl, dq, gl);
+            chain_step_adjoint<T, DEG>(p, h, dl, gl);
             if (sorted) {
                 T *val = sval + (tt & 1) * (DEG * kBwdBlock);  // two buffers: one barrier per step is enough
 #pragma unroll
