@@ -11,14 +11,11 @@
 // letter and sent to memory by atomics in the order of the output, whole cache lines at a time (atomics from the lanes
 // that add the rows, four paths and a few letters to an instruction, took a third of the kernel's time).
 //
-// 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32: 643 us against 959 us with the cells; fp64 step
-// 1749 against 2368 us.  The chains alone take 70 % of that.  Not bound by memory, nor by the vector ALU's own rate: a
-// SIMD issues a vector instruction every 1.7 ns, where four resident waves can issue one in 0.9.  The LDS works for
-// 0.35 of the 0.64 ms, 36 % of that in bank conflicts (a staged letter is 34 words after the one before, so the parity
-// of a letter decides which half of the banks its 32 words take, and the four words of a wave have letters of their
-// own), and two barriers per two increments and blocks of unequal length (912 on 1024 places) add to it.  The same sums on the matrix cores (16x16x4 fp32, the entries times a matrix of zeros and ones) were built
-// and are slower: fp32 matrix instructions take as long as the vector
-// ALU would for sixteen letters and do not run beside it.
+// 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32: 585 us against 959 us with the cells (step of
+// fp64 1641 against 2368 us).  Not bound by memory, nor by the vector ALU's own rate: four resident waves can issue a vector
+// instruction every 0.9 ns.  Two barriers per two increments and blocks of unequal length (912 on 1024 places) add to the
+// chains.  The same sums on the matrix cores (16x16x4 fp32, the entries times a matrix of zeros and ones) were built and
+// are slower: fp32 matrix instructions take as long as the vector ALU would for sixteen letters and do not run beside it.
 #include <type_traits>
 
 #include "common.hpp"
@@ -35,9 +32,26 @@ constexpr int kThreads = kWaves * kWave;
 constexpr int kLetters = 16;  // at most
 constexpr int kTile = 2;      // increments between barriers: two waves add up the rows of each
 constexpr int kRows = 32;     // rows of entries: sixteen lanes' worth for two waves
-constexpr int kStage = 8;     // increments staged at once
-constexpr int kLetterRow = 2 * kGroup + 2;  // staged increments: [pair][letter][path][increment of the pair]
-static_assert(kTile == 2 && kStage % kTile == 0, "the increments of a tile are read as a pair");
+// Staged increments: [pair][letter][path][increment of the pair].  In fp32 half a wave reads the pairs of two words at once,
+// 32 LDS banks for each: they lie there twice, in the lower 32 banks for the even words of a wave and in the upper 32 for the
+// odd ones, and the paths of a letter are rotated by the letter, so that the lanes that stage neighbouring letters store to
+// different banks.  (Once, 34 elements apart, so that the parity of a letter chose its half of the banks, half the reads met in
+// one: step of the example above 815 us, now 796; a third of the LDS time was bank conflicts.)  In fp64 a word's sixteen
+// pairs fill the banks by themselves.
+template <typename T>
+struct Staged {
+    static constexpr int kCopies = sizeof(T) == 4 ? 2 : 1;
+    static constexpr int kStage = 8 / kCopies;  // increments staged at once: the same room for both types
+    static constexpr int kLetterRow = kCopies == 2 ? 4 * kGroup : 2 * kGroup + 2;
+    static constexpr int kPair = kLetters * kLetterRow;  // from one pair of staged increments to the next
+    static_assert(kStage % kTile == 0 && kStage * kLetters % kWave == 0, "whole tiles and whole waves");
+    // element of the pair of a letter and path that the words of parity `copy` read
+    static __device__ __forceinline__ int at(int letter, int path, int copy) {
+        return kCopies == 2 ? letter * kLetterRow + 2 * kGroup * copy + 2 * ((path + letter) % kGroup)
+                            : letter * kLetterRow + 2 * path;
+    }
+};
+static_assert(kTile == 2, "the increments of a tile are read as a pair");
 static_assert(kTile * kRows * 4 == kThreads, "a thread per increment of the tile, row and four paths");
 
 // Entries of a lane: with twelve, four blocks share a CU's LDS and the registers of four waves to a SIMD suffice
@@ -61,7 +75,7 @@ struct alignas(32) Increment {
 template <typename T>
 struct ListShared {
     Increment<T> inc[kTile];
-    alignas(16) T steps[kStage / 2][kLetters][kLetterRow];
+    alignas(16) T steps[Staged<T>::kStage / 2][Staged<T>::kPair];
     alignas(16) uint32_t place[kRows][kRowLen];    // byte offsets of entries in an increment
     alignas(32) T sums[kTile][kRows][kGroup + 4];       // of the rows, for every path
     int count[kLetters], first_row[kLetters];
@@ -75,7 +89,7 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
                                                    int64_t unit, ListShared<T> &sh) {
     constexpr int WPL = list_words(DEG);
     constexpr int kPaths = kGroup / kWaves;  // paths that a wave stages
-    constexpr int kPair = kLetters * kLetterRow;  // from one pair of staged increments to the next
+    constexpr int kStage = Staged<T>::kStage, kPair = Staged<T>::kPair, kCopies = Staged<T>::kCopies;
     typedef T Pair __attribute__((ext_vector_type(2)));
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const int slot = lane / kGroup, pl = lane % kGroup;
@@ -111,7 +125,7 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
         p[i][0] = T(1);
 #pragma unroll
         for (int k = 0; k < DEG; ++k) {
-            aoff[i][k] = l[k] * kLetterRow + 2 * pl;
+            aoff[i][k] = Staged<T>::at(l[k], pl, slot % kCopies);
             nth[i][k] = have && pl == 0 ? atomicAdd(&sh.count[l[k]], 1) : -1;
             p[i][k + 1] = T(0);
             h[i][k] = T(0);
@@ -146,7 +160,7 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
 #pragma unroll
             for (int k = 0; k < DEG; ++k)
                 if (nth[i][k] >= 0) {
-                    const int to = sh.first_row[aoff[i][k] / kLetterRow] * kRowLen + nth[i][k];
+                    const int to = sh.first_row[aoff[i][k] / Staged<T>::kLetterRow] * kRowLen + nth[i][k];
                     (&sh.place[0][0])[to] =
                         (uint32_t)(((wave * kEntries + i * DEG + k) * kWave + slot * kGroup) * (int)sizeof(T));
                 }
@@ -158,12 +172,13 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
     // issued before them too.)
     constexpr int kChunks = kStage * kLetters / kWave;
     T hi[kPaths][kChunks], lo[kPaths][kChunks];
-    int stage_at[kChunks], stage_step[kChunks];
+    int stage_at[kChunks], stage_step[kChunks], stage_letter[kChunks];
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) {
         const int j = lane + c * kWave, st = j / d;
         stage_step[c] = st;
-        stage_at[c] = (st / 2) * kPair + (j - st * d) * kLetterRow + st % 2 + 2 * wave;
+        stage_letter[c] = j - st * d;
+        stage_at[c] = (st / 2) * kPair + st % 2;
     }
     auto fetch = [&](int64_t t0, int nt) {
 #pragma unroll
@@ -178,15 +193,18 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
             }
         }
     };
-    T *steps = &sh.steps[0][0][0];
+    T *steps = &sh.steps[0][0];
     auto commit = [&](int nt) {
 #pragma unroll
         for (int c = 0; c < kChunks; ++c)
             if (stage_step[c] < nt)
 #pragma unroll
-                for (int pp = 0; pp < kPaths; ++pp)
-                    steps[stage_at[c] + 2 * pp * kWaves] =
-                        b0 + wave + pp * kWaves < shape.B ? hi[pp][c] - lo[pp][c] : T(0);
+                for (int pp = 0; pp < kPaths; ++pp) {
+                    const T dx = b0 + wave + pp * kWaves < shape.B ? hi[pp][c] - lo[pp][c] : T(0);
+#pragma unroll
+                    for (int copy = 0; copy < kCopies; ++copy)
+                        steps[stage_at[c] + Staged<T>::at(stage_letter[c], wave + pp * kWaves, copy)] = dx;
+                }
     };
     const int64_t nstages = (span.steps + kStage - 1) / kStage;
     auto stage_steps = [&](int64_t si) {
