@@ -44,18 +44,44 @@ __device__ void forward_body(const T *__restrict__ path, T *__restrict__ sig, co
 #pragma unroll
     for (int k = 1; k <= DEG; ++k) p[k] = T(0);
 
+    // Increments are staged in pairs, [pair][letter][increment of the pair]: a read, and the address that it takes, bring a
+    // letter of two of them, which matters because a word of length n takes n reads beside some n^2 instructions of its chain.
+    // Forward launch, one increment / two to a read: 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32
+    // 205 / 181 us, fp64 345 / 313; 200 paths of 700, 1020 words up to length 8 over 12 letters, 300 / 279.
+    typedef T Pair __attribute__((ext_vector_type(2)));
+    const int width = (int)d;
+    int at[DEG];
+#pragma unroll
+    for (int k = 0; k < DEG; ++k) at[k] = 2 * l[k];
     for (int64_t t0 = 0; t0 < span.steps; t0 += tile) {
         const int nt = (int)((span.steps - t0) < tile ? (span.steps - t0) : tile);
         const T *xw = x + t0 * d;
         __syncthreads();
-        for (int64_t idx = tid; idx < (int64_t)nt * d; idx += kBlock) sdx[idx] = xw[idx + d] - xw[idx];
+        for (int idx = tid; idx < (nt + 1) / 2 * width; idx += kBlock) {
+            const int pair = (int)((uint32_t)idx / (uint32_t)width);
+            const T *from = xw + (int64_t)pair * d + idx;  // point 2 * pair, letter idx - pair * d
+            const T mid = from[d], first = mid - from[0];
+            const T second = 2 * pair + 1 < nt ? from[2 * d] - mid : T(0);
+            reinterpret_cast<Pair *>(sdx)[idx] = Pair{first, second};
+        }
         __syncthreads();
         if (active) {
-            for (int tt = 0; tt < nt; ++tt) {
-                const T *dxr = sdx + (int64_t)tt * d;
-                T dl[DEG];
+            const T *dxr = sdx;
+            T dl[DEG];
+            for (int tt = 0; tt + 1 < nt; tt += 2, dxr += 2 * width) {
+                Pair both[DEG];
 #pragma unroll
-                for (int k = 0; k < DEG; ++k) dl[k] = dxr[l[k]];
+                for (int k = 0; k < DEG; ++k) both[k] = *reinterpret_cast<const Pair *>(dxr + at[k]);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                    for (int k = 0; k < DEG; ++k) dl[k] = both[k][i];
+                    chain_step<T, DEG, DEG>(p, dl);
+                }
+            }
+            if (nt % 2) {
+#pragma unroll
+                for (int k = 0; k < DEG; ++k) dl[k] = dxr[at[k]];
                 chain_step<T, DEG, DEG>(p, dl);
             }
         }
@@ -405,7 +431,9 @@ hipError_t launch_words_forward(const T *path, T *sig, const SigShape &shape, co
     const int64_t per_row = plan.block_begin[plan.depth + 1];
     const int64_t blocks = per_row * shape.B * shape.W;
     if (blocks == 0) return hipSuccess;
-    const int tile = pick_tile(shape.d, sizeof(T), shape.L - 1, 1, 16384);
+    int tile = pick_tile(shape.d, sizeof(T), shape.L - 1, 1, 16384);
+    // whole pairs (a row of letters takes 8 KB at most, so one always fits)
+    if (tile % 2) tile += (tile + 1) * shape.d * (int64_t)sizeof(T) <= 16384 ? 1 : -1;
     const size_t lds = (size_t)tile * shape.d * sizeof(T);
 #define PSIG_LAUNCH(MAXDEG)                                                                                    \
     hipLaunchKernelGGL((words_forward_kernel<T, MAXDEG>), dim3((unsigned)blocks), dim3(kBlock), lds, stream, path, sig, \
