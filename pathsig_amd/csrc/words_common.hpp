@@ -94,29 +94,41 @@ __device__ __forceinline__ void chain_step(T (&p)[DEG + 1], const T (&dl)[DEG]) 
     }
 }
 
+// Horner values of target level M over what their next product asks for: with r_0 = 1/M and T_J = S(w_1..w_J) + r_(J-1) dl_J,
+// r_J = T_J / (M - J) for J < M.
+template <typename T, int M, int DEG, int J = 1>
+__device__ __forceinline__ void divided_values(const T (&p)[DEG + 1], const T (&dl)[DEG], T (&r)[DEG + 1]) {
+    if constexpr (J == 1) r[0] = Recip<T>::of(M);
+    if constexpr (J < M) {
+        r[J] = fma_t<T>(r[J - 1], dl[J - 1], p[J]);
+        if constexpr (M - J > 1) r[J] *= Recip<T>::of(M - J);
+        divided_values<T, M, DEG, J + 1>(p, dl, r);
+    }
+}
+
 // One Chen step on the chain back, and its adjoint.  p is the chain after the step (levels < DEG) and becomes the one
 // before it; h, the adjoint of the chain after the step, becomes the one before it, and gl[k] holds the step's
 // dL/d(dl[k]).  Targets ascend: h[M] is still the adjoint after the step when target M reads it, and the levels below
 // M have been taken back, so the Horner values of target M are those of the forward step: they serve the adjoint and
-// take level M back, S(w_1..w_M) -= t_(M-1) dl.  The adjoint of t_J is u_J = h[M] dl_(J+1) .. dl_M: letter J gets
-// u_J t_(J-1) of it and the chain u_J / (M - J)!.
-// A word of six letters takes 81 vector instructions (101 with the letters at every scale, 111 rolled back in a pass of its
-// own with exp(-dl)).  256 paths of 512 points, 16 letters, 2320 words up to length 6, us a step, scales on the letters / on
-// the chain: fp32 840 / 815, fp64 1715 / 1665; 1020 words up to length 8 over 12 letters, 200 paths of 700, 1093 / 1080, of it
-// forward 312 / 301.  Gradients against 64 bits are off by 2.0e-6 of their norm both ways, values by 3.6e-7.
+// take level M back, S(w_1..w_M) -= r_(M-1) dl_M.  The adjoint of T_J is v_J = v_(J+1) dl_(J+1) / (M - J): the chain gets
+// v_J of it and letter J v_J r_(J-1).  v and r are divided at every node, so that both stay within what ends up in a
+// result: with products of letters in place of v, divided once at the end, a word of eight letters overflowed 5040 times
+// earlier than its gradient.  The divisions take 10 of 91 vector instructions of a word of six letters (101 with the letters
+// at every scale in their place) and 15 of 781 us a step, 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32.
 template <typename T, int DEG, int M = 1>
 __device__ __forceinline__ void chain_step_adjoint(T (&p)[DEG + 1], T (&h)[DEG + 1], const T (&dl)[DEG], T (&gl)[DEG]) {
     if constexpr (M <= DEG) {
-        T t[DEG + 1];
-        horner_values<T, M, DEG>(p, dl, t);
-        if (M < DEG) p[M] = M == 1 ? p[1] - dl[0] : fma_t<T>(-t[M - 1], dl[M - 1], p[M]);
-        T u = h[M];
-        gl[M - 1] = M == 1 ? u : u * t[M - 1];
+        T r[DEG + 1];
+        divided_values<T, M, DEG>(p, dl, r);
+        if (M < DEG) p[M] = M == 1 ? p[1] - dl[0] : fma_t<T>(-r[M - 1], dl[M - 1], p[M]);
+        T v = h[M];
+        gl[M - 1] = M == 1 ? v : v * r[M - 1];
 #pragma unroll
         for (int j = M - 1; j >= 1; --j) {
-            u *= dl[j];
-            h[j] = M - j == 1 ? h[j] + u : fma_t<T>(u, RecipFactorial<T>::of(M - j), h[j]);
-            gl[j - 1] = fma_t<T>(u, t[j - 1], gl[j - 1]);
+            if (M - j > 1) v *= Recip<T>::of(M - j);
+            v *= dl[j];
+            h[j] += v;
+            gl[j - 1] = fma_t<T>(v, r[j - 1], gl[j - 1]);
         }
         chain_step_adjoint<T, DEG, M + 1>(p, h, dl, gl);
     }
