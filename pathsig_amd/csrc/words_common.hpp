@@ -52,34 +52,18 @@ __device__ __forceinline__ void decode_letters(uint64_t code, uint64_t d, int (&
     }
 }
 
-template <typename T>
-struct RecipFactorial {
-    // 1/k! for k = 1..12 as compile-time constants of type T
-    static __device__ constexpr T of(int k) {
-        double f = 1.0;
-        for (int i = 2; i <= k; ++i) f *= i;
-        return T(1.0 / f);
-    }
-};
-
-// Horner value of target level M after position J of the chain p, over (M - J)!: with t_0 = 1/M!,
-//     t_J = S(w_1..w_J) / (M - J)! + t_(J-1) dl_J   and   S_new(w_1..w_M) = S(w_1..w_M) + t_(M-1) dl_M.
-// The scales are constants on the chain instead of divisors of the letters: two instructions for M - J > 1 and one for
-// M - J = 1, where letters at the M scales that a word asks for take one each beside the one of the node.  The rounded product
-// is the smaller of the two terms.
-template <typename T, int M, int J, int DEG>
-__device__ __forceinline__ T horner_value(const T (&p)[DEG + 1], const T (&dl)[DEG], T before) {
-    if constexpr (M - J > 1) return fma_t<T>(p[J], RecipFactorial<T>::of(M - J), before * dl[J - 1]);
-    else return fma_t<T>(before, dl[J - 1], p[J]);
-}
-
-// Horner values t[1..M-1] of target level M
+// Horner values of target level M over what their next product asks for: with r_0 = 1/M and T_J = S(w_1..w_J) + r_(J-1) dl_J,
+// r_J = T_J / (M - J) for J < M; S_new(w_1..w_M) = S(w_1..w_M) + r_(M-1) dl_M.  Two instructions for M - J > 1 and one for M - J = 1,
+// as many as letters at the M scales that a word asks for would take, and constants in place of those.  (1/(M - J)! in place of
+// 1/(M - J), with r_0 = 1/M!, takes as many: the first of them are 5040 times smaller at depth 8, and a word that begins with
+// an increment below 5e-34 then lost digits to the smallest floats.)
 template <typename T, int M, int DEG, int J = 1>
-__device__ __forceinline__ void horner_values(const T (&p)[DEG + 1], const T (&dl)[DEG], T (&t)[DEG + 1]) {
-    if constexpr (J == 1) t[0] = RecipFactorial<T>::of(M);
+__device__ __forceinline__ void horner_values(const T (&p)[DEG + 1], const T (&dl)[DEG], T (&r)[DEG + 1]) {
+    if constexpr (J == 1) r[0] = Recip<T>::of(M);
     if constexpr (J < M) {
-        t[J] = horner_value<T, M, J, DEG>(p, dl, t[J - 1]);
-        horner_values<T, M, DEG, J + 1>(p, dl, t);
+        r[J] = fma_t<T>(r[J - 1], dl[J - 1], p[J]);
+        if constexpr (M - J > 1) r[J] *= Recip<T>::of(M - J);
+        horner_values<T, M, DEG, J + 1>(p, dl, r);
     }
 }
 
@@ -87,22 +71,10 @@ __device__ __forceinline__ void horner_values(const T (&p)[DEG + 1], const T (&d
 template <typename T, int DEG, int TOP>
 __device__ __forceinline__ void chain_step(T (&p)[DEG + 1], const T (&dl)[DEG]) {
     if constexpr (TOP >= 1) {
-        T t[DEG + 1];
-        horner_values<T, TOP, DEG>(p, dl, t);
-        p[TOP] = TOP == 1 ? p[1] + dl[0] : fma_t<T>(t[TOP - 1], dl[TOP - 1], p[TOP]);
+        T r[DEG + 1];
+        horner_values<T, TOP, DEG>(p, dl, r);
+        p[TOP] = TOP == 1 ? p[1] + dl[0] : fma_t<T>(r[TOP - 1], dl[TOP - 1], p[TOP]);
         chain_step<T, DEG, TOP - 1>(p, dl);
-    }
-}
-
-// Horner values of target level M over what their next product asks for: with r_0 = 1/M and T_J = S(w_1..w_J) + r_(J-1) dl_J,
-// r_J = T_J / (M - J) for J < M.
-template <typename T, int M, int DEG, int J = 1>
-__device__ __forceinline__ void divided_values(const T (&p)[DEG + 1], const T (&dl)[DEG], T (&r)[DEG + 1]) {
-    if constexpr (J == 1) r[0] = Recip<T>::of(M);
-    if constexpr (J < M) {
-        r[J] = fma_t<T>(r[J - 1], dl[J - 1], p[J]);
-        if constexpr (M - J > 1) r[J] *= Recip<T>::of(M - J);
-        divided_values<T, M, DEG, J + 1>(p, dl, r);
     }
 }
 
@@ -119,7 +91,7 @@ template <typename T, int DEG, int M = 1>
 __device__ __forceinline__ void chain_step_adjoint(T (&p)[DEG + 1], T (&h)[DEG + 1], const T (&dl)[DEG], T (&gl)[DEG]) {
     if constexpr (M <= DEG) {
         T r[DEG + 1];
-        divided_values<T, M, DEG>(p, dl, r);
+        horner_values<T, M, DEG>(p, dl, r);
         if (M < DEG) p[M] = M == 1 ? p[1] - dl[0] : fma_t<T>(-r[M - 1], dl[M - 1], p[M]);
         T v = h[M];
         gl[M - 1] = M == 1 ? v : v * r[M - 1];

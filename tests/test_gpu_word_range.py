@@ -32,3 +32,20 @@ def test_gradient_of_large_increments(set_option, B, d, depth, size, upstream):
     want = torch.stack([-letters, letters]).expand(B, 2, d)
     # taking the step back leaves 2^-24 of each prefix value, which weighs binomial(N, m) in a gradient; 4 N roundings
     assert strict_rel_err(grad, want) < (2 ** depth + 4 * depth) * 2 ** -23
+
+
+# A word that begins with an increment close to the smallest normal float, the others large: its value is an ordinary number,
+# and the values on the way to it are not smaller than that increment over the first two divisors of the recurrence,
+# 1.2e-38 / 56 = 1.5e5 steps of the smallest float: relative 3e-6, and 1e-6 of ordinary roundings.
+@pytest.mark.parametrize("depth,size", [(8, 1e4), (6, 1e5)])
+def test_value_of_a_word_that_begins_small(set_option, depth, size):
+    import pathsig_amd as ps
+    set_option("tiled", 0)
+    B, d = 40, 3
+    proj = ps.projections.words([(0,) + (1,) * (depth - 1)], depth=depth, path_dim=d)
+    path = torch.zeros(B, 2, d)
+    path[:, 1, 0] = torch.logspace(math.log10(1.2e-38), -36, B, dtype=torch.float64).float()
+    path[:, 1, 1] = size
+    out = ps.Signature(depth=depth, projection=proj)(path.cuda())[:, 0].double().cpu()
+    want = path[:, 1, 0].double() * size ** (depth - 1) / math.factorial(depth)
+    assert float(((out - want).abs() / want).max()) < 1e-5
