@@ -1662,28 +1662,41 @@ __global__ void __launch_bounds__(kWave) chunk_level1_kernel(const T *__restrict
 // gathered there the lanes read the slab back across the lanes, eight 16-byte reads each, and leave eight
 // partial sums per increment and letter in `sg`.
 // Units of five to eight waves do so too where a lane's state leaves no more than two waves to a SIMD: one such block
-// then fills a CU whatever LDS it takes.  (8, 5), fp32, 256 paths of 2048 points: reverse sweep 1734 -> 1588 us (307
-// -> 293 vector instructions per increment and wave); letters 16 bytes apart instead of 32, which halves the bank
-// conflicts, 1631.
+// then fills a CU whatever LDS it takes.  (8, 5), fp32, 256 paths of 2048 points: reverse sweep 1666 -> 1601 us (1722 ->
+// 1617 with the signature taken back in a pass of its own; 307 -> 293 vector instructions per increment and wave); letters 16
+// bytes apart instead of 32, which halves the bank conflicts, are slower by 43.  Up to 110 values below a prefix: with the 132
+// of eleven letters the slab form spills (15 registers, none with DPP; (11, 5), 128 paths of 65 points, 221 / 233 us).
 // fp64: the exchanges move two registers to a value, the slab 16 bytes to two letters, and the chain's terms are added
-// to the lane's row there.  It pays from seven letters on, with eight values to exchange, and over two: a step of 512
-// paths of 2000 points, us, DPP / slab: (7, 2) 489 / 372, (8, 3) 543 / 480, (10, 2) 726 / 570, (9, 3) 1640 / 1268,
-// (2, 4) 267 / 249; (8, 5) with letter bounds, 128 of 1024, 951 / 905.  Not over three to six letters ((4, 3) 244 /
-// 332, (6, 3) 315 / 375) nor, with sixteen padded letters, for thirteen letters and more at depth 3 ((15, 3) 1388 /
-// 1483) and nine and more at depth 4 and 5 ((9, 4) 526 / 570).
-template <typename T, int D, int N, int P, int MAXW = 0>
+// to the lane's row there.  It pays from seven letters on, with eight values to exchange.  Reverse sweep, us, DPP / slab:
+// 512 paths of 300 points (7, 2) 74 / 49, (8, 3) 83 / 73, (10, 2) 109 / 98, (11, 3) 262 / 160; 32768 rows of 64 points
+// (8, 3) 687 / 575, (11, 3) 2396 / 1896, (14, 2) 1164 / 779.  Over two and twelve letters it pays as long as a CU has few
+// waves, which rows cut into chunks see to: (2, 4), 512 of 300, 41 / 37, (12, 3), 64 of 300, 38 / 33; where the rows or
+// windows are many, the 8 KB to a wave keep others out that small states would let in: (2, 3), 32768 rows of 64 points, 196 /
+// 255, as windows 197 / 254, 480 windows of 64 10.7 / 12.7; (12, 3) 2419 / 2812, 2414 / 2782, 54 / 58; from depth 8 on the state
+// of two letters lets no more in ((2, 8) windows 987 / 942).  Over nine at depth 2 windows in one piece alone lose (792 / 852,
+// in rows 764 / 749).  Not over three to six letters (512 of 1000 points: (4, 3) 104 / 142, (6, 3) 137 / 148; but (6, 4) 400 /
+// 238, its windows 85 / 66, so the line is not drawn for every depth here), nor at depth 4 and 5 from nine letters on
+// ((9, 4), 128 of 300, 123 / 132; (10, 4) 174 / 178), nor for thirteen and more at depth 3, where either side wins: 512 of 1000
+// 922 / 845, (14, 3) 1078 / 1020, and windows of (14, 3) 223 / 247.
+// ACCUMULATE, CHUNKED, MAXW: as for the kernel.
+template <typename T, int D, int N, int P, bool ACCUMULATE, bool CHUNKED, int MAXW = 0>
 struct BackwardShape {
     using G = Geometry<D, N, P, sizeof(T), MAXW>;
     static constexpr int KS = N - P;
     static constexpr int kVW = 16 / (int)sizeof(T);  // letters of a 16-byte piece
     // letters padded to a power of two of whole 16-byte pieces
     static constexpr int kDP = D <= kVW ? kVW : D <= 4 ? 4 : D <= 8 ? 8 : 16;
+    static constexpr bool kFewWaves = CHUNKED && !ACCUMULATE;  // (rows cut so that two waves to a SIMD come of them)
     static constexpr bool kSlabLetters =
-        sizeof(T) == 4 || D == 2 || D == 7 || D == 8 || (D >= 9 && (N == 2 || (N == 3 && D <= 12)));
+        sizeof(T) == 4 || (D == 2 && (N >= 8 || kFewWaves)) || D == 7 || D == 8 ||
+        (D == 9 && N == 2 && (CHUNKED || !ACCUMULATE)) || (D >= 10 && N == 2) || ((D >= 9 && D <= 11) && N == 3) ||
+        (D == 12 && N == 3 && kFewWaves);
     static constexpr bool kSlab = kSlabLetters && D <= 15 && !G::kSplit &&
-                                  (G::kWaves <= 4 || (G::kWaves <= 8 && G::kSubTrie > 40));
+                                  (G::kWaves <= 4 || (G::kWaves <= 8 && G::kSubTrie > 40 && G::kSubTrie <= 110));
     static constexpr int kGroups = kDP / kVW;      // 16-byte pieces per lane and increment
-    static constexpr bool kByPiece = sizeof(T) == 8 || kGroups >= 4;  // layout of the slab: [piece][lane]
+    // layout of the slab: [piece][lane].  (fp32 not over thirteen letters at depth 5, where it leaves a lane 214 registers in the
+    // upper half instead of 56: 32 paths of 65 points 256 us, side by side 228.)
+    static constexpr bool kByPiece = sizeof(T) == 8 || (kGroups >= 4 && !(D == 13 && N == 5));
     static constexpr int kSubTile = 8 / kGroups;   // increments that wait in the slab: 8, 4, 2 or 1 (8 KB per wave)
     static constexpr int kSlabElems = kSlab ? G::kWaves * kSubTile * kWave * kDP : 4;
     static constexpr int kParts = kSlab ? 8 : 4;
@@ -1724,18 +1737,17 @@ struct BackwardShape {
 // its own / shared: fp32 (8, 5), 256 paths of 2048 points, 1728 / 1691; (4, 6), 128 of 1024, 88.8 / 85.2; (3, 6), 4 of
 // 20001, 177 / 167; (6, 5), 64 of 2048 in windows of 64, 340 / 335; (8, 5) with letter bounds 337 / 327; fp64 (6, 5) 95.3 /
 // 90.9, (3, 6) 54.5 / 50.8, (8, 4) 123.5 / 120.6.  Not shared: see run_backward.
-template <typename T, int D, int N, int P, bool ACCUMULATE, bool CHUNKED, int BOUND, int MAXW = 0, bool SHARED = true>
+template <typename T, int D, int N, int P, bool ACCUMULATE, bool CHUNKED, int BOUND, int MAXW = 0, bool SHARED = true,
+          typename BS = BackwardShape<T, D, N, P, ACCUMULATE, CHUNKED, MAXW>>
 __device__ __forceinline__ void dense_backward_body(
     const T *__restrict__ path, const T *__restrict__ sig, const T *__restrict__ grad_sig, const T *__restrict__ edgeA,
     const T *__restrict__ edgeZ, T *__restrict__ grad_inc, const SigShape &shape, int chunks, T *__restrict__ grad_path,
     const int pu_unit,  // index of the thread within its unit (its prefix, unless the first level is split)
     const int tid,      // index of the thread within its block
-    T (&sdx_all)[BackwardShape<T, D, N, P, MAXW>::kStage],
-    T (&sg)[BackwardShape<T, D, N, P, MAXW>::kSums][BackwardShape<T, D, N, P, MAXW>::kSumRow],
-    T (&cells)[BackwardShape<T, D, N, P, MAXW>::kCells], T (&slab)[BackwardShape<T, D, N, P, MAXW>::kSlabElems], T (&carry)[D],
+    T (&sdx_all)[BS::kStage], T (&sg)[BS::kSums][BS::kSumRow], T (&cells)[BS::kCells], T (&slab)[BS::kSlabElems],
+    T (&carry)[D],
     const T *__restrict__ edgeL = nullptr, const T *__restrict__ edgeR = nullptr) {
     using G = Geometry<D, N, P, sizeof(T), MAXW>;
-    using BS = BackwardShape<T, D, N, P, MAXW>;
     constexpr int KS = N - P;
     constexpr int kParts = BS::kParts;
     constexpr int kBwdTile = BS::kBwdTile;
@@ -2237,7 +2249,7 @@ __global__ void __launch_bounds__((Geometry<D, N, P, sizeof(T), MAXW>::kBlock))
                           SigShape shape, int chunks, T *__restrict__ grad_path = nullptr,
                           const int *__restrict__ bounds = nullptr, const T *__restrict__ edgeL = nullptr,
                           const T *__restrict__ edgeR = nullptr) {
-    using BS = BackwardShape<T, D, N, P, MAXW>;
+    using BS = BackwardShape<T, D, N, P, ACCUMULATE, CHUNKED, MAXW>;
     static_assert(!BOUNDED || LetterBounds<D, P>::kUsable, "letter bounds need one first letter per wave");
     __shared__ __align__(16) T sdx[BS::kStage];
     __shared__ __align__(16) T sg[BS::kSums][BS::kSumRow];
@@ -2379,7 +2391,7 @@ constexpr bool grouped_handover_ok() {
         return false;
     } else {
         using G = Geometry<D, N, P, 4>;
-        using BS = BackwardShape<float, D, N, P>;
+        using BS = BackwardShape<float, D, N, P, false, true>;  // (the sweep that takes the groups)
         constexpr bool staged = 2 * Geometry<D, N, PC>::kSigSize * sizeof(float) <= 48 * 1024;
         return ForwardShape<float, D, N, P, 4>::kGrouped && G::kBlock * 4 <= 1024 && staged &&
                EdgesShape<float, D, N, PS, PC>::kUsable && scan_fits<float, D, N, PS>() && BS::kSlab &&
@@ -2930,7 +2942,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         // (letter blocks: twice the waves that fit the GPU at once, so that the short ones fill in behind the long)
         const int64_t want_waves = dc.bounded && elem == 4 ? 4096 : 2048;
         int chunks = pick_chunks(rows, v.block, L, want_waves, many && may_chain);
-        // deep fp32 shapes: the reverse sweep rebuilds A_t = A_{t+1} (x) exp(-dx_t) step by step, and over a span of
+        // deep fp32 shapes: the reverse sweep rebuilds A_t from A_{t+1} step by step, and over a span of
         // large increments that roll-back loses digits at depth 9 and more (d = 2, depth 12, five increments of
         // size 0.8: gradient off by 1.5e-5 in one piece, 1e-6 in two or more); four chunks at least
         if (elem == 4 && depth >= 9 && chunks < 4) chunks = (int)std::max<int64_t>(1, std::min<int64_t>(4, L - 1));
