@@ -1727,16 +1727,30 @@ struct BackwardShape {
     // constants instead where those fit the register file.
     static constexpr bool kChainCells = sizeof(T) == 8 && !kSlab && D <= 8 && D * G::kBlock * (int)sizeof(T) <= 32 * 1024;
     static constexpr int kCells = kChainCells ? D * G::kBlock : 1;
+    // The signature is taken back inside the adjoint (see SHARED below) up to sixteen letters.  Not where the levels of A that are
+    // held until their target comes leave the registers: us, inside / in a pass of its own, fp64 (8, 5) 256 paths of 300 points
+    // 493 / 463 (in 120 windows of 64 101 / 103), (8, 6) 32 of 65 184 / 158, (11, 5) 304 / 288; fp32 (15, 4) in chunks 256 of 300
+    // 1382 / 1241, 120 windows of 64 214 / 206, (14, 4) 7232 windows 4368 / 4051 (in chunks 623 / 649; rows of (15, 4) in one piece
+    // 5445 / 5788).  Over wider alphabets a roll-back is little beside the top level, and either side wins by how its
+    // registers fall: 8 paths of 257 points (30, 3) 595 / 526, fp64 (25, 4) 1302 / 1116, (24, 4) 1118 / 1008, the other way round
+    // fp64 (32, 4) 1746 / 1822, (28, 4) 487 / 501; but fp64 at depth 3 from 28 to 64 letters inside, (64, 3) 995 / 1097, 120
+    // windows of (32, 3) 202 / 362, the others even.
+    static constexpr bool kWideState = G::kSubTrie > 200 && N == 4;  // (14 and 15 letters, prefixes of two)
+    static constexpr bool kFitsInside =
+        G::kLetterBlocks ||
+        (sizeof(T) == 4 ? !(kWideState && (ACCUMULATE || (CHUNKED && D == 15)))
+                        : !((D == 8 && (N >= 6 || (N == 5 && !ACCUMULATE))) || (D == 11 && N == 5)));
+    static constexpr bool kTakenBackInside = D <= 16 ? kFitsInside : sizeof(T) == 8 && N == 3 && D >= 28 && D <= 64;
 };
 
 // BOUND: the upstream gradient is zero on every top-level word that has a letter below BOUND after the
 // prefix's first letter, and the sweep leaves those words out; the LDS arrays belong to the calling kernel.
 // SHARED: A_t = A_{t+1} (x) exp(-dx_t) is taken back target by target inside the adjoint of the step, on the Horner values
 // that the adjoint computes anyway (AdjTargets: BACK), in place of a pass with exp(-dx) that computes such values of its
-// own: 12 of 293 vector instructions less per increment for (8, 5), 22 of some 260 for (4, 6).  Reverse sweeps, us, a pass of
-// its own / shared: fp32 (8, 5), 256 paths of 2048 points, 1728 / 1691; (4, 6), 128 of 1024, 88.8 / 85.2; (3, 6), 4 of
-// 20001, 177 / 167; (6, 5), 64 of 2048 in windows of 64, 340 / 335; (8, 5) with letter bounds 337 / 327; fp64 (6, 5) 95.3 /
-// 90.9, (3, 6) 54.5 / 50.8, (8, 4) 123.5 / 120.6.  Not shared: see run_backward.
+// own.  Reverse sweeps, us, a pass of its own / shared: fp32 (8, 5), 256 paths of 2048 points, 1617 / 1601 (with the sums by
+// DPP 1722 / 1666); (4, 6), 128 of 1024, 85.5 / 82.8; (3, 6), 8 of 4001, 27.3 / 26.3; (6, 5), 64 of 2048 in windows of 64, 323 /
+// 320; (8, 5) with letter bounds 337 / 327; (2, 8), 512 of 300, 62.1 / 56.0; fp64 (3, 6) 98 / 92, (5, 6), 256 of 300, 517 / 487.  Not shared: BackwardShape::kTakenBackInside, and
+// the launches of run_backward.
 template <typename T, int D, int N, int P, bool ACCUMULATE, bool CHUNKED, int BOUND, int MAXW = 0, bool SHARED = true,
           typename BS = BackwardShape<T, D, N, P, ACCUMULATE, CHUNKED, MAXW>>
 __device__ __forceinline__ void dense_backward_body(
@@ -1748,6 +1762,7 @@ __device__ __forceinline__ void dense_backward_body(
     T (&carry)[D],
     const T *__restrict__ edgeL = nullptr, const T *__restrict__ edgeR = nullptr) {
     using G = Geometry<D, N, P, sizeof(T), MAXW>;
+    constexpr bool kInside = SHARED && BS::kTakenBackInside;
     constexpr int KS = N - P;
     constexpr int kParts = BS::kParts;
     constexpr int kBwdTile = BS::kBwdTile;
@@ -1964,7 +1979,7 @@ __device__ __forceinline__ void dense_backward_body(
         const T *sdx = sdx_all + (t0 - staged_from) * (KS * D);
         lds_barrier();
         auto step = [&](int tt, const T (&dxs)[KS][D], const T (&dxp)[P], const T (&dxf)[FQ][FK]) {
-            if constexpr (!SHARED) {
+            if constexpr (!kInside) {
                 // A_t = A_{t+1} (x) exp(-dx_t), levels < N
                 if constexpr (G::kSplit)
                     StepTargets<T, D, P, N - 1, true, 0, KF>::template run<kAS, KS>(a, asub, dxs, dxf, dxp);
@@ -1984,10 +1999,10 @@ __device__ __forceinline__ void dense_backward_body(
 #pragma unroll
             for (int j = 0; j < P; ++j) gpre[j] = T(0);
             if constexpr (G::kSplit)
-                AdjTargets<T, D, N, P, 1, BOUND, KF, SHARED>::template run<kAS, G::kFwdSub, KS>(a, asub, hc, hsub, dxs, dxf, dxp,
+                AdjTargets<T, D, N, P, 1, BOUND, KF, kInside>::template run<kAS, G::kFwdSub, KS>(a, asub, hc, hsub, dxs, dxf, dxp,
                                                                                         gdxk, gdxf, gpre);
             else
-                AdjTargets<T, D, N, P, 1, BOUND, D, SHARED>::template run<kAS, G::kFwdSub, KS>(a, asub, hc, hsub, dxs, dxs, dxp,
+                AdjTargets<T, D, N, P, 1, BOUND, D, kInside>::template run<kAS, G::kFwdSub, KS>(a, asub, hc, hsub, dxs, dxs, dxp,
                                                                                     gdxk, gdxk, gpre);
             // letter k collects the sub-trie sums (with the 1/(q+1) of their increments) and the chain
             // positions whose letter is k
@@ -2468,16 +2483,20 @@ constexpr int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
 size_t pad256(size_t n) { return (n + 255) / 256 * 256; }
 
-// fp32 calls keep to 64 chunks, to one product after the other and to a roll-back of its own beyond this length: a
-// cautious limit, not one that precision asks for.  A path gradient is the difference of neighbouring increment sums,
+// fp32 calls without windows whose rows are longer than this and cut into chunks keep to 64 chunks and to one product after
+// the other, and their sweeps take the signature back in a pass of its own: a cautious limit, not one that precision asks
+// for, which keeps the results of the long rows that few chunks serve.  It holds nothing else in place: rows in one piece,
+// windows and letter blocks of any length take the signature back inside the adjoint, and the letter sums of some shapes are
+// added in another order than they were, at any length.  A path gradient is the difference of neighbouring increment sums,
 // sqrt(L) times smaller than they are for a Brownian path, so fp32 gradients are off by about 1e-7 sqrt(L) of their
 // norm, and two ways of cutting a path differ by as much from each other.  Against 64 bits neither is the better one:
 // (3, 6), 4 paths of 20001 points, largest error of three draws 1.10e-5 with 64 chunks (values 3.6e-7) and 1.10e-5 with
-// 512 in chains (1.0e-7); (2, 8) 1.25e-5 both, (4, 4) 1.08e-5 both, (5, 5), 2 of 10001, 9.3e-6 and 9.4e-6.  What the
-// limit costs, us a step: 302 against 135, 288 against 139, 135 against 85, 162 against 83; (3, 6) 120 against 73 at
-// 4098 points, so there is a step in time at 4097 increments.  The other way round (8, 3), 8 of 12001: 100 us here, 107
-// without the limit. The shared roll-back alone would take 10 of the 177 us of the reverse sweep at (3, 6).
-constexpr int64_t kSameBitsFromSteps = 4096;
+// 512 in chains (1.0e-7); (2, 8) 1.25e-5 both, (4, 4) 1.08e-5 both, (5, 5), 2 of 10001, 9.3e-6 and 9.4e-6; nor of the two
+// ways back: (3, 6), 2 of 9001 in one piece, 1.04e-5 in a pass of its own and 1.02e-5 inside, (2, 8) 1.34e-5 and 1.35e-5, (8, 5)
+// 8.7e-6 and 8.6e-6.  What the limit costs, us a step: 302 against 135, 288 against 139, 135 against 85, 162 against 83;
+// (3, 6) 120 against 73 at 4098 points, so there is a step in time at 4097 increments.  The other way round (8, 3), 8 of
+// 12001: 100 us here, 107 without the limit, which the estimate of make_dense_choice would have to see first.
+constexpr int64_t kLongRowSteps = 4096;
 
 #if PSIG_GROUP < 0
 struct SweepProfile {
@@ -2835,9 +2854,9 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
                                        dim3((unsigned)units), dim3(G::kBlock), 0, stream, path, sig, grad_sig, dumpA, dumpH,
                                        grad_inc, shape, chunks, grad_path, (const int *)nullptr, edgeL, edgeR);
                 };
-                if constexpr (sizeof(T) == 4) {
-                    // Rows beyond kSameBitsFromSteps keep the order of operations that they had: see there.
-                    if (shape.L - 1 > kSameBitsFromSteps) launch(std::false_type{});
+                if constexpr (sizeof(T) == 4 && BackwardShape<T, D, N, P, false, true>::kTakenBackInside) {
+                    // (longer rows: see kLongRowSteps)
+                    if (shape.L - 1 > kLongRowSteps) launch(std::false_type{});
                     else launch(std::true_type{});
                 } else {
                     launch(std::true_type{});
@@ -2930,7 +2949,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         // in fp64
         const double step_us = (0.2 + 0.013 * v.sub_size) * (elem == 8 ? 2.0 : 1.0);
         const double low_bytes = (double)v.low_size * elem;
-        const bool may_chain = !plain && (elem == 8 || L - 1 <= kSameBitsFromSteps);
+        const bool may_chain = !plain && (elem == 8 || L - 1 <= kLongRowSteps);
         bool many = false;  // more than 64 chunks
         if (chunks_ok && !windowed && L - 1 > 2048) {
             // what the shorter sweeps save against what the longer chains of products cost
