@@ -361,7 +361,7 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
     return PATHSIG_OK;
 }
 
-// Deep fp32 calls.  The reverse sweep rebuilds the signature of every earlier time by multiplying with exp(-dx_t),
+// Deep fp32 calls.  The reverse sweep rebuilds the signature of every earlier time from that of the later one,
 // and the gradient of a top-level coefficient sums thousands of terms of mixed sign: from depth 9 on, fp32 rounding
 // in those two places passes 1e-5 of the largest gradient (over a span of increments of size one, swept in one
 // piece: 1.0e-5 to 1.5e-5 at depth 9, up to 3.5e-5 at depth 12).  Such a backward runs in fp64 on copies of the

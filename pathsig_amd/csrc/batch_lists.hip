@@ -11,8 +11,8 @@
 // letter and sent to memory by atomics in the order of the output, whole cache lines at a time (atomics from the lanes
 // that add the rows, four paths and a few letters to an instruction, took a third of the kernel's time).
 //
-// 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32: 585 us against 959 us with the cells (step of
-// fp64 1641 against 2368 us).  Not bound by memory, nor by the vector ALU's own rate: four resident waves can issue a vector
+// 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32: 599 us against 959 us with the cells (fp64,
+// forward and backward, 1631 against 2368 us).  Not bound by memory, nor by the vector ALU's own rate: four resident waves can issue a vector
 // instruction every 0.9 ns.  Two barriers per two increments and blocks of unequal length (912 on 1024 places) add to the
 // chains.  The same sums on the matrix cores (16x16x4 fp32, the entries times a matrix of zeros and ones) were built and
 // are slower: fp32 matrix instructions take as long as the vector ALU would for sixteen letters and do not run beside it.
@@ -36,7 +36,8 @@ constexpr int kRows = 32;     // rows of entries: sixteen lanes' worth for two w
 // 32 LDS banks for each: they lie there twice, in the lower 32 banks for the even words of a wave and in the upper 32 for the
 // odd ones, and the paths of a letter are rotated by the letter, so that the lanes that stage neighbouring letters store to
 // different banks.  (Once, 34 elements apart, so that the parity of a letter chose its half of the banks, half the reads met in
-// one: step of the example above 815 us, now 796; a third of the LDS time was bank conflicts.)  In fp64 a word's sixteen
+// one: step of the example above 815 us, in both halves 796; LDS clocks lost to conflicts 78 -> 59 M of 216 -> 201 M, the rest of
+// them where the rows of entries are read and stored.)  In fp64 a word's sixteen
 // pairs fill the banks by themselves.
 template <typename T>
 struct Staged {

@@ -1929,7 +1929,7 @@ __device__ __forceinline__ void dense_backward_body(
     a[0] = T(1);
     // onehot[j][k] = 1 when the j-th letter of the lane's prefix is k (kept in registers only where
     // registers are plentiful; otherwise the letters are compared every time, which also keeps an infinite term of one
-    // letter out of the sums of the others)
+    // letter out of the sums of the others, where a product with zero carries it into them as NaN)
     constexpr bool kOneHot = sizeof(T) == 4 && P * D <= 24;
     T onehot[kOneHot ? P : 1][kOneHot ? D : 1];
     // Wide alphabets compare every letter with the prefix letters to route the chain's terms (P * D selects and

@@ -5,10 +5,11 @@
 // A lane that owns the word w = (w_1..w_n) carries the signature values of the prefixes of w
 // (a chain of n+1 numbers) and sweeps the window once.  Per increment it evaluates, for every
 // target level m = n..1, the Horner chain
-//     s_1 = 1/m,  tmp_j = p_j + s_j * dx[w_j],  s_{j+1} = tmp_j / (m - j),   p_m += s_m * dx[w_m]
+//     r_0 = 1/m,  T_j = p_j + r_{j-1} * dx[w_j],  r_j = T_j / (m - j),   p_m += r_{m-1} * dx[w_m]
 // which is S <- S (x) exp(dx) restricted to the chain (reference: src/pathsig/forward/sig_kernels.cu:129-154).
-// The backward lane carries the chain rolled back with exp(-dx) and the adjoint of the chain, and
-// back-propagates through the same Horner chains; this needs O(n^2) work per increment
+// The backward lane carries the chain and its adjoint and takes both back an increment at a time: target by target, the
+// Horner values of the forward step serve the adjoint and return the chain to what it was before the step
+// (words_common.hpp); this needs O(n^2) work per increment
 // (the reference assembles prefix x segment x suffix products in O(n^3),
 // src/pathsig/backward/sig_backward_kernels.cu:204-253).  Increments of a tile of time steps are
 // staged once per block in LDS; per-letter gradient sums are collected in LDS and flushed to the
