@@ -48,9 +48,11 @@ __device__ void forward_body(const T *__restrict__ path, T *__restrict__ sig, co
     // Increments are staged in pairs, [pair][letter][increment of the pair]: a read, and the address that it takes, bring a
     // letter of two of them, which matters because a word of length n takes n reads beside some n^2 instructions of its chain.
     // Forward launch, one increment / two to a read: 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32
-    // 205 / 181 us, fp64 345 / 313; 200 paths of 700, 1020 words up to length 8 over 12 letters, 300 / 279.
+    // 205 / 181 us, fp64 345 / 313; 200 paths of 700, 1020 words up to length 8 over 12 letters, 300 / 279.  (The letter and pair
+    // of an element are carried along: a division for each costs 3 of 34 us over 100 letters, 2000 words, 256 paths of 128.)
     typedef T Pair __attribute__((ext_vector_type(2)));
     const int width = (int)d;
+    const int first_letter = tid % width, first_pair = tid / width;
     int at[DEG];
 #pragma unroll
     for (int k = 0; k < DEG; ++k) at[k] = 2 * l[k];
@@ -58,9 +60,13 @@ __device__ void forward_body(const T *__restrict__ path, T *__restrict__ sig, co
         const int nt = (int)((span.steps - t0) < tile ? (span.steps - t0) : tile);
         const T *xw = x + t0 * d;
         __syncthreads();
-        for (int idx = tid; idx < (nt + 1) / 2 * width; idx += kBlock) {
-            const int pair = (int)((uint32_t)idx / (uint32_t)width);
-            const T *from = xw + (int64_t)pair * d + idx;  // point 2 * pair, letter idx - pair * d
+        int letter = first_letter, pair = first_pair;  // of element idx
+        for (int idx = tid; idx < (nt + 1) / 2 * width; idx += kBlock, letter += kBlock % width, pair += kBlock / width) {
+            if (letter >= width) {
+                letter -= width;
+                ++pair;
+            }
+            const T *from = xw + (int64_t)pair * 2 * d + letter;
             const T mid = from[d], first = mid - from[0];
             const T second = 2 * pair + 1 < nt ? from[2 * d] - mid : T(0);
             reinterpret_cast<Pair *>(sdx)[idx] = Pair{first, second};
