@@ -1,4 +1,4 @@
-"""Per-increment sums over the letters in the reverse sweep, against the CPU checker: the lanes leave their terms in a slab
+"""Per-increment sums over the letters in the reverse sweep, against the oracle: the lanes leave their terms in a slab
 in LDS (fp32 up to fifteen letters, fp64 over the alphabets where that is the faster way) or exchange them."""
 import pytest
 import torch

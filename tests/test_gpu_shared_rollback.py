@@ -1,6 +1,6 @@
 """Reverse sweep: the signature is taken back inside the adjoint of a step, or in a pass of its own (rows of more than 4096
 increments in time chunks in fp32; shapes whose state would not fit the registers; wide alphabets).  Both sides of that
-length and rows that are not cut, against the CPU checker."""
+length and rows that are not cut, against the oracle."""
 import pytest
 import torch
 
