@@ -211,6 +211,47 @@ __global__ void __launch_bounds__(kTopWaves *kWave)
     }
 }
 
+// Adjoints of the chunks.  Grid: x over (row, chunk), y over slices of the words.  A word of level m sums over the d + d^2 +
+// .. + d^(depth - m) words that continue it: by a group of lanes, as many as that number keeps at work, the more the fewer
+// words a level has.  Bandwidth of L2: every level is read once per shorter level.
+template <typename T>
+__global__ void __launch_bounds__(kChainThreads)
+    chunk_adjoints_kernel(const T *__restrict__ grad, const T *__restrict__ right, T *__restrict__ out, int n, ChainLevels lv) {
+    const uint32_t unit = blockIdx.x, row = unit / (uint32_t)n;
+    const int depth = lv.depth;
+    const int64_t all = (int64_t)lv.low + lv.width[depth];
+    const T *g = grad + row * all;
+    const T *z = right + (int64_t)unit * lv.low;
+    T *to = out + (int64_t)unit * all;
+    const uint32_t tid = blockIdx.y * kChainThreads + threadIdx.x, threads = gridDim.y * kChainThreads;
+    if (unit - row * (uint32_t)n == (uint32_t)n - 1) {
+        // nothing follows the last chunk (and a product with what is zero there would turn an infinite gradient into NaN)
+        for (int64_t i = tid; i < all; i += threads) to[i] = g[i];
+        return;
+    }
+    for (uint32_t i = tid; i < lv.width[depth]; i += threads) to[lv.low + i] = g[lv.low + i];
+    uint32_t longer = 0;
+    for (int m = depth - 1; m >= 1; --m) {
+        longer += lv.width[depth - m];
+        const uint32_t lanes = longer >= 256 ? kWave : longer >= 32 ? 16 : longer >= 8 ? 4 : 1;
+        const uint32_t part = tid % lanes, step = threads / lanes;
+        // (whole waves stay together: the shuffles below need all lanes of a group)
+        for (uint32_t w = tid / lanes; w < (lv.width[m] + step - 1) / step * step; w += step) {
+            T sum = T(0);
+            if (w < lv.width[m]) {
+                for (int q = 1; q <= depth - m; ++q) {
+                    const T *from = g + lv.off[m + q] + w * lv.width[q], *by = z + lv.off[q];
+                    T level = T(0);
+                    for (uint32_t s = part; s < lv.width[q]; s += lanes) level += from[s] * by[s];
+                    sum += level;
+                }
+            }
+            for (uint32_t o = lanes / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, (int)o, kWave);
+            if (part == 0 && w < lv.width[m]) to[lv.off[m] + w] = g[lv.off[m] + w] + sum;
+        }
+    }
+}
+
 }  // namespace
 
 namespace {
@@ -330,7 +371,34 @@ hipError_t launch_chain_top(const T *elements, int64_t stride, const ChainLeft<T
     });
 }
 
+namespace {
+// blocks to a chunk: enough for a few thousand waves, none without 1024 words of its own
+unsigned adjoint_slices(int64_t units, uint32_t top) {
+    int64_t slices = 1;
+    while (slices * units < 2048 && slices * 2048 <= (int64_t)top) slices *= 2;
+    return (unsigned)slices;
+}
+}  // namespace
+
+template <typename T>
+hipError_t launch_chunk_adjoints(const T *grad, const T *right, T *out, int64_t rows, int n, int64_t d, int depth,
+                                 hipStream_t stream) {
+    ChainLevels lv;
+    if (!chain_levels(d, depth, &lv)) return hipErrorNotSupported;
+    hipLaunchKernelGGL(chunk_adjoints_kernel<T>, dim3((unsigned)(rows * n), adjoint_slices(rows * n, lv.width[depth])),
+                       dim3(kChainThreads), 0, stream, grad, right, out, n, lv);
+    return hipGetLastError();
+}
+
+// 4 us, and what it reads and writes at 4 TB/s
+double chunk_adjoints_us(size_t elem, int64_t rows, int n, int64_t d, int depth) {
+    ChainLevels lv;
+    if (!chain_levels(d, depth, &lv)) return 1e9;
+    return 4.0 + 0.25e-6 * (double)rows * n * lv.width[depth] * (depth + 1) * (double)elem;
+}
+
 #define PSIG_INSTANTIATE(T)                                                                                         \
+    template hipError_t launch_chunk_adjoints<T>(const T *, const T *, T *, int64_t, int, int64_t, int, hipStream_t); \
     template hipError_t launch_chain<T>(const T *, int64_t, int64_t, int, int64_t, int, T *, bool, T *, T *, int64_t, \
                                         T *, int64_t, hipStream_t);                                                 \
     template hipError_t launch_chain_top<T>(const T *, int64_t, const ChainLeft<T> &, T *, int64_t, int64_t, int, int64_t, int, \

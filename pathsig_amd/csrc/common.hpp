@@ -226,6 +226,12 @@ struct ChainLeft {
 template <typename T>
 hipError_t launch_chain_top(const T *elements, int64_t stride, const ChainLeft<T> &left, T *out, int64_t out_stride, int64_t rows,
                             int n, int64_t d, int depth, hipStream_t stream);
+// Adjoint at the right edge of every chunk: out[row, c](w) = sum over s of grad[row](w s) right[row, c](s), with right the
+// product of the chunks after c below the top level (`launch_chain`); dense-layout rows, out: [rows, n, all levels].
+template <typename T>
+hipError_t launch_chunk_adjoints(const T *grad, const T *right, T *out, int64_t rows, int n, int64_t d, int depth,
+                                 hipStream_t stream);
+double chunk_adjoints_us(size_t elem, int64_t rows, int n, int64_t d, int depth);
 // whether these launches exist for a chain of n elements, and what they take (estimates, us)
 bool chain_possible(int64_t rows, int n, int64_t d, int depth);
 double chain_us(size_t elem, int64_t rows, int n, int64_t d, int depth, int directions);

@@ -28,6 +28,11 @@ struct DenseChoice {
     bool chain_groups;          // grouped: those of the groups, and the top level of the row as a sum over the groups
     bool chain_top;             // not grouped: the top level of the row as a sum over the partial signatures
     bool forward_chains;        // any of them in the forward
+    // Far chunks: a shape whose kernels sweep a row in one piece (units of several blocks, split children, fp64 rows too long
+    // for the scan kernel) is cut into time chunks all the same.  Forward: those kernels sweep the chunks, the products are
+    // formed in memory (chain_kernels.hip).  Backward: one launch contracts the upstream gradient with what follows each
+    // chunk, and every chunk is swept as a row of its own, from its own state and adjoint.
+    bool far;
 };
 
 // While one that is on lives, the choices made on its thread take at most 64 chunks to a row and no launches for long

@@ -562,7 +562,7 @@ struct Geometry {
     static constexpr int kLanes = kSplit ? kParts * kPartLanes : kPrefixes;
     // A unit needs kUnitWaves waves.  Up to sixteen of them form one block; a larger unit is spread over
     // kUnitBlocks blocks (its lanes never talk to each other inside a sweep; the per-increment sums of the
-    // backward then meet in memory).  Such shapes are swept in one piece, without time chunks.
+    // backward then meet in memory).  Such shapes are swept in one piece, or in far chunks (DenseChoice::far).
     static constexpr int kUnitWaves = (kLanes + kWave - 1) / kWave;
     // waves of one block: sixteen at most, eight when the lane's sub-trie is large (a block of sixteen waves leaves
     // each lane 128 registers, which the reverse sweep of such a shape overflows), four from 160 values on (one
@@ -591,8 +591,8 @@ struct Geometry {
     static constexpr int kBlock = kWaves * kWave;
     static constexpr int kFwdSub = sub_size(D, kK, N - P);    // sub-trie levels P+1..N
     static constexpr int kASub = sub_size(D, kK, N - 1 - P);  // levels P+1..N-1
-    // swept in one piece, never cut into time chunks: units of several blocks, and units with split children (the
-    // products of chunk signatures are not written for them)
+    // swept in one piece, or in far chunks (DenseChoice::far): units of several blocks, and units with split children (the
+    // products of chunk signatures inside the kernels are not written for them)
     static constexpr bool kOnePiece = kUnitBlocks > 1 || kSplit;
     // Sweeps with letter bounds: the waves of a unit differ in the words they leave out, by a factor of ten and
     // more between the first letter 0 and the last, and a wave cannot issue faster than every fourth clock, so
@@ -1810,7 +1810,8 @@ __device__ __forceinline__ void dense_backward_body(
     chunk_range(span.steps, chunks, c, begin, end);
     const T *x = path + (b * shape.L + span.start) * D;
     T *ginc = grad_inc + (b * (shape.L - 1) + span.start) * D;
-    const T *grow = grad_sig + row * G::kSigSize;
+    // (a sweep in one piece over a time chunk, run_backward's far chunks: a state and an adjoint of its own per chunk)
+    const T *grow = grad_sig + (CHUNKED ? row : unit) * G::kSigSize;
 
     // A chunk that writes the path gradient itself (kToPath) owns the points begin .. end - 1 of its row (the last
     // chunk also the final point): dL/dx[t] = g[t-1] - g[t] with g the per-increment sums.  The sum of the last
@@ -1922,7 +1923,8 @@ __device__ __forceinline__ void dense_backward_body(
             contract_right<T, D, N, P, G::kFwdSub>(hc, hsub, edgeZ + unit * G::kLowSize, sw);
         }
     } else {
-        load_state<T, D, P, N - 1, kAS, KF>(sig + row * G::kSigSize, pu, active, a, asub, a0);
+        const T *state_row = edgeA != nullptr ? edgeA + unit * G::kLowSize : sig + unit * G::kSigSize;
+        load_state<T, D, P, N - 1, kAS, KF>(state_row, pu, active, a, asub, a0);
         if (ntiles > 0) stage_for(ntiles - 1);
         adjoint_chain_of_lane<T, D, P>(pu, a0, hc);
     }
@@ -2570,6 +2572,26 @@ hipError_t launch_scan(const T *chunk_low, T *edgeA, T *edgeZ, int64_t rows, int
     return hipGetLastError();
 }
 
+// Shapes that the launches over time chunks do not serve: units of several blocks or with split children, rows too long for
+// the scan kernel's LDS in this type.  Their calls are cut into far chunks where that pays (DenseChoice::far).
+template <typename T, int D, int N, int P, int PS>
+constexpr bool kFarChunks = Geometry<D, N, P, sizeof(T)>::kOnePiece || !scan_fits<T, D, N, PS>();
+
+// Signatures of all chunks (chunk_sig: [rows, chunks, all levels]), and the products of the chunks up to and including each
+// (edgeA) and, unless null, of those after each (edgeZ), below the top level.  temp: two arrays like edgeA.
+template <typename T, int D, int N, int P>
+hipError_t launch_far_chunks(const T *path, const SigShape &shape, int chunks, T *chunk_sig, T *edgeA, T *edgeZ, T *temp,
+                             hipStream_t stream) {
+    using G = Geometry<D, N, P, sizeof(T)>;
+    const int64_t rows = shape.B * shape.W;
+    hipLaunchKernelGGL((dense_forward_kernel<T, D, N, P, 1>), dim3((unsigned)(rows * chunks * G::kUnitBlocks)),
+                       dim3(G::kBlock), 0, stream, path, chunk_sig, shape, chunks);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    return launch_chain<T>((const T *)chunk_sig, G::kSigSize, rows, chunks, D, N, edgeA, true, edgeZ, (T *)nullptr, 0, temp,
+                           rows * chunks * G::kLowSize, stream);
+}
+
 // keep (optional): receives the prefix and suffix products of the chunk signatures below the top level, which the
 // time-chunked backward of the same call starts its chunks from: [rows, chunks, low] twice, the second array
 // pad256 bytes after the start of the first.
@@ -2595,8 +2617,20 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, const Dense
                            dim3(G::kBlock), 0, stream, path, sig, shape, 1);
         return hipGetLastError();
     }
-    if constexpr (G::kOnePiece) {
-        return hipErrorNotSupported;  // such shapes are never cut into time chunks (dense_choice)
+    if constexpr (kFarChunks<T, D, N, P, PS>) {
+        // far chunks (DenseChoice::far): the signatures of all chunks go to memory, where their products are formed
+        if (!dc.far) return hipErrorNotSupported;
+        T *chunk_sig = (T *)workspace;
+        const int64_t low_elems = rows * chunks * G::kLowSize;
+        const size_t low_bytes = pad256((size_t)low_elems * sizeof(T));
+        T *low_space = (T *)((unsigned char *)workspace + pad256((size_t)rows * chunks * G::kSigSize * sizeof(T)));
+        T *edgeA = keep ? keep : low_space;
+        T *edgeZ = keep ? (T *)((unsigned char *)keep + low_bytes) : (T *)nullptr;
+        hipError_t e = launch_far_chunks<T, D, N, P>(path, shape, chunks, chunk_sig, edgeA, edgeZ,
+                                                     (T *)((unsigned char *)low_space + low_bytes), stream);
+        if (e != hipSuccess) return e;
+        return launch_chain_top<T>((const T *)chunk_sig, G::kSigSize, ChainLeft<T>{edgeA, chunks, 1, -1, true}, sig,
+                                   G::kSigSize, rows, chunks, D, N, stream);
     } else {
     // chunks are swept GW to a block when that divides the chunk count and fits the block and LDS limits;
     // a row that fits one block goes straight to the output, without the combine launch
@@ -2759,25 +2793,49 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
         if (e != hipSuccess) return e;
     }
     if (rows == 0) return hipSuccess;
-    if (chunks <= 1) {
+    // one piece: the signature and the upstream gradient of the row; far chunks: a state and an adjoint per chunk
+    const T *state = nullptr, *adjoint = grad_sig;
+    if constexpr (kFarChunks<T, D, N, P, PS>) {
+        if (chunks > 1) {
+            if (!dc.far) return hipErrorNotSupported;
+            // workspace: [rows, chunks] adjoints (before them, without kept products, the chunk signatures), then the products
+            T *dense = (T *)workspace;
+            const size_t low_bytes = pad256((size_t)(rows * chunks * G::kLowSize) * sizeof(T));
+            const T *edgeZ;
+            if (kept) {
+                state = kept;
+                edgeZ = (const T *)((const unsigned char *)kept + low_bytes);
+            } else {
+                unsigned char *low_space =
+                    (unsigned char *)workspace + pad256((size_t)rows * chunks * G::kSigSize * sizeof(T));
+                e = launch_far_chunks<T, D, N, P>(path, shape, chunks, dense, (T *)low_space, (T *)(low_space + low_bytes),
+                                                  (T *)(low_space + 2 * low_bytes), stream);
+                if (e != hipSuccess) return e;
+                state = (const T *)low_space;
+                edgeZ = (const T *)(low_space + low_bytes);
+            }
+            e = launch_chunk_adjoints<T>(grad_sig, edgeZ, dense, rows, chunks, D, N, stream);
+            if (e != hipSuccess) return e;
+            adjoint = dense;
+        }
+    }
+    if (chunks <= 1 || kFarChunks<T, D, N, P, PS>) {
+        const int pieces = chunks <= 1 ? 1 : chunks;
+        const dim3 grid((unsigned)(rows * pieces * G::kUnitBlocks));
         profile_bracket(true, stream);
         if (accumulate) {
-            hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, false>),
-                               dim3((unsigned)(rows * G::kUnitBlocks)), dim3(G::kBlock), 0, stream, path, sig, grad_sig,
-                               (const T *)nullptr, (const T *)nullptr, grad_inc, shape, 1);
+            hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, false>), grid, dim3(G::kBlock), 0, stream, path, sig,
+                               adjoint, state, (const T *)nullptr, grad_inc, shape, pieces);
         } else {
             if constexpr (G::kUnitBlocks == 1)
-                hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, false, false>), dim3((unsigned)rows),
-                                   dim3(G::kBlock), 0, stream, path, sig, grad_sig, (const T *)nullptr,
-                                   (const T *)nullptr, grad_inc, shape, 1, grad_path);
+                hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, false, false>), grid, dim3(G::kBlock), 0, stream, path,
+                                   sig, adjoint, state, (const T *)nullptr, grad_inc, shape, pieces, grad_path);
             *wrote_path = true;
         }
         profile_bracket(false, stream);
         return hipGetLastError();
     }
-    if constexpr (G::kOnePiece || !scan_fits<T, D, N, PS>()) {
-        // never cut into time chunks (dense_choice): shapes whose units take several blocks, rows too long for
-        // the scan kernel's LDS in this type
+    if constexpr (kFarChunks<T, D, N, P, PS>) {
         return hipErrorNotSupported;
     } else {
         const int64_t units = rows * chunks;
@@ -2887,6 +2945,57 @@ float profile_sweep_ms() {
     return ms;
 }
 
+// Estimate of both sweeps of a call, us.  An increment takes some 0.2 us and 0.013 us for every value below a lane's prefix,
+// twice that in fp64, as long as a SIMD has one wave; more waves, of one block or of many, overlap in part.
+static double step_us_of(const VariantInfo &v, size_t elem) { return (0.2 + 0.013 * v.sub_size) * (elem == 8 ? 2.0 : 1.0); }
+static double sweeps_us(const VariantInfo &v, size_t elem, int64_t rows, int64_t L, int chunks) {
+    const double unit_waves = (double)(v.block / kWave);
+    const double to_simd = std::max(unit_waves / v.unit_blocks / 4, (double)rows * chunks * unit_waves / 1024);
+    return (double)(L - 1) / chunks * step_us_of(v, elem) * std::max(1.0, 0.4 + 0.6 * to_simd);
+}
+
+// Far chunks (DenseChoice::far) of a call without windows, 0 where one piece is as good: about two waves to a SIMD, chunks of
+// sixteen increments at least, half a gigabyte of chunk signatures at most.  fp32 rows of more than 4096 increments stay in
+// one piece for the reason given at kLongRowSteps.  A step, us, in one piece / in far chunks: fp32 (16, 4), 2 paths of 4000
+// points, 4744 / 363, 1 of 300 365 / 85; (9, 5), 4 of 1000, 1361 / 243; (6, 6), 2 of 500, 449 / 134, 16 of 500 454 / 247 (64 of
+// 500 fill the GPU in one piece: 456); (5, 7), 3 of 2000, 3406 / 411; fp64 (4, 7), 13 of 2799, 4374 / 744, (16, 4), 5 of 847,
+// 2153 / 386; a forward alone, fp64 (16, 4), 1 of 410, 130 / 48.  The estimates are cautious: fp64 (4, 7), 20 of 200, stays in
+// one piece, where a forward takes 74 us and 92 in chunks.
+static int far_chunks(const VariantInfo &v, size_t elem, int64_t rows, int64_t L) {
+    if (v.depth > 8 || (elem == 4 && L - 1 > kLongRowSteps)) return 0;
+    const int64_t unit_waves = v.block / kWave;
+    int64_t c = (2048 + rows * unit_waves - 1) / (rows * unit_waves);
+    c = std::min({c, (L - 1) / 16, kMostChunks});
+    const int64_t forced = options().chunks;
+    if (forced >= 1 && forced <= kMostChunks) c = forced;
+    c = std::min<int64_t>(c, (int64_t(1) << 29) / (rows * v.sig_size * (int64_t)elem));
+    if (c < 2 || rows * c * v.unit_blocks >= (int64_t(1) << 30) || !chain_possible(rows, (int)c, v.d, v.depth)) return 0;
+    // (a forward alone is a quarter of the sweeps, and must not lose by it either)
+    const double saved = sweeps_us(v, elem, rows, L, 1) - sweeps_us(v, elem, rows, L, (int)c);
+    const double products = chain_us(elem, rows, (int)c, v.d, v.depth, 2) + chain_top_us(elem, rows, (int)c, v.d, v.depth);
+    if (forced < 1 && (0.25 * saved < products + 6.0 ||
+                       saved < products + chunk_adjoints_us(elem, rows, (int)c, v.d, v.depth) + 8.0))
+        return 0;
+    return (int)c;
+}
+
+// What a call without windows takes with the kernels of an entry of the table, cut as it would be.  (Log-signature of (14, 4), 2
+// paths of 2176 points, fp32: 3437 us a step with prefixes of three in one piece, 277 with prefixes of two in 64 chunks.)
+static double entry_us(const VariantInfo &v, size_t elem, int64_t rows, int64_t L) {
+    if (v.chunks_ok[elem == 8 ? 1 : 0]) {
+        const int chunks = pick_chunks(rows, v.block, L, 2048, false);
+        const bool staged = 2 * (size_t)v.sig_size * elem <= 48 * 1024;
+        const double products = chunks == 1 ? 0.0
+                                            : scan_us(chunks, v.depth, (double)v.low_size * elem) +
+                                                  combine_us(elem, chunks, v.depth, v.sig_size, staged);
+        return sweeps_us(v, elem, rows, L, chunks) + products;
+    }
+    const int far = far_chunks(v, elem, rows, L);
+    if (far == 0) return sweeps_us(v, elem, rows, L, 1);
+    return sweeps_us(v, elem, rows, L, far) + chain_us(elem, rows, far, v.d, v.depth, 2) +
+           chain_top_us(elem, rows, far, v.d, v.depth) + chunk_adjoints_us(elem, rows, far, v.d, v.depth);
+}
+
 static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes,
                                      int64_t B, int64_t L, int64_t W, bool windowed, bool plain) {
     DenseChoice dc{};
@@ -2901,17 +3010,26 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
             // a later entry for the same (d, depth) has more lanes per row: take it when this one cannot
             // put about a wave on every SIMD even with the most time chunks the path allows
             bool later = false;
-            for (int j = i + 1; j < kNumVariants; ++j) later = later || (kVariants[j].d == d && kVariants[j].depth == depth);
+            int other = i;
+            for (int j = i + 1; j < kNumVariants; ++j)
+                if (kVariants[j].d == d && kVariants[j].depth == depth) later = true, other = j;
             const int64_t max_chunks = (L - 1) / 16 < 1 ? 1 : ((L - 1) / 16 > 64 ? 64 : (L - 1) / 16);
             // (a shape that is not cut into chunks has its rows only; half a wave per SIMD is then enough to take it,
             // the later entry being two to three times slower per coefficient)
             const bool cut = v.chunks_ok[elem == 8 ? 1 : 0];
-            if (later && rows * (v.block / kWave) * (cut ? max_chunks : 1) < (cut ? 1024 : 512)) continue;
+            // .. unless the estimates say that this one is the faster all the same: the later entry's rows may be
+            // dozens of waves swept in one piece
+            if (later && rows * (v.block / kWave) * (cut ? max_chunks : 1) < (cut ? 1024 : 512) &&
+                (windowed || plain || (elem == 4 && L - 1 > kLongRowSteps) ||
+                 entry_us(v, elem, rows, L) > 0.7 * entry_us(kVariants[other], elem, rows, L)))
+                continue;
             // the short prefixes of the wide alphabets hold 68 to 240 values per lane: fp64 up to 132 (d = 11) and
             // wherever the children are split
             if (later && elem == 8 && !v.fp64_fits) continue;
         }
         const bool chunks_ok = v.chunks_ok[elem == 8 ? 1 : 0];
+        const int far = chunks_ok || windowed || plain ? 0 : far_chunks(v, elem, rows, L);
+        const bool one_piece = !chunks_ok && far == 0;
         if (!all_dense) {
             // A word projection is computed densely and gathered when that is the cheaper way: when its top level
             // keeps a fair share of the dense one (the top level dominates the cost), or when the dense sweep is
@@ -2938,16 +3056,14 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
                                        (elem == 8 ? 2.0 : 1.0));
                 if (dense_us > 0.8 * per_word_us) return dc;
             }
-            if ((double)rows * (double)v.sig_size * (double)elem * (chunks_ok ? 1.0 : 2.0) > 4e9) return dc;
+            if ((double)rows * (double)v.sig_size * (double)elem * (one_piece ? 2.0 : 1.0) > 4e9) return dc;
             dc.embed = true;
-            dc.resweep = !chunks_ok;
+            dc.resweep = one_piece;
             dc.dense_bytes = pad256((size_t)rows * v.sig_size * elem);
             dc.bounded = chunks_ok && v.bounds_ok && level_sizes[depth] > 0 && level_sizes[depth] < top_dense &&
                          options().letter_bounds != 0;
         }
-        // an increment takes some 0.2 us of both sweeps and 0.013 us for every value below a lane's prefix, twice that
-        // in fp64
-        const double step_us = (0.2 + 0.013 * v.sub_size) * (elem == 8 ? 2.0 : 1.0);
+        const double step_us = step_us_of(v, elem);
         const double low_bytes = (double)v.low_size * elem;
         const bool may_chain = !plain && (elem == 8 || L - 1 <= kLongRowSteps);
         bool many = false;  // more than 64 chunks
@@ -2968,7 +3084,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         if (const int64_t forced = options().chunks; forced >= 1 && forced <= 1024) chunks = (int)forced;
         // not chunked: units of several blocks (a row is dozens of waves already), rows too long for the scan
         // kernel's LDS
-        if (!chunks_ok) chunks = 1;
+        if (!chunks_ok) chunks = far > 0 ? far : 1;
         if (rows * (chunks + 1) >= (int64_t(1) << 31)) return dc;
         dc.usable = true;
         dc.variant = i;
@@ -2976,6 +3092,20 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         dc.bwd_chunks = (dc.embed && !dc.resweep && chunks < 2) ? 2 : chunks;
         dc.forward_workspace = dc.dense_bytes + (dc.bounded ? kBoundsBytes : 0);
         dc.backward_workspace = (dc.resweep ? 2 : 1) * dc.dense_bytes + (dc.bounded ? kBoundsBytes : 0);
+        if (far > 0) {
+            // forward: chunk signatures, products (where none are kept) and two arrays of scratch; backward: adjoints (first
+            // the chunk signatures, where nothing was kept), both products and the scratch
+            const size_t all = pad256((size_t)rows * far * v.sig_size * elem), low = pad256((size_t)rows * far * v.low_size * elem);
+            dc.far = true;
+            dc.forward_chains = true;
+            dc.forward_workspace += all + 3 * low;
+            dc.backward_workspace += all + 4 * low;
+            // (sized as the products of ordinary chunks are, below)
+            const size_t unit = (size_t)rows * v.low_size * elem;
+            const size_t spare = unit % 256 == 0 ? 0 : 2 * ((512 + unit - 1) / unit);
+            dc.keep_bytes = unit * (spare + (size_t)far * 2);
+            return dc;
+        }
         // the forward can hand those products to the backward when both cut the rows the same way
         if (dc.bwd_chunks > 1 && dc.fwd_chunks == dc.bwd_chunks) {
             // grouped hand-over (see grouped_handover_ok): whole groups of four chunks, two groups at least
