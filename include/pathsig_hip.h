@@ -54,6 +54,10 @@ const char *pathsig_last_error(void);
  */
 size_t pathsig_sig_forward_workspace(int dtype, int64_t B, int64_t L, int64_t d, int depth,
                                      const int64_t *level_sizes, int64_t W);
+/* Scratch with which a forward that keeps nothing is fastest, at least what pathsig_sig_forward_workspace asks for: the
+ * per-word kernels cut few words on few paths into time chunks where they get it. */
+size_t pathsig_sig_forward_scratch(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
+                                   int64_t W);
 int pathsig_sig_forward(const void *path, void *sig, int dtype, int64_t B, int64_t L, int64_t d, int depth,
                         const int64_t *level_sizes, const int64_t *encoded_words, int64_t n_encoded,
                         const int32_t *windows, int64_t W, void *workspace, size_t workspace_bytes,
@@ -102,6 +106,7 @@ int pathsig_sig_backward_noalloc(const void *path, const void *sig, const void *
  * See the "grouped" option.)  The per-word kernels hand over, in the same buffer, the
  * prefix values of the words whose prefixes are not all part of the signature (the backward otherwise
  * rebuilds them with a forward sweep, as src/pathsig/backward/sig_backward_kernels.cu:134-157 does).
+ * Where they cut the paths into time chunks, they hand over the signatures of the chunks at all factors of the words.
  * A word projection that is computed through a register-tiled shape which is swept in one piece (depth 2,
  * shapes with more than 1024 lanes per row) hands over its dense signature, which the backward otherwise
  * sweeps again.

@@ -24,6 +24,7 @@ TORCH_LIB = PKG / "libpathsig_torch.so"
 DENSE_GROUPS = 8  # kDenseGroups of csrc/dense.hpp
 UNITS = ([("dense_kernels.hip", f"dense_kernels_g{g}.o", [f"-DPSIG_GROUP={g}"]) for g in range(DENSE_GROUPS)]
          + [("batch_kernels.hip", "batch_kernels.o", []), ("batch_lists.hip", "batch_lists.o", []), ("words_kernels.hip", "words_kernels.o", []),
+            ("words_chunks.hip", "words_chunks.o", []),
             ("logsig_kernels.hip", "logsig_kernels.o", []), ("chain_kernels.hip", "chain_kernels.o", []),
             ("logsig_rows.hip", "logsig_rows_f32.o", ["-DPSIG_ROWS_TYPE=float"]),
             ("logsig_rows.hip", "logsig_rows_f64.o", ["-DPSIG_ROWS_TYPE=double"]), ("dense_kernels.hip", "dense_kernels.o", []),

@@ -201,6 +201,33 @@ size_t words_keep_bytes(const LevelPlan &plan, int64_t rows, int64_t d, size_t e
     return (size_t)count * elem;
 }
 
+// Time chunks of a per-word call (none while PlainChunks is active), the bytes of the table of factors and of an array of
+// values at the chunks' edges, and what a forward keeps: the table, and one or two elements more where the size would be
+// that of another layout (words_keep_bytes).
+WordChunks chunks_of_words(const LevelPlan &plan, size_t elem, int64_t B, int64_t L, int64_t d, bool windowed) {
+    if (PlainChunks::active()) return WordChunks{};
+    return word_chunks(elem, B, L, d, plan.depth, plan.size, windowed);
+}
+size_t word_table_bytes(const WordChunks &wc, int64_t B, size_t elem) {
+    return align_up((size_t)(B * wc.chunks * wc.table_size) * elem);
+}
+size_t word_edge_bytes(const WordChunks &wc, int64_t B, size_t elem) {
+    return align_up((size_t)(B * wc.chunks * wc.edge_size) * elem);
+}
+size_t words_kept_bytes(const LevelPlan &plan, const WordChunks &wc, int64_t B, int64_t rows, int64_t d, size_t elem) {
+    const size_t chains = words_keep_bytes(plan, rows, d, elem);
+    if (!wc.chunks) return chains;
+    uint64_t low = 0, top = 1;
+    for (int k = 1; k <= plan.depth; ++k) {
+        if (k > 1) low += top;
+        top *= (uint64_t)d;
+    }
+    const uint64_t unit = (uint64_t)rows * low, dense = unit + (uint64_t)rows * top;
+    uint64_t count = (uint64_t)(word_table_bytes(wc, B, elem) / elem);
+    while ((unit > 1 && (count % unit == 0 || count == dense)) || count * elem == chains) ++count;
+    return (size_t)count * elem;
+}
+
 template <typename T>
 int sig_forward_t(const void *path, void *sig, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
                   const int64_t *codes, int64_t n_encoded, const int32_t *windows, int64_t W, void *keep,
@@ -214,7 +241,8 @@ int sig_forward_t(const void *path, void *sig, int64_t B, int64_t L, int64_t d, 
     rc = check_grid(plan, B * shape.W);
     if (rc != PATHSIG_OK) return rc;
     const DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
-    const size_t keep_need = dc.usable ? dc.keep_bytes : words_keep_bytes(plan, B * shape.W, d, sizeof(T));
+    WordChunks wc = dc.usable ? WordChunks{} : chunks_of_words(plan, sizeof(T), B, L, d, windows != nullptr);
+    const size_t keep_need = dc.usable ? dc.keep_bytes : words_kept_bytes(plan, wc, B, B * shape.W, d, sizeof(T));
     if (keep && (keep_need == 0 || keep_bytes < keep_need)) {
         set_error("chunk buffer: this call keeps %zu bytes, got %zu", keep_need, keep_bytes);
         return PATHSIG_ERR_ARGUMENT;
@@ -237,6 +265,14 @@ int sig_forward_t(const void *path, void *sig, int64_t B, int64_t L, int64_t d, 
             e = launch_gather_columns<T>(dense, (T *)sig, plan, d, codes, B * shape.W, stream);
             if (e != hipSuccess) return launch_failed(e, "gather launch");
         }
+        return PATHSIG_OK;
+    }
+    // (a call that keeps nothing and brings no scratch for the table is swept in one piece)
+    if (wc.chunks && (keep || (workspace && workspace_bytes >= word_table_bytes(wc, B, sizeof(T))))) {
+        T *table = (T *)(keep ? keep : workspace);
+        hipError_t e = launch_word_factors<T>((const T *)path, table, shape, plan, codes, wc, stream);
+        if (e == hipSuccess) e = launch_word_products<T>(table, (T *)sig, (T *)nullptr, (T *)nullptr, shape, plan, wc, stream);
+        if (e != hipSuccess) return launch_failed(e, "forward launch");
         return PATHSIG_OK;
     }
     plan.keep = keep;  // the per-word forward leaves the prefix values its backward would recompute
@@ -264,7 +300,8 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
     rc = check_grid(plan, B * shape.W);
     if (rc != PATHSIG_OK) return rc;
     const DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
-    const size_t keep_need = dc.usable ? dc.keep_bytes : words_keep_bytes(plan, B * shape.W, d, sizeof(T));
+    WordChunks wc = dc.usable ? WordChunks{} : chunks_of_words(plan, sizeof(T), B, L, d, windows != nullptr);
+    const size_t keep_need = dc.usable ? dc.keep_bytes : words_kept_bytes(plan, wc, B, B * shape.W, d, sizeof(T));
     // The layout of what a forward keeps follows from the choice of kernels, which the tuning switches can change
     // between the two calls.  A buffer of another size than this call would have kept comes from a forward that
     // chose differently and is refused (no two choices keep the same number of bytes).
@@ -273,7 +310,7 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
                   kept_bytes);
         return PATHSIG_ERR_ARGUMENT;
     }
-    plan.keep = const_cast<void *>(kept);
+    plan.keep = wc.chunks ? nullptr : const_cast<void *>(kept);
     const bool words_kernel = !dc.usable && !batch_backward_usable(sizeof(T), B, d, shape.W);
     const bool batch_wide = !dc.usable && !words_kernel && batch_wide_sums(sizeof(T), plan);
     const size_t inc_bytes = inc_buffer_bytes(sizeof(T), B, L, d, words_kernel || batch_wide);
@@ -284,6 +321,21 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
     }
     T *ginc = (T *)workspace;
     hipError_t e;
+    if (wc.chunks) {
+        const size_t table = word_table_bytes(wc, B, sizeof(T)), edge = word_edge_bytes(wc, B, sizeof(T));
+        if (workspace_bytes < need + 2 * edge + (kept ? 0 : table)) {
+            wc = WordChunks{};  // (a caller that brings no more scratch than one piece takes)
+        } else {
+            unsigned char *at = (unsigned char *)workspace + need;
+            T *left = (T *)at, *right = (T *)(at + edge), *made = (T *)(at + 2 * edge);
+            e = kept ? hipSuccess : launch_word_factors<T>((const T *)path, made, shape, plan, codes, wc, stream);
+            if (e == hipSuccess)
+                e = launch_word_products<T>(kept ? (const T *)kept : made, (T *)nullptr, left, right, shape, plan, wc, stream);
+            if (e != hipSuccess) return launch_failed(e, "forward launch");
+            wc.left = left;
+            wc.right = right;
+        }
+    }
     if (dc.usable) {
         unsigned char *extra = (unsigned char *)workspace + inc_bytes;
         const T *gdense = (const T *)grad_sig;
@@ -335,10 +387,10 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
             profile_bracket(true, stream);
             if (words_kernel)
                 e = launch_words_backward<T>((const T *)path, (const T *)sig, (const T *)grad_sig, ginc64, shape, plan,
-                                             codes, stream);
+                                             codes, wc, stream);
             else
                 e = launch_batch_backward<T, double>((const T *)path, (const T *)sig, (const T *)grad_sig, ginc64, shape,
-                                                     plan, codes, stream);
+                                                     plan, codes, wc, stream);
             profile_bracket(false, stream);
             if (e != hipSuccess) return launch_failed(e, "backward launch");
         }
@@ -351,7 +403,7 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
         if (shape.W > 0 && plan.sig_size > 0) {
             profile_bracket(true, stream);
             e = launch_batch_backward<T, T>((const T *)path, (const T *)sig, (const T *)grad_sig, ginc, shape, plan, codes,
-                                            stream);
+                                            wc, stream);
             profile_bracket(false, stream);
             if (e != hipSuccess) return launch_failed(e, "backward launch");
         }
@@ -756,6 +808,17 @@ size_t pathsig_sig_forward_workspace(int dtype, int64_t B, int64_t L, int64_t d,
     return dc.usable ? dc.forward_workspace : 0;
 }
 
+size_t pathsig_sig_forward_scratch(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
+                                   int64_t W) {
+    const size_t needed = pathsig_sig_forward_workspace(dtype, B, L, d, depth, level_sizes, W);
+    if (needed > 0 || check_common(dtype, B, L, d, depth) != PATHSIG_OK) return needed;
+    LevelPlan plan;
+    bool all_dense;
+    if (build_plan(d, depth, level_sizes, INT64_MAX, true, &plan, &all_dense) != PATHSIG_OK) return 0;
+    if (dense_choice(elem_size(dtype), d, depth, all_dense, level_sizes, B, L, W > 0 ? W : 1, W > 0).usable) return 0;
+    return word_table_bytes(chunks_of_words(plan, elem_size(dtype), B, L, d, W > 0), B, elem_size(dtype));
+}
+
 size_t pathsig_sig_chunks_bytes(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
                                 int64_t W) {
     if (check_common(dtype, B, L, d, depth) != PATHSIG_OK) return 0;
@@ -765,7 +828,8 @@ size_t pathsig_sig_chunks_bytes(int dtype, int64_t B, int64_t L, int64_t d, int 
     const DenseChoice dc =
         dense_choice(elem_size(dtype), d, depth, all_dense, level_sizes, B, L, W > 0 ? W : 1, W > 0);
     if (dc.usable) return dc.keep_bytes;
-    return words_keep_bytes(plan, B * (W > 0 ? W : 1), d, elem_size(dtype));
+    const WordChunks wc = chunks_of_words(plan, elem_size(dtype), B, L, d, W > 0);
+    return words_kept_bytes(plan, wc, B, B * (W > 0 ? W : 1), d, elem_size(dtype));
 }
 
 int pathsig_sig_forward(const void *path, void *sig, int dtype, int64_t B, int64_t L, int64_t d, int depth,
@@ -830,8 +894,10 @@ size_t pathsig_sig_backward_workspace(int dtype, int64_t B, int64_t L, int64_t d
     }
     const bool words_kernel = !dc.usable && !batch_backward_usable(elem_size(dtype), B, d, W > 0 ? W : 1);
     const bool batch_wide = !dc.usable && !words_kernel && batch_wide_sums(elem_size(dtype), plan);
+    const WordChunks wc = dc.usable ? WordChunks{} : chunks_of_words(plan, elem_size(dtype), B, L, d, W > 0);
     return inc_buffer_bytes(elem_size(dtype), B, L, d, words_kernel || batch_wide) +
-           (dc.usable ? dc.backward_workspace : 0) + 256;
+           (dc.usable ? dc.backward_workspace : 0) + word_table_bytes(wc, B, elem_size(dtype)) +
+           2 * word_edge_bytes(wc, B, elem_size(dtype)) + 256;
 }
 
 int pathsig_sig_backward(const void *path, const void *sig, const void *grad_sig, void *grad_path, int dtype,

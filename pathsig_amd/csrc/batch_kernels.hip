@@ -301,9 +301,10 @@ bool batch_backward_usable(size_t elem, int64_t B, int64_t d, int64_t W) {
 
 template <typename T, typename ACC>
 hipError_t launch_batch_backward(const T *path, const T *sig, const T *grad_sig, ACC *grad_inc, const SigShape &shape,
-                                 const LevelPlan &plan_in, const int64_t *codes, hipStream_t stream) {
+                                 const LevelPlan &plan_in, const int64_t *codes, const WordChunks &wc, hipStream_t stream) {
     // (over sixteen letters and fewer the entries are sorted by letter once and added up in rows: 599 against 959 us)
-    if (shape.d <= 16) return launch_batch_lists<T, ACC>(path, sig, grad_sig, grad_inc, shape, plan_in, codes, stream);
+    if (shape.d <= 16) return launch_batch_lists<T, ACC>(path, sig, grad_sig, grad_inc, shape, plan_in, codes, wc, stream);
+    if (wc.chunks) return hipErrorInvalidValue;
     const int G = batch_group<T>(shape.B);
     LevelPlan plan = plan_in;
     int64_t blocks = 0;
@@ -356,12 +357,12 @@ bool batch_wide_sums(size_t elem, const LevelPlan &plan) { return elem == 4 && p
 
 template hipError_t launch_batch_backward<float, float>(const float *, const float *, const float *, float *,
                                                         const SigShape &, const LevelPlan &, const int64_t *,
-                                                        hipStream_t);
+                                                        const WordChunks &, hipStream_t);
 template hipError_t launch_batch_backward<float, double>(const float *, const float *, const float *, double *,
                                                          const SigShape &, const LevelPlan &, const int64_t *,
-                                                         hipStream_t);
+                                                         const WordChunks &, hipStream_t);
 template hipError_t launch_batch_backward<double, double>(const double *, const double *, const double *, double *,
                                                           const SigShape &, const LevelPlan &, const int64_t *,
-                                                          hipStream_t);
+                                                          const WordChunks &, hipStream_t);
 
 }  // namespace psig

@@ -82,12 +82,12 @@ struct ListShared {
     int count[kLetters], first_row[kLetters];
 };
 
-template <typename T, int DEG, typename ACC>
+template <typename T, int DEG, typename ACC, bool CHUNKED>
 __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, const T *__restrict__ sig,
                                                    const T *__restrict__ grad_sig, ACC *__restrict__ grad_inc,
                                                    const SigShape &shape, const LevelPlan &plan,
                                                    const int64_t *__restrict__ codes, int64_t blk_in_level,
-                                                   int64_t unit, ListShared<T> &sh) {
+                                                   int64_t unit, ListShared<T> &sh, const WordChunks &wc) {
     constexpr int WPL = list_words(DEG);
     constexpr int kPaths = kGroup / kWaves;  // paths that a wave stages
     constexpr int kStage = Staged<T>::kStage, kPair = Staged<T>::kPair, kCopies = Staged<T>::kCopies;
@@ -95,11 +95,15 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const int slot = lane / kGroup, pl = lane % kGroup;
     const int d = (int)shape.d;
-    const int64_t group = unit / shape.W, w = unit - group * shape.W;
+    // (a unit is a window of a group of paths, or a time chunk of paths without windows)
+    const int64_t per_group = CHUNKED ? wc.chunks : shape.W;
+    const int64_t group = unit / per_group, part = unit - group * per_group;
+    const int64_t w = CHUNKED ? 0 : part;
     const int64_t b0 = group * kGroup;
     const bool path_ok = b0 + pl < shape.B;
     const int64_t b = path_ok ? b0 + pl : shape.B - 1;
-    const WindowSpan span = window_span(shape, w);
+    WindowSpan span = window_span(shape, w);
+    if constexpr (CHUNKED) span = chunk_of_span(span, wc.chunks, (int)part);
     const int64_t row = b * shape.W + w;
     const T *srow = sig + row * plan.sig_size;
     const T *grow = grad_sig + row * plan.sig_size;
@@ -111,7 +115,7 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
     __syncthreads();
 
     // per word: offsets of the lane's increments, chain at the right end of the window, chain adjoint
-    const bool kept_chain = DEG > 1 && !plan.from_saved[DEG] && plan.keep != nullptr && plan.keep_off[DEG] >= 0;
+    const bool kept_chain = DEG > 1 && !CHUNKED && !plan.from_saved[DEG] && plan.keep != nullptr && plan.keep_off[DEG] >= 0;
     const int64_t word0 = ((blk_in_level * kWaves + wave) * kSlots + slot) * WPL;
     int aoff[WPL][DEG], nth[WPL][DEG];
     T p[WPL][DEG + 1], h[WPL][DEG + 1];
@@ -132,7 +136,9 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
             h[i][k] = T(0);
         }
         h[i][DEG] = (have && path_ok) ? grow[plan.out_off[DEG] + word_idx] : T(0);
-        if (plan.from_saved[DEG] && have) {
+        if (CHUNKED) {
+            if (have && path_ok) word_chunk_edges<T, DEG>(wc, plan, row * wc.chunks + part, word_idx, p[i], h[i]);
+        } else if (plan.from_saved[DEG] && have) {
             uint64_t off = 0, width = (uint64_t)d, pref = 0;
 #pragma unroll
             for (int k = 1; k < DEG; ++k) {
@@ -213,7 +219,7 @@ __device__ __forceinline__ void list_backward_body(const T *__restrict__ path, c
         return (int)(left < kStage ? left : kStage);
     };
 
-    if (!plan.from_saved[DEG] && DEG > 1 && nstages > 0 && !kept_chain) {
+    if (!plan.from_saved[DEG] && DEG > 1 && nstages > 0 && !kept_chain && !CHUNKED) {
         // chain at the right end of the window by a forward sweep (levels < DEG)
         fetch(0, stage_steps(0));
         commit(stage_steps(0));
@@ -335,11 +341,11 @@ __device__ __forceinline__ int level_of_block(const LevelPlan &plan, int64_t blk
 
 // Consecutive blocks work on the same words of consecutive groups of paths: the blocks of the longest words, which
 // take longest, start first and spread over the device.
-template <typename T, int MAXDEG, typename ACC>
+template <typename T, int MAXDEG, typename ACC, bool CHUNKED>
 __global__ void __launch_bounds__(kThreads, sizeof(T) == 8 || MAXDEG > 8 ? 2 : MAXDEG > 6 ? 3 : 4)
     list_backward_kernel(const T *__restrict__ path, const T *__restrict__ sig, const T *__restrict__ grad_sig,
                          ACC *__restrict__ grad_inc, SigShape shape, LevelPlan plan,
-                         const int64_t *__restrict__ codes) {
+                         const int64_t *__restrict__ codes, WordChunks wc) {
     __shared__ ListShared<T> sh;
     const int64_t linear = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
     const int64_t blk = linear / gridDim.y, unit = linear - blk * gridDim.y;
@@ -349,7 +355,7 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 8 || MAXDEG > 8 ? 2 : M
 #define PSIG_CASE(N)                                                                                               \
     case N:                                                                                                        \
         if constexpr (N <= MAXDEG)                                                                                 \
-            list_backward_body<T, N, ACC>(path, sig, grad_sig, grad_inc, shape, plan, codes, bl, unit, sh);        \
+            list_backward_body<T, N, ACC, CHUNKED>(path, sig, grad_sig, grad_inc, shape, plan, codes, bl, unit, sh, wc);    \
         break;
         PSIG_CASE(1) PSIG_CASE(2) PSIG_CASE(3) PSIG_CASE(4) PSIG_CASE(5) PSIG_CASE(6)
         PSIG_CASE(7) PSIG_CASE(8) PSIG_CASE(9) PSIG_CASE(10) PSIG_CASE(11) PSIG_CASE(12)
@@ -362,9 +368,9 @@ __global__ void __launch_bounds__(kThreads, sizeof(T) == 8 || MAXDEG > 8 ? 2 : M
 
 template <typename T, typename ACC>
 hipError_t launch_batch_lists(const T *path, const T *sig, const T *grad_sig, ACC *grad_inc, const SigShape &shape,
-                              const LevelPlan &plan_in, const int64_t *codes, hipStream_t stream) {
+                              const LevelPlan &plan_in, const int64_t *codes, const WordChunks &wc, hipStream_t stream) {
     LevelPlan plan = plan_in;
-    const int64_t units = (shape.B + kGroup - 1) / kGroup * shape.W;
+    const int64_t units = (shape.B + kGroup - 1) / kGroup * (wc.chunks ? wc.chunks : shape.W);
     int64_t blocks = 0;
     for (int k = plan.depth; k >= 1; --k) {
         const int64_t per_block = (int64_t)kWaves * kSlots * list_words(k);
@@ -376,8 +382,12 @@ hipError_t launch_batch_lists(const T *path, const T *sig, const T *grad_sig, AC
     if (shape.d > kLetters || blocks >= (int64_t(1) << 31) || units > 65535) return hipErrorInvalidValue;
     const dim3 grid((unsigned)blocks, (unsigned)units);
 #define PSIG_LAUNCH(MAXDEG)                                                                                         \
-    hipLaunchKernelGGL((list_backward_kernel<T, MAXDEG, ACC>), grid, dim3(kThreads), 0, stream, path, sig, grad_sig, \
-                       grad_inc, shape, plan, codes)
+    if (wc.chunks)                                                                                                  \
+        hipLaunchKernelGGL((list_backward_kernel<T, MAXDEG, ACC, true>), grid, dim3(kThreads), 0, stream, path, sig, \
+                           grad_sig, grad_inc, shape, plan, codes, wc);                                             \
+    else                                                                                                            \
+        hipLaunchKernelGGL((list_backward_kernel<T, MAXDEG, ACC, false>), grid, dim3(kThreads), 0, stream, path, sig, \
+                           grad_sig, grad_inc, shape, plan, codes, wc)
     if (plan.depth <= 4)
         PSIG_LAUNCH(4);
     else if (plan.depth <= 6)
@@ -392,10 +402,19 @@ hipError_t launch_batch_lists(const T *path, const T *sig, const T *grad_sig, AC
 
 #define PSIG_INSTANCE(T, ACC)                                                                                     \
     template hipError_t launch_batch_lists<T, ACC>(const T *, const T *, const T *, ACC *, const SigShape &,      \
-                                                   const LevelPlan &, const int64_t *, hipStream_t);
+                                                   const LevelPlan &, const int64_t *, const WordChunks &, hipStream_t);
 PSIG_INSTANCE(float, float)
 PSIG_INSTANCE(float, double)
 PSIG_INSTANCE(double, double)
 #undef PSIG_INSTANCE
+
+int64_t list_waves(int64_t B, int depth, const int64_t *level_sizes) {
+    int64_t blocks = 0;
+    for (int k = 1; k <= depth; ++k) {
+        const int64_t per_block = (int64_t)kWaves * kSlots * list_words(k);
+        blocks += (level_sizes[k] + per_block - 1) / per_block;
+    }
+    return blocks * kWaves * ((B + kGroup - 1) / kGroup);
+}
 
 }  // namespace psig

@@ -41,6 +41,15 @@ struct SigShape {
     const int32_t *windows;
 };
 
+// Time chunks of a per-word call (words_chunks.hip); level n has its words side by side.
+struct WordChunks {
+    int chunks;                          // of every path; 0: swept in one piece
+    int64_t table_size, edge_size;       // elements per (path, chunk)
+    int64_t table_off[kMaxDepth + 1];    // signature of the chunk at the factors w_(i+1)..w_j of every word, 0 <= i < j <= n
+    int64_t edge_off[kMaxDepth + 1];     // at the factors w_1..w_k (left) and w_(k+1)..w_n (right), 1 <= k <= n
+    const void *left, *right;            // [paths, chunks, edge_size]: of everything up to the chunk's right edge, and after it
+};
+
 void set_error(const char *fmt, ...);
 
 // Tuning switches of the library (pathsig_set_option).  Their initial values come from the environment, read
@@ -154,7 +163,20 @@ hipError_t launch_words_forward(const T *path, T *sig, const SigShape &shape, co
 // (its per-increment sums are fp64 whatever T is: one term per block of words and cell)
 template <typename T>
 hipError_t launch_words_backward(const T *path, const T *sig, const T *grad_sig, double *grad_inc,
-                                 const SigShape &shape, const LevelPlan &plan, const int64_t *codes, hipStream_t stream);
+                                 const SigShape &shape, const LevelPlan &plan, const int64_t *codes, const WordChunks &wc,
+                                 hipStream_t stream);
+// The choice of time chunks for a call (chunks == 0: none); the signatures of the chunks at all factors of the words (table:
+// paths * chunks * table_size elements); their products: the signature (where not null), and (left, right not null) the
+// values that the backward starts its chunks from.
+WordChunks word_chunks(size_t elem, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes, bool windowed);
+template <typename T>
+hipError_t launch_word_factors(const T *path, T *table, const SigShape &shape, const LevelPlan &plan, const int64_t *codes,
+                               const WordChunks &wc, hipStream_t stream);
+template <typename T>
+hipError_t launch_word_products(const T *table, T *sig, T *left, T *right, const SigShape &shape, const LevelPlan &plan,
+                                const WordChunks &wc, hipStream_t stream);
+// waves of the list backward (batch_lists.hip) in one piece
+int64_t list_waves(int64_t B, int depth, const int64_t *level_sizes);
 // backward with lanes on paths (batch_kernels.hip): same contract as launch_words_backward; usable for
 // batches of at least a dozen paths of moderate dimension
 bool batch_backward_usable(size_t elem, int64_t B, int64_t d, int64_t W);
@@ -162,11 +184,11 @@ bool batch_backward_usable(size_t elem, int64_t B, int64_t d, int64_t W);
 bool batch_wide_sums(size_t elem, const LevelPlan &plan);
 template <typename T, typename ACC>
 hipError_t launch_batch_backward(const T *path, const T *sig, const T *grad_sig, ACC *grad_inc, const SigShape &shape,
-                                 const LevelPlan &plan, const int64_t *codes, hipStream_t stream);
+                                 const LevelPlan &plan, const int64_t *codes, const WordChunks &wc, hipStream_t stream);
 // the same over at most sixteen letters (batch_lists.hip)
 template <typename T, typename ACC>
 hipError_t launch_batch_lists(const T *path, const T *sig, const T *grad_sig, ACC *grad_inc, const SigShape &shape,
-                               const LevelPlan &plan, const int64_t *codes, hipStream_t stream);
+                               const LevelPlan &plan, const int64_t *codes, const WordChunks &wc, hipStream_t stream);
 template <typename T>
 hipError_t launch_fill_zero(T *ptr, int64_t n, hipStream_t stream);
 // Grid of the kernels that run x over the columns of a row (256 threads to a block, a thread per column while

@@ -3055,6 +3055,15 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
                     std::max(80.0, 10.0 * (double)v.sig_size * (double)rows * steps / (v.d <= 8 ? 40e6 : 25e6) *
                                        (elem == 8 ? 2.0 : 1.0));
                 if (dense_us > 0.8 * per_word_us) return dc;
+                // Few words on few paths are swept in time chunks (words_chunks.hip), whatever their number, while the dense
+                // sweep may have a handful of waves.  (A step, us, dense / words in chunks: fp64, 1 path of 300 points, 16
+                // words of (12, 5), 926 / 69; 3 of 1000, 2000 words of (10, 6), 3925 / 127; 10 of 396, 542 of (12, 5), 708 / 76.)
+                const WordChunks wc = plain ? WordChunks{} : word_chunks(elem, B, L, d, depth, level_sizes, windowed);
+                if (wc.chunks) {
+                    const double chunked_us =
+                        25.0 + 2.0 * steps / wc.chunks + 0.6 * wc.chunks + 5e-6 * words * (double)rows * steps;
+                    if (chunked_us < 0.6 * std::max(dense_us, entry_us(v, elem, rows, L) + 20.0)) return dc;
+                }
             }
             if ((double)rows * (double)v.sig_size * (double)elem * (one_piece ? 2.0 : 1.0) > 4e9) return dc;
             dc.embed = true;

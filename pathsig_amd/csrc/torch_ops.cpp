@@ -131,7 +131,9 @@ std::tuple<Tensor, Tensor> sig_forward(const Tensor &path_in, int64_t depth, boo
         chunk_bytes = pathsig_sig_chunks_bytes(c.dt, c.B, c.L, c.d, (int)c.depth, c.sizes, c.W);
         chunks = at::empty({(int64_t)(chunk_bytes / c.path.element_size())}, c.path.options());
     }
-    const size_t ws_bytes = pathsig_sig_forward_workspace(c.dt, c.B, c.L, c.d, (int)c.depth, c.sizes, c.W);
+    // (what a forward keeps serves it as scratch too)
+    const size_t ws_bytes = (chunk_bytes ? pathsig_sig_forward_workspace : pathsig_sig_forward_scratch)(
+        c.dt, c.B, c.L, c.d, (int)c.depth, c.sizes, c.W);
     Tensor ws = scratch(ws_bytes, c.path);
     check_rc(pathsig_sig_forward_keep(ptr(c.path), ptr(out), c.dt, c.B, c.L, c.d, (int)c.depth, c.sizes,
                                       (const int64_t *)ptr(c.words), c.n_words,

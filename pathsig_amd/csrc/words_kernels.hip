@@ -23,86 +23,6 @@ namespace {
 
 constexpr int kBlock = 256;
 
-template <typename T, int DEG>
-__device__ void forward_body(const T *__restrict__ path, T *__restrict__ sig, const SigShape &shape,
-                             const LevelPlan &plan, const int64_t *__restrict__ codes, int64_t row, int64_t blk_in_level,
-                             int tile, T *sdx) {
-    const int tid = threadIdx.x;
-    const int64_t d = shape.d;
-    const int64_t word_idx = blk_in_level * kBlock + tid;
-    const bool active = word_idx < plan.size[DEG];
-    uint64_t code = 0;
-    if (active) code = plan.code_off[DEG] >= 0 ? (uint64_t)codes[plan.code_off[DEG] + word_idx] : (uint64_t)word_idx;
-    int l[DEG];
-    decode_letters<DEG>(code, (uint64_t)d, l);
-
-    const int64_t b = row / shape.W, w = row - b * shape.W;
-    const WindowSpan span = window_span(shape, w);
-    const T *x = path + (b * shape.L + span.start) * d;
-
-    T p[DEG + 1];
-    p[0] = T(1);
-#pragma unroll
-    for (int k = 1; k <= DEG; ++k) p[k] = T(0);
-
-    // Increments are staged in pairs, [pair][letter][increment of the pair]: a read, and the address that it takes, bring a
-    // letter of two of them, which matters because a word of length n takes n reads beside some n^2 instructions of its chain.
-    // Forward launch, one increment / two to a read: 256 paths of 512 points, 16 letters, 2320 words up to length 6, fp32
-    // 205 / 181 us, fp64 345 / 313; 200 paths of 700, 1020 words up to length 8 over 12 letters, 300 / 279.  (The letter and pair
-    // of an element are carried along: a division for each costs 3 of 34 us over 100 letters, 2000 words, 256 paths of 128.)
-    typedef T Pair __attribute__((ext_vector_type(2)));
-    const int width = (int)d;
-    const int first_letter = tid % width, first_pair = tid / width;
-    int at[DEG];
-#pragma unroll
-    for (int k = 0; k < DEG; ++k) at[k] = 2 * l[k];
-    for (int64_t t0 = 0; t0 < span.steps; t0 += tile) {
-        const int nt = (int)((span.steps - t0) < tile ? (span.steps - t0) : tile);
-        const T *xw = x + t0 * d;
-        __syncthreads();
-        int letter = first_letter, pair = first_pair;  // of element idx
-        for (int idx = tid; idx < (nt + 1) / 2 * width; idx += kBlock, letter += kBlock % width, pair += kBlock / width) {
-            if (letter >= width) {
-                letter -= width;
-                ++pair;
-            }
-            const T *from = xw + (int64_t)pair * 2 * d + letter;
-            const T mid = from[d], first = mid - from[0];
-            const T second = 2 * pair + 1 < nt ? from[2 * d] - mid : T(0);
-            reinterpret_cast<Pair *>(sdx)[idx] = Pair{first, second};
-        }
-        __syncthreads();
-        if (active) {
-            const T *dxr = sdx;
-            T dl[DEG];
-            for (int tt = 0; tt + 1 < nt; tt += 2, dxr += 2 * width) {
-                Pair both[DEG];
-#pragma unroll
-                for (int k = 0; k < DEG; ++k) both[k] = *reinterpret_cast<const Pair *>(dxr + at[k]);
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-#pragma unroll
-                    for (int k = 0; k < DEG; ++k) dl[k] = both[k][i];
-                    chain_step<T, DEG, DEG>(p, dl);
-                }
-            }
-            if (nt % 2) {
-#pragma unroll
-                for (int k = 0; k < DEG; ++k) dl[k] = dxr[at[k]];
-                chain_step<T, DEG, DEG>(p, dl);
-            }
-        }
-    }
-    if (active) {
-        sig[row * plan.sig_size + plan.out_off[DEG] + word_idx] = p[DEG];
-        if (plan.keep && plan.keep_off[DEG] >= 0) {
-            T *kept = (T *)plan.keep + row * plan.keep_size + plan.keep_off[DEG] + word_idx * (DEG - 1);
-#pragma unroll
-            for (int k = 1; k < DEG; ++k) kept[k - 1] = p[k];
-        }
-    }
-}
-
 template <typename T, int MAXDEG>
 __global__ void __launch_bounds__(kBlock) words_forward_kernel(const T *__restrict__ path, T *__restrict__ sig,
                                                                SigShape shape, LevelPlan plan,
@@ -117,7 +37,7 @@ __global__ void __launch_bounds__(kBlock) words_forward_kernel(const T *__restri
     switch (deg) {
 #define PSIG_CASE(N)                                                                                  \
     case N:                                                                                           \
-        if constexpr (N <= MAXDEG) forward_body<T, N>(path, sig, shape, plan, codes, row, bl, tile, sdx); \
+        if constexpr (N <= MAXDEG) forward_body<T, N, kBlock>(path, sig, shape, plan, codes, row, bl, tile, sdx); \
         break;
         PSIG_CASE(1) PSIG_CASE(2) PSIG_CASE(3) PSIG_CASE(4) PSIG_CASE(5) PSIG_CASE(6)
         PSIG_CASE(7) PSIG_CASE(8) PSIG_CASE(9) PSIG_CASE(10) PSIG_CASE(11) PSIG_CASE(12)
@@ -133,11 +53,12 @@ __global__ void __launch_bounds__(kBlock) words_forward_kernel(const T *__restri
 constexpr int kBwdBlock = kWave;
 constexpr int kSortedMax = 64;
 
-template <typename T, int DEG>
+// CHUNKED: `unit` counts time chunks of the paths (WordChunks), not rows.
+template <typename T, int DEG, bool CHUNKED>
 __device__ void backward_body(const T *__restrict__ path, const T *__restrict__ sig, const T *__restrict__ grad_sig,
                               double *__restrict__ grad_inc, const SigShape &shape, const LevelPlan &plan,
-                              const int64_t *__restrict__ codes, int64_t row, int64_t blk_in_level, int tile, T *sdx,
-                              T *sacc, T *sval, int *sorder, int *scnt) {
+                              const int64_t *__restrict__ codes, int64_t unit, int64_t blk_in_level, int tile, T *sdx,
+                              T *sacc, T *sval, int *sorder, int *scnt, const WordChunks &wc) {
     const int lane = threadIdx.x;
     const int64_t d = shape.d;
     const int64_t word_idx = blk_in_level * kBwdBlock + lane;
@@ -188,8 +109,10 @@ __device__ void backward_body(const T *__restrict__ path, const T *__restrict__ 
     }
     const bool two_runs = sorted && __all(changes <= 1);
 
+    const int64_t row = CHUNKED ? unit / wc.chunks : unit;
     const int64_t b = row / shape.W, w = row - b * shape.W;
-    const WindowSpan span = window_span(shape, w);
+    WindowSpan span = window_span(shape, w);
+    if constexpr (CHUNKED) span = chunk_of_span(span, wc.chunks, (int)(unit - row * wc.chunks));
     const T *x = path + (b * shape.L + span.start) * d;
     double *ginc = grad_inc + (b * (shape.L - 1) + span.start) * d;
     const T *srow = sig + row * plan.sig_size;
@@ -199,7 +122,9 @@ __device__ void backward_body(const T *__restrict__ path, const T *__restrict__ 
     p[0] = T(1);
 #pragma unroll
     for (int k = 1; k <= DEG; ++k) p[k] = T(0);
-    if (plan.from_saved[DEG]) {
+    if (CHUNKED) {
+        // (below, with the adjoint)
+    } else if (plan.from_saved[DEG]) {
         if (active) {
             uint64_t off = 0, width = (uint64_t)d, pref = 0;
 #pragma unroll
@@ -239,6 +164,7 @@ __device__ void backward_body(const T *__restrict__ path, const T *__restrict__ 
 #pragma unroll
     for (int k = 0; k <= DEG; ++k) h[k] = T(0);
     h[DEG] = active ? grad_sig[row * plan.sig_size + plan.out_off[DEG] + word_idx] : T(0);
+    if (CHUNKED && active) word_chunk_edges<T, DEG>(wc, plan, unit, word_idx, p, h);
 
     const int64_t ntiles = (span.steps + tile - 1) / tile;
     for (int64_t ti = ntiles - 1; ti >= 0; --ti) {
@@ -306,12 +232,12 @@ __device__ void backward_body(const T *__restrict__ path, const T *__restrict__ 
 
 // MAXDEG bounds the word lengths compiled into one kernel: the register budget of a kernel is that of its
 // longest chain, so shallow signatures get a kernel with more waves per SIMD.
-template <typename T, int MAXDEG>
+template <typename T, int MAXDEG, bool CHUNKED>
 __global__ void __launch_bounds__(kBwdBlock) words_backward_kernel(const T *__restrict__ path, const T *__restrict__ sig,
                                                                    const T *__restrict__ grad_sig,
                                                                    double *__restrict__ grad_inc, SigShape shape,
                                                                    LevelPlan plan, const int64_t *__restrict__ codes,
-                                                                   int tile) {
+                                                                   int tile, WordChunks wc) {
     extern __shared__ __align__(16) unsigned char smem[];
     T *sdx = reinterpret_cast<T *>(smem);
     T *sacc = sdx + (int64_t)tile * shape.d;
@@ -327,8 +253,8 @@ __global__ void __launch_bounds__(kBwdBlock) words_backward_kernel(const T *__re
 #define PSIG_CASE(N)                                                                                              \
     case N:                                                                                                       \
         if constexpr (N <= MAXDEG)                                                                                \
-            backward_body<T, N>(path, sig, grad_sig, grad_inc, shape, plan, codes, row, bl, tile, sdx, sacc, sval, \
-                                sorder, scnt);                                                                    \
+            backward_body<T, N, CHUNKED>(path, sig, grad_sig, grad_inc, shape, plan, codes, row, bl, tile, sdx, sacc, sval, \
+                                sorder, scnt, wc);                                                                \
         break;
         PSIG_CASE(1) PSIG_CASE(2) PSIG_CASE(3) PSIG_CASE(4) PSIG_CASE(5) PSIG_CASE(6)
         PSIG_CASE(7) PSIG_CASE(8) PSIG_CASE(9) PSIG_CASE(10) PSIG_CASE(11) PSIG_CASE(12)
@@ -454,7 +380,7 @@ hipError_t launch_words_forward(const T *path, T *sig, const SigShape &shape, co
 
 template <typename T>
 hipError_t launch_words_backward(const T *path, const T *sig, const T *grad_sig, double *grad_inc, const SigShape &shape,
-                                 const LevelPlan &plan_in, const int64_t *codes, hipStream_t stream) {
+                                 const LevelPlan &plan_in, const int64_t *codes, const WordChunks &wc, hipStream_t stream) {
     // same levels, blocks of one wave
     LevelPlan plan = plan_in;
     int64_t per_row = 0;
@@ -463,7 +389,7 @@ hipError_t launch_words_backward(const T *path, const T *sig, const T *grad_sig,
         per_row += (plan.size[k] + kBwdBlock - 1) / kBwdBlock;
     }
     plan.block_begin[plan.depth + 1] = per_row;
-    const int64_t blocks = per_row * shape.B * shape.W;
+    const int64_t blocks = per_row * shape.B * shape.W * (wc.chunks ? wc.chunks : 1);
     if (blocks == 0) return hipSuccess;
     if (blocks >= (int64_t(1) << 31)) return hipErrorInvalidValue;
     // one wave per block: a small tile keeps many blocks resident on a CU
@@ -471,8 +397,12 @@ hipError_t launch_words_backward(const T *path, const T *sig, const T *grad_sig,
     const size_t lds = (size_t)2 * tile * shape.d * sizeof(T) + (size_t)2 * plan.depth * kBwdBlock * sizeof(T) +
                        (size_t)plan.depth * kBwdBlock * sizeof(int) + (size_t)(kSortedMax + 1) * sizeof(int);
 #define PSIG_LAUNCH(MAXDEG)                                                                                       \
-    hipLaunchKernelGGL((words_backward_kernel<T, MAXDEG>), dim3((unsigned)blocks), dim3(kBwdBlock), lds, stream, path, \
-                       sig, grad_sig, grad_inc, shape, plan, codes, tile)
+    if (wc.chunks)                                                                                                \
+        hipLaunchKernelGGL((words_backward_kernel<T, MAXDEG, true>), dim3((unsigned)blocks), dim3(kBwdBlock), lds, stream, \
+                           path, sig, grad_sig, grad_inc, shape, plan, codes, tile, wc);                          \
+    else                                                                                                          \
+        hipLaunchKernelGGL((words_backward_kernel<T, MAXDEG, false>), dim3((unsigned)blocks), dim3(kBwdBlock), lds, stream, \
+                           path, sig, grad_sig, grad_inc, shape, plan, codes, tile, wc)
     if (plan.depth <= 3) PSIG_LAUNCH(3);
     else if (plan.depth <= 4) PSIG_LAUNCH(4);
     else if (plan.depth <= 6) PSIG_LAUNCH(6);
@@ -529,7 +459,7 @@ hipError_t launch_scatter_columns(const T *grad, T *dense, const LevelPlan &plan
     template hipError_t launch_words_forward<T>(const T *, T *, const SigShape &, const LevelPlan &, const int64_t *, \
                                                 hipStream_t);                                                       \
     template hipError_t launch_words_backward<T>(const T *, const T *, const T *, double *, const SigShape &,       \
-                                                 const LevelPlan &, const int64_t *, hipStream_t);                  \
+                                                 const LevelPlan &, const int64_t *, const WordChunks &, hipStream_t); \
     template hipError_t launch_fill_zero<T>(T *, int64_t, hipStream_t);                                             \
     template hipError_t launch_increments_to_path<T, T>(const T *, T *, int64_t, int64_t, int64_t, hipStream_t);
 PSIG_INSTANTIATE(float)
