@@ -46,8 +46,9 @@ public:
     static bool active();
 };
 
+// far_ok: far chunks may be chosen, or another entry of the table for the sake of its chunks.
 DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes, int64_t B,
-                         int64_t L, int64_t W, bool windowed);
+                         int64_t L, int64_t W, bool windowed, bool far_ok = true);
 
 // `sig` / `grad_sig` are dense-layout rows; `workspace` is the part of the scratch after any dense buffer.
 // top_codes / top_count: the word list of the top level (device memory), read only when dc.bounded.

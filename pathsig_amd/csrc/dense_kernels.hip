@@ -2997,7 +2997,7 @@ static double entry_us(const VariantInfo &v, size_t elem, int64_t rows, int64_t 
 }
 
 static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes,
-                                     int64_t B, int64_t L, int64_t W, bool windowed, bool plain) {
+                                     int64_t B, int64_t L, int64_t W, bool windowed, bool plain, bool far_ok) {
     DenseChoice dc{};
     dc.variant = -1;
     dc.fwd_chunks = dc.bwd_chunks = 1;
@@ -3020,7 +3020,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
             // .. unless the estimates say that this one is the faster all the same: the later entry's rows may be
             // dozens of waves swept in one piece
             if (later && rows * (v.block / kWave) * (cut ? max_chunks : 1) < (cut ? 1024 : 512) &&
-                (windowed || plain || (elem == 4 && L - 1 > kLongRowSteps) ||
+                (windowed || plain || !far_ok || (elem == 4 && L - 1 > kLongRowSteps) ||
                  entry_us(v, elem, rows, L) > 0.7 * entry_us(kVariants[other], elem, rows, L)))
                 continue;
             // the short prefixes of the wide alphabets hold 68 to 240 values per lane: fp64 up to 132 (d = 11) and
@@ -3028,7 +3028,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
             if (later && elem == 8 && !v.fp64_fits) continue;
         }
         const bool chunks_ok = v.chunks_ok[elem == 8 ? 1 : 0];
-        const int far = chunks_ok || windowed || plain ? 0 : far_chunks(v, elem, rows, L);
+        const int far = chunks_ok || windowed || plain || !far_ok ? 0 : far_chunks(v, elem, rows, L);
         const bool one_piece = !chunks_ok && far == 0;
         if (!all_dense) {
             // A word projection is computed densely and gathered when that is the cheaper way: when its top level
@@ -3181,9 +3181,9 @@ bool PlainChunks::active() { return plain_chunks(); }
 // A step of training asks for the same choice seven times (sizes of buffers, then the launches), and a small call is
 // bound by its host time: the last few choices of a thread are remembered.
 DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes, int64_t B,
-                         int64_t L, int64_t W, bool windowed) {
+                         int64_t L, int64_t W, bool windowed, bool far_ok) {
     struct Key {
-        int64_t elem, d, depth, all_dense, B, L, W, windowed, plain, options, sizes[kMaxDepth];
+        int64_t elem, d, depth, all_dense, B, L, W, windowed, plain, far_ok, options, sizes[kMaxDepth];
     };
     constexpr int kRemembered = 8;
     thread_local Key keys[kRemembered];
@@ -3200,11 +3200,12 @@ DenseChoice dense_choice(size_t elem, int64_t d, int depth, bool all_dense, cons
     key.W = W;
     key.windowed = windowed ? 1 : 0;
     key.plain = PlainChunks::active() ? 1 : 0;
+    key.far_ok = far_ok ? 1 : 0;
     key.options = options_epoch();
     if (!all_dense && level_sizes) std::memcpy(key.sizes, level_sizes + 1, (size_t)depth * sizeof(int64_t));
     for (unsigned i = 0; i < used; ++i)
         if (!std::memcmp(&keys[i], &key, sizeof key)) return choices[i];
-    const DenseChoice dc = make_dense_choice(elem, d, depth, all_dense, level_sizes, B, L, W, windowed, key.plain != 0);
+    const DenseChoice dc = make_dense_choice(elem, d, depth, all_dense, level_sizes, B, L, W, windowed, key.plain != 0, far_ok);
     keys[next] = key;
     choices[next] = dc;
     next = (next + 1) % kRemembered;
