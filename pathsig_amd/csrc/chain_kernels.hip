@@ -212,8 +212,8 @@ __global__ void __launch_bounds__(kTopWaves *kWave)
 }
 
 // Adjoints of the chunks.  Grid: x over (row, chunk), y over slices of the words.  A word of level m sums over the d + d^2 +
-// .. + d^(depth - m) words that continue it: by a group of lanes, as many as that number keeps at work, the more the fewer
-// words a level has.  Bandwidth of L2: every level is read once per shorter level.
+// .. + d^(depth - m) words that continue it: by a block, or by a group of lanes, as many as that number keeps at work, the
+// more the fewer words a level has.  Bandwidth of L2: every level is read once per shorter level.
 template <typename T>
 __global__ void __launch_bounds__(kChainThreads)
     chunk_adjoints_kernel(const T *__restrict__ grad, const T *__restrict__ right, T *__restrict__ out, int n, ChainLevels lv) {
@@ -230,9 +230,35 @@ __global__ void __launch_bounds__(kChainThreads)
         return;
     }
     for (uint32_t i = tid; i < lv.width[depth]; i += threads) to[lv.low + i] = g[lv.low + i];
+    __shared__ T part_sums[kChainThreads / kWave];
     uint32_t longer = 0;
     for (int m = depth - 1; m >= 1; --m) {
         longer += lv.width[depth - m];
+        if (longer >= 1024) {
+            // the short words: a block each, four products of a lane in flight
+            for (uint32_t w = blockIdx.y; w < lv.width[m]; w += gridDim.y) {
+                T sum = T(0);
+                for (int q = 1; q <= depth - m; ++q) {
+                    const T *from = g + lv.off[m + q] + w * lv.width[q], *by = z + lv.off[q];
+                    T level[4] = {T(0), T(0), T(0), T(0)};
+                    uint32_t s = threadIdx.x;
+                    for (; s + 3 * kChainThreads < lv.width[q]; s += 4 * kChainThreads)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) level[r] += from[s + r * kChainThreads] * by[s + r * kChainThreads];
+                    for (; s < lv.width[q]; s += kChainThreads) level[0] += from[s] * by[s];
+                    sum += (level[0] + level[1]) + (level[2] + level[3]);
+                }
+                for (uint32_t o = kWave / 2; o > 0; o >>= 1) sum += __shfl_xor(sum, (int)o, kWave);
+                if (threadIdx.x % kWave == 0) part_sums[threadIdx.x / kWave] = sum;
+                __syncthreads();
+                if (threadIdx.x == 0) {
+                    for (int v = 1; v < kChainThreads / kWave; ++v) sum += part_sums[v];
+                    to[lv.off[m] + w] = g[lv.off[m] + w] + sum;
+                }
+                __syncthreads();
+            }
+            continue;
+        }
         const uint32_t lanes = longer >= 256 ? kWave : longer >= 32 ? 16 : longer >= 8 ? 4 : 1;
         const uint32_t part = tid % lanes, step = threads / lanes;
         // (whole waves stay together: the shuffles below need all lanes of a group)

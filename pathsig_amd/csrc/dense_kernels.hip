@@ -2979,21 +2979,32 @@ static int far_chunks(const VariantInfo &v, size_t elem, int64_t rows, int64_t L
     return (int)c;
 }
 
-// What a call without windows takes with the kernels of an entry of the table, cut as it would be.  (Log-signature of (14, 4), 2
+// What a call without windows takes with the kernels of an entry of the table, cut as it would be: both sweeps, and the products
+// of the chunks.  (Log-signature of (14, 4), 2
 // paths of 2176 points, fp32: 3437 us a step with prefixes of three in one piece, 277 with prefixes of two in 64 chunks.)
-static double entry_us(const VariantInfo &v, size_t elem, int64_t rows, int64_t L) {
+struct EntryUs {
+    double sweeps, products;
+    double total() const { return sweeps + products; }
+};
+static EntryUs entry_us(const VariantInfo &v, size_t elem, int64_t rows, int64_t L) {
     if (v.chunks_ok[elem == 8 ? 1 : 0]) {
         const int chunks = pick_chunks(rows, v.block, L, 2048, false);
         const bool staged = 2 * (size_t)v.sig_size * elem <= 48 * 1024;
         const double products = chunks == 1 ? 0.0
                                             : scan_us(chunks, v.depth, (double)v.low_size * elem) +
                                                   combine_us(elem, chunks, v.depth, v.sig_size, staged);
-        return sweeps_us(v, elem, rows, L, chunks) + products;
+        return {sweeps_us(v, elem, rows, L, chunks), products};
     }
     const int far = far_chunks(v, elem, rows, L);
-    if (far == 0) return sweeps_us(v, elem, rows, L, 1);
-    return sweeps_us(v, elem, rows, L, far) + chain_us(elem, rows, far, v.d, v.depth, 2) +
-           chain_top_us(elem, rows, far, v.d, v.depth) + chunk_adjoints_us(elem, rows, far, v.d, v.depth);
+    if (far == 0) return {sweeps_us(v, elem, rows, L, 1), 0.0};
+    return {sweeps_us(v, elem, rows, L, far), chain_us(elem, rows, far, v.d, v.depth, 2) +
+                                                  chain_top_us(elem, rows, far, v.d, v.depth) +
+                                                  chunk_adjoints_us(elem, rows, far, v.d, v.depth)};
+}
+// (a forward alone is a quarter of the sweeps, and must not lose by the choice either)
+static bool entry_pays(const EntryUs &short_prefix, const EntryUs &long_prefix) {
+    return short_prefix.total() < 0.7 * long_prefix.total() &&
+           0.25 * short_prefix.sweeps + short_prefix.products + 4.0 < 0.25 * long_prefix.sweeps + long_prefix.products;
 }
 
 static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes,
@@ -3021,7 +3032,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
             // dozens of waves swept in one piece
             if (later && rows * (v.block / kWave) * (cut ? max_chunks : 1) < (cut ? 1024 : 512) &&
                 (windowed || plain || !far_ok || (elem == 4 && L - 1 > kLongRowSteps) ||
-                 entry_us(v, elem, rows, L) > 0.7 * entry_us(kVariants[other], elem, rows, L)))
+                 !entry_pays(entry_us(v, elem, rows, L), entry_us(kVariants[other], elem, rows, L))))
                 continue;
             // the short prefixes of the wide alphabets hold 68 to 240 values per lane: fp64 up to 132 (d = 11) and
             // wherever the children are split
@@ -3062,7 +3073,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
                 if (wc.chunks) {
                     const double chunked_us =
                         25.0 + 2.0 * steps / wc.chunks + 0.6 * wc.chunks + 5e-6 * words * (double)rows * steps;
-                    if (chunked_us < 0.6 * std::max(dense_us, entry_us(v, elem, rows, L) + 20.0)) return dc;
+                    if (chunked_us < 0.6 * std::max(dense_us, entry_us(v, elem, rows, L).total() + 20.0)) return dc;
                 }
             }
             if ((double)rows * (double)v.sig_size * (double)elem * (one_piece ? 2.0 : 1.0) > 4e9) return dc;

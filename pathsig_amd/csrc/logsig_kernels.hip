@@ -27,6 +27,7 @@
 //   * scatter form (any size): every word pushes its terms to its prefixes and suffixes with atomics.
 #include <cmath>
 #include <cstdlib>
+#include <algorithm>
 #include <type_traits>
 
 #include "common.hpp"
@@ -512,7 +513,8 @@ __device__ void block_matvec(const T *A, const T *B, const MatvecShape &sh, T *r
 // computes T(v) = sum_u g(uv) Qc(u) for the suffixes v of length N - j, where
 // Qc(u) = -sum_{k=2}^{|u|+1} Q_{k-1}(u) / k! is entry |u| of u's cache row (the forward puts it there).  R goes to its own workspace array, T
 // initialises the gradient.
-template <typename T>
+// SPLIT: the outputs of a product are shared by several blocks (few rows of a large layout).
+template <typename T, bool SPLIT>
 __global__ void __launch_bounds__(kLogBlock) logsig_gather_top_kernel(const T *__restrict__ logsig,
                                                                       const T *__restrict__ cache,
                                                                       const T *__restrict__ gtop_all, T *grad_sig,
@@ -521,7 +523,8 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_top_kernel(const T *_
     __shared__ T red[kLogBlock];
     const int N = hp.depth;
     const int64_t row = blockIdx.x;
-    const int j = (int)blockIdx.y + 1, i = N - j;
+    // (y: the split, and which slice of its outputs)
+    const int j = (SPLIT ? (int)blockIdx.y % (N - 1) : (int)blockIdx.y) + 1, i = N - j;
     const bool suffix_side = blockIdx.z == 1;
     if (!hp.summed) {
         // the gradient of a top-level word is its upstream gradient: every block of the row copies a slice
@@ -538,13 +541,20 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_top_kernel(const T *_
     int64_t wi = 1, wj = 1;
     for (int k = 0; k < i; ++k) wi *= hp.d;
     for (int k = 0; k < j; ++k) wj *= hp.d;
+    int64_t begin = 0, count = suffix_side ? wi : wj;
+    if constexpr (SPLIT) {
+        const int64_t outputs = count, part = (int64_t)blockIdx.y / (N - 1), parts = (int64_t)gridDim.y / (N - 1);
+        begin = outputs * part / parts;
+        count = outputs * (part + 1) / parts - begin;
+        if (count == 0) return;
+    }
     if (!suffix_side) {
-        T *R = R_all + row * hp.lower + hp.off[j];
-        block_matvec<T>(gtop, lgs + hp.off[i], MatvecShape{1, wj, wi, 1, 0, wi, 1, 0, 0, 1, 0}, red,
+        T *R = R_all + row * hp.lower + hp.off[j] + begin;
+        block_matvec<T>(gtop + begin * wi, lgs + hp.off[i], MatvecShape{1, count, wi, 1, 0, wi, 1, 0, 0, 1, 0}, red,
                         [&](int64_t, int64_t o, T r) { R[o] = r; });
     } else {
-        T *gsi = grad_sig + row * hp.total + hp.off[i];
-        block_matvec<T>(gtop, cache + row * hp.cache_stride + hp.off[j] * N + j, MatvecShape{1, wi, wj, 1, 0, 1, wi, 0, 0, N, 0},
+        T *gsi = grad_sig + row * hp.total + hp.off[i] + begin;
+        block_matvec<T>(gtop + begin, cache + row * hp.cache_stride + hp.off[j] * N + j, MatvecShape{1, count, wj, 1, 0, 1, wi, 0, 0, N, 0},
                         red, [&](int64_t, int64_t o, T r) { gsi[o] = hp.summed ? gsi[o] + r : r; });
     }
 }
@@ -586,19 +596,18 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_top_rows_kernel(
     }
 }
 
-// Levels below the top, one block per row, going down.  `a` ([lower columns][depth]) holds a_k: in LDS when the
-// launch provides room for it (A_IN_LDS; the kernel is a chain of short dependent passes over `a`, so their
-// latency is what it costs), else in the workspace.  `R` ([lower columns], workspace) are the top-level sums of
-// logsig_gather_top_kernel, which has also stored the top-level part of the gradient in grad_sig.
-// STAGED (with A_IN_LDS): everything else the passes read or update is brought to LDS in one burst of loads at the
+// Levels below the top, one block per row, going down.  `a` ([lower columns][depth]) holds a_k in LDS (the kernel is a
+// chain of short dependent passes over `a`, so their latency is what it costs).  `R` ([lower columns], workspace) are the
+// top-level sums of logsig_gather_top_kernel, which has also stored the top-level part of the gradient in grad_sig.
+// STAGED: everything else the passes read or update is brought to LDS in one burst of loads at the
 // start (the gradient of the levels below the top with the upstream gradient already added, the log-signature and
 // the cache rows of the levels 1 .. depth - 2), so that no pass waits for memory; the gradient goes back to memory
 // at the end.  For calls of a few hundred rows at most, where a row's latency is all there is.
-template <typename T, bool A_IN_LDS, bool STAGED = false>
+template <typename T, bool STAGED>
 __global__ void __launch_bounds__(kLogBlock) logsig_gather_kernel(const T *__restrict__ logsig,
                                                                   const T *__restrict__ cache,
                                                                   const T *__restrict__ grad_logsig, T *grad_sig,
-                                                                  T *a_all, const T *__restrict__ R_all, HybridPlan hp,
+                                                                  const T *__restrict__ R_all, HybridPlan hp,
                                                                   bool copy_top) {
     extern __shared__ __align__(16) unsigned char gather_smem[];
     __shared__ T red[kLogBlock];
@@ -609,11 +618,7 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_kernel(const T *__res
     const T *gl = grad_logsig + row * hp.total;
     T *gs = grad_sig + row * hp.total;
     const bool summed = hp.summed;  // gs holds the upstream gradient already
-    // the address space of `a` is fixed at compile time, so that its loads are LDS loads and not generic ones
-    static_assert(A_IN_LDS || !STAGED, "the staged form keeps `a` in LDS too");
-    T *a;
-    if constexpr (A_IN_LDS) a = reinterpret_cast<T *>(gather_smem);
-    else a = a_all + row * hp.lower * N;
+    T *a = reinterpret_cast<T *>(gather_smem);
     const T *R = R_all + row * hp.lower;
     const int64_t few = N >= 2 ? hp.off[N - 1] : 0;  // columns of the levels 1 .. N - 2
     const T *lgsp, *Crp;
@@ -753,6 +758,98 @@ __global__ void __launch_bounds__(kLogBlock) logsig_gather_kernel(const T *__res
     }
     if constexpr (STAGED)
         for (int64_t i = threadIdx.x; i < hp.lower; i += (int)blockDim.x) gs[i] = gsp[i];
+}
+
+// The same, a launch per level, for rows whose `a` does not fit a block's LDS: one block per row would wait for memory in every
+// pass, and a few rows leave most of the GPU idle.  A word's sums take `lanes` lanes (up to a wave, or the block), one term of
+// either sum each at a time.  Bound by the latency of those loads and of the launches.  us for all levels, one block per row /
+// launches: fp32 (6, 6), 2 rows, 123 / 44, (9, 5), 402 rows, 182 / 138; fp64 (9, 5), 1 row, 76 / 38, (8, 5), 128 rows, 70 / 46.
+// (Not for `a` in LDS: (3, 8), 85 rows, 76 in one launch and 76 in seven.)
+constexpr int kLevelThreads = 256;
+template <typename T, int DEG>
+__device__ __forceinline__ void adjoint_level(const T *lgs, const T *Cr, const T *gl, T *gs, T *a, const T *R,
+                                              const HybridPlan &hp, int64_t block, int lanes, T *red) {
+    const int N = hp.depth, tid = (int)threadIdx.x;
+    const int at = (int)block * kLevelThreads + tid, w = at / lanes, part = tid % lanes;
+    int wn = 1;
+    for (int k = 0; k < DEG; ++k) wn *= (int)hp.d;
+    const bool have = w < wn;
+    T sums[DEG + 1];  // sum_v a_{k+1}(w v) L(v), k = 1 .. DEG; sum_u sum_k a_k(u w) Q_{k-1}(u)
+#pragma unroll
+    for (int k = 0; k <= DEG; ++k) sums[k] = T(0);
+    if (have) {
+        int wi = 1;
+        for (int i = 1; i < N - DEG; ++i) {
+            wi *= (int)hp.d;
+            const T *av = a + (hp.off[DEG + i] + (int64_t)w * wi) * N + 1, *lv = lgs + hp.off[i];
+#pragma unroll 4
+            for (int v = part; v < wi; v += lanes) {
+                const T l = lv[v];
+#pragma unroll
+                for (int k = 0; k < DEG; ++k) sums[k] += av[(int64_t)v * N + k] * l;
+            }
+            const T *au = a + (hp.off[DEG + i] + w) * N + 1, *cu = Cr + hp.off[i] * N;
+            const int64_t apart = (int64_t)wn * N;
+#pragma unroll 2
+            for (int u = part; u < wi; u += lanes)
+                for (int m = 0; m < i; ++m) sums[DEG] += au[u * apart + m] * cu[(int64_t)u * N + m];
+        }
+    }
+    for (int o = (lanes < kWave ? lanes : kWave) / 2; o >= 1; o /= 2) {
+#pragma unroll
+        for (int k = 0; k <= DEG; ++k) sums[k] += __shfl_xor(sums[k], o);
+    }
+    if (lanes > kWave) {
+        // the block's waves share one word
+        constexpr int kWaves = kLevelThreads / kWave;
+        if (tid % kWave == 0) {
+#pragma unroll
+            for (int k = 0; k <= DEG; ++k) red[(tid / kWave) * (kMaxDepth + 1) + k] = sums[k];
+        }
+        __syncthreads();
+        if (tid == 0) {
+#pragma unroll
+            for (int k = 0; k <= DEG; ++k)
+                for (int q = 1; q < kWaves; ++q) sums[k] += red[q * (kMaxDepth + 1) + k];
+        }
+    }
+    if (!have || part != 0) return;
+    // a_k(w) starts from its top-level part, -R(w) / (k + 1)!; lam(w) = g(w) + a_1(w) + the other sums is the gradient of
+    // the word; a_k(w) -= lam(w) / k! for k >= 2
+    const int64_t col = hp.off[DEG] + w;
+    const T r = R[col];
+    T *aw = a + col * N;
+    const T first = sums[0] - inv_factorial<T>(2) * r;
+    const T lam = (hp.summed ? T(0) : gl[col]) + first + (gs[col] + sums[DEG]);
+    gs[col] = lam;
+    aw[0] = first;
+#pragma unroll
+    for (int k = 2; k <= DEG; ++k) aw[k - 1] = sums[k - 1] - inv_factorial<T>(k + 1) * r - inv_factorial<T>(k) * lam;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kLevelThreads)
+    logsig_level_kernel(const T *__restrict__ logsig, const T *__restrict__ cache, const T *__restrict__ grad_logsig,
+                        T *grad_sig, T *a_all, const T *__restrict__ R_all, HybridPlan hp, int level, int lanes,
+                        int64_t blocks, bool copy_top) {
+    __shared__ T red[kLevelThreads / kWave * (kMaxDepth + 1)];
+    const int64_t row = blockIdx.x / blocks, block = blockIdx.x - row * blocks;  // `blocks` to a row
+    const T *lgs = logsig + row * hp.lg_stride, *Cr = cache + row * hp.cache_stride;
+    const T *gl = grad_logsig + row * hp.total;
+    T *gs = grad_sig + row * hp.total, *a = a_all + row * hp.lower * hp.depth;
+    const T *R = R_all + row * hp.lower;
+    if (copy_top) {
+        for (int64_t i = block * kLevelThreads + threadIdx.x; i < hp.size[hp.depth]; i += blocks * kLevelThreads)
+            gs[hp.off[hp.depth] + i] = gl[hp.off[hp.depth] + i];
+    }
+    switch (level) {
+#define PSIG_CASE(N) \
+    case N: adjoint_level<T, N>(lgs, Cr, gl, gs, a, R, hp, block, lanes, red); break;
+        PSIG_CASE(1) PSIG_CASE(2) PSIG_CASE(3) PSIG_CASE(4) PSIG_CASE(5) PSIG_CASE(6)
+        PSIG_CASE(7) PSIG_CASE(8) PSIG_CASE(9) PSIG_CASE(10) PSIG_CASE(11)
+#undef PSIG_CASE
+        default: break;
+    }
 }
 
 // dense[row][code of word e] += grad_logsig[row][top column e]; dense must be zero on entry
@@ -938,9 +1035,16 @@ hipError_t launch_adjoint(const T *logsig, const T *cache, const T *grad_logsig,
                 gtop = dense;
                 top_stride = lp.top_dense;
             }
-            hipLaunchKernelGGL(logsig_gather_top_kernel<T>, dim3((unsigned)rows, (unsigned)(depth - 1), 2),
-                               dim3(kLogBlock), 0, stream, logsig, cache, gtop, grad_sig, R, hp, top_stride,
-                               grad_logsig);
+            // A thousand blocks: few rows of a large layout split the outputs of a product, up to sixteen ways (fp64 (9, 5), 1 row,
+            // 56 us whole, 29 split; fp32 (6, 6), 2 rows, 38 / 29).
+            const int64_t parts = std::min<int64_t>(1024 / (rows * (depth - 1) * 2), 16);
+            if (parts >= 4 && lp.top_dense >= 32768)
+                hipLaunchKernelGGL((logsig_gather_top_kernel<T, true>),
+                                   dim3((unsigned)rows, (unsigned)((depth - 1) * parts), 2), dim3(kLogBlock), 0, stream, logsig,
+                                   cache, gtop, grad_sig, R, hp, top_stride, grad_logsig);
+            else
+                hipLaunchKernelGGL((logsig_gather_top_kernel<T, false>), dim3((unsigned)rows, (unsigned)(depth - 1), 2),
+                                   dim3(kLogBlock), 0, stream, logsig, cache, gtop, grad_sig, R, hp, top_stride, grad_logsig);
         }
         e = hipGetLastError();
         if (e != hipSuccess) return e;
@@ -951,21 +1055,36 @@ hipError_t launch_adjoint(const T *logsig, const T *cache, const T *grad_logsig,
         const size_t staged_bytes = a_bytes + (size_t)(hp.lower + few * (1 + depth)) * sizeof(T);
         if (a_in_lds && rows <= 512 && staged_bytes <= 150 * 1024) {
             if (staged_bytes > 32 * 1024) {
-                e = allow_dynamic_lds<logsig_gather_kernel<T, true, true>>(staged_bytes);
+                e = allow_dynamic_lds<logsig_gather_kernel<T, true>>(staged_bytes);
                 if (e != hipSuccess) return e;
             }
-            hipLaunchKernelGGL((logsig_gather_kernel<T, true, true>), dim3((unsigned)rows), dim3(blk), staged_bytes,
-                               stream, logsig, cache, grad_logsig, grad_sig, gradP, (const T *)R, hp, copy_top);
+            hipLaunchKernelGGL((logsig_gather_kernel<T, true>), dim3((unsigned)rows), dim3(blk), staged_bytes,
+                               stream, logsig, cache, grad_logsig, grad_sig, (const T *)R, hp, copy_top);
         } else if (a_in_lds) {
             if (a_bytes > 32 * 1024) {
-                e = allow_dynamic_lds<logsig_gather_kernel<T, true>>(a_bytes);
+                e = allow_dynamic_lds<logsig_gather_kernel<T, false>>(a_bytes);
                 if (e != hipSuccess) return e;
             }
-            hipLaunchKernelGGL((logsig_gather_kernel<T, true>), dim3((unsigned)rows), dim3(blk), a_bytes, stream,
-                               logsig, cache, grad_logsig, grad_sig, gradP, (const T *)R, hp, copy_top);
+            hipLaunchKernelGGL((logsig_gather_kernel<T, false>), dim3((unsigned)rows), dim3(blk), a_bytes, stream,
+                               logsig, cache, grad_logsig, grad_sig, (const T *)R, hp, copy_top);
         } else {
-            hipLaunchKernelGGL((logsig_gather_kernel<T, false>), dim3((unsigned)rows), dim3(blk), 0, stream, logsig,
-                               cache, grad_logsig, grad_sig, gradP, (const T *)R, hp, copy_top);
+            int64_t words = hp.lower - (depth >= 2 ? hp.off[depth - 1] : 0), longer = 0;  // of the level; that continue a word
+            for (int n = depth - 1; n >= 1; --n) {
+                // four terms and more to a lane, sixteen where the words alone fill the GPU
+                const int64_t each = rows * words >= 65536 ? 16 : 4;
+                int lanes = 1;
+                while (lanes < kWave && lanes * 2 * each <= longer) lanes *= 2;
+                if (longer >= 1024 && rows * words <= 4096) lanes = kLevelThreads;
+                const int64_t blocks = (words * lanes + kLevelThreads - 1) / kLevelThreads;
+                if (rows * blocks >= (int64_t(1) << 31)) return hipErrorInvalidValue;
+                hipLaunchKernelGGL(logsig_level_kernel<T>, dim3((unsigned)(rows * blocks)), dim3(kLevelThreads), 0, stream,
+                                   logsig, cache, grad_logsig, grad_sig, gradP, (const T *)R, hp, n, lanes, blocks,
+                                   copy_top && n == depth - 1);
+                e = hipGetLastError();
+                if (e != hipSuccess) return e;
+                longer = (longer + 1) * d;
+                words /= d;
+            }
         }
         return hipGetLastError();
     }
@@ -1006,10 +1125,22 @@ hipError_t launch_picked_logsig(const T *sig, int64_t sig_stride, T *lg, T *cach
     int64_t slices = (n_out + 4 * blk - 1) / (4 * blk);
     if (slices > 16) slices = 16;
     const bool together = slices < 2;
+    // few rows: the level below the top, if it is a large one, is shared by several blocks too (fp64 (9, 5), 1 row: 35 us in two
+    // launches, 15 in three)
+    int64_t below = (hp.lower - hp.off[depth - 1] + blk - 1) / blk;
+    if (below > 64) below = 64;
+    const bool split = !together && depth >= 3 && below >= 8 && rows <= 64;
+    if (split) slices = std::min<int64_t>((n_out + blk - 1) / blk, 64);
     hipLaunchKernelGGL((logsig_picked_kernel<T, uint32_t>), dim3((unsigned)rows), dim3(blk), 0, stream, sig, sig_stride, lg,
-                       cache, out, n_out, hp, top, top_words, picked, 1, depth - 1, together);
+                       cache, out, n_out, hp, top, top_words, picked, 1, split ? depth - 2 : depth - 1, together);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || together) return e;
+    if (split) {
+        hipLaunchKernelGGL((logsig_picked_kernel<T, uint32_t>), dim3((unsigned)rows, (unsigned)below), dim3(blk), 0, stream,
+                           sig, sig_stride, lg, cache, out, n_out, hp, top, top_words, picked, depth - 1, depth - 1, false);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
     hipLaunchKernelGGL((logsig_picked_kernel<T, uint32_t>), dim3((unsigned)rows, (unsigned)slices), dim3(blk), 0, stream,
                        sig, sig_stride, lg, cache, out, n_out, hp, top, top_words, picked, 1, 0, true);
     return hipGetLastError();
