@@ -1645,6 +1645,128 @@ __global__ void __launch_bounds__(kWave) chunk_level1_kernel(const T *__restrict
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Depth 2 in windows.  A row has no more lanes than letters, so the sweeps above leave most of a wave idle, and nothing at
+// this depth needs a sweep: with x' = x - x_start, u' the midpoint of an increment and dx the increment itself,
+//     S(ab) = sum_t u'_a dx_b,     dL/d(dx_b) = g(b) + sum_c g(bc) x'_end,c + sum_a u'_a (g(ab) - g(ba)).
+// Several windows share a wave, a lane to each of their letters (padded to a power of two); an increment's letters reach the
+// lanes of its window through LDS.  Bound by vector issue for long windows, by the rows of the signature in memory for short
+// ones.  us, a lane to a letter of one window / several windows to a wave: a step, fp64, 237 427 windows of 9 points, 12 letters
+// (log-signature) 1373 / 714, 2674 of 204, 15 letters, 391 / 186; fp32, 12 400 of 64, 8 letters, 145 / 63; a forward, 7936 of 128,
+// 13 letters, 59 / 20, fp64, 97 405 of 23, 5 letters, 84 / 25.
+// ---------------------------------------------------------------------------------------------
+constexpr int kPairsThreads = 256;
+constexpr int pairs_lanes(int d) { return d <= 2 ? 2 : d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : 32; }
+
+// The lanes of a window, its path and its steps; all lanes of a wave run `most` rounds.
+template <typename T, int D>
+struct PairsLane {
+    static constexpr int G = pairs_lanes(D), kRows = kPairsThreads / G;
+    int64_t row, b;
+    Span span;
+    int letter;
+    int64_t most;
+    bool have;  // a letter of a window
+    __device__ __forceinline__ explicit PairsLane(const SigShape &shape) {
+        letter = (int)threadIdx.x % G;
+        row = (int64_t)blockIdx.x * kRows + (int)threadIdx.x / G;
+        have = row < shape.B * shape.W && letter < D;
+        int64_t w;
+        divide_index(have ? row : 0, shape.W, b, w);
+        span = unit_span(shape, w);
+        if (!have) span.steps = 0;
+        most = span.steps;
+        for (int o = kWave / 2; o >= 1; o /= 2) {
+            const int64_t other = __shfl_xor((long long)most, o);
+            most = other > most ? other : most;
+        }
+    }
+};
+
+// the values that the lanes of a window hold, one to a letter, in all of them
+template <typename T, int D>
+__device__ __forceinline__ void share_letters(T *mine, int letter, T v, T (&all)[D]) {
+    mine[letter] = v;
+    // (the LDS operations of a wave complete in order; the fences keep the compiler from moving them)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int k = 0; k < D; ++k) all[k] = mine[k];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <typename T, int D>
+__global__ void __launch_bounds__(kPairsThreads) pairs_forward_kernel(const T *__restrict__ path, T *__restrict__ sig, SigShape shape) {
+    using PL = PairsLane<T, D>;
+    __shared__ __align__(16) T letters[PL::kRows][PL::G];
+    const PL pl(shape);
+    T *mine = letters[(int)threadIdx.x / PL::G];
+    const T *x = path + (pl.b * shape.L + pl.span.start) * D + (pl.have ? pl.letter : 0);
+    const int64_t steps = pl.span.steps;
+    T acc[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) acc[k] = T(0);
+    const T start = steps > 0 ? x[0] : T(0);
+    T from = start, to = steps > 0 ? x[D] : start;
+    for (int64_t t = 0; t < pl.most; ++t) {
+        const T ahead = t + 1 < steps ? x[(t + 2) * D] : to;
+        const T dx = to - from, mid = (from - start) + dx * T(0.5);
+        T all[D];
+        share_letters<T, D>(mine, pl.letter, dx, all);
+#pragma unroll
+        for (int k = 0; k < D; ++k) acc[k] = fmad<T>(mid, all[k], acc[k]);
+        from = to;  // (beyond the window: increments of zero)
+        to = ahead;
+    }
+    if (!pl.have) return;
+    T *out = sig + pl.row * (D + D * D);
+    out[pl.letter] = from - start;
+#pragma unroll
+    for (int k = 0; k < D; ++k) out[D + pl.letter * D + k] = acc[k];
+}
+
+// adds the sums of its windows to the per-increment gradients
+template <typename T, int D>
+__global__ void __launch_bounds__(kPairsThreads)
+    pairs_backward_kernel(const T *__restrict__ path, const T *__restrict__ grad_sig, T *__restrict__ grad_inc, SigShape shape) {
+    using PL = PairsLane<T, D>;
+    __shared__ __align__(16) T letters[PL::kRows][PL::G];
+    const PL pl(shape);
+    T *mine = letters[(int)threadIdx.x / PL::G];
+    const int letter = pl.have ? pl.letter : 0;
+    const int64_t steps = pl.span.steps;
+    const T *x = path + (pl.b * shape.L + pl.span.start) * D + letter;
+    T *ginc = grad_inc + (pl.b * (shape.L - 1) + pl.span.start) * D + letter;
+    const T *g = grad_sig + (pl.have ? pl.row : 0) * (D + D * D);
+    const T start = steps > 0 ? x[0] : T(0);
+    T turn[D], fixed = g[letter];  // g(ab) - g(ba) for this letter b; what all increments of the window get
+    {
+        T whole[D];
+        share_letters<T, D>(mine, pl.letter, steps > 0 ? x[steps * D] - start : T(0), whole);
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            const T own = g[D + letter * D + a];
+            fixed = fmad<T>(own, whole[a], fixed);
+            turn[a] = g[D + a * D + letter] - own;
+        }
+    }
+    T from = start, to = steps > 0 ? x[D] : start;
+    for (int64_t t = 0; t < pl.most; ++t) {
+        const T ahead = t + 1 < steps ? x[(t + 2) * D] : to;
+        T mid[D];
+        share_letters<T, D>(mine, pl.letter, (from - start) + (to - from) * T(0.5), mid);
+        T v = fixed;
+#pragma unroll
+        for (int a = 0; a < D; ++a) v = fmad<T>(mid[a], turn[a], v);
+        if (pl.have && t < steps) atomicAdd(&ginc[t * D], v);
+        from = to;
+        to = ahead;
+    }
+}
+
 // LDS layout of the reverse sweep.  Per-increment sums leave a wave as four row sums (eight partial sums where the
 // slab below is used); the tile flush adds the parts of all waves in a fixed order.  The tile is shortened until
 // the parts fit 48 KB of LDS (128 KB for the widest alphabets, whose parts of sixteen increments would not fit a
@@ -2606,6 +2728,14 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, const Dense
     const int chunks = dc.fwd_chunks;
     if (bounds && !kBoundsOk) return hipErrorInvalidValue;
     if (chunks <= 1) {
+        if constexpr (N == 2 && D <= 32) {
+            if (shape.windows) {
+                const int64_t per_block = PairsLane<T, D>::kRows;
+                hipLaunchKernelGGL((pairs_forward_kernel<T, D>), dim3((unsigned)((rows + per_block - 1) / per_block)),
+                                   dim3(kPairsThreads), 0, stream, path, sig, shape);
+                return hipGetLastError();
+            }
+        }
         if constexpr (kBoundsOk) {
             if (bounds) {
                 hipLaunchKernelGGL((dense_forward_kernel<T, D, N, P, 1, true>), dim3((unsigned)rows), dim3(G::kBlock),
@@ -2824,8 +2954,14 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
         const dim3 grid((unsigned)(rows * pieces * G::kUnitBlocks));
         profile_bracket(true, stream);
         if (accumulate) {
-            hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, false>), grid, dim3(G::kBlock), 0, stream, path, sig,
-                               adjoint, state, (const T *)nullptr, grad_inc, shape, pieces);
+            if constexpr (N == 2 && D <= 32) {  // (units of one block: windows)
+                const int64_t per_block = PairsLane<T, D>::kRows;
+                hipLaunchKernelGGL((pairs_backward_kernel<T, D>), dim3((unsigned)((rows + per_block - 1) / per_block)),
+                                   dim3(kPairsThreads), 0, stream, path, grad_sig, grad_inc, shape);
+            } else {
+                hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, false>), grid, dim3(G::kBlock), 0, stream, path, sig,
+                                   adjoint, state, (const T *)nullptr, grad_inc, shape, pieces);
+            }
         } else {
             if constexpr (G::kUnitBlocks == 1)
                 hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, false, false>), grid, dim3(G::kBlock), 0, stream, path,
@@ -3097,6 +3233,9 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         // (letter blocks: twice the waves that fit the GPU at once, so that the short ones fill in behind the long)
         const int64_t want_waves = dc.bounded && elem == 4 ? 4096 : 2048;
         int chunks = pick_chunks(rows, v.block, L, want_waves, many && may_chain);
+        // depth 2 in windows: several share a wave, and nothing is swept (pairs_forward_kernel); few of them, of lengths that
+        // are not known here, are cut into chunks all the same
+        if (windowed && depth == 2 && d <= 32 && (rows >= 512 || L <= 128)) chunks = 1;
         // deep fp32 shapes: the reverse sweep rebuilds A_t from A_{t+1} step by step, and over a span of
         // large increments that roll-back loses digits at depth 9 and more (d = 2, depth 12, five increments of
         // size 0.8: gradient off by 1.5e-5 in one piece, 1e-6 in two or more); four chunks at least
