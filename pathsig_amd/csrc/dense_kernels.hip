@@ -1652,7 +1652,7 @@ __global__ void __launch_bounds__(kWave) chunk_level1_kernel(const T *__restrict
 // Several windows share a wave, a lane to each of their letters (padded to a power of two); an increment's letters reach the
 // lanes of its window through LDS.  Bound by vector issue for long windows, by the rows of the signature in memory for short
 // ones.  us, a lane to a letter of one window / several windows to a wave: a step, fp64, 237 427 windows of 9 points, 12 letters
-// (log-signature) 1373 / 714, 2674 of 204, 15 letters, 391 / 186; fp32, 12 400 of 64, 8 letters, 145 / 63; a forward, 7936 of 128,
+// (log-signature) 1373 / 714, 2674 of 204, 15 letters, 391 / 131; fp32, 12 400 of 64, 8 letters, 145 / 63; a forward, 7936 of 128,
 // 13 letters, 59 / 20, fp64, 97 405 of 23, 5 letters, 84 / 25.
 // ---------------------------------------------------------------------------------------------
 constexpr int kPairsThreads = 256;
@@ -1683,43 +1683,56 @@ struct PairsLane {
     }
 };
 
-// the values that the lanes of a window hold, one to a letter, in all of them
-template <typename T, int D>
-__device__ __forceinline__ void share_letters(T *mine, int letter, T v, T (&all)[D]) {
-    mine[letter] = v;
-    // (the LDS operations of a wave complete in order; the fences keep the compiler from moving them)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-    for (int k = 0; k < D; ++k) all[k] = mine[k];
+// Orders a wave's LDS stores before its reads, and these before the next stores.  (The LDS operations of a wave complete in
+// order; the fences keep the compiler from moving them.)
+__device__ __forceinline__ void pairs_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <typename T, int D>
+// Increments that meet in LDS at a time (U of the kernels): the round trip, and the points fetched ahead, are waited for once
+// for all of them, which pays while the SIMDs have little else to do.  us, one / four: 2674 windows of 204 points, 15 letters,
+// fp64, forward and backward kernel 66 + 100 / 40 + 72 (669 waves); a forward of 7936 of 128, 13 letters, fp32, 19.8 / 22.8 (1984
+// waves), of 97 405 of 23, 5 letters, fp64, 24.5 / 29.0.
+inline bool pairs_few(int64_t rows, int lanes) { return rows * lanes < 1536 * kWave; }
+
+template <typename T, int D, int U>
 __global__ void __launch_bounds__(kPairsThreads) pairs_forward_kernel(const T *__restrict__ path, T *__restrict__ sig, SigShape shape) {
     using PL = PairsLane<T, D>;
-    __shared__ __align__(16) T letters[PL::kRows][PL::G];
+    __shared__ __align__(16) T letters[PL::kRows][U][PL::G];
     const PL pl(shape);
-    T *mine = letters[(int)threadIdx.x / PL::G];
+    T(*mine)[PL::G] = letters[(int)threadIdx.x / PL::G];
     const T *x = path + (pl.b * shape.L + pl.span.start) * D + (pl.have ? pl.letter : 0);
     const int64_t steps = pl.span.steps;
-    T acc[D];
+    // (points beyond the window are its last one: increments of zero)
+    auto point = [&](int64_t t) { return steps > 0 ? x[(t < steps ? t : steps) * D] : T(0); };
+    T acc[D], to[U];
 #pragma unroll
     for (int k = 0; k < D; ++k) acc[k] = T(0);
-    const T start = steps > 0 ? x[0] : T(0);
-    T from = start, to = steps > 0 ? x[D] : start;
-    for (int64_t t = 0; t < pl.most; ++t) {
-        const T ahead = t + 1 < steps ? x[(t + 2) * D] : to;
-        const T dx = to - from, mid = (from - start) + dx * T(0.5);
-        T all[D];
-        share_letters<T, D>(mine, pl.letter, dx, all);
+    const T start = point(0);
+    T from = start;
 #pragma unroll
-        for (int k = 0; k < D; ++k) acc[k] = fmad<T>(mid, all[k], acc[k]);
-        from = to;  // (beyond the window: increments of zero)
-        to = ahead;
+    for (int u = 0; u < U; ++u) to[u] = point(u + 1);
+    for (int64_t t = 0; t < pl.most; t += U) {
+        T mid[U], ahead[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) ahead[u] = point(t + U + u + 1);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const T dx = to[u] - from;
+            mid[u] = (from - start) + dx * T(0.5);
+            mine[u][pl.letter] = dx;
+            from = to[u];
+        }
+        pairs_fence();
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int k = 0; k < D; ++k) acc[k] = fmad<T>(mid[u], mine[u][k], acc[k]);
+        pairs_fence();
+#pragma unroll
+        for (int u = 0; u < U; ++u) to[u] = ahead[u];
     }
     if (!pl.have) return;
     T *out = sig + pl.row * (D + D * D);
@@ -1729,41 +1742,53 @@ __global__ void __launch_bounds__(kPairsThreads) pairs_forward_kernel(const T *_
 }
 
 // adds the sums of its windows to the per-increment gradients
-template <typename T, int D>
+template <typename T, int D, int U>
 __global__ void __launch_bounds__(kPairsThreads)
     pairs_backward_kernel(const T *__restrict__ path, const T *__restrict__ grad_sig, T *__restrict__ grad_inc, SigShape shape) {
     using PL = PairsLane<T, D>;
-    __shared__ __align__(16) T letters[PL::kRows][PL::G];
+    __shared__ __align__(16) T letters[PL::kRows][U][PL::G];
     const PL pl(shape);
-    T *mine = letters[(int)threadIdx.x / PL::G];
+    T(*mine)[PL::G] = letters[(int)threadIdx.x / PL::G];
     const int letter = pl.have ? pl.letter : 0;
     const int64_t steps = pl.span.steps;
     const T *x = path + (pl.b * shape.L + pl.span.start) * D + letter;
     T *ginc = grad_inc + (pl.b * (shape.L - 1) + pl.span.start) * D + letter;
     const T *g = grad_sig + (pl.have ? pl.row : 0) * (D + D * D);
-    const T start = steps > 0 ? x[0] : T(0);
+    auto point = [&](int64_t t) { return steps > 0 ? x[(t < steps ? t : steps) * D] : T(0); };
+    const T start = point(0);
+    T from = start, to[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) to[u] = point(u + 1);
     T turn[D], fixed = g[letter];  // g(ab) - g(ba) for this letter b; what all increments of the window get
-    {
-        T whole[D];
-        share_letters<T, D>(mine, pl.letter, steps > 0 ? x[steps * D] - start : T(0), whole);
+    mine[0][pl.letter] = point(steps) - start;
+    pairs_fence();
 #pragma unroll
-        for (int a = 0; a < D; ++a) {
-            const T own = g[D + letter * D + a];
-            fixed = fmad<T>(own, whole[a], fixed);
-            turn[a] = g[D + a * D + letter] - own;
-        }
+    for (int a = 0; a < D; ++a) {
+        const T own = g[D + letter * D + a];
+        fixed = fmad<T>(own, mine[0][a], fixed);
+        turn[a] = g[D + a * D + letter] - own;
     }
-    T from = start, to = steps > 0 ? x[D] : start;
-    for (int64_t t = 0; t < pl.most; ++t) {
-        const T ahead = t + 1 < steps ? x[(t + 2) * D] : to;
-        T mid[D];
-        share_letters<T, D>(mine, pl.letter, (from - start) + (to - from) * T(0.5), mid);
-        T v = fixed;
+    pairs_fence();
+    for (int64_t t = 0; t < pl.most; t += U) {
+        T ahead[U];
 #pragma unroll
-        for (int a = 0; a < D; ++a) v = fmad<T>(mid[a], turn[a], v);
-        if (pl.have && t < steps) atomicAdd(&ginc[t * D], v);
-        from = to;
-        to = ahead;
+        for (int u = 0; u < U; ++u) ahead[u] = point(t + U + u + 1);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            mine[u][pl.letter] = (from - start) + (to[u] - from) * T(0.5);
+            from = to[u];
+        }
+        pairs_fence();
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            T v = fixed;
+#pragma unroll
+            for (int a = 0; a < D; ++a) v = fmad<T>(mine[u][a], turn[a], v);
+            if (pl.have && t + u < steps) atomicAdd(&ginc[(t + u) * D], v);
+        }
+        pairs_fence();
+#pragma unroll
+        for (int u = 0; u < U; ++u) to[u] = ahead[u];
     }
 }
 
@@ -2731,8 +2756,11 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, const Dense
         if constexpr (N == 2 && D <= 32) {
             if (shape.windows) {
                 const int64_t per_block = PairsLane<T, D>::kRows;
-                hipLaunchKernelGGL((pairs_forward_kernel<T, D>), dim3((unsigned)((rows + per_block - 1) / per_block)),
-                                   dim3(kPairsThreads), 0, stream, path, sig, shape);
+                const dim3 grid((unsigned)((rows + per_block - 1) / per_block));
+                if (pairs_few(rows, PairsLane<T, D>::G))
+                    hipLaunchKernelGGL((pairs_forward_kernel<T, D, 4>), grid, dim3(kPairsThreads), 0, stream, path, sig, shape);
+                else
+                    hipLaunchKernelGGL((pairs_forward_kernel<T, D, 1>), grid, dim3(kPairsThreads), 0, stream, path, sig, shape);
                 return hipGetLastError();
             }
         }
@@ -2956,8 +2984,13 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
         if (accumulate) {
             if constexpr (N == 2 && D <= 32) {  // (units of one block: windows)
                 const int64_t per_block = PairsLane<T, D>::kRows;
-                hipLaunchKernelGGL((pairs_backward_kernel<T, D>), dim3((unsigned)((rows + per_block - 1) / per_block)),
-                                   dim3(kPairsThreads), 0, stream, path, grad_sig, grad_inc, shape);
+                const dim3 blocks((unsigned)((rows + per_block - 1) / per_block));
+                if (pairs_few(rows, PairsLane<T, D>::G))
+                    hipLaunchKernelGGL((pairs_backward_kernel<T, D, 4>), blocks, dim3(kPairsThreads), 0, stream, path,
+                                       grad_sig, grad_inc, shape);
+                else
+                    hipLaunchKernelGGL((pairs_backward_kernel<T, D, 1>), blocks, dim3(kPairsThreads), 0, stream, path,
+                                       grad_sig, grad_inc, shape);
             } else {
                 hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, false>), grid, dim3(G::kBlock), 0, stream, path, sig,
                                    adjoint, state, (const T *)nullptr, grad_inc, shape, pieces);

@@ -13,8 +13,10 @@ TOL = {torch.float32: 1e-5, torch.float64: 1e-12}
 # letters around the padded group sizes; windows that are empty, of one point, of one increment, overlapping, of very
 # different lengths inside one wave, out of range; more windows than a block holds; a path far from the origin
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
-@pytest.mark.parametrize("d", [2, 3, 4, 5, 8, 9, 15, 16, 17, 32, 33])
-@pytest.mark.parametrize("B,far", [(1, False), (40, False), (7, True)])
+# (3000 paths: windows enough to take one increment at a time)
+@pytest.mark.parametrize("d,B,far", [(d, B, far) for d in (2, 3, 4, 5, 8, 9, 15, 16, 17, 32, 33)
+                                     for B, far in ((1, False), (40, False), (7, True))]
+                         + [(4, 3000, False), (9, 3000, False), (17, 3000, False)])
 def test_depth_two_windows(dtype, d, B, far):
     import pathsig_amd as ps
     L = 60
