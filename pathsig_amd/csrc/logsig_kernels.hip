@@ -1036,9 +1036,10 @@ hipError_t launch_adjoint(const T *logsig, const T *cache, const T *grad_logsig,
                 top_stride = lp.top_dense;
             }
             // A thousand blocks: few rows of a large layout split the outputs of a product, up to sixteen ways (fp64 (9, 5), 1 row,
-            // 56 us whole, 29 split; fp32 (6, 6), 2 rows, 38 / 29).
+            // 56 us whole, 29 split; fp32 (6, 6), 2 rows, 38 / 29).  Not up to (8, 5) and (14, 4), 32 768 and 38 416 words,
+            // whose steps lose 4 to 13 % by it (fp32, 13 rows, 96 / 109 us and 93 / 107).
             const int64_t parts = std::min<int64_t>(1024 / (rows * (depth - 1) * 2), 16);
-            if (parts >= 4 && lp.top_dense >= 32768)
+            if (parts >= 4 && lp.top_dense >= 45000)
                 hipLaunchKernelGGL((logsig_gather_top_kernel<T, true>),
                                    dim3((unsigned)rows, (unsigned)((depth - 1) * parts), 2), dim3(kLogBlock), 0, stream, logsig,
                                    cache, gtop, grad_sig, R, hp, top_stride, grad_logsig);
