@@ -1648,7 +1648,7 @@ __global__ void __launch_bounds__(kWave) chunk_level1_kernel(const T *__restrict
 // ---------------------------------------------------------------------------------------------
 // Depth 2 in windows.  A row has no more lanes than letters, so the sweeps above leave most of a wave idle, and nothing at
 // this depth needs a sweep: with x' = x - x_start, u' the midpoint of an increment and dx the increment itself,
-//     S(ab) = sum_t u'_a dx_b,     dL/d(dx_b) = g(b) + sum_c g(bc) x'_end,c + sum_a u'_a (g(ab) - g(ba)).
+//     S(ab) = sum_t u'_a dx_b,     dL/d(dx_b) = g(b) + sum_a u'_a g(ab) + sum_c (x'_end - u')_c g(bc).
 // Several windows share a wave, a lane to each of their letters (padded to a power of two); an increment's letters reach the
 // lanes of its window through LDS.  Bound by vector issue for long windows, by the rows of the signature in memory for short
 // ones.  us, a lane to a letter of one window / several windows to a wave: a step, fp64, 237 427 windows of 9 points, 12 letters
@@ -1697,6 +1697,24 @@ __device__ __forceinline__ void pairs_fence() {
 // waves), of 97 405 of 23, 5 letters, fp64, 24.5 / 29.0.
 inline bool pairs_few(int64_t rows, int lanes) { return rows * lanes < 1536 * kWave; }
 
+// Letter of a window's running point, relative to the first.  The difference of the points is exact to a rounding; where either
+// is not finite, the sum of the increments says what the sweeps say: a point that is not finite stays visible in what follows it.
+template <typename T>
+struct PairsPoint {
+    T start, sum = T(0);
+    __device__ __forceinline__ T reached(T at) const {
+        const T apart = at - start;
+        return __builtin_elementwise_abs(apart - sum) < T(INFINITY) ? apart : sum;
+    }
+    // midpoint of the increment from `at` to `to`, which is passed; zero beyond the window
+    __device__ __forceinline__ T pass(T at, T to, bool in, T &dx) {
+        dx = in ? to - at : T(0);
+        const T mid = in ? reached(at) + dx * T(0.5) : T(0);
+        sum += dx;
+        return mid;
+    }
+};
+
 template <typename T, int D, int U>
 __global__ void __launch_bounds__(kPairsThreads) pairs_forward_kernel(const T *__restrict__ path, T *__restrict__ sig, SigShape shape) {
     using PL = PairsLane<T, D>;
@@ -1705,13 +1723,13 @@ __global__ void __launch_bounds__(kPairsThreads) pairs_forward_kernel(const T *_
     T(*mine)[PL::G] = letters[(int)threadIdx.x / PL::G];
     const T *x = path + (pl.b * shape.L + pl.span.start) * D + (pl.have ? pl.letter : 0);
     const int64_t steps = pl.span.steps;
-    // (points beyond the window are its last one: increments of zero)
+    // (points beyond the window are its last one)
     auto point = [&](int64_t t) { return steps > 0 ? x[(t < steps ? t : steps) * D] : T(0); };
     T acc[D], to[U];
 #pragma unroll
     for (int k = 0; k < D; ++k) acc[k] = T(0);
-    const T start = point(0);
-    T from = start;
+    PairsPoint<T> at{point(0)};
+    T from = at.start;
 #pragma unroll
     for (int u = 0; u < U; ++u) to[u] = point(u + 1);
     for (int64_t t = 0; t < pl.most; t += U) {
@@ -1720,8 +1738,8 @@ __global__ void __launch_bounds__(kPairsThreads) pairs_forward_kernel(const T *_
         for (int u = 0; u < U; ++u) ahead[u] = point(t + U + u + 1);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const T dx = to[u] - from;
-            mid[u] = (from - start) + dx * T(0.5);
+            T dx;
+            mid[u] = at.pass(from, to[u], t + u < steps, dx);
             mine[u][pl.letter] = dx;
             from = to[u];
         }
@@ -1736,55 +1754,61 @@ __global__ void __launch_bounds__(kPairsThreads) pairs_forward_kernel(const T *_
     }
     if (!pl.have) return;
     T *out = sig + pl.row * (D + D * D);
-    out[pl.letter] = from - start;
+    out[pl.letter] = at.reached(from);
 #pragma unroll
     for (int k = 0; k < D; ++k) out[D + pl.letter * D + k] = acc[k];
 }
 
-// adds the sums of its windows to the per-increment gradients
+// Adds the sums of its windows to the per-increment gradients.  sig: the signature of the windows, read at level 1.  (The terms
+// of g(ab) and g(ba) are kept apart: their difference would be NaN for an infinite gradient.)
 template <typename T, int D, int U>
 __global__ void __launch_bounds__(kPairsThreads)
-    pairs_backward_kernel(const T *__restrict__ path, const T *__restrict__ grad_sig, T *__restrict__ grad_inc, SigShape shape) {
+    pairs_backward_kernel(const T *__restrict__ path, const T *__restrict__ sig, const T *__restrict__ grad_sig,
+                          T *__restrict__ grad_inc, SigShape shape) {
     using PL = PairsLane<T, D>;
-    __shared__ __align__(16) T letters[PL::kRows][U][PL::G];
+    __shared__ __align__(16) T letters[PL::kRows][U][2][PL::G];  // of an increment: its midpoint, and what follows that
     const PL pl(shape);
-    T(*mine)[PL::G] = letters[(int)threadIdx.x / PL::G];
+    T(*mine)[2][PL::G] = letters[(int)threadIdx.x / PL::G];
     const int letter = pl.have ? pl.letter : 0;
     const int64_t steps = pl.span.steps;
     const T *x = path + (pl.b * shape.L + pl.span.start) * D + letter;
     T *ginc = grad_inc + (pl.b * (shape.L - 1) + pl.span.start) * D + letter;
     const T *g = grad_sig + (pl.have ? pl.row : 0) * (D + D * D);
+    const T end = sig[(pl.have ? pl.row : 0) * (D + D * D) + letter];
     auto point = [&](int64_t t) { return steps > 0 ? x[(t < steps ? t : steps) * D] : T(0); };
-    const T start = point(0);
-    T from = start, to[U];
+    PairsPoint<T> at{point(0)};
+    T from = at.start, to[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) to[u] = point(u + 1);
-    T turn[D], fixed = g[letter];  // g(ab) - g(ba) for this letter b; what all increments of the window get
-    mine[0][pl.letter] = point(steps) - start;
-    pairs_fence();
+    T before[D], after[D];  // g(ab) and g(bc), for this letter b
+    const T fixed = g[letter];
 #pragma unroll
     for (int a = 0; a < D; ++a) {
-        const T own = g[D + letter * D + a];
-        fixed = fmad<T>(own, mine[0][a], fixed);
-        turn[a] = g[D + a * D + letter] - own;
+        before[a] = g[D + a * D + letter];
+        after[a] = g[D + letter * D + a];
     }
-    pairs_fence();
     for (int64_t t = 0; t < pl.most; t += U) {
         T ahead[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) ahead[u] = point(t + U + u + 1);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            mine[u][pl.letter] = (from - start) + (to[u] - from) * T(0.5);
+            T dx;
+            const T mid = at.pass(from, to[u], t + u < steps, dx);
+            mine[u][0][pl.letter] = mid;
+            mine[u][1][pl.letter] = end - mid;
             from = to[u];
         }
         pairs_fence();
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            T v = fixed;
+            T v = fixed, w = T(0);
 #pragma unroll
-            for (int a = 0; a < D; ++a) v = fmad<T>(mine[u][a], turn[a], v);
-            if (pl.have && t + u < steps) atomicAdd(&ginc[(t + u) * D], v);
+            for (int a = 0; a < D; ++a) {
+                v = fmad<T>(mine[u][0][a], before[a], v);
+                w = fmad<T>(mine[u][1][a], after[a], w);
+            }
+            if (pl.have && t + u < steps) atomicAdd(&ginc[(t + u) * D], v + w);
         }
         pairs_fence();
 #pragma unroll
@@ -2986,10 +3010,10 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
                 const int64_t per_block = PairsLane<T, D>::kRows;
                 const dim3 blocks((unsigned)((rows + per_block - 1) / per_block));
                 if (pairs_few(rows, PairsLane<T, D>::G))
-                    hipLaunchKernelGGL((pairs_backward_kernel<T, D, 4>), blocks, dim3(kPairsThreads), 0, stream, path,
+                    hipLaunchKernelGGL((pairs_backward_kernel<T, D, 4>), blocks, dim3(kPairsThreads), 0, stream, path, sig,
                                        grad_sig, grad_inc, shape);
                 else
-                    hipLaunchKernelGGL((pairs_backward_kernel<T, D, 1>), blocks, dim3(kPairsThreads), 0, stream, path,
+                    hipLaunchKernelGGL((pairs_backward_kernel<T, D, 1>), blocks, dim3(kPairsThreads), 0, stream, path, sig,
                                        grad_sig, grad_inc, shape);
             } else {
                 hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, false>), grid, dim3(G::kBlock), 0, stream, path, sig,

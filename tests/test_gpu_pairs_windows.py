@@ -34,3 +34,65 @@ def test_depth_two_windows(dtype, d, B, far):
     assert rel_err(grad, TO.signature_vjp(path, G, 2, None, None, windows)) < TOL[dtype]
     log = ps.LogSignature(depth=2, windows=torch.tensor(windows, device="cuda"))(x)
     assert torch.isfinite(log).all() and rel_err(log[..., :d], want[..., :d]) < TOL[dtype]
+
+
+# 16 rows, and more than the windows that share a wave start from
+@pytest.mark.parametrize("B", [2, 2100])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("d", [3, 9])
+def test_points_that_are_not_finite_show(dtype, d, B):
+    """A point that is not finite shows in every coefficient of its letter in its windows, level 1 among them, and in the gradient
+    of all of these windows; no other window has it."""
+    import pathsig_amd as ps
+    windows = torch.tensor([(0, 20), (0, 8), (5, 12), (12, 20), (3, 19), (8, 20), (8, 9), (1, 7)])
+    holds = torch.tensor([a <= 7 < b and b - a > 1 for a, b in windows.tolist()])
+    path = brownian_path(B, 20, d, seed=1340).to(dtype)
+    module = ps.Signature(depth=2, windows=windows.cuda())
+    of_letter = torch.zeros(d + d * d, dtype=torch.bool)
+    of_letter[1] = True
+    of_letter[d:].view(d, d)[1, :] = True
+    of_letter[d:].view(d, d)[:, 1] = True
+    for bad in (float("nan"), float("inf"), -float("inf")):
+        x = path.clone()
+        x[1, 7, 1] = bad
+        x = x.cuda().requires_grad_(True)
+        out = module(x)
+        finite = torch.isfinite(out.detach()).cpu()
+        want = torch.ones_like(finite)
+        want[1] = ~(holds[:, None] & of_letter[None, :])
+        assert torch.equal(finite, want)
+        (grad,) = torch.autograd.grad(out, x, randn(tuple(out.shape), seed=134).to(dtype).cuda())
+        finite = torch.isfinite(grad).all(dim=2).cpu()
+        assert finite[0].all() and finite[2:].all() and not finite[1].any()
+    # the last point of the window (0, 8): what a very large one there gives, at its limit
+    x, large = path.clone(), path.double().clone()
+    x[1, 7, 1], large[1, 7, 1] = float("inf"), 1e12
+    got = module(x.cuda())[1, 1].double().cpu()
+    want = TO.compute_signature(large[1:2], 2, None, None, [(0, 8)])[0, 0]
+    assert torch.equal(torch.isinf(got), of_letter) and torch.equal(torch.sign(got)[of_letter], torch.sign(want)[of_letter])
+
+
+@pytest.mark.parametrize("B", [2, 2100])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("word", [(1,), (1, 1), (0, 1), (1, 0)])
+def test_an_infinite_gradient_stays_with_its_letters(dtype, word, B):
+    """The gradient of the first and of the last point of a window (of one increment sum each) has the sign that a finite upstream
+    gradient of its coefficient gives it; the other letters get none."""
+    import pathsig_amd as ps
+    d, windows = 3, [(0, 20), (5, 12), (12, 20), (2, 5), (3, 19), (8, 20), (8, 9), (0, 8)]
+    path = brownian_path(B, 20, d, seed=1350)
+    x = path.to(dtype).cuda().requires_grad_(True)
+    out = ps.Signature(depth=2, windows=torch.tensor(windows, device="cuda"))(x)
+    column = word[0] if len(word) == 1 else d + word[0] * d + word[1]
+    grads = []
+    for value in (1.0, float("inf")):
+        G = torch.zeros_like(out)
+        G[1, 1, column] = value
+        grads.append(torch.autograd.grad(out, x, G, retain_graph=True)[0].cpu())
+    one, infinite = grads
+    others = [k for k in range(d) if k not in word]
+    assert torch.equal(infinite[..., others], torch.zeros_like(infinite[..., others]))
+    assert torch.equal(infinite[0], torch.zeros_like(infinite[0]))
+    for at in (5, 11):
+        for k in set(word):
+            assert one[1, at, k] != 0 and infinite[1, at, k] == torch.sign(one[1, at, k]) * float("inf")
