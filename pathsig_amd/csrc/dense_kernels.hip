@@ -1651,9 +1651,9 @@ __global__ void __launch_bounds__(kWave) chunk_level1_kernel(const T *__restrict
 //     S(ab) = sum_t u'_a dx_b,     dL/d(dx_b) = g(b) + sum_a u'_a g(ab) + sum_c (x'_end - u')_c g(bc).
 // Several windows share a wave, a lane to each of their letters (padded to a power of two); an increment's letters reach the
 // lanes of its window through LDS.  Bound by vector issue for long windows, by the rows of the signature in memory for short
-// ones.  us, a lane to a letter of one window / several windows to a wave: a step, fp64, 237 427 windows of 9 points, 12 letters
-// (log-signature) 1373 / 714, 2674 of 204, 15 letters, 391 / 131; fp32, 12 400 of 64, 8 letters, 145 / 63; a forward, 7936 of 128,
-// 13 letters, 59 / 20, fp64, 97 405 of 23, 5 letters, 84 / 25.
+// ones.  us, a lane to a letter of one window / several windows to a wave: a step, fp64, 234 184 windows of 9 points, 12 letters
+// (log-signature) 1406 / 784, 2688 of 204, 15 letters, 403 / 174; fp32, 12 600 of 64, 8 letters, 160 / 78; a forward, 8192 of
+// 128, 13 letters, 63 / 42, fp64, 97 000 of 23, 5 letters, 91 / 27.
 // ---------------------------------------------------------------------------------------------
 constexpr int kPairsThreads = 256;
 constexpr int pairs_lanes(int d) { return d <= 2 ? 2 : d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : 32; }
@@ -1692,9 +1692,9 @@ __device__ __forceinline__ void pairs_fence() {
 }
 
 // Increments that meet in LDS at a time (U of the kernels): the round trip, and the points fetched ahead, are waited for once
-// for all of them, which pays while the SIMDs have little else to do.  us, one / four: 2674 windows of 204 points, 15 letters,
-// fp64, forward and backward kernel 66 + 100 / 40 + 72 (669 waves); a forward of 7936 of 128, 13 letters, fp32, 19.8 / 22.8 (1984
-// waves), of 97 405 of 23, 5 letters, fp64, 24.5 / 29.0.
+// for all of them, which pays while the SIMDs have little else to do.  us, one / four, forward and backward: windows of 129
+// points, fp32, 8192 over 2 letters 16.9 + 41.5 / 12.8 + 35.7, 4096 over 15 letters 25.4 + 54.9 / 24.8 + 50.8, 16 384 of them
+// 37.4 + 108 / 48.4 + 118; fp64, 65 536 over 4 letters 36.8 + 92.7 / 38.9 + 144.
 inline bool pairs_few(int64_t rows, int lanes) { return rows * lanes < 1536 * kWave; }
 
 // Letter of a window's running point, relative to the first.  The difference of the points is exact to a rounding; where either
@@ -1759,23 +1759,68 @@ __global__ void __launch_bounds__(kPairsThreads) pairs_forward_kernel(const T *_
     for (int k = 0; k < D; ++k) out[D + pl.letter * D + k] = acc[k];
 }
 
+// Increments whose sums a wave collects in LDS before they go to memory.
+template <typename T>
+constexpr int pairs_tile(int d) { return d <= 3 && sizeof(T) == 4 ? 32 : 16; }
+
 // Adds the sums of its windows to the per-increment gradients.  sig: the signature of the windows, read at level 1.  (The terms
 // of g(ab) and g(ba) are kept apart: their difference would be NaN for an infinite gradient.)
+// The sums of a tile of increments meet in LDS and leave the wave a window at a time, side by side in memory; those of windows
+// that start at the same point (whole paths, expanding windows) are added up before, else the lanes of such windows would wait
+// for each other at every address.  (us, an atomic addition per window, letter and increment / this way: fp32, 16 384 windows of
+// 129 points over 2 letters 1220 / 37, over 15 letters 1290 / 108, of 64 points at their own places, 2 letters, 72 / 23.)
 template <typename T, int D, int U>
 __global__ void __launch_bounds__(kPairsThreads)
     pairs_backward_kernel(const T *__restrict__ path, const T *__restrict__ sig, const T *__restrict__ grad_sig,
                           T *__restrict__ grad_inc, SigShape shape) {
     using PL = PairsLane<T, D>;
+    constexpr int kTile = pairs_tile<T>(D), kCells = kTile * D, kStride = kCells + D, kRounds = (kCells + kWave - 1) / kWave;
+    constexpr int kShare = kWave / PL::G;  // windows of a wave
     __shared__ __align__(16) T letters[PL::kRows][U][2][PL::G];  // of an increment: its midpoint, and what follows that
+    __shared__ T sums[PL::kRows][kStride];
     const PL pl(shape);
-    T(*mine)[2][PL::G] = letters[(int)threadIdx.x / PL::G];
+    const int lane = (int)threadIdx.x % kWave, slot = (int)threadIdx.x / PL::G;
+    T(*mine)[2][PL::G] = letters[slot];
+    T *tile = sums[slot];
+    const T *tiles = sums[(int)threadIdx.x / kWave * kShare];
     const int letter = pl.have ? pl.letter : 0;
     const int64_t steps = pl.span.steps;
     const T *x = path + (pl.b * shape.L + pl.span.start) * D + letter;
-    T *ginc = grad_inc + (pl.b * (shape.L - 1) + pl.span.start) * D + letter;
+    const int64_t first = (pl.b * (shape.L - 1) + pl.span.start) * D;  // of the window's cells
     const T *g = grad_sig + (pl.have ? pl.row : 0) * (D + D * D);
     const T end = sig[(pl.have ? pl.row : 0) * (D + D * D) + letter];
     auto point = [&](int64_t t) { return steps > 0 ? x[(t < steps ? t : steps) * D] : T(0); };
+    auto first_of = [&](int q) {
+        const unsigned low = (unsigned)__builtin_amdgcn_readlane((int)(uint32_t)first, q * PL::G);
+        const unsigned high = (unsigned)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)first >> 32), q * PL::G);
+        return (int64_t)((uint64_t)high << 32 | low);
+    };
+    auto flush = [&](int64_t t0) {
+        pairs_fence();
+        T sum[kRounds];
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) sum[r] = T(0);
+        int most = 0;
+        int64_t at = first_of(0);
+        for (int q = 0; q < kShare; ++q) {
+            const int64_t left = __builtin_amdgcn_readlane((int)steps, q * PL::G) - t0;
+            const int cells = (int)(left < 0 ? 0 : left < kTile ? left : kTile) * D;
+            most = cells > most ? cells : most;
+#pragma unroll
+            for (int r = 0; r < kRounds; ++r)
+                if (r * kWave + lane < cells) sum[r] += tiles[q * kStride + r * kWave + lane];
+            const int64_t next = q + 1 < kShare ? first_of(q + 1) : -1;
+            if (next == at) continue;
+#pragma unroll
+            for (int r = 0; r < kRounds; ++r) {
+                if (r * kWave + lane < most) atomicAdd(&grad_inc[at + t0 * D + r * kWave + lane], sum[r]);
+                sum[r] = T(0);
+            }
+            most = 0;
+            at = next;
+        }
+        pairs_fence();
+    };
     PairsPoint<T> at{point(0)};
     T from = at.start, to[U];
 #pragma unroll
@@ -1787,32 +1832,37 @@ __global__ void __launch_bounds__(kPairsThreads)
         before[a] = g[D + a * D + letter];
         after[a] = g[D + letter * D + a];
     }
-    for (int64_t t = 0; t < pl.most; t += U) {
-        T ahead[U];
+    for (int64_t t0 = 0; t0 < pl.most; t0 += kTile) {
+        const int used = (int)(pl.most - t0 < kTile ? pl.most - t0 : kTile);
+        for (int i = 0; i < used; i += U) {
+            const int64_t t = t0 + i;
+            T ahead[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) ahead[u] = point(t + U + u + 1);
+            for (int u = 0; u < U; ++u) ahead[u] = point(t + U + u + 1);
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            T dx;
-            const T mid = at.pass(from, to[u], t + u < steps, dx);
-            mine[u][0][pl.letter] = mid;
-            mine[u][1][pl.letter] = end - mid;
-            from = to[u];
-        }
-        pairs_fence();
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            T v = fixed, w = T(0);
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                v = fmad<T>(mine[u][0][a], before[a], v);
-                w = fmad<T>(mine[u][1][a], after[a], w);
+            for (int u = 0; u < U; ++u) {
+                T dx;
+                const T mid = at.pass(from, to[u], t + u < steps, dx);
+                mine[u][0][pl.letter] = mid;
+                mine[u][1][pl.letter] = end - mid;
+                from = to[u];
             }
-            if (pl.have && t + u < steps) atomicAdd(&ginc[(t + u) * D], v + w);
-        }
-        pairs_fence();
+            pairs_fence();
 #pragma unroll
-        for (int u = 0; u < U; ++u) to[u] = ahead[u];
+            for (int u = 0; u < U; ++u) {
+                T v = fixed, w = T(0);
+#pragma unroll
+                for (int a = 0; a < D; ++a) {
+                    v = fmad<T>(mine[u][0][a], before[a], v);
+                    w = fmad<T>(mine[u][1][a], after[a], w);
+                }
+                if (pl.letter < D) tile[(i + u) * D + pl.letter] = v + w;
+            }
+            pairs_fence();
+#pragma unroll
+            for (int u = 0; u < U; ++u) to[u] = ahead[u];
+        }
+        flush(t0);
     }
 }
 

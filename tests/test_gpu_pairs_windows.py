@@ -98,3 +98,23 @@ def test_an_infinite_gradient_stays_with_its_letters(dtype, word, B):
     for at in (5, 11):
         for k in set(word):
             assert one[1, at, k] != 0 and infinite[1, at, k] == torch.sign(one[1, at, k]) * float("inf")
+
+
+# Windows that start at the same point add their sums up before these go to memory: groups of equal starts that end inside a
+# wave, at its end and beyond it, with lengths that differ by more than a tile of increments; tiles that are not full
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("d,B", [(d, B) for d in (2, 3, 4, 7, 8, 12, 16, 20, 32) for B in (2, 420)])
+def test_windows_with_equal_starts(dtype, d, B):
+    import pathsig_amd as ps
+    L = 70
+    windows = ([(0, n) for n in (2, 70, 18, 17, 33, 34, 1, 50)] + [(1, 70)] * 3 + [(40, 70), (40, 41), (40, 57)]
+               + [(0, 70), (69, 70), (0, 16), (0, 0), (0, 49), (1, 10)])
+    path = brownian_path(B, L, d, seed=1360 + d).to(dtype).double()
+    x = path.to(dtype).cuda().requires_grad_(True)
+    out = ps.Signature(depth=2, windows=torch.tensor(windows, device="cuda"))(x)
+    some = torch.tensor([0, 1, B // 2, B - 1]).unique()  # (all of a large batch would take the checker a minute)
+    assert rel_err(out[some], TO.compute_signature(path[some], 2, None, None, windows)) < TOL[dtype]
+    G = randn(tuple(out.shape), seed=136)
+    (grad,) = torch.autograd.grad(out, x, G.to(dtype).cuda())
+    assert rel_err(grad[some], TO.signature_vjp(path[some], G[some], 2, None, None, windows)) < TOL[dtype]
+    assert torch.isfinite(grad).all()
