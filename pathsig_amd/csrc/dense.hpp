@@ -33,6 +33,8 @@ struct DenseChoice {
     // formed in memory (chain_kernels.hip).  Backward: one launch contracts the upstream gradient with what follows each
     // chunk, and every chunk is swept as a row of its own, from its own state and adjoint.
     bool far;
+    // Depth 2 in windows that are swept in one piece: several windows to a wave (pairs_forward_kernel, pairs_backward_kernel).
+    bool pairs_forward, pairs_backward;
 };
 
 // While one that is on lives, the choices made on its thread take at most 64 chunks to a row and no launches for long

@@ -2828,7 +2828,7 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, const Dense
     if (bounds && !kBoundsOk) return hipErrorInvalidValue;
     if (chunks <= 1) {
         if constexpr (N == 2 && D <= 32) {
-            if (shape.windows) {
+            if (dc.pairs_forward) {
                 const int64_t per_block = PairsLane<T, D>::kRows;
                 const dim3 grid((unsigned)((rows + per_block - 1) / per_block));
                 if (pairs_few(rows, PairsLane<T, D>::G))
@@ -3055,8 +3055,8 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
         const int pieces = chunks <= 1 ? 1 : chunks;
         const dim3 grid((unsigned)(rows * pieces * G::kUnitBlocks));
         profile_bracket(true, stream);
-        if (accumulate) {
-            if constexpr (N == 2 && D <= 32) {  // (units of one block: windows)
+        if constexpr (N == 2 && D <= 32) {
+            if (dc.pairs_backward) {
                 const int64_t per_block = PairsLane<T, D>::kRows;
                 const dim3 blocks((unsigned)((rows + per_block - 1) / per_block));
                 if (pairs_few(rows, PairsLane<T, D>::G))
@@ -3065,10 +3065,13 @@ hipError_t run_backward(const T *path, const T *sig, const T *grad_sig, T *grad_
                 else
                     hipLaunchKernelGGL((pairs_backward_kernel<T, D, 1>), blocks, dim3(kPairsThreads), 0, stream, path, sig,
                                        grad_sig, grad_inc, shape);
-            } else {
-                hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, false>), grid, dim3(G::kBlock), 0, stream, path, sig,
-                                   adjoint, state, (const T *)nullptr, grad_inc, shape, pieces);
+                profile_bracket(false, stream);
+                return hipGetLastError();
             }
+        }
+        if (accumulate) {
+            hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, true, false>), grid, dim3(G::kBlock), 0, stream, path, sig,
+                               adjoint, state, (const T *)nullptr, grad_inc, shape, pieces);
         } else {
             if constexpr (G::kUnitBlocks == 1)
                 hipLaunchKernelGGL((dense_backward_kernel<T, D, N, P, false, false>), grid, dim3(G::kBlock), 0, stream, path,
@@ -3250,6 +3253,22 @@ static bool entry_pays(const EntryUs &short_prefix, const EntryUs &long_prefix) 
            0.25 * short_prefix.sweeps + short_prefix.products + 4.0 < 0.25 * long_prefix.sweeps + long_prefix.products;
 }
 
+// Whether windows of depth 2 share waves (pairs_forward_kernel, pairs_backward_kernel).  Their lengths are not known here, and a
+// wave walks its longest one an LDS round trip after the other (fp32, forward 0.07 us an increment over 2 letters, 0.16 over 15,
+// backward 0.23 and 0.32), so there have to be windows enough that the sweeps, a wave and more to a window, take longer.  Lines
+// where the new way is the faster one for whole paths, expanding windows up to 4097 points, windows at their own places and
+// windows of 9 points alike.  us, swept (in chunks, where rows are few) / shared:
+//   forward, whole paths of 1025 points, fp32, 2 letters: 512 rows 18.7 / 83, 4096 64 / 84, 8192 102 / 85; 15 letters: 2048 149 /
+//   168, 4096 266 / 169; fp64, 15 letters: 512 70 / 187, 4096 464 / 191;
+//   backward, the same: fp32, 2 letters 42 / 237, 346 / 238, 608 / 239 (expanding, 4096 rows 841 / 914); 8 letters: 512 128 / 288,
+//   2048 488 / 292, 4096 745 / 293 (expanding, 2048 rows 1081 / 1113); 15 letters: 512 140 / 330, 2048 549 / 332; fp64, 15
+//   letters: 512 249 / 392, 2048 962 / 398.
+// (Over twelve letters, fp32, 4096 expanding windows take 538 / 559 forward, whole paths of 129 points 22.3 / 21.4.)
+static bool pairs_forward_pays(int64_t d, int64_t rows) { return rows >= 8192 || (rows >= 4096 && pairs_lanes((int)d) >= 16); }
+static bool pairs_backward_pays(size_t elem, int64_t d, int64_t rows) {
+    return rows >= 8192 || (rows >= 2048 && rows * pairs_lanes((int)d) * (int64_t)elem >= 131072);
+}
+
 static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all_dense, const int64_t *level_sizes,
                                      int64_t B, int64_t L, int64_t W, bool windowed, bool plain, bool far_ok) {
     DenseChoice dc{};
@@ -3340,9 +3359,6 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         // (letter blocks: twice the waves that fit the GPU at once, so that the short ones fill in behind the long)
         const int64_t want_waves = dc.bounded && elem == 4 ? 4096 : 2048;
         int chunks = pick_chunks(rows, v.block, L, want_waves, many && may_chain);
-        // depth 2 in windows: several share a wave, and nothing is swept (pairs_forward_kernel); few of them, of lengths that
-        // are not known here, are cut into chunks all the same
-        if (windowed && depth == 2 && d <= 32 && (rows >= 512 || L <= 128)) chunks = 1;
         // deep fp32 shapes: the reverse sweep rebuilds A_t from A_{t+1} step by step, and over a span of
         // large increments that roll-back loses digits at depth 9 and more (d = 2, depth 12, five increments of
         // size 0.8: gradient off by 1.5e-5 in one piece, 1e-6 in two or more); four chunks at least
@@ -3356,6 +3372,10 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         dc.variant = i;
         dc.fwd_chunks = chunks;
         dc.bwd_chunks = (dc.embed && !dc.resweep && chunks < 2) ? 2 : chunks;
+        if (windowed && depth == 2 && d <= 32) {
+            dc.pairs_forward = pairs_forward_pays(d, rows);
+            dc.pairs_backward = pairs_backward_pays(elem, d, rows);
+        }
         dc.forward_workspace = dc.dense_bytes + (dc.bounded ? kBoundsBytes : 0);
         dc.backward_workspace = (dc.resweep ? 2 : 1) * dc.dense_bytes + (dc.bounded ? kBoundsBytes : 0);
         if (far > 0) {

@@ -52,3 +52,15 @@ def test_windows_are_not_taken_for_rows_as_long_as_the_path(lib, dtype, elem, B,
     products = (2 + arrays) * (rows * 64 * low * elem + 256)
     assert lib.pathsig_sig_backward_workspace(dtype, B, L, d, depth, None, W) <= B * (L - 1) * d * elem + 256 + products
     assert lib.pathsig_sig_forward_workspace(dtype, B * W, L, d, depth, None, 0) == whole
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("d", [2, 4, 8, 15, 32])
+@pytest.mark.parametrize("rows", [512, 1024, 1536])
+@pytest.mark.parametrize("L", [257, 1025, 4097])
+def test_few_windows_of_depth_two_are_cut_into_chunks(lib, dtype, d, rows, L):
+    """512 windows over two letters would be 16 waves of several windows each, every one of which walks its longest window alone:
+    up to 2048 rows, calls keep to time chunks."""
+    assert lib.pathsig_sig_forward_workspace(dtype, 8, L, d, 2, None, rows // 8) > 0
+    assert lib.pathsig_sig_chunks_bytes(dtype, 8, L, d, 2, None, rows // 8) > 0
+    assert lib.pathsig_sig_forward_workspace(dtype, 8, L, d, 2, None, 1024) == 0
