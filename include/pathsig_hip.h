@@ -54,8 +54,9 @@ const char *pathsig_last_error(void);
  */
 size_t pathsig_sig_forward_workspace(int dtype, int64_t B, int64_t L, int64_t d, int depth,
                                      const int64_t *level_sizes, int64_t W);
-/* Scratch with which a forward that keeps nothing is fastest, at least what pathsig_sig_forward_workspace asks for: the
- * per-word kernels cut few words on few paths into time chunks where they get it. */
+/* The same, and the scratch of few words on few paths, whose forward the per-word kernels cut into time chunks where they get
+ * it and sweep in one piece where they do not.  (pathsig_sig_forward_workspace asks for that scratch where such a call would
+ * otherwise be computed through a dense shape, which takes scratch too.) */
 size_t pathsig_sig_forward_scratch(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
                                    int64_t W);
 int pathsig_sig_forward(const void *path, void *sig, int dtype, int64_t B, int64_t L, int64_t d, int depth,
@@ -116,6 +117,9 @@ int pathsig_sig_backward_noalloc(const void *path, const void *sig, const void *
  */
 size_t pathsig_sig_chunks_bytes(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
                                 int64_t W);
+/* Workspace of pathsig_sig_forward_keep beside its buffer; no more than pathsig_sig_forward_workspace, which serves as well. */
+size_t pathsig_sig_forward_keep_workspace(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
+                                          int64_t W);
 int pathsig_sig_forward_keep(const void *path, void *sig, int dtype, int64_t B, int64_t L, int64_t d, int depth,
                              const int64_t *level_sizes, const int64_t *encoded_words, int64_t n_encoded,
                              const int32_t *windows, int64_t W, void *chunks, size_t chunks_bytes, void *workspace,

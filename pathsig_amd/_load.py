@@ -42,6 +42,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.pathsig_sig_forward_workspace.argtypes = [_INT, _I64, _I64, _I64, _INT, _PTR, _I64]
     lib.pathsig_sig_forward_scratch.restype = _SIZE
     lib.pathsig_sig_forward_scratch.argtypes = [_INT, _I64, _I64, _I64, _INT, _PTR, _I64]
+    lib.pathsig_sig_forward_keep_workspace.restype = _SIZE
+    lib.pathsig_sig_forward_keep_workspace.argtypes = [_INT, _I64, _I64, _I64, _INT, _PTR, _I64]
     lib.pathsig_sig_forward.restype = _INT
     lib.pathsig_sig_forward.argtypes = [_PTR, _PTR, _INT, _I64, _I64, _I64, _INT, _PTR, _PTR, _I64, _PTR, _I64,
                                         _PTR, _SIZE, _PTR]

@@ -797,30 +797,41 @@ int pathsig_set_option(const char *name, int64_t value) {
     return PATHSIG_OK;
 }
 
-size_t pathsig_sig_forward_workspace(int dtype, int64_t B, int64_t L, int64_t d, int depth,
-                                     const int64_t *level_sizes, int64_t W) {
+namespace {
+// Scratch of a forward.  keeps: its buffer serves the per-word kernels as their table; every: the table also where the call
+// would not be computed through a dense shape either.
+size_t forward_scratch(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes, int64_t W, bool keeps,
+                       bool every) {
     if (check_common(dtype, B, L, d, depth) != PATHSIG_OK) return 0;
+    const size_t elem = elem_size(dtype);
     LevelPlan plan;
     bool all_dense;
     if (build_plan(d, depth, level_sizes, INT64_MAX, true, &plan, &all_dense) != PATHSIG_OK) return 0;
-    if (const int64_t D = wide_pad_dim(elem_size(dtype), d, depth, all_dense, B, L, W > 0 ? W : 1, W > 0)) {
-        const WideLayout lay = wide_layout(elem_size(dtype), B, L, d, D, B * (W > 0 ? W : 1));
+    const int64_t windows = W > 0 ? W : 1;
+    if (const int64_t D = wide_pad_dim(elem, d, depth, all_dense, B, L, windows, W > 0)) {
+        const WideLayout lay = wide_layout(elem, B, L, d, D, B * windows);
         return lay.path_bytes + lay.sig_bytes + pathsig_sig_forward_workspace(dtype, B, L, D, depth, nullptr, W);
     }
-    const DenseChoice dc =
-        dense_choice(elem_size(dtype), d, depth, all_dense, level_sizes, B, L, W > 0 ? W : 1, W > 0);
-    return dc.usable ? dc.forward_workspace : 0;
+    const DenseChoice dc = dense_choice(elem, d, depth, all_dense, level_sizes, B, L, windows, W > 0);
+    if (dc.usable) return dc.forward_workspace;
+    if (keeps || !(every || dc.words_in_chunks)) return 0;
+    return word_table_bytes(chunks_of_words(plan, elem, B, L, d, W > 0), B, elem);
+}
+}  // namespace
+
+size_t pathsig_sig_forward_workspace(int dtype, int64_t B, int64_t L, int64_t d, int depth,
+                                     const int64_t *level_sizes, int64_t W) {
+    return forward_scratch(dtype, B, L, d, depth, level_sizes, W, false, false);
 }
 
 size_t pathsig_sig_forward_scratch(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
                                    int64_t W) {
-    const size_t needed = pathsig_sig_forward_workspace(dtype, B, L, d, depth, level_sizes, W);
-    if (needed > 0 || check_common(dtype, B, L, d, depth) != PATHSIG_OK) return needed;
-    LevelPlan plan;
-    bool all_dense;
-    if (build_plan(d, depth, level_sizes, INT64_MAX, true, &plan, &all_dense) != PATHSIG_OK) return 0;
-    if (dense_choice(elem_size(dtype), d, depth, all_dense, level_sizes, B, L, W > 0 ? W : 1, W > 0).usable) return 0;
-    return word_table_bytes(chunks_of_words(plan, elem_size(dtype), B, L, d, W > 0), B, elem_size(dtype));
+    return forward_scratch(dtype, B, L, d, depth, level_sizes, W, false, true);
+}
+
+size_t pathsig_sig_forward_keep_workspace(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
+                                          int64_t W) {
+    return forward_scratch(dtype, B, L, d, depth, level_sizes, W, true, false);
 }
 
 size_t pathsig_sig_chunks_bytes(int dtype, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,

@@ -7,6 +7,8 @@ namespace psig {
 
 struct DenseChoice {
     bool usable;                // a register-tiled kernel exists for this call
+    bool words_in_chunks;       // not usable: one does, but the per-word kernels in time chunks (word_chunks) are taken to be
+                                // faster, so that the forward's scratch has to hold their table
     bool embed;                 // the call is a word projection that is computed densely and then gathered
     bool bounded;               // embed: the sweeps leave out top-level words by the letter bounds of the word list
     bool resweep;               // embed with a shape that is not cut into time chunks: the backward needs the dense

@@ -3335,7 +3335,8 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
                 if (wc.chunks) {
                     const double chunked_us =
                         25.0 + 2.0 * steps / wc.chunks + 0.6 * wc.chunks + 5e-6 * words * (double)rows * steps;
-                    if (chunked_us < 0.6 * std::max(dense_us, entry_us(v, elem, rows, L).total() + 20.0)) return dc;
+                    dc.words_in_chunks = chunked_us < 0.6 * std::max(dense_us, entry_us(v, elem, rows, L).total() + 20.0);
+                    if (dc.words_in_chunks) return dc;
                 }
             }
             if ((double)rows * (double)v.sig_size * (double)elem * (one_piece ? 2.0 : 1.0) > 4e9) return dc;

@@ -132,7 +132,7 @@ std::tuple<Tensor, Tensor> sig_forward(const Tensor &path_in, int64_t depth, boo
         chunks = at::empty({(int64_t)(chunk_bytes / c.path.element_size())}, c.path.options());
     }
     // (what a forward keeps serves it as scratch too)
-    const size_t ws_bytes = (chunk_bytes ? pathsig_sig_forward_workspace : pathsig_sig_forward_scratch)(
+    const size_t ws_bytes = (chunk_bytes ? pathsig_sig_forward_keep_workspace : pathsig_sig_forward_scratch)(
         c.dt, c.B, c.L, c.d, (int)c.depth, c.sizes, c.W);
     Tensor ws = scratch(ws_bytes, c.path);
     check_rc(pathsig_sig_forward_keep(ptr(c.path), ptr(out), c.dt, c.B, c.L, c.d, (int)c.depth, c.sizes,

@@ -142,3 +142,26 @@ def test_logsignature_in_one_call_checks_its_sizes(lib, n_out, picked, windows, 
     assert b"log-signature in one call" in lib.pathsig_last_error()
     assert lib.pathsig_logsignature_backward(ptr(1), ptr(1), saved, ptr(1), ptr(1), *shape, ptr(1), backward, None) == -1
     assert b"log-signature in one call" in lib.pathsig_last_error()
+
+
+def test_the_documented_scratch_of_words_in_chunks(lib):
+    """Few words on few long paths that would be computed through a dense shape are swept in time chunks instead: the size that
+    pathsig_sig_forward_workspace asks for holds the table of that route, and a keeping forward needs it in its buffer alone."""
+    for dtype, B, L, d, depth, words, full in ((0, 1, 1000, 6, 5, 16, 2), (1, 2, 3000, 6, 5, 60, 2), (1, 1, 4000, 3, 8, 16, 3),
+                                               (0, 3, 1000, 10, 5, 2000, 2), (1, 16, 3070, 15, 4, 50, 0)):
+        top = d ** depth
+        listed = [0] * (full + 1) + [min(d ** k, words // (depth - full)) for k in range(full + 1, depth + 1)]
+        sizes = (ctypes.c_int64 * (depth + 1))(*[d ** k if 1 <= k <= full else listed[k] for k in range(depth + 1)])
+        assert sizes[depth] < top
+        call = (dtype, B, L, d, depth, sizes, 0)
+        table = sum(n * sizes[n] * (n + 1) // 2 for n in range(1, depth + 1)) * (4, 8)[dtype]  # of one chunk of one path
+        asked = lib.pathsig_sig_forward_workspace(*call)
+        assert asked >= 2 * B * table and asked == lib.pathsig_sig_forward_scratch(*call)
+        assert lib.pathsig_sig_forward_keep_workspace(*call) == 0
+        assert lib.pathsig_sig_chunks_bytes(*call) >= asked
+    # calls that would not be computed densely either ask for nothing, as a forward without scratch sweeps them in one piece
+    sizes = (ctypes.c_int64 * 7)(0, 16, 0, 0, 0, 0, 20)
+    assert lib.pathsig_sig_forward_workspace(0, 1, 300, 16, 6, sizes, 0) == 0
+    assert lib.pathsig_sig_forward_scratch(0, 1, 300, 16, 6, sizes, 0) > 0
+    # dense calls: the keeping forward needs what the plain one does
+    assert lib.pathsig_sig_forward_keep_workspace(0, 128, 1024, 4, 6, None, 0) == lib.pathsig_sig_forward_workspace(0, 128, 1024, 4, 6, None, 0) > 0

@@ -134,3 +134,36 @@ def test_scratch_that_holds_one_piece_only(ps):
         torch.cuda.synchronize()
         results.append((sig, grad))
     assert rel_err(results[0][0], results[1][0]) < 1e-12 and rel_err(results[0][1], results[1][1]) < 1e-12
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_a_plain_forward_with_the_scratch_it_asks_for_is_swept_in_chunks(ps, dtype):
+    """Words that would be computed through a dense shape: with the workspace that the query asks for, the forward gives the bits of
+    one that keeps the table of the chunks; with none it is swept in one piece."""
+    from pathsig_amd import _load
+    lib = _load.lib()
+    B, L, d, depth, code = 2, 1000, 6, 5, 0 if dtype == torch.float32 else 1
+    words = random_word_set(d, 3, depth, 16, seed=994)
+    proj = ps.projections.words(words, depth=depth, path_dim=d, full_levels=(1, 2))
+    sizes = (ctypes.c_int64 * len(proj.level_sizes))(*proj.level_sizes)
+    call = (code, B, L, d, depth, sizes, 0)
+    need, keeps = lib.pathsig_sig_forward_workspace(*call), lib.pathsig_sig_chunks_bytes(*call)
+    assert need > 0 and lib.pathsig_sig_forward_keep_workspace(*call) == 0
+    path = brownian_path(B, L, d, seed=995)
+    x, codes = path.to(dtype).cuda(), proj.encoded_words
+    ws, table = (torch.empty(n, dtype=torch.uint8, device="cuda") for n in (need, keeps))
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    sigs = [torch.full((B, proj.sig_size), float("nan"), dtype=dtype, device="cuda") for _ in range(3)]
+    words_arg = (sizes, p(codes), codes.numel(), None, 0)
+    assert lib.pathsig_sig_forward(p(x), p(sigs[0]), code, B, L, d, depth, *words_arg, p(ws), need, stream) == 0
+    assert lib.pathsig_sig_forward_keep(p(x), p(sigs[1]), code, B, L, d, depth, *words_arg, p(table), keeps, None, 0, stream) == 0
+    assert lib.pathsig_sig_forward(p(x), p(sigs[2]), code, B, L, d, depth, *words_arg, None, 0, stream) == 0
+    torch.cuda.synchronize()
+    offs, listed, cols = TO.dense_level_offsets(d, depth), iter(proj._codes), []
+    for k in range(1, depth + 1):
+        size = proj.level_sizes[k]
+        cols += [offs[k] + (j if size == d ** k else next(listed)) for j in range(size)]
+    want = TO.signature(path, depth)[:, torch.tensor(cols)]
+    assert torch.equal(sigs[0], sigs[1]) and not torch.equal(sigs[0], sigs[2])
+    assert all(rel_err(s, want) < TOL[dtype] for s in sigs)
