@@ -228,6 +228,16 @@ size_t words_kept_bytes(const LevelPlan &plan, const WordChunks &wc, int64_t B, 
     return (size_t)count * elem;
 }
 
+// The choice for a call that hands nothing over and brings `room` bytes for it: far chunks, and the entries of the table that are
+// taken for their chunks' sake, are there for speed, and a caller that brings the scratch of the sweep in one piece gets that.
+DenseChoice choice_within(const DenseChoice &dc, size_t room, bool forward, size_t elem, int64_t d, int depth, bool all_dense,
+                          const int64_t *level_sizes, int64_t B, int64_t L, int64_t W, bool windowed) {
+    const auto need = [forward](const DenseChoice &c) { return forward ? c.forward_workspace : c.backward_workspace; };
+    if (!dc.usable || need(dc) <= room) return dc;
+    const DenseChoice plainer = dense_choice(elem, d, depth, all_dense, level_sizes, B, L, W, windowed, false);
+    return plainer.usable && need(plainer) <= room ? plainer : dc;
+}
+
 template <typename T>
 int sig_forward_t(const void *path, void *sig, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes,
                   const int64_t *codes, int64_t n_encoded, const int32_t *windows, int64_t W, void *keep,
@@ -240,13 +250,16 @@ int sig_forward_t(const void *path, void *sig, int64_t B, int64_t L, int64_t d, 
     if (B == 0 || shape.W == 0 || plan.sig_size == 0) return PATHSIG_OK;
     rc = check_grid(plan, B * shape.W);
     if (rc != PATHSIG_OK) return rc;
-    const DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
+    DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
     WordChunks wc = dc.usable ? WordChunks{} : chunks_of_words(plan, sizeof(T), B, L, d, windows != nullptr);
     const size_t keep_need = dc.usable ? dc.keep_bytes : words_kept_bytes(plan, wc, B, B * shape.W, d, sizeof(T));
     if (keep && (keep_need == 0 || keep_bytes < keep_need)) {
         set_error("chunk buffer: this call keeps %zu bytes, got %zu", keep_need, keep_bytes);
         return PATHSIG_ERR_ARGUMENT;
     }
+    if (!keep)
+        dc = choice_within(dc, workspace ? workspace_bytes : 0, true, sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W,
+                           windows != nullptr);
     if (dc.usable) {
         if (workspace_bytes < dc.forward_workspace || (dc.forward_workspace && !workspace)) {
             set_error("workspace too small: need %zu bytes, got %zu", dc.forward_workspace, workspace_bytes);
@@ -299,7 +312,7 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
     if (B == 0) return PATHSIG_OK;
     rc = check_grid(plan, B * shape.W);
     if (rc != PATHSIG_OK) return rc;
-    const DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
+    DenseChoice dc = dense_choice(sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W, windows != nullptr);
     WordChunks wc = dc.usable ? WordChunks{} : chunks_of_words(plan, sizeof(T), B, L, d, windows != nullptr);
     const size_t keep_need = dc.usable ? dc.keep_bytes : words_kept_bytes(plan, wc, B, B * shape.W, d, sizeof(T));
     // The layout of what a forward keeps follows from the choice of kernels, which the tuning switches can change
@@ -314,6 +327,9 @@ int sig_backward_t(const void *path, const void *sig, const void *grad_sig, void
     const bool words_kernel = !dc.usable && !batch_backward_usable(sizeof(T), B, d, shape.W);
     const bool batch_wide = !dc.usable && !words_kernel && batch_wide_sums(sizeof(T), plan);
     const size_t inc_bytes = inc_buffer_bytes(sizeof(T), B, L, d, words_kernel || batch_wide);
+    if (!kept && workspace_bytes >= inc_bytes)
+        dc = choice_within(dc, workspace_bytes - inc_bytes, false, sizeof(T), d, depth, all_dense, level_sizes, B, L, shape.W,
+                           windows != nullptr);
     const size_t need = inc_bytes + (dc.usable ? dc.backward_workspace : 0);
     if (!workspace || workspace_bytes < need) {
         set_error("workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
@@ -515,9 +531,9 @@ int wide_forward(const void *path, void *sig, int64_t B, int64_t L, int64_t d, i
                  int64_t W, void *workspace, size_t workspace_bytes, hipStream_t stream) {
     const int64_t rows = B * (windows ? W : 1);
     const WideLayout lay = wide_layout(sizeof(T), B, L, d, D, rows);
-    const size_t inner = pathsig_sig_forward_workspace(sizeof(T) == 8 ? PATHSIG_F64 : PATHSIG_F32, B, L, D, 3, nullptr,
-                                                       windows ? W : 0);
-    const size_t need = lay.path_bytes + lay.sig_bytes + inner;
+    // (the least that the inner call takes: see choice_within)
+    const size_t need = lay.path_bytes + lay.sig_bytes +
+                        dense_choice(sizeof(T), D, 3, true, nullptr, B, L, windows ? W : 1, windows != nullptr, false).forward_workspace;
     if (!workspace || workspace_bytes < need) {
         set_error("workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
         return PATHSIG_ERR_WORKSPACE;
@@ -528,7 +544,7 @@ int wide_forward(const void *path, void *sig, int64_t B, int64_t L, int64_t d, i
     if (e == hipSuccess) e = launch_wide_copy<T, true, false>((const T *)path, wide_path, B * L, d, d, D, d, D, stream);
     if (e != hipSuccess) return launch_failed(e, "wide path launch");
     const int rc = sig_forward_t<T>(wide_path, wide_sig, B, L, D, 3, nullptr, nullptr, 0, windows, W, nullptr, 0,
-                                    at + lay.path_bytes + lay.sig_bytes, inner, stream);
+                                    at + lay.path_bytes + lay.sig_bytes, workspace_bytes - lay.path_bytes - lay.sig_bytes, stream);
     if (rc != PATHSIG_OK) return rc;
     e = launch_wide_copy<T, false, true>((const T *)sig, wide_sig, rows, lay.sig_size, lay.sig_size, lay.wide_sig_size, d,
                                          D, stream);
@@ -548,7 +564,8 @@ int wide_backward(const void *path, const void *sig, const void *grad_sig, void 
                   hipStream_t stream) {
     const int64_t rows = B * (windows ? W : 1);
     const WideLayout lay = wide_layout(sizeof(T), B, L, d, D, rows);
-    const size_t need = wide_backward_bytes(sizeof(T), B, L, d, D, windows ? W : 0);
+    const size_t need = 2 * lay.path_bytes + 2 * lay.sig_bytes + inc_buffer_bytes(sizeof(T), B, L, D, false) +
+                        dense_choice(sizeof(T), D, 3, true, nullptr, B, L, windows ? W : 1, windows != nullptr, false).backward_workspace;
     if (!workspace || workspace_bytes < need) {
         set_error("workspace too small: need %zu bytes, got %zu", need, workspace_bytes);
         return PATHSIG_ERR_WORKSPACE;
@@ -572,7 +589,7 @@ int wide_backward(const void *path, const void *sig, const void *grad_sig, void 
                                             lay.wide_sig_size, d, D, stream);
     if (e != hipSuccess) return launch_failed(e, "wide scatter launch");
     const int rc = sig_backward_t<T>(wide_path, wide_sig, wide_grad, wide_gpath, B, L, D, 3, nullptr, nullptr, 0, windows, W,
-                                     nullptr, 0, inner_ws, need - 2 * lay.path_bytes - 2 * lay.sig_bytes, stream);
+                                     nullptr, 0, inner_ws, workspace_bytes - 2 * lay.path_bytes - 2 * lay.sig_bytes, stream);
     if (rc != PATHSIG_OK) return rc;
     e = launch_wide_copy<T, false, false>((const T *)grad_path, wide_gpath, B * L, d, d, D, d, D, stream);
     if (e != hipSuccess) return launch_failed(e, "wide gradient launch");

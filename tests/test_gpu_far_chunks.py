@@ -1,5 +1,7 @@
 """Time chunks of the shapes whose kernels sweep a row in one piece (several blocks to a unit, children split between lanes,
 fp64 rows that the scan kernel does not take), against the CPU checker."""
+import ctypes
+
 import pytest
 import torch
 
@@ -89,3 +91,49 @@ def test_infinite_gradient_after_the_last_chunk(ps, set_option):
     (grad,) = torch.autograd.grad(out, x, G)
     others = [k for k in range(16) if k != 3]
     assert torch.isfinite(grad[0, -5:, others]).all()
+
+
+# (16, 4): far chunks; (14, 4): the entry with the shorter prefix, for its chunks; (4, 7) fp64: rows that the scan kernel does not
+# take; 70 letters at depth 3: on copies over 72; a word projection of (9, 5), through its dense rows
+@pytest.mark.parametrize("dtype,B,L,d,depth,listed", [
+    (torch.float32, 2, 400, 16, 4, False), (torch.float64, 2, 400, 16, 4, False), (torch.float32, 2, 500, 14, 4, False),
+    (torch.float64, 2, 700, 4, 7, False), (torch.float32, 1, 500, 70, 3, False), (torch.float32, 2, 300, 9, 5, True)])
+def test_scratch_that_holds_one_piece_only(ps, dtype, B, L, d, depth, listed):
+    """Far chunks are there for speed: a forward or backward that hands nothing over and brings what a sweep in one piece takes is
+    swept in one piece, and one that brings less is refused."""
+    from pathsig_amd import _load
+    lib = _load.lib()
+    code, elem = (0, 4) if dtype == torch.float32 else (1, 8)
+    pad = lambda n: (n + 255) // 256 * 256
+    top = d ** depth
+    codes = torch.arange(0, top, 3) if listed else torch.empty(0, dtype=torch.int64)
+    sizes = (ctypes.c_int64 * (depth + 1))(0, *[d ** k for k in range(1, depth)], len(codes)) if listed else None
+    S = sum(d ** k for k in range(1, depth)) + (len(codes) if listed else top)
+    wide = (d + 7) // 8 * 8 if d > 64 else d
+    copies = [0, 0] if wide == d else [pad(B * L * wide * elem), pad(B * sum(wide ** k for k in range(1, depth + 1)) * elem)]
+    dense = pad(B * sum(d ** k for k in range(1, depth + 1)) * elem) if listed else 0
+    forward = sum(copies) + dense
+    backward = 2 * sum(copies) + 2 * dense + pad(B * (L - 1) * wide * elem)
+    call = (code, B, L, d, depth, sizes, 0)
+    asked = lib.pathsig_sig_forward_workspace(*call), lib.pathsig_sig_backward_workspace(*call)
+    assert asked[0] > forward and asked[1] > backward + 256
+    path = brownian_path(B, L, d, seed=960 + d).to(dtype).double()
+    x = path.to(dtype).cuda()
+    G = randn((B, S), seed=96)
+    g, words = G.to(dtype).cuda(), codes.cuda()
+    p = lambda t: ctypes.c_void_p(t.data_ptr() if t.numel() else 0)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ws = torch.empty(max(asked), dtype=torch.uint8, device="cuda")
+    tail = (code, B, L, d, depth, sizes, p(words) if listed else None, len(codes), None, 0)
+    cols = torch.cat([torch.arange(S - len(codes)), S - len(codes) + codes]) if listed else torch.arange(S)
+    full = TO.signature(path, depth)
+    want_grad = TO.signature_vjp(path, torch.zeros_like(full).index_add_(1, cols, G), depth)
+    for fws, bws in (asked, (forward, backward)):
+        sig, grad = torch.full((B, S), float("nan"), dtype=dtype, device="cuda"), torch.full_like(x, float("nan"))
+        assert lib.pathsig_sig_forward(p(x), p(sig), *tail, p(ws) if fws else None, fws, stream) == 0, lib.pathsig_last_error()
+        assert lib.pathsig_sig_backward(p(x), p(sig), p(g), p(grad), *tail, p(ws), bws, stream) == 0, lib.pathsig_last_error()
+        torch.cuda.synchronize()
+        assert rel_err(sig, full[:, cols]) < TOL[dtype] and rel_err(grad, want_grad) < TOL[dtype]
+    if forward:
+        assert lib.pathsig_sig_forward(p(x), p(sig), *tail, p(ws), forward - 256, stream) == -3
+    assert lib.pathsig_sig_backward(p(x), p(sig), p(g), p(grad), *tail, p(ws), backward - 256, stream) == -3
