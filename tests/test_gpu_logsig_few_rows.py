@@ -55,3 +55,19 @@ def test_modules(dtype, rows, d, depth, lyndon):
     want = TO.signature_vjp(path, TO.logsig_vjp(sig, dense, depth, d, d ** depth, None), depth)
     (grad,) = torch.autograd.grad(out, x, G.to(dtype).cuda())
     assert rel_err(grad, want) < 2 * TOL[dtype]
+
+
+# The outputs of a product over the top level in parts: two, three, five (fewer than one output to some of a wide alphabet's
+# parts), sixteen, and rows that are just too many for any
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("rows,d,depth", [(51, 6, 6), (52, 6, 6), (42, 9, 5), (13, 16, 4), (1, 64, 3), (3, 49, 3)])
+def test_parts_of_the_top_products(dtype, rows, d, depth):
+    import pathsig_amd  # noqa: F401
+    sig = TO.signature(brownian_path(rows, 8, d, seed=1300 + d) * 1.5, depth)
+    G = randn(tuple(sig.shape), seed=130)
+    x = sig.to(dtype).cuda().requires_grad_(True)
+    none = torch.empty(0, dtype=torch.int64, device="cuda")
+    got = torch.ops.pathsig.sig_to_logsig(x, depth, d, False, none, [0] + [d ** k for k in range(1, depth + 1)])[0]
+    (grad,) = torch.autograd.grad(got, x, G.to(dtype).cuda())
+    some = torch.tensor([0, rows - 1]).unique()
+    assert rel_err(grad[some], TO.logsig_vjp(sig[some], G[some], depth, d, d ** depth, None)) < TOL[dtype]
