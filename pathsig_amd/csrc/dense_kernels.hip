@@ -3200,13 +3200,21 @@ static double sweeps_us(const VariantInfo &v, size_t elem, int64_t rows, int64_t
     return (double)(L - 1) / chunks * step_us_of(v, elem) * std::max(1.0, 0.4 + 0.6 * to_simd);
 }
 
+// A forward in one piece, an increment, us, counted low.
+static double forward_step_us(const VariantInfo &v, size_t elem) {
+    return (elem == 8 ? 0.33 : 0.22) * (v.sub_size < 116 ? 1.0 : elem == 8 ? 2.0 : 1.7);
+}
+
 // Far chunks (DenseChoice::far) of a call without windows, 0 where one piece is as good: about two waves to a SIMD, chunks of
 // sixteen increments at least, half a gigabyte of chunk signatures at most.  fp32 rows of more than 4096 increments stay in
 // one piece for the reason given at kLongRowSteps.  A step, us, in one piece / in far chunks: fp32 (16, 4), 2 paths of 4000
 // points, 4744 / 363, 1 of 300 365 / 85; (9, 5), 4 of 1000, 1361 / 243; (6, 6), 2 of 500, 449 / 134, 16 of 500 454 / 247 (64 of
 // 500 fill the GPU in one piece: 456); (5, 7), 3 of 2000, 3406 / 411; fp64 (4, 7), 13 of 2799, 4374 / 744, (16, 4), 5 of 847,
-// 2153 / 386; a forward alone, fp64 (16, 4), 1 of 410, 130 / 48.  The estimates are cautious: fp64 (4, 7), 20 of 200, stays in
-// one piece, where a forward takes 74 us and 92 in chunks.
+// 2153 / 386; a forward alone, fp64 (16, 4), 1 of 410, 130 / 48.
+// A forward alone must not lose by it: in one piece it takes 0.2 to 0.5 us an increment, whatever the shape (twice that from 116
+// values below a lane's prefix on; counted low), in chunks the products, whose estimate is high by a third and more.  (As a
+// quarter of both sweeps against the products it lost in 8 of 260 calls of random shapes: fp64 (56, 3), 7 paths of 109 points,
+// 58 / 114; (4, 8), 5 of 220, 91 / 118; fp32 (60, 3), 7 of 196, 65 / 77.)
 static int far_chunks(const VariantInfo &v, size_t elem, int64_t rows, int64_t L) {
     if (v.depth > 8 || (elem == 4 && L - 1 > kLongRowSteps)) return 0;
     const int64_t unit_waves = v.block / kWave;
@@ -3216,12 +3224,11 @@ static int far_chunks(const VariantInfo &v, size_t elem, int64_t rows, int64_t L
     if (forced >= 1 && forced <= kMostChunks) c = forced;
     c = std::min<int64_t>(c, (int64_t(1) << 29) / (rows * v.sig_size * (int64_t)elem));
     if (c < 2 || rows * c * v.unit_blocks >= (int64_t(1) << 30) || !chain_possible(rows, (int)c, v.d, v.depth)) return 0;
-    // (a forward alone is a quarter of the sweeps, and must not lose by it either)
-    const double saved = sweeps_us(v, elem, rows, L, 1) - sweeps_us(v, elem, rows, L, (int)c);
-    const double products = chain_us(elem, rows, (int)c, v.d, v.depth, 2) + chain_top_us(elem, rows, (int)c, v.d, v.depth);
-    if (forced < 1 && (0.25 * saved < products + 6.0 ||
-                       saved < products + chunk_adjoints_us(elem, rows, (int)c, v.d, v.depth) + 8.0))
-        return 0;
+    if (forced >= 1) return (int)c;
+    const double one_piece = sweeps_us(v, elem, rows, L, 1), saved = one_piece - sweeps_us(v, elem, rows, L, (int)c);
+    const double chain = chain_us(elem, rows, (int)c, v.d, v.depth, 2), top = chain_top_us(elem, rows, (int)c, v.d, v.depth);
+    if (saved < chain + top + chunk_adjoints_us(elem, rows, (int)c, v.d, v.depth) + 8.0) return 0;
+    if ((double)(L - 1) * forward_step_us(v, elem) * saved / one_piece < 0.6 * chain + top + 6.0) return 0;
     return (int)c;
 }
 
@@ -3247,10 +3254,13 @@ static EntryUs entry_us(const VariantInfo &v, size_t elem, int64_t rows, int64_t
                                                   chain_top_us(elem, rows, far, v.d, v.depth) +
                                                   chunk_adjoints_us(elem, rows, far, v.d, v.depth)};
 }
-// (a forward alone is a quarter of the sweeps, and must not lose by the choice either)
-static bool entry_pays(const EntryUs &short_prefix, const EntryUs &long_prefix) {
+// (A forward alone is a quarter of the sweeps, and must not lose by the choice either; in fp64 at depth 4 the long prefix takes a
+// seventh: (16, 4), 21 paths of 937 points, 298 us where the short one took 445, 27 of 2176, 687 and 804, (18, 4), 10 of 697, 254
+// and 301.)
+static bool entry_pays(const EntryUs &short_prefix, const EntryUs &long_prefix, size_t elem, int depth) {
+    const double share = elem == 8 && depth == 4 ? 0.14 : 0.25;
     return short_prefix.total() < 0.7 * long_prefix.total() &&
-           0.25 * short_prefix.sweeps + short_prefix.products + 4.0 < 0.25 * long_prefix.sweeps + long_prefix.products;
+           0.25 * short_prefix.sweeps + short_prefix.products + 4.0 < share * long_prefix.sweeps + long_prefix.products;
 }
 
 // Whether windows of depth 2 share waves (pairs_forward_kernel, pairs_backward_kernel).  Their lengths are not known here, and a
@@ -3294,7 +3304,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
             // dozens of waves swept in one piece
             if (later && rows * (v.block / kWave) * (cut ? max_chunks : 1) < (cut ? 1024 : 512) &&
                 (windowed || plain || !far_ok || (elem == 4 && L - 1 > kLongRowSteps) ||
-                 !entry_pays(entry_us(v, elem, rows, L), entry_us(kVariants[other], elem, rows, L))))
+                 !entry_pays(entry_us(v, elem, rows, L), entry_us(kVariants[other], elem, rows, L), elem, depth)))
                 continue;
             // the short prefixes of the wide alphabets hold 68 to 240 values per lane: fp64 up to 132 (d = 11) and
             // wherever the children are split

@@ -1039,9 +1039,9 @@ hipError_t launch_adjoint(const T *logsig, const T *cache, const T *grad_logsig,
             // letters: the shortest product has as many outputs as there are letters, and a block with one or two of them has
             // no terms for its lanes.  us, whole / 2 / 4 / 8 / 16 parts, 1 row: fp32 (6, 6) 75 / 59 / 63 / 63 / 63, (9, 5) 75 / 56 /
             // 50 / 58 / 58, (16, 4) 50 / 40 / 36 / 42 / 50, (64, 3) 118 / 69 / 44 / 32 / 27; 13 rows: (16, 4) 54 / 47 / 40 / 50 / 73;
-            // fp64 (9, 5), 1 row, 87 / 64 / 54 / 61 / 62.  Layouts of fewer words gain less and lose sooner: fp32 (8, 5), 32 768
+            // fp64 (9, 5), 1 row, 87 / 64 / 54 / 61 / 62, (7, 6), 1 row, 132 / 97 / 83 / 84 / 84 (3 parts 85).  Layouts of fewer words gain less and lose sooner: fp32 (8, 5), 32 768
             // words, 2 parts 45 / 41 with 1 row, 49 / 53 with 50; (7, 5), 16 807 words, 35 / 33 and 36 / 42.
-            const int64_t parts = std::min<int64_t>({16, std::max<int64_t>(2, d / 3), 1024 / (rows * (depth - 1) * 2)});
+            const int64_t parts = std::min<int64_t>({16, std::max<int64_t>(2, (d + 2) / 3), 1024 / (rows * (depth - 1) * 2)});
             if (parts >= 2 && lp.top_dense >= 45000)
                 hipLaunchKernelGGL((logsig_gather_top_kernel<T, true>),
                                    dim3((unsigned)rows, (unsigned)((depth - 1) * parts), 2), dim3(kLogBlock), 0, stream, logsig,

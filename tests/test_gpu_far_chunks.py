@@ -19,6 +19,33 @@ def ps():
     return pathsig_amd
 
 
+def _columns(proj, d, depth):
+    """Places of a projection's words in the dense layout."""
+    if proj is None:
+        return torch.arange(sum(d ** k for k in range(1, depth + 1)))
+    return torch.tensor(TO.projection_columns(d, depth, proj.level_sizes, proj._codes))
+
+
+def _kept_chunks(dtype, B, L, d, depth, level_sizes, logarithm):
+    """Time chunks whose products a forward of the call hands to its backward (0: none)."""
+    from pathsig_amd import _load
+    lib, code, elem = _load.lib(), 0 if dtype == torch.float32 else 1, 4 if dtype == torch.float32 else 8
+    if logarithm:  # (levels below the top are full in what the call computes; the size counts the chunks, four elements each)
+        sizes = None if level_sizes is None else [0, *[d ** k for k in range(1, depth)], level_sizes[depth]]
+        host = None if sizes is None else (ctypes.c_int64 * len(sizes))(*sizes)
+        out = [ctypes.c_size_t() for _ in range(3)]
+        lib.pathsig_logsignature_sizes.argtypes = [ctypes.c_int] + [ctypes.c_int64] * 3 + [
+            ctypes.c_int, ctypes.c_void_p, ctypes.c_int64] + [ctypes.POINTER(ctypes.c_size_t)] * 3
+        assert lib.pathsig_logsignature_sizes(code, B, L, d, depth, host, 0, *out) == 0
+        tag = out[0].value // elem % 4096
+        return tag // 4 if tag % 4 == 1 else 0
+    host = None if level_sizes is None else (ctypes.c_int64 * len(level_sizes))(*level_sizes)
+    low = B * sum(d ** k for k in range(1, depth)) * elem
+    kept = lib.pathsig_sig_chunks_bytes(code, B, L, d, depth, host, 0)
+    dense = low + B * d ** depth * elem  # (a projection that is swept in one piece keeps its dense rows)
+    return 0 if kept == dense else kept // low // 2
+
+
 # (16, 4): split children in one block; (12, 5): split, beyond what the products are compiled for (one piece); (9, 5), (5, 7):
 # several blocks; (13, 4): several blocks in fp64; (4, 7): fp64 rows too long for the scan kernel.  Six chunks are the least
 # that are multiplied; fewer increments than chunks leave some empty.
@@ -52,7 +79,7 @@ def test_forced_chunks(ps, set_option, dtype, d, depth, chunks, L):
 @pytest.mark.parametrize("d,depth,L,name", [(14, 4, 600, "lyndon"), (9, 5, 400, "lyndon"), (9, 5, 500, "words"),
                                             (16, 4, 300, None), (14, 4, 500, None), (4, 7, 700, None)])
 def test_own_choice(ps, dtype, d, depth, L, name):
-    """The library's choice for one path, with projections that are swept in the dense layout."""
+    """The library's choice for one path is far chunks, with projections that are swept in the dense layout too."""
     path = brownian_path(1, L, d, seed=930 + d)
     x = path.to(dtype).cuda().requires_grad_(True)
     proj = None
@@ -64,21 +91,16 @@ def test_own_choice(ps, dtype, d, depth, L, name):
     module = ps.LogSignature if name == "lyndon" else ps.Signature
     out = module(depth=depth, projection=proj)(x)
     full = (TO.logsignature if name == "lyndon" else TO.signature)(path, depth)
-    offs = TO.dense_level_offsets(d, depth)
-    cols = torch.arange(full.shape[1])
-    if proj is not None:
-        listed, cols = iter(proj._codes), []
-        for k in range(1, depth + 1):
-            size = proj.level_sizes[k]
-            cols += [offs[k] + (j if size == d ** k else next(listed)) for j in range(size)]
-        cols = torch.tensor(cols)
+    cols = _columns(proj, d, depth)
+    assert _kept_chunks(dtype, 1, L, d, depth, None if proj is None else proj.level_sizes, name == "lyndon") > 1
     assert rel_err(out, full[:, cols]) < TOL[dtype]
-    if name != "lyndon":
-        G = randn(tuple(out.shape), seed=93)
-        dense = torch.zeros_like(full)
-        dense.index_add_(1, cols, G)
-        (grad,) = torch.autograd.grad(out, x, G.to(dtype).cuda())
-        assert rel_err(grad, TO.signature_vjp(path, dense, depth)) < TOL[dtype]
+    G = randn(tuple(out.shape), seed=93)
+    dense = torch.zeros_like(full)
+    dense.index_add_(1, cols, G)
+    (grad,) = torch.autograd.grad(out, x, G.to(dtype).cuda())
+    if name == "lyndon":
+        dense = TO.logsig_vjp(TO.signature(path, depth), dense, depth, d, d ** depth, None)
+    assert rel_err(grad, TO.signature_vjp(path, dense, depth)) < TOL[dtype]
 
 
 def test_infinite_gradient_after_the_last_chunk(ps, set_option):
@@ -137,3 +159,27 @@ def test_scratch_that_holds_one_piece_only(ps, dtype, B, L, d, depth, listed):
     if forward:
         assert lib.pathsig_sig_forward(p(x), p(sig), *tail, p(ws), forward - 256, stream) == -3
     assert lib.pathsig_sig_backward(p(x), p(sig), p(g), p(grad), *tail, p(ws), backward - 256, stream) == -3
+
+
+# In chunks by force and by the library's choice; the last lengths that an fp32 call of a depth has its chunks for, and the first
+# that it has not (LogPlan)
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("d,depth,L,chunks,lyndon", [(9, 5, 90, 7, False), (9, 5, 90, 7, True), (16, 4, 90, 7, False), (16, 4, 90, 7, True),
+                                                     (9, 5, 300, 0, False), (16, 4, 300, 0, True), (9, 5, 1025, 0, True),
+                                                     (9, 5, 1026, 0, True), (16, 4, 2049, 0, False), (16, 4, 2050, 0, False)])
+def test_gradient_of_the_logarithm(ps, set_option, dtype, d, depth, L, chunks, lyndon):
+    set_option("chunks", chunks)
+    path = brownian_path(1, L, d, seed=970 + d + L).to(dtype).double()
+    proj = ps.projections.lyndon(depth=depth, path_dim=d) if lyndon else None
+    in_chunks = _kept_chunks(dtype, 1, L, d, depth, proj.level_sizes if lyndon else None, True)
+    one_piece = dtype == torch.float32 and L - 1 > 2048 >> (depth - 4)
+    assert in_chunks == chunks if chunks else (in_chunks > 1) != one_piece
+    x = path.to(dtype).cuda().requires_grad_(True)
+    out = ps.LogSignature(depth=depth, projection=proj)(x)
+    sig, cols = TO.signature(path, depth), _columns(proj, d, depth)
+    assert rel_err(out, TO.sig_to_logsig(sig, depth, d, d ** depth, None)[0][:, cols]) < TOL[dtype]
+    G = randn(tuple(out.shape), seed=97)
+    dense = torch.zeros_like(sig).index_add_(1, cols, G)
+    want = TO.signature_vjp(path, TO.logsig_vjp(sig, dense, depth, d, d ** depth, None), depth)
+    (grad,) = torch.autograd.grad(out, x, G.to(dtype).cuda())
+    assert rel_err(grad, want) < TOL[dtype]
