@@ -134,23 +134,29 @@ constexpr int64_t kChunkSteps = 16;  // increments of a chunk, at least
 }  // namespace
 
 // Chunks of sixteen increments and more, at most 64 and no more than fill the GPU, if the forward gains by them (a backward
-// gains more).  An increment of a word takes a wave 0.3 us, of which it keeps its SIMD busy for instructions only; the
-// launches take 8 us and the products 0.15 (depth 1) to 0.5 us (depth 8) a chunk.  fp32 rows of more than 4096 increments keep to one piece, as those of the dense kernels keep
-// to 64 chunks.
+// gains more).  In one piece an increment takes 0.010 us and 0.019 for every letter of the longest words, or what keeps the
+// SIMDs busy; in chunks that latency is divided, but suffixes and the staging of all letters for blocks of one wave keep them
+// busy for longer, the launches take 4.5 us more, the products 0.15 (depth 1) to 0.5 us (depth 8) a chunk, and the table is written and
+// read (1 us a megabyte, of short paths more than they sweep).  (With 0.3 us an increment, staging and table left out, a
+// forward lost in 23 of 240 random calls, now in one, by 3 us: fp32, 3 paths of 2436 points, 58 057 words of (38, 4), 174 / 515 us; fp64, 2 of 105, 31 029 words of
+// (31, 4), 11 / 27.)  fp32 rows of more than 4096 increments keep to one piece, as those of the dense kernels keep to 64 chunks.
 WordChunks word_chunks(size_t elem, int64_t B, int64_t L, int64_t d, int depth, const int64_t *level_sizes, bool windowed) {
     WordChunks wc{};
     if (windowed || !level_sizes || depth > 8 || B < 1 || L - 1 < 2 * kChunkSteps || (elem == 4 && L - 1 > 4096)) return wc;
+    int longest = 0;
     int64_t waves = 0, longer = 0;
-    double work = 0, factor_work = 0;  // us of a SIMD per increment, of one path
+    double work = 0, factor_work = 0, staged_work = 0;  // us of a SIMD per increment, of one path
     for (int n = depth; n >= 1; --n) {
         const int64_t size = level_sizes[n], of_level = (size + kWave - 1) / kWave;
         if (size > (int64_t(1) << 24)) return wc;
         // (1 ns to an instruction, twice that in fp64)
         const double us = 1e-3 * (10.0 + 0.85 * n * (n + 1) + n) * ((double)elem / 4);
+        if (longest == 0 && size > 0) longest = n;
         longer += size;
         waves += of_level;
         work += us * (double)of_level;
         factor_work += us * (double)((longer + kWave - 1) / kWave);
+        staged_work += (0.8 * us + 0.3e-3 * (double)d * ((double)elem / 4)) * (double)((longer + kWave - 1) / kWave);
         wc.table_off[n] = wc.table_size;
         wc.edge_off[n] = wc.edge_size;
         wc.table_size += size * n * (n + 1) / 2;
@@ -173,10 +179,11 @@ WordChunks word_chunks(size_t elem, int64_t B, int64_t L, int64_t d, int depth, 
     if (c * B * wc.table_size * (int64_t)elem > (int64_t(1) << 28)) c = (int64_t(1) << 28) / (B * wc.table_size * (int64_t)elem);
     if (c * ((B + 15) / 16) > 65535) c = 65535 / ((B + 15) / 16);
     if (c < 2) return WordChunks{};
-    const double steps = (double)(L - 1), simds = 1.0 / 1024;
-    const double one_piece = steps * std::max(0.3, (double)B * work * simds);
-    const double in_chunks = steps * std::max(0.3 / (double)c, (double)B * factor_work * simds) + 8.0 + product_us * (double)c;
-    if (in_chunks > 0.7 * one_piece) return WordChunks{};
+    const double steps = (double)(L - 1), simds = 1.0 / 1024, latency = 0.010 + 0.019 * longest;
+    const double one_piece = 3.0 + steps * std::max(latency, (double)B * work * simds);
+    const double in_chunks = 7.5 + product_us * (double)c + steps * std::max(latency / (double)c, (double)B * staged_work * simds) +
+                             1e-6 * (double)c * (double)B * (double)wc.table_size * (double)elem;
+    if (in_chunks > one_piece) return WordChunks{};
     wc.chunks = (int)c;
     return wc;
 }

@@ -1,5 +1,7 @@
 """Scratch of the launches for long chains of time chunks: asked for where they are taken, and never at the price of a call
 that the allocation-free backward can serve without them."""
+import ctypes
+
 import pytest
 import torch
 
@@ -64,3 +66,14 @@ def test_few_windows_of_depth_two_are_cut_into_chunks(lib, dtype, d, rows, L):
     assert lib.pathsig_sig_forward_workspace(dtype, 8, L, d, 2, None, rows // 8) > 0
     assert lib.pathsig_sig_chunks_bytes(dtype, 8, L, d, 2, None, rows // 8) > 0
     assert lib.pathsig_sig_forward_workspace(dtype, 8, L, d, 2, None, 1024) == 0
+
+
+# Words whose table takes longer to write and read than a short path to sweep, and words that keep the SIMDs busy as it is, are
+# swept in one piece; few words of long paths in chunks.
+@pytest.mark.parametrize("dtype,B,L,d,depth,top,chunks", [
+    (1, 2, 105, 31, 4, 31000, False), (0, 3, 2436, 38, 4, 58000, False), (1, 68, 154, 37, 3, 1400, False), (0, 19, 75, 15, 1, 15, False),
+    (0, 2, 2616, 35, 5, 300, True), (1, 40, 2976, 9, 5, 60, True), (0, 1, 928, 23, 8, 90, True)])
+def test_words_are_cut_into_chunks_where_a_forward_gains(lib, dtype, B, L, d, depth, top, chunks):
+    sizes = (ctypes.c_int64 * (depth + 1))(*[0] * depth, top)
+    assert (lib.pathsig_sig_forward_scratch(dtype, B, L, d, depth, sizes, 0) > 0) == chunks
+    assert lib.pathsig_sig_forward_workspace(dtype, B, L, d, depth, sizes, 0) == 0
