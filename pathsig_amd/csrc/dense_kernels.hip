@@ -1850,13 +1850,13 @@ __global__ void __launch_bounds__(kPairsThreads)
             pairs_fence();
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                T v = fixed, w = T(0);
+                T v = T(0), w = T(0);  // (the largest term last: fewer roundings of its size)
 #pragma unroll
                 for (int a = 0; a < D; ++a) {
                     v = fmad<T>(mine[u][0][a], before[a], v);
                     w = fmad<T>(mine[u][1][a], after[a], w);
                 }
-                if (pl.letter < D) tile[(i + u) * D + pl.letter] = v + w;
+                if (pl.letter < D) tile[(i + u) * D + pl.letter] = fixed + (v + w);
             }
             pairs_fence();
 #pragma unroll
