@@ -663,8 +663,9 @@ LogPlan log_plan(int dtype, int64_t B, int64_t L, int64_t d, int depth, const in
     for (int k = 1; k < depth; ++k)
         if (plan.code_off[k] >= 0) return lp;
     // The gradient of a logarithm is a difference of larger terms: in fp32 a sweep in one piece is off by 1e-5 and more of its
-    // norm from some 1000 increments on ((6, 6), 2 paths of 1000 points, 1.3e-5, in far chunks 0.9e-5; of 4000 2.5e-5 and
-    // 1.9e-5), so that two ways of cutting long rows would differ by 2e-5 and more.  They stay as they are.
+    // norm from some 1000 increments on, and two ways of cutting differ by as much.  Longer rows stay in one piece so that their
+    // results stay what they were, not because precision asked for it: far chunks are the nearer to 64 bits ((6, 6), 2 paths of
+    // 1000 points, 1.3e-5 in one piece and 0.9e-5 in far chunks; of 4000, 2.5e-5 and 1.9e-5).
     const bool far_ok = elem == 8 || L - 1 <= (int64_t(2048) >> (depth > 4 ? depth - 4 : 0));
     lp.dc = dense_choice(elem, d, depth, all_dense, level_sizes, B, L, windows, W > 0, far_ok);
     if (!lp.dc.usable) return lp;

@@ -2989,7 +2989,7 @@ hipError_t run_forward(const T *path, T *sig, const SigShape &shape, const Dense
                                          stream);
             if (e != hipSuccess) return e;
         } else {
-            return hipErrorNotSupported;  // such shapes are never cut into time chunks (dense_choice)
+            return hipErrorNotSupported;  // (such shapes are cut into far chunks only, above)
         }
     }
     if (groups == 1) return hipSuccess;
@@ -3269,12 +3269,16 @@ static bool entry_pays(const EntryUs &short_prefix, const EntryUs &long_prefix, 
 // where the new way is the faster one for whole paths, expanding windows up to 4097 points, windows at their own places and
 // windows of 9 points alike.  us, swept (in chunks, where rows are few) / shared:
 //   forward, whole paths of 1025 points, fp32, 2 letters: 512 rows 18.7 / 83, 4096 64 / 84, 8192 102 / 85; 15 letters: 2048 149 /
-//   168, 4096 266 / 169; fp64, 15 letters: 512 70 / 187, 4096 464 / 191;
+//   168, 4096 266 / 169; fp64, 15 letters: 512 70 / 187, 4096 464 / 191; the sweeps take longer over an odd number of letters:
+//   fp64, 2048 rows, 15 letters 246 / 189, 16 letters 172 / 201, fp32, 2672 rows, 19 letters 257 / 170, 20 letters 172 / 208;
 //   backward, the same: fp32, 2 letters 42 / 237, 346 / 238, 608 / 239 (expanding, 4096 rows 841 / 914); 8 letters: 512 128 / 288,
 //   2048 488 / 292, 4096 745 / 293 (expanding, 2048 rows 1081 / 1113); 15 letters: 512 140 / 330, 2048 549 / 332; fp64, 15
 //   letters: 512 249 / 392, 2048 962 / 398.
 // (Over twelve letters, fp32, 4096 expanding windows take 538 / 559 forward, whole paths of 129 points 22.3 / 21.4.)
-static bool pairs_forward_pays(int64_t d, int64_t rows) { return rows >= 8192 || (rows >= 4096 && pairs_lanes((int)d) >= 16); }
+static bool pairs_forward_pays(size_t elem, int64_t d, int64_t rows) {
+    const bool wide_and_odd = d % 2 == 1 && pairs_lanes((int)d) * (int64_t)elem >= 128;
+    return rows >= 8192 || (rows >= 4096 && pairs_lanes((int)d) >= 16) || (rows >= 2048 && wide_and_odd);
+}
 static bool pairs_backward_pays(size_t elem, int64_t d, int64_t rows) {
     return rows >= 8192 || (rows >= 2048 && rows * pairs_lanes((int)d) * (int64_t)elem >= 131072);
 }
@@ -3375,8 +3379,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         // size 0.8: gradient off by 1.5e-5 in one piece, 1e-6 in two or more); four chunks at least
         if (elem == 4 && depth >= 9 && chunks < 4) chunks = (int)std::max<int64_t>(1, std::min<int64_t>(4, L - 1));
         if (const int64_t forced = options().chunks; forced >= 1 && forced <= 1024) chunks = (int)forced;
-        // not chunked: units of several blocks (a row is dozens of waves already), rows too long for the scan
-        // kernel's LDS
+        // units of several blocks, split children, rows too long for the scan kernel's LDS: far chunks or one piece
         if (!chunks_ok) chunks = far > 0 ? far : 1;
         if (rows * (chunks + 1) >= (int64_t(1) << 31)) return dc;
         dc.usable = true;
@@ -3384,7 +3387,7 @@ static DenseChoice make_dense_choice(size_t elem, int64_t d, int depth, bool all
         dc.fwd_chunks = chunks;
         dc.bwd_chunks = (dc.embed && !dc.resweep && chunks < 2) ? 2 : chunks;
         if (windowed && depth == 2 && d <= 32) {
-            dc.pairs_forward = pairs_forward_pays(d, rows);
+            dc.pairs_forward = pairs_forward_pays(elem, d, rows);
             dc.pairs_backward = pairs_backward_pays(elem, d, rows);
         }
         dc.forward_workspace = dc.dense_bytes + (dc.bounded ? kBoundsBytes : 0);

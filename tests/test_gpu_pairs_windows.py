@@ -125,7 +125,7 @@ def test_windows_with_equal_starts(dtype, d, B):
 # Both sides of the lines between sweeps (in chunks, where rows are few) and shared waves, 2048, 4096 and 8192 windows, on paths
 # longer than a chunk takes
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
-@pytest.mark.parametrize("d", [2, 4, 8, 15, 32])
+@pytest.mark.parametrize("d", [2, 4, 8, 15, 17, 32])
 @pytest.mark.parametrize("B", [64, 255, 256, 511, 512, 1023, 1024])
 def test_rows_on_both_sides_of_the_lines(dtype, d, B):
     import pathsig_amd as ps
