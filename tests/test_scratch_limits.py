@@ -77,3 +77,12 @@ def test_words_are_cut_into_chunks_where_a_forward_gains(lib, dtype, B, L, d, de
     sizes = (ctypes.c_int64 * (depth + 1))(*[0] * depth, top)
     assert (lib.pathsig_sig_forward_scratch(dtype, B, L, d, depth, sizes, 0) > 0) == chunks
     assert lib.pathsig_sig_forward_workspace(dtype, B, L, d, depth, sizes, 0) == 0
+
+
+# Far chunks, and short prefixes for their chunks' sake, only where a forward alone gains too.
+@pytest.mark.parametrize("dtype,B,L,d,depth,chunks", [
+    (1, 7, 109, 56, 3, False), (1, 5, 220, 4, 8, False), (0, 7, 196, 60, 3, False), (1, 21, 937, 16, 4, False), (1, 10, 697, 18, 4, False),
+    (0, 2, 4000, 16, 4, True), (1, 13, 2799, 4, 7, True), (1, 8, 1091, 9, 5, True), (1, 35, 500, 32, 3, True), (0, 4, 1000, 9, 5, True)])
+def test_far_chunks_are_taken_where_a_forward_gains(lib, dtype, B, L, d, depth, chunks):
+    assert (lib.pathsig_sig_forward_workspace(dtype, B, L, d, depth, None, 0) > 0) == chunks
+    assert (lib.pathsig_sig_chunks_bytes(dtype, B, L, d, depth, None, 0) > 0) == chunks
